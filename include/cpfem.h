@@ -148,6 +148,17 @@ int cpfem_update_state(cpfem_ctx* ctx, void* stream, const double* dofs, const C
 int cpfem_solve(cpfem_ctx* ctx, void* stream, const double* mat, const double* b, double* x, double tol,
                 double atol, int32_t maxiter, int32_t precond, int32_t precision, CpfemSolveInfo* info);
 
+/* cpfem_solve with a geometric multigrid V-cycle in the place of the Jacobi scaling, where that
+   applies: systems of at least 1500 rows on meshes whose nodes are numbered as a full box (see
+   cpfem_box_numbering; every node, on the faces too, coupled to all its neighbours).  Same
+   recurrence, stopping rule, arguments and errors; info->iterations counts its (far fewer)
+   iterations.  precision CPFEM_MIXED: FP32 values inside the preconditioner, FP64 operator.  On
+   other systems, and from x0 anew where the multigrid solve breaks down, does not meet the
+   stopping rule within 60 iterations or leaves |A x - b| >= 0.1, the call is cpfem_solve with
+   precond = 1.  Dirichlet dofs are those of cpfem_set_dirichlet. */
+int cpfem_solve_mg(cpfem_ctx* ctx, void* stream, const double* mat, const double* b, double* x, double tol, double atol,
+                   int32_t maxiter, int32_t precision, CpfemSolveInfo* info);
+
 /* cpfem_solve in FP64 without any device allocation.  No counterpart in the reference: it is
    for callers that cannot allocate device memory (code under HIP graph capture, tight serving
    loops, harnesses that forbid hipMalloc).  The Krylov workspace (scalars, partial sums,
@@ -273,8 +284,10 @@ int cpfem_transpose(cpfem_ctx* ctx, void* stream, const double* mat, double* mat
    resets the counters.  Classes (index): 0 point update (local Newton, P), 1 element
    stiffness/residual, 2 matrix gather, 3 residual gather, 4 Krylov SpMV kernels, 5 Krylov
    vector kernels, 6 point stress/history, 7 copy, 8 residual replacement of the mixed form,
-   9 parked points of the point kernel, 10 consistent tangent of the assembly.  No counterpart
-   in the reference. */
+   9 parked points of the point kernel, 10 consistent tangent of the assembly, 11 passes over the
+   finest matrix inside the multigrid preconditioner, 12 the rest of the preconditioner, 13 its
+   setup (11 and 12 are sampled too; in a multigrid solve 4 and 5 are the BiCGSTAB products and
+   vector kernels).  No counterpart in the reference. */
 int cpfem_profile(cpfem_ctx* ctx, int32_t enable, int32_t sample);
 int cpfem_profile_read(cpfem_ctx* ctx, int32_t n, double* ms, int64_t* launches, int64_t* timed);
 

@@ -79,6 +79,8 @@ _SIGS = {
                                    ctypes.c_int32, ctypes.c_int32, ctypes.POINTER(CpfemSolveInfo)]),
     "cpfem_solve_noalloc": (ctypes.c_int, [vp, vp, vp, vp, vp, ctypes.c_double, ctypes.c_double, ctypes.c_int32,
                                            ctypes.c_int32, ctypes.POINTER(CpfemSolveInfo)]),
+    "cpfem_solve_mg": (ctypes.c_int, [vp, vp, vp, vp, vp, ctypes.c_double, ctypes.c_double, ctypes.c_int32,
+                                      ctypes.c_int32, ctypes.POINTER(CpfemSolveInfo)]),
     "cpfem_spmv": (ctypes.c_int, [vp, vp, vp, vp, vp]),
     "cpfem_solve_direct": (ctypes.c_int, [vp, vp, vp, vp, vp, ctypes.c_int32, ctypes.POINTER(CpfemSolveInfo)]),
     "cpfem_band_order": (ctypes.c_int, [ctypes.c_int64, vp, vp, vp, vp]),
@@ -102,7 +104,7 @@ _SIGS = {
 }
 
 PROF_CLASSES = ("element_qp", "element_K", "gather_matrix", "gather_residual", "krylov_spmv", "krylov_vector",
-                "point_local", "copy", "krylov_replace", "element_qp_park", "point_tangent")
+                "point_local", "copy", "krylov_replace", "element_qp_park", "point_tangent", "mg_fine", "mg_coarse", "mg_setup")
 
 EXPORTED = tuple(_SIGS)
 _lib = None

@@ -5,15 +5,17 @@ Follows crystal_plasticity_OR_design/solver.py:310-437 (and linear_incremental_s
 Dirichlet row elimination and the Krylov solve all run in libcpfem_hip.so; this module only
 sequences the calls and reads back norms.
 
-solver_options keys (as in the reference): 'jax_solver': {'precond': bool}, 'umfpack_solver',
+solver_options keys (as in the reference): 'jax_solver': {'precond': bool or 'jacobi'}, 'umfpack_solver',
 'petsc_solver', 'custom_solver', 'initial_guess', 'tol' (1e-6), 'rel_tol' (1e-8),
 'line_search_flag' (False).  Added: 'precision': 'fp64' (default) | 'mixed' (FP32 Krylov matrix
 with FP64 refinement), 'krylov_tol'/'krylov_atol' (1e-10), 'krylov_maxiter' (10000),
 'max_newton' (200; the reference loop has no cap and spins forever on a stagnating residual).
 'umfpack_solver' is served by the device banded direct solver (cpfem_solve_direct: unpivoted
 band LU under a bandwidth-reducing node order plus FP64 iterative refinement, 'refine' steps,
-default 2); 'petsc_solver' (an iterative Krylov solve in the reference, bcgsl + ilu by default)
-by the device Krylov solver at the same 1e-10 tolerance.
+default 2); 'jax_solver' with precond True (the default) runs the reference's BiCGSTAB to its
+stopping rule with a multigrid cycle in the place of the Jacobi scaling on box-numbered meshes
+(multigrid_solve; 'jacobi', or a 'krylov_maxiter', keeps the scaling); 'petsc_solver' (an iterative Krylov solve in the reference, bcgsl + ilu by default)
+by the same solve at the same 1e-10 tolerance.
 """
 import ctypes
 import logging
@@ -55,17 +57,35 @@ def _precision(solver_options):
     return N.MIXED if p == "mixed" else N.FP64
 
 
+def _krylov_args(mat, b, x, solver_options):
+    return (ptr(mat), ptr(b), ptr(x), float(solver_options.get("krylov_tol", 1e-10)),
+            float(solver_options.get("krylov_atol", 1e-10)), int(solver_options.get("krylov_maxiter", 10000)))
+
+
 def krylov_solve(problem, mat, b, x0, solver_options=None, precond=True):
     """jax_solve (solver.py:19-48) on the device: Jacobi-BiCGSTAB, tol = atol = 1e-10,
     maxiter 10000, then the |Ax - b| < 0.1 assertion."""
     solver_options = solver_options or {}
     x = x0.clone()
     info = N.CpfemSolveInfo()
-    rc = problem.ctx._lib.cpfem_solve(problem.ctx.h, stream_handle(), ptr(mat), ptr(b), ptr(x),
-                                      float(solver_options.get("krylov_tol", 1e-10)),
-                                      float(solver_options.get("krylov_atol", 1e-10)),
-                                      int(solver_options.get("krylov_maxiter", 10000)), 1 if precond else 0,
-                                      _precision(solver_options), ctypes.byref(info))
+    rc = problem.ctx._lib.cpfem_solve(problem.ctx.h, stream_handle(), *_krylov_args(mat, b, x, solver_options),
+                                      1 if precond else 0, _precision(solver_options), ctypes.byref(info))
+    return _krylov_result(problem, x, rc, info)
+
+
+def multigrid_solve(problem, mat, b, x0, solver_options=None):
+    """krylov_solve with the multigrid preconditioner where the mesh allows it (cpfem_solve_mg):
+    the same system to the same stopping rule in about ten iterations; elsewhere, and where it
+    does not converge, the Jacobi-preconditioned solve."""
+    solver_options = solver_options or {}
+    x = x0.clone()
+    info = N.CpfemSolveInfo()
+    rc = problem.ctx._lib.cpfem_solve_mg(problem.ctx.h, stream_handle(), *_krylov_args(mat, b, x, solver_options),
+                                         _precision(solver_options), ctypes.byref(info))
+    return _krylov_result(problem, x, rc, info)
+
+
+def _krylov_result(problem, x, rc, info):
     stats = dict(iterations=info.iterations, outer=info.outer, residual=info.residual, b_norm=info.b_norm)
     problem.solver_info.append(stats)
     if rc == N.EKRYLOV:
@@ -96,10 +116,15 @@ def linear_solver(problem, mat, b, x0, solver_options):
         solver_options["jax_solver"] = {}
     if "jax_solver" in solver_options:
         precond = solver_options["jax_solver"].get("precond", True)
+        # a caller who bounds the iterations, or names the preconditioner, gets the plain iteration
+        if precond is True and "krylov_maxiter" not in solver_options:
+            return multigrid_solve(problem, mat, b, x0, solver_options)
         return krylov_solve(problem, mat, b, x0, solver_options, precond)
     if "umfpack_solver" in solver_options:
         return direct_solve(problem, mat, b, solver_options)
     if "petsc_solver" in solver_options:
+        if "krylov_maxiter" not in solver_options:
+            return multigrid_solve(problem, mat, b, x0, solver_options)
         return krylov_solve(problem, mat, b, x0, solver_options, True)
     if "custom_solver" in solver_options:
         return solver_options["custom_solver"](BlockEllMatrix(problem.ctx, mat), b, x0, solver_options)

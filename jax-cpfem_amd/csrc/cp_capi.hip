@@ -30,7 +30,7 @@ static hipEvent_t prof_event(Prof* p) {
 // launches per load step) are sampled; every launch of the point and assembly classes (a few
 // hundred of milliseconds-long launches, several kernels sharing a class) is timed.
 static int prof_every(const Prof* p, int cls) {
-  return (cls == PC_SPMV || cls == PC_KVEC || cls == PC_KREPLACE) ? p->sample : 1;
+  return (cls == PC_SPMV || cls == PC_KVEC || cls == PC_KREPLACE || cls == PC_MG_FINE || cls == PC_MG_COARSE) ? p->sample : 1;
 }
 
 int prof_begin(Prof* p, int cls, hipStream_t st) {
@@ -141,7 +141,7 @@ struct cpfem_ctx {
   // Krylov
   KrylovScalars* d_ksc = nullptr;
   double* d_kpartial = nullptr;  // [PS_COUNT][krylov blocks]
-  double* kv64[12] = {};  // r rhat (spare) q phat (spare) (spare) t invd (spare) rp rq; rp, rq hold 2 n
+  double* kv64[12] = {};  // r rhat p q phat s shat t invd x0 rp rq (p, s, shat, x0: multigrid solve); rp, rq hold 2 n
   float* d_mat32 = nullptr;
   double *d_r64 = nullptr, *d_tmp64 = nullptr;
   // pinned host staging
@@ -158,6 +158,10 @@ struct cpfem_ctx {
   int spmv_form = -1;  // BiCGSTAB SpMV form: -1 = picked by size (krylov_spmv_form), else forced
   int64_t box[3] = {0, 0, 0};  // box numbering (nx, ny, nz) of the pattern, or zeros
   int box_cols = 1;            // the flat SpMV computes the box numbering's columns (0: loads them)
+  Multigrid mg;                // multigrid preconditioner (buffers allocated on first use)
+  std::vector<void*> mg_mem;   // its device allocations
+  bool box_full = false;       // every row of the pattern holds exactly the node's neighbours in the box
+  uint64_t* h_flag = nullptr;  // progress word written by its BiCGSTAB (pinned)
   double* scratch = nullptr;  // device address of the fixed workspace array on this context's device
 
   int krylov_form() const { return spmv_form >= 0 ? spmv_form : krylov_spmv_form(n_dofs, n_slots); }
@@ -310,6 +314,25 @@ static void box_numbering(int64_t nn, const int32_t* col, const int32_t* nslot, 
   dims[2] = nz;
 }
 
+// Whether every node of a box-numbered pattern, on its faces too, has exactly its neighbours in
+// the box as columns, ascending (the slots the multigrid coarsening computes).
+static bool box_pattern_full(int64_t nn, const int32_t* col, const int32_t* nslot, const int64_t dims[3]) {
+  if (dims[0] == 0) return false;
+  const int64_t B = dims[0], A = dims[0] * dims[1];
+  int64_t i = 0;
+  for (int64_t z = 0; z < dims[2]; ++z)
+    for (int64_t y = 0; y < dims[1]; ++y)
+      for (int64_t x = 0; x < dims[0]; ++x, ++i) {
+        int s = 0;
+        for (int64_t dz = z > 0 ? -1 : 0; dz <= (z + 1 < dims[2] ? 1 : 0); ++dz)
+          for (int64_t dy = y > 0 ? -1 : 0; dy <= (y + 1 < dims[1] ? 1 : 0); ++dy)
+            for (int64_t dx = x > 0 ? -1 : 0; dx <= (x + 1 < dims[0] ? 1 : 0); ++dx, ++s)
+              if (s >= nslot[i] || (int64_t)col[(int64_t)s * nn + i] != i + dz * A + dy * B + dx) return false;
+        if (s != nslot[i]) return false;
+      }
+  return true;
+}
+
 static int build_maps(cpfem_ctx* c, const int32_t* cells) {
   const int64_t nn = c->n_nodes, nc = c->n_cells;
   // node -> (cell, local) list, ascending cell
@@ -347,6 +370,7 @@ static int build_maps(cpfem_ctx* c, const int32_t* cells) {
     c->h_dslot[i] = (int32_t)(std::lower_bound(v.begin(), v.end(), (int32_t)i) - v.begin());
   }
   box_numbering(nn, c->h_col.data(), c->h_nslot.data(), c->box);
+  c->box_full = box_pattern_full(nn, c->h_col.data(), c->h_nslot.data(), c->box);
   // transpose map: slot s of row j points at node i; tslot gives the slot of node j in row i
   std::vector<int32_t> tslot((size_t)maxs * nn, 0);
   for (int64_t j = 0; j < nn; ++j)
@@ -664,6 +688,119 @@ static int solve_impl(cpfem_ctx* c, hipStream_t st, const KBufs& kb, const doubl
   return CPFEM_OK;
 }
 
+// ------------------------------------------------------------------------- multigrid solve
+// Systems of at least MG_MIN_ROWS rows on full box patterns take the multigrid preconditioner.
+constexpr int64_t MG_MIN_ROWS = 1500;
+// Iterations it gets before the Jacobi-preconditioned solve takes over (it needs about 10).
+constexpr int MG_MAXITER = 60;
+
+static void mg_free(cpfem_ctx* c) {
+  for (void* p : c->mg_mem) (void)hipFree(p);
+  c->mg_mem.clear();
+}
+
+// Buffers of the multigrid levels; false (and no buffers) if it does not apply to this mesh or
+// the device is out of memory for it.
+static bool ensure_mg(cpfem_ctx* c) {
+  Multigrid& mg = c->mg;
+  if (mg.state) return mg.state > 0;
+  mg.state = -1;
+  if (!c->box_full || c->n_slots != 27 || c->n_dofs < MG_MIN_ROWS || !mg_plan(c->box, &mg)) return false;
+  const auto get = [&](size_t doubles) -> double* {
+    void* p = nullptr;
+    if (hipMalloc(&p, doubles * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      return nullptr;
+    }
+    c->mg_mem.push_back(p);
+    return static_cast<double*>(p);
+  };
+  bool ok = true;
+  for (int l = 0; l < mg.nl && ok; ++l) {
+    MgLevel& L = mg.lv[l];
+    const size_t n = (size_t)L.g.n;
+    double* v = get(5 * n);
+    ok = v != nullptr;
+    L.minv = v;
+    L.b = v + n;
+    L.x0 = v + 2 * n;
+    L.x1 = v + 3 * n;
+    L.r = v + 4 * n;
+    if (l > 0 && ok) ok = (L.A = get(81 * n)) != nullptr;
+  }
+  int64_t n1 = 0, n2 = 0;
+  mg_scratch(mg, &n1, &n2);
+  ok = ok && (mg.rap1 = get((size_t)n1)) && (mg.rap2 = get((size_t)n2)) && (mg.lam = get(8)) &&
+       (mg.inv = get((size_t)mg.lv[mg.nl - 1].g.n * mg.lv[mg.nl - 1].g.n));
+  if (ok && !c->h_flag && hipHostMalloc((void**)&c->h_flag, sizeof(uint64_t)) != hipSuccess) {
+    (void)hipGetLastError();
+    ok = false;
+  }
+  if (!ok) {
+    mg_free(c);
+    return false;
+  }
+  mg.state = 1;
+  return true;
+}
+
+// BiCGSTAB with the multigrid preconditioner; *converged: to the stopping rule, with a true
+// residual that the reference's check accepts.
+template <typename TM>
+static int run_mg(cpfem_ctx* c, hipStream_t st, const double* mat, const TM* matp, const double* b, double* x, double tol,
+                  double atol, int maxiter, CpfemSolveInfo* inf, bool* converged) {
+  const Multigrid& mg = c->mg;
+  const BellView M = c->bell();
+  launch_inv_diag(M, mat, c->d_dslot, c->kv64[8], 1, st);
+  int sl = prof_begin(&c->prof, PC_MG_SETUP, st);
+  mg_setup<TM>(mg, mat, c->kv64[8], c->d_isbc, c->d_kpartial, st);
+  prof_end(&c->prof, sl, st);
+  KrylovWork w{};
+  w.n = c->n_dofs;
+  w.nb = krylov_blocks(c->n_dofs);
+  w.nbs = mg_spmv_blocks(c->n_dofs);
+  w.ps = std::max(w.nb, w.nbs);
+  w.partial = c->d_kpartial;
+  w.sc = c->d_ksc;
+  double** k = c->kv64;
+  const MgVec v{x, k[0], k[1], k[2], k[3], k[4], k[5], k[6], k[7], k[8]};
+  __atomic_store_n(c->h_flag, (uint64_t)0, __ATOMIC_RELEASE);
+  mg_krylov_init(mg, M, mat, b, v, w, tol, atol, std::min(maxiter, MG_MAXITER), st);
+  HIPCHK(hipGetLastError());
+  // An iteration's first kernel reports the convergence test in the pinned word; the next
+  // iteration is queued once it has, while the rest of this one runs.
+  uint64_t f = 0;
+  for (int it = 0; it <= MG_MAXITER + 1; ++it) {
+    mg_krylov_iteration<TM>(mg, M, mat, matp, v, w, it, c->h_flag, st, &c->prof);
+    HIPCHK(hipGetLastError());
+    for (unsigned spin = 0;; ++spin) {
+      f = __atomic_load_n(c->h_flag, __ATOMIC_ACQUIRE);
+      if ((f >> 33) > (uint64_t)it || (f >> 32 & 1)) break;
+      if ((spin & 0xfff) == 0xfff) {
+        const hipError_t e = hipStreamQuery(st);
+        if (e == hipErrorNotReady) continue;
+        HIPCHK(e);
+        f = __atomic_load_n(c->h_flag, __ATOMIC_ACQUIRE);
+        if ((f >> 33) > (uint64_t)it || (f >> 32 & 1)) break;
+        return fail(CPFEM_EHIP, "multigrid solve: no progress report from the device");
+      }
+    }
+    if (f >> 32 & 1) break;
+  }
+  launch_residual64(M, mat, x, b, c->d_tmp64, st);
+  launch_residual_norm(c->n_dofs, c->d_tmp64, c->d_tmp64, c->d_partial, c->nb, c->d_scalar, st);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipMemcpyAsync(c->h_dbl, c->d_scalar, sizeof(double), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipMemcpyAsync(c->h_ksc, c->d_ksc, sizeof(KrylovScalars), hipMemcpyDeviceToHost, st));
+  HIPCHK(hipStreamSynchronize(st));
+  inf->iterations = c->h_ksc->k;
+  inf->outer = 1;
+  inf->residual = std::sqrt(c->h_dbl[0]);
+  inf->b_norm = std::sqrt(c->h_ksc->bs);
+  *converged = c->h_ksc->k >= 0 && c->h_ksc->rs <= c->h_ksc->atol2 && inf->residual < 0.1;
+  return CPFEM_OK;
+}
+
 // ------------------------------------------------------------------------- C ABI
 extern "C" {
 
@@ -754,6 +891,8 @@ void cpfem_destroy(cpfem_ctx* c) {
   dfree(c->d_kpartial);
   for (int i = 0; i < 12; ++i) dfree(c->kv64[i]);
   dfree(c->d_mat32); dfree(c->d_r64); dfree(c->d_tmp64);
+  mg_free(c);
+  if (c->h_flag) (void)hipHostFree(c->h_flag);
   if (c->h_ksc) (void)hipHostFree(c->h_ksc);
   if (c->h_dbl) (void)hipHostFree(c->h_dbl);
   if (c->h_int) (void)hipHostFree(c->h_int);
@@ -1084,6 +1223,34 @@ int cpfem_solve(cpfem_ctx* c, void* stream, const double* mat, const double* b, 
   int rc;
   if ((rc = ensure_krylov(c, precision == CPFEM_MIXED))) return rc;
   return solve_impl(c, (hipStream_t)stream, ctx_bufs(c), mat, b, x, tol, atol, maxiter, precond, precision, info);
+}
+
+int cpfem_solve_mg(cpfem_ctx* c, void* stream, const double* mat, const double* b, double* x, double tol, double atol,
+                   int32_t maxiter, int32_t precision, CpfemSolveInfo* info) {
+  if (!c || !mat || !b || !x) return fail(CPFEM_EBADARG, "null argument");
+  if (precision != CPFEM_FP64 && precision != CPFEM_MIXED) return fail(CPFEM_EBADARG, "unknown precision");
+  if (maxiter < 0) return fail(CPFEM_EBADARG, "maxiter must be >= 0");
+  if (ensure_mg(c)) {
+    int rc;
+    hipStream_t st = (hipStream_t)stream;
+    if ((rc = ensure_krylov(c, precision == CPFEM_MIXED))) return rc;
+    launch_copy(c->n_dofs, x, c->kv64[9], st);  // x0, for the solve that takes over
+    CpfemSolveInfo inf{};
+    bool converged = false;
+    if (precision == CPFEM_FP64) {
+      rc = run_mg<double>(c, st, mat, mat, b, x, tol, atol, maxiter, &inf, &converged);
+    } else {
+      launch_cast_f32(c->mat_len(), mat, c->d_mat32, st);
+      rc = run_mg<float>(c, st, mat, c->d_mat32, b, x, tol, atol, maxiter, &inf, &converged);
+    }
+    if (rc) return rc;
+    if (converged) {
+      if (info) *info = inf;
+      return CPFEM_OK;
+    }
+    launch_copy(c->n_dofs, c->kv64[9], x, st);
+  }
+  return cpfem_solve(c, stream, mat, b, x, tol, atol, maxiter, 1, precision, info);
 }
 
 int cpfem_solve_noalloc(cpfem_ctx* c, void* stream, const double* mat, const double* b, double* x, double tol, double atol,

@@ -144,6 +144,9 @@ enum ProfClass {
   PC_KREPLACE,        // residual replacement of the mixed form (k_kreplace)
   PC_ELEMENT_PARK,    // parked points of the assembly's point kernel (k_element_qp_park)
   PC_TANGENT,         // consistent tangent from the converged stresses (k_point_tangent)
+  PC_MG_FINE,         // products with the finest matrix in the multigrid preconditioner
+  PC_MG_COARSE,       // the rest of the preconditioner (coarse levels, transfers)
+  PC_MG_SETUP,        // coarse operators and the spectral bound
   PC_COUNT
 };
 
@@ -211,6 +214,52 @@ struct KVec {
   double2 *rp, *rq;
   const double* invd;
 };
+
+// ---------------------------------------------------------------- multigrid (cp_mg.hip)
+// Node grid of one level, x fastest; n = 3 nx ny nz rows.
+struct MgGrid {
+  int32_t nx, ny, nz, n;
+  double inv_a, inv_b;  // 1 / (nx ny), 1 / nx
+};
+constexpr int MG_MAXL = 12;
+// One level: operator (level 0: the caller's block-ELL matrix; coarser levels: 27 offsets in
+// lexicographic order, value (o, k) of row r at (3 o + k) n + r, zero outside the box), the
+// inverse diagonal (0 on Dirichlet dofs), right-hand side, two iterates and the residual.
+struct MgLevel {
+  MgGrid g;
+  void* A;
+  double *minv, *b, *x0, *x1, *r;
+};
+struct Multigrid {
+  int nl = 0;    // levels
+  int tail = 0;  // first level of the one-block kernel
+  MgLevel lv[MG_MAXL];
+  void *rap1 = nullptr, *rap2 = nullptr;  // triple-product intermediates
+  double* inv = nullptr;                  // inverse of the last level's operator
+  double* lam = nullptr;                  // [0] = 1 / lambda_max of the scaled operator
+  int state = 0;                          // 0: no buffers yet, 1: allocated, -1: does not apply
+};
+// Levels of a box of nx x ny x nz nodes (host; no buffers). False if the box is too thin.
+bool mg_plan(const int64_t box[3], Multigrid* mg);
+// Doubles of the two triple-product intermediates of the plan.
+void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2);
+// Coarse operators, diagonals and the spectral bound for the matrix vals (fine values in TM).
+template <typename TM>
+void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const uint8_t* is_bc, double* partial,
+              hipStream_t st);
+// Vectors of the multigrid-preconditioned BiCGSTAB.
+struct MgVec {
+  double *x, *r, *rhat, *p, *q, *phat, *s, *shat, *t;
+  const double* invd;
+};
+void mg_krylov_init(const Multigrid& mg, const BellView& M, const double* vals, const double* b, MgVec v, KrylovWork w,
+                    double tol, double atol, int maxiter, hipStream_t st);
+// One iteration; vals: FP64 operator, valsp: the preconditioner's values of the same matrix.
+// flag: host word that the first kernel sets to (iteration + 1) << 33 | done << 32 | k.
+template <typename TM>
+void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w,
+                         int iter, uint64_t* flag, hipStream_t st, Prof* prof);
+int mg_spmv_blocks(int64_t n);
 
 // Banded LU of the Newton matrix (direct-solve option): n dofs, half bandwidths kl = ku,
 // row-major band of width W = kl + ku + 1 under the node map ip (old -> new), work vector y,

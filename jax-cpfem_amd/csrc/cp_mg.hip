@@ -1,0 +1,1065 @@
+// Geometric multigrid preconditioner for the Newton matrices of box-numbered meshes, and the
+// BiCGSTAB that uses it.
+//
+// The reference solves every Newton system by Jacobi-preconditioned BiCGSTAB
+// (crystal_plasticity_OR_design/solver.py:19-48), whose iteration count grows with the number of
+// elements per side (about 200 at 16^3, 370 at 32^3, 900 at 64^3 to 1e-12), each iteration two
+// passes over the whole matrix.  Here the same recurrence runs to the same stopping rule with
+// one multigrid V-cycle in the place of the diagonal scaling: about 10 iterations at every
+// size, in the elastic and in the plastic state.
+//
+// Cycle: levels coarsen every direction by two (node 2I; an odd last element stays as one),
+// trilinear interpolation P, coarse operators P^T A P, Dirichlet dofs masked out on every level
+// (they are scaled by the diagonal alone); before the coarse correction a Chebyshev polynomial
+// of the diagonally scaled operator over [0.1, 1.1] lambda_max, none after it.  With
+// scalar-diagonal smoothing before the correction only, degree 4 on the finest and 3 on the
+// coarser levels needs the fewest matrix passes (per iteration 2 + 2 x 4 on the finest level;
+// degree 2 takes 16 iterations, 3 takes 12, 4 takes 10; smoothing after the correction as well,
+// 3x3 block diagonals and W-cycles gain nothing).  The last level (at most 81 rows) is inverted.
+// lambda_max comes from a power iteration on the second level (the levels' values differ by a
+// few percent, the polynomial's range by ten).  Levels of at most TAIL_ROWS rows run in one
+// block, whose barriers are cheaper than launches.
+//
+// The polynomial is run as the three-term recurrence on the iterate,
+//   x' = x + c1 (x - x_prev) + c2 D^-1 (b - A x),
+// which reads and writes two vectors fewer per pass than the form that carries the residual.
+#include <hip/hip_ext.h>
+
+#include <algorithm>
+#include <type_traits>
+
+#include "cp_krylov.hpp"
+
+namespace cpfem {
+
+constexpr int DEG_FINE = 4, DEG_COARSE = 3;
+constexpr int TAIL_ROWS = 384, TAIL_LAST = 81, TAIL_SUM = 768, TAIL_BS = 2 * TAIL_ROWS;
+constexpr int POWER_STEPS = 12;
+constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
+constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
+
+// Chebyshev recurrence over [lo, 1.1] lambda_max in units of 1 / lambda_max (the kernels multiply
+// by the device-resident 1 / lambda_max): x1 = ith D^-1 b, then step k uses c1[k], c2[k].
+struct Cheb {
+  double ith;
+  double c1[4], c2[4];
+};
+
+static Cheb cheb(int deg, double lo) {
+  Cheb c{};
+  const double hi = 1.1, th = 0.5 * (hi + lo), de = 0.5 * (hi - lo), sg = th / de;
+  double rho = 1.0 / sg;
+  c.ith = 1.0 / th;
+  for (int k = 0; k + 1 < deg; ++k) {
+    const double rn = 1.0 / (2.0 * sg - rho);
+    c.c1[k] = rn * rho;
+    c.c2[k] = 2.0 * rn / de;
+    rho = rn;
+  }
+  return c;
+}
+
+// ---------------------------------------------------------------------------------
+// Grids (host)
+static MgGrid make_grid(int64_t nx, int64_t ny, int64_t nz) {
+  MgGrid g;
+  g.nx = (int32_t)nx;
+  g.ny = (int32_t)ny;
+  g.nz = (int32_t)nz;
+  g.n = (int32_t)(3 * nx * ny * nz);
+  g.inv_a = 1.0 / (double)(nx * ny);
+  g.inv_b = 1.0 / (double)nx;
+  return g;
+}
+static int64_t coarse_nodes(int64_t m) { return (m - 1 + 1) / 2 + 1; }  // m nodes, ceil((m - 1) / 2) + 1
+
+bool mg_plan(const int64_t box[3], Multigrid* mg) {
+  if (box[0] < 3 || box[1] < 3 || box[2] < 3 || 3 * box[0] * box[1] * box[2] >= (1LL << 28)) return false;
+  mg->nl = 0;
+  int64_t m[3] = {box[0], box[1], box[2]};
+  for (;;) {
+    mg->lv[mg->nl] = MgLevel{};
+    mg->lv[mg->nl].g = make_grid(m[0], m[1], m[2]);
+    ++mg->nl;
+    const int64_t c[3] = {coarse_nodes(m[0]), coarse_nodes(m[1]), coarse_nodes(m[2])};
+    if (3 * m[0] * m[1] * m[2] <= 81 || (c[0] == m[0] && c[1] == m[1] && c[2] == m[2])) break;
+    if (mg->nl == MG_MAXL) break;
+    for (int d = 0; d < 3; ++d) m[d] = c[d];
+  }
+  mg->tail = mg->nl - 1;
+  int64_t sum = mg->lv[mg->tail].g.n;
+  if (sum > TAIL_LAST) return false;
+  // the first level of the block holds its matrix in registers (two threads per row), the others
+  // take three threads per row
+  while (mg->tail > 1 && mg->lv[mg->tail].g.n * 3 <= TAIL_BS && mg->lv[mg->tail - 1].g.n <= TAIL_ROWS &&
+         sum + mg->lv[mg->tail - 1].g.n <= TAIL_SUM)
+    sum += mg->lv[--mg->tail].g.n;
+  return mg->nl >= 2;
+}
+
+void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2) {
+  const MgGrid &f = mg.lv[0].g, &c = mg.lv[1].g;
+  *n1 = 81LL * 3 * c.nx * f.ny * f.nz;
+  *n2 = 81LL * 3 * c.nx * c.ny * f.nz;
+}
+
+// ---------------------------------------------------------------------------------
+// Interpolation in one direction with n elements: fine node of coarse node X, and the weight of
+// coarse node X at fine node i.
+__device__ __forceinline__ int mg_fine(int X, int n) { return min(2 * X, n); }
+__device__ __forceinline__ double mg_weight(int i, int f, int n) {
+  if (i == f) return 1.0;
+  return (i & 1) && i != n && (i == f + 1 || i == f - 1) ? 0.5 : 0.0;
+}
+
+struct NodeXYZ {
+  int x, y, z;
+};
+// Node coordinates of node i: (i + 0.5) / A lies at least 0.5 / A from an integer, far beyond the
+// product's rounding.
+__device__ __forceinline__ NodeXYZ mg_node(const MgGrid& g, int i) {
+  NodeXYZ p;
+  p.z = (int)(((double)i + 0.5) * g.inv_a);
+  const int rz = i - p.z * g.nx * g.ny;
+  p.y = (int)(((double)rz + 0.5) * g.inv_b);
+  p.x = rz - p.y * g.nx;
+  return p;
+}
+
+// A x of row r over the slots of one part (27 / P of them): FINE: the caller's block-ELL matrix
+// (columns of face nodes loaded, the others computed), else a coarse operator in offset order.
+template <typename TM, bool FINE, int P>
+__device__ __forceinline__ double mg_dot(const BellView& M, const MgGrid& g, const TM* __restrict__ A,
+                                         const double* __restrict__ x, int r, int part) {
+  constexpr int NSL = 27 / P;
+  const int i = (int)((uint32_t)r / 3u);
+  const NodeXYZ p = mg_node(g, i);
+  const int a = g.nx * g.ny, b = g.nx;
+  const int s0 = P == 1 ? 0 : NSL * part;
+  const bool inner = (uint32_t)(p.x - 1) < (uint32_t)(g.nx - 2) && (uint32_t)(p.y - 1) < (uint32_t)(g.ny - 2) &&
+                     (uint32_t)(p.z - 1) < (uint32_t)(g.nz - 2);
+  int32_t j[NSL];
+  if (inner) {
+    const int base = P == 1 ? i - a : i + (part - 1) * a;
+#pragma unroll
+    for (int k = 0; k < NSL; ++k) j[k] = base + (k / 9) * a + (k / 3 % 3 - 1) * b + (k % 3 - 1);
+  } else if (FINE) {
+#pragma unroll
+    for (int k = 0; k < NSL; ++k) j[k] = M.col[(int64_t)(s0 + k) * M.n_nodes + i];
+  } else {  // an offset out of the box holds zeros: any node of the box will do
+    const int xm = p.x > 0 ? 1 : 0, xp = p.x < g.nx - 1 ? 1 : 0, ym = p.y > 0 ? b : 0, yp = p.y < g.ny - 1 ? b : 0;
+    const int zm = p.z > 0 ? a : 0, zp = p.z < g.nz - 1 ? a : 0;
+#pragma unroll
+    for (int k = 0; k < NSL; ++k) {
+      const int dz = P == 1 ? k / 9 - 1 : part - 1, dy = k / 3 % 3 - 1, dx = k % 3 - 1;
+      j[k] = i + (dz < 0 ? -zm : dz > 0 ? zp : 0) + (dy < 0 ? -ym : dy > 0 ? yp : 0) + (dx < 0 ? -xm : dx > 0 ? xp : 0);
+    }
+  }
+  const int64_t n = g.n;
+  const TM* __restrict__ v = A + 3 * (int64_t)s0 * n + r;
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < NSL; ++k) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc += (double)v[(3 * k + c) * n] * x[3 * j[k] + c];
+  }
+  return acc;
+}
+
+// Rows of a block: P = 1: 256 rows, one per thread; P = 3: 64 rows, the slots of each split over
+// the block's three waves (planes of the stencil), so that small levels fill more of the device.
+template <int P>
+struct MgShape {
+  static constexpr int BS = P == 1 ? 256 : 64 * P;
+  static constexpr int ROWS = P == 1 ? 256 : 64;
+};
+
+// order: bit 0: row blocks in reverse, bit 1: XCD-local ranges.  Consecutive passes over the same
+// matrix alternate their direction, so that each starts on the rows the last one read last (the
+// matrix outgrows the 256 MB Infinity Cache at 56^3).
+template <int P>
+__device__ __forceinline__ int mg_row0(int order) {
+  int b = (order & 2) ? xcd_rank((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+  if (order & 1) b = (int)gridDim.x - 1 - b;
+  return b * MgShape<P>::ROWS;
+}
+
+// A x of this thread's row; true in the thread that owns the row (whose acc is complete).
+template <typename TM, bool FINE, int P>
+__device__ __forceinline__ bool mg_row(const BellView& M, const MgGrid& g, const TM* __restrict__ A,
+                                       const double* __restrict__ x, int order, int& r, double& acc, double* red) {
+  if constexpr (P == 1) {
+    r = mg_row0<1>(order) + (int)threadIdx.x;
+    acc = 0.0;
+    if (r < g.n) acc = mg_dot<TM, FINE, 1>(M, g, A, x, r, 0);
+    return r < g.n;
+  } else {
+    const int lane = threadIdx.x & 63, part = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    r = mg_row0<P>(order) + lane;
+    acc = 0.0;
+    if (r < g.n) acc = mg_dot<TM, FINE, P>(M, g, A, x, r, part);
+    if (part) red[(part - 1) * 64 + lane] = acc;
+    __syncthreads();
+    if (part) return false;
+#pragma unroll
+    for (int k = 0; k < P - 1; ++k) acc += red[k * 64 + lane];
+    return r < g.n;
+  }
+}
+
+// One Chebyshev step: xo <- x + c1 (x - xo) + c2 D^-1 (b - A x) (first: xo counts as zero).
+template <typename TM, bool FINE, int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mg_smooth(BellView M, const TM* __restrict__ A, MgGrid g,
+                                                             const double* __restrict__ minv, const double* __restrict__ b,
+                                                             const double* __restrict__ x, double* __restrict__ xo, int first,
+                                                             double c1, double c2, const double* __restrict__ lam,
+                                                             const int32_t* __restrict__ done, int order) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  const int dn = *done;  // tested when the product is there: one round trip less per pass
+  const double c2l = c2 * lam[0];
+  int r;
+  double acc;
+  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red) || dn) return;
+  const double xv = x[r], xp = first ? 0.0 : xo[r];
+  xo[r] = xv + (c1 * (xv - xp) + c2l * minv[r] * (b[r] - acc));
+}
+
+// r = b - A x on the free dofs, 0 on Dirichlet dofs.
+template <typename TM, bool FINE, int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mg_resid(BellView M, const TM* __restrict__ A, MgGrid g,
+                                                            const double* __restrict__ minv, const double* __restrict__ b,
+                                                            const double* __restrict__ x, double* __restrict__ out,
+                                                            const int32_t* __restrict__ done, int order) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  const int dn = *done;
+  int r;
+  double acc;
+  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red) || dn) return;
+  out[r] = minv[r] != 0.0 ? b[r] - acc : 0.0;
+}
+
+// Power iteration: xo = D^-1 A x, and the partial sums of <xo, xo> and <x, x>.
+template <typename TM, int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mg_power(BellView M, const TM* __restrict__ A, MgGrid g,
+                                                            const double* __restrict__ minv, const double* __restrict__ x,
+                                                            double* __restrict__ xo, double* __restrict__ partial, int ps) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  __shared__ double sh[2 * (MgShape<P>::BS / 64)];
+  int r;
+  double acc, v[2] = {0.0, 0.0};
+  if (mg_row<TM, false, P>(M, g, A, x, 0, r, acc, red)) {
+    const double y = minv[r] * acc;
+    xo[r] = y;
+    v[0] = y * y;
+    v[1] = x[r] * x[r];
+  }
+  put_partials<MgShape<P>::BS, 2>(v, {0, 1}, partial, ps, sh);
+}
+// Start vector: an alternating sign per node with a hashed amplitude (the largest eigenvectors
+// oscillate from node to node).
+__global__ void __launch_bounds__(256) k_mg_power_start(MgGrid g, const double* __restrict__ minv, double* __restrict__ x) {
+  const int r = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (r >= g.n) return;
+  const NodeXYZ p = mg_node(g, (int)((uint32_t)r / 3u));
+  uint32_t h = (uint32_t)r * 2654435761u;
+  h ^= h >> 15;
+  h *= 2246822519u;
+  h ^= h >> 13;
+  const double s = ((p.x + p.y + p.z) & 1) ? -1.0 : 1.0;
+  x[r] = minv[r] != 0.0 ? s * (0.5 + (double)(h >> 8) * (1.0 / 16777216.0)) : 0.0;
+}
+__global__ void __launch_bounds__(256) k_mg_power_finish(const double* __restrict__ partial, int count, int ps,
+                                                        double* __restrict__ lam) {
+  __shared__ double sh[2 * 4];
+  double v[2] = {0.0, 0.0};
+  for (int i = threadIdx.x; i < count; i += 256) {
+    v[0] += partial[i];
+    v[1] += partial[ps + i];
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const double s = wave_sum(v[j]);
+    if (lane == 0) sh[j * 4 + wid] = s;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) lam[0] = sqrt((sh[4] + sh[5] + sh[6] + sh[7]) / (sh[0] + sh[1] + sh[2] + sh[3]));
+}
+
+// P^T r at coarse row t (res: the residual of grid f).
+__device__ __forceinline__ double mg_restrict_row(const MgGrid& f, const MgGrid& g, int t, const double* __restrict__ res) {
+  const int I = (int)((uint32_t)t / 3u), c = t - 3 * I;
+  const NodeXYZ p = mg_node(g, I);
+  const int ex = f.nx - 1, ey = f.ny - 1, ez = f.nz - 1;
+  const int fx = mg_fine(p.x, ex), fy = mg_fine(p.y, ey), fz = mg_fine(p.z, ez);
+  double acc = 0.0;
+#pragma unroll
+  for (int dz = -1; dz <= 1; ++dz) {
+    const int z = fz + dz;
+    const bool okz = z >= 0 && z <= ez;
+    const double wz = okz ? mg_weight(z, fz, ez) : 0.0;
+#pragma unroll
+    for (int dy = -1; dy <= 1; ++dy) {
+      const int y = fy + dy;
+      const bool oky = okz && y >= 0 && y <= ey;
+      const double wy = oky ? wz * mg_weight(y, fy, ey) : 0.0;
+#pragma unroll
+      for (int dx = -1; dx <= 1; ++dx) {
+        const int xx = fx + dx;
+        const bool ok = oky && xx >= 0 && xx <= ex;
+        const double w = ok ? wy * mg_weight(xx, fx, ex) : 0.0;
+        const int node = ok ? xx + f.nx * (y + f.ny * z) : fx + f.nx * (fy + f.ny * fz);
+        acc += w * res[3 * node + c];
+      }
+    }
+  }
+  return acc;
+}
+
+// Restriction b_c = P^T r and the first coarse iterate x_c = ith D^-1 b_c.
+__global__ void __launch_bounds__(256) k_mg_restrict(MgGrid f, MgGrid g, const double* __restrict__ rf,
+                                                    const double* __restrict__ minv, double* __restrict__ b,
+                                                    double* __restrict__ x, double ith, const double* __restrict__ lam,
+                                                    const int32_t* __restrict__ done) {
+  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t >= g.n) return;
+  const int dn = *done;
+  const double il = ith * lam[0], mi = minv[t];
+  double acc = mg_restrict_row(f, g, t, rf);
+  if (dn) return;
+  acc = mi != 0.0 ? acc : 0.0;
+  b[t] = acc;
+  x[t] = il * mi * acc;
+}
+
+// P e at fine node (x, y, z), component c.
+__device__ __forceinline__ double mg_interp(const MgGrid& f, const MgGrid& g, const NodeXYZ& p, int c,
+                                            const double* __restrict__ e) {
+  // the one or two parents of a direction: first, step to the second (0: none), weight
+  const auto par = [](int i, int n, int& X, int& d) {
+    if (!(i & 1)) {
+      X = i >> 1;
+      d = 0;
+    } else if (i == n) {
+      X = (i + 1) >> 1;
+      d = 0;
+    } else {
+      X = i >> 1;
+      d = 1;
+    }
+  };
+  int X, Y, Z, dx, dy, dz;
+  par(p.x, f.nx - 1, X, dx);
+  par(p.y, f.ny - 1, Y, dy);
+  par(p.z, f.nz - 1, Z, dz);
+  const int b = 3 * (X + g.nx * (Y + g.ny * Z)) + c;
+  const int sx = 3 * dx, sy = 3 * dy * g.nx, sz = 3 * dz * g.nx * g.ny;
+  // a direction without a second parent reads the first one twice: the mean is its value
+  const double v0 = 0.5 * (e[b] + e[b + sx]), v1 = 0.5 * (e[b + sy] + e[b + sy + sx]);
+  const double v2 = 0.5 * (e[b + sz] + e[b + sz + sx]), v3 = 0.5 * (e[b + sz + sy] + e[b + sz + sy + sx]);
+  return 0.5 * (0.5 * (v0 + v1) + 0.5 * (v2 + v3));
+}
+
+// out = x + P e on the free dofs; on Dirichlet dofs b / diagonal (finest level) or 0.
+__global__ void __launch_bounds__(256) k_mg_prolong(MgGrid f, MgGrid g, const double* __restrict__ e, const double* __restrict__ x,
+                                                   const double* __restrict__ minv, const double* __restrict__ b,
+                                                   const double* __restrict__ invd, double* __restrict__ out,
+                                                   const int32_t* __restrict__ done) {
+  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t >= f.n) return;
+  const int dn = *done;
+  const int i = (int)((uint32_t)t / 3u);
+  const NodeXYZ p = mg_node(f, i);
+  const double v = x[t] + mg_interp(f, g, p, t - 3 * i, e);
+  if (dn) return;
+  out[t] = minv[t] != 0.0 ? v : (invd ? b[t] * invd[t] : 0.0);
+}
+
+// The levels of at most TAIL_ROWS rows in one block, their vectors in LDS.  Bound by latency: one
+// CU reads 64 B per clock from the L2, so the first of these levels (375 rows, 243 KB at 64^3)
+// keeps its matrix in registers, half a row per thread, and reads it once per cycle instead
+// of once per product; the last level (at most 81 rows) is solved with its inverse, staged in LDS.
+// (Reading it for each product, one thread per row: 56 us per cycle.)
+struct MgTail {
+  int nl;
+  MgGrid f;  // the level above, whose residual is restricted first
+  const double* rf;
+  MgGrid g[MG_MAXL];
+  const void* A[MG_MAXL];
+  const double* minv[MG_MAXL];
+  int off[MG_MAXL];
+};
+
+// One thread's share of a row of the block's first level: slots [S0, S0 + 14) (13 in the second
+// half).  Rows off the box read a node of the box against a zero.
+constexpr int TAIL_SLOTS = 14;
+struct TailRow {
+  int i3, xm, xp, ym, yp, zm, zp;  // three times the node, and the steps to its neighbours (0: none)
+  __device__ TailRow(const MgGrid& g, int r) {
+    const int i = (int)((uint32_t)r / 3u);
+    const NodeXYZ p = mg_node(g, i);
+    i3 = 3 * i;
+    xm = p.x > 0 ? 3 : 0;
+    xp = p.x < g.nx - 1 ? 3 : 0;
+    ym = p.y > 0 ? 3 * g.nx : 0;
+    yp = p.y < g.ny - 1 ? 3 * g.nx : 0;
+    zm = p.z > 0 ? 3 * g.nx * g.ny : 0;
+    zp = p.z < g.nz - 1 ? 3 * g.nx * g.ny : 0;
+  }
+};
+template <typename TM, int S0>
+__device__ __forceinline__ void tail_load(const TM* __restrict__ A, int n, int r, TM (&a)[3 * TAIL_SLOTS]) {
+#pragma unroll
+  for (int k = 0; k < 3 * TAIL_SLOTS; ++k) a[k] = 3 * S0 + k < 81 ? A[(3 * S0 + k) * (int64_t)n + r] : (TM)0;
+}
+template <typename TM, int S0>
+__device__ __forceinline__ double tail_dot(const TailRow& t, const TM (&a)[3 * TAIL_SLOTS], const double* __restrict__ v) {
+  double acc = 0.0;
+#pragma unroll
+  for (int k = 0; k < TAIL_SLOTS; ++k) {
+    constexpr int last = 26;
+    const int s = S0 + k < last ? S0 + k : last;
+    const int dz = s / 9 - 1, dy = s / 3 % 3 - 1, dx = s % 3 - 1;
+    const double* w = v + t.i3 + (dz < 0 ? -t.zm : dz > 0 ? t.zp : 0) + (dy < 0 ? -t.ym : dy > 0 ? t.yp : 0) +
+                      (dx < 0 ? -t.xm : dx > 0 ? t.xp : 0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc += (double)a[3 * k + c] * w[c];
+  }
+  return acc;
+}
+
+template <typename TM>
+__global__ void __launch_bounds__(TAIL_BS) k_mg_tail(MgTail T, double* __restrict__ x, Cheb cc, const double* __restrict__ inv,
+                                                     const double* __restrict__ lam, const int32_t* __restrict__ done) {
+  __shared__ double sb[TAIL_SUM], sx[TAIL_SUM], so[TAIL_SUM], red[TAIL_BS];
+  __shared__ double sI[TAIL_LAST * TAIL_LAST];
+  const int tid = threadIdx.x;
+  const int dn = *done;
+  const double il = lam[0];
+  const BellView none{};
+  const int last = T.nl - 1;
+  // the first level's matrix (threads below TAIL_ROWS: first half of the row's slots), the last
+  // level's inverse into LDS
+  const int n0 = T.g[0].n, half = __builtin_amdgcn_readfirstlane(tid >= TAIL_ROWS ? 1 : 0), r0 = tid - half * TAIL_ROWS;
+  const bool own0 = r0 < n0 && last > 0;
+  const TailRow row0(T.g[0], own0 ? r0 : 0);
+  TM a0[3 * TAIL_SLOTS];
+  if (own0) {
+    if (half)
+      tail_load<TM, TAIL_SLOTS>(static_cast<const TM*>(T.A[0]), n0, r0, a0);
+    else
+      tail_load<TM, 0>(static_cast<const TM*>(T.A[0]), n0, r0, a0);
+  }
+  for (int k = tid; k < T.g[last].n * T.g[last].n; k += TAIL_BS) sI[k] = inv[k];
+  if (tid < n0) {
+    const double v = mg_restrict_row(T.f, T.g[0], tid, T.rf);
+    sb[tid] = T.minv[0][tid] != 0.0 ? v : 0.0;
+  }
+  if (dn) return;  // uniform
+  // A v of the level's rows in the threads tid < n
+  const auto product = [&](int l, const double* v) -> double {
+    const int n = T.g[l].n;
+    double a = 0.0, y = 0.0;
+    if (l == 0 && last > 0) {
+      if (own0) a = half ? tail_dot<TM, TAIL_SLOTS>(row0, a0, v) : tail_dot<TM, 0>(row0, a0, v);
+      red[tid] = a;
+      __syncthreads();
+      if (tid < n) y = a + red[tid + TAIL_ROWS];
+    } else {
+      const TM* A = static_cast<const TM*>(T.A[l]);
+      const int part = tid / n, r = tid - part * n;  // 3 n <= TAIL_BS below the first level
+      if (part < 3) a = mg_dot<TM, false, 3>(none, T.g[l], A, v, r, part);
+      red[tid] = a;
+      __syncthreads();
+      if (tid < n) y = a + red[tid + n] + red[tid + 2 * n];
+    }
+    __syncthreads();
+    return y;
+  };
+  // Chebyshev polynomial of degree deg from zero; the result's buffer alternates between sx and so
+  const auto smooth = [&](int l, int deg, const Cheb& c) -> double* {
+    const int n = T.g[l].n, o = T.off[l];
+    double *cur = sx + o, *oth = so + o;
+    const double mi = tid < n ? T.minv[l][tid] : 0.0;
+    if (tid < n) {
+      cur[tid] = c.ith * il * mi * sb[o + tid];
+      oth[tid] = 0.0;
+    }
+    __syncthreads();
+    for (int k = 0; k + 1 < deg; ++k) {
+      const double y = product(l, cur);
+      if (tid < n) oth[tid] = cur[tid] + (c.c1[k] * (cur[tid] - oth[tid]) + c.c2[k] * il * mi * (sb[o + tid] - y));
+      __syncthreads();
+      double* s = cur;
+      cur = oth;
+      oth = s;
+    }
+    return cur;
+  };
+  __syncthreads();
+  for (int l = 0; l < last; ++l) {
+    const double* cur = smooth(l, DEG_COARSE, cc);
+    const int n = T.g[l].n, o = T.off[l];
+    const double y = product(l, cur);
+    double v = 0.0;
+    if (tid < n) {
+      v = cur[tid];
+      so[o + tid] = T.minv[l][tid] != 0.0 ? sb[o + tid] - y : 0.0;  // residual
+      sx[o + tid] = v;                                               // iterate
+    }
+    __syncthreads();
+    const int nc = T.g[l + 1].n;
+    if (tid < nc) sb[T.off[l + 1] + tid] = T.minv[l + 1][tid] != 0.0 ? mg_restrict_row(T.g[l], T.g[l + 1], tid, so + o) : 0.0;
+    __syncthreads();
+  }
+  {  // the last level exactly, a row's columns over three threads
+    const int n = T.g[last].n, o = T.off[last], w = (n + 2) / 3;
+    const int part = tid / n, r = tid - part * n;
+    double a = 0.0;
+    if (part < 3) {
+      for (int c = part * w; c < min(n, (part + 1) * w); ++c) a += sI[c * n + r] * sb[o + c];
+    }
+    red[tid] = a;
+    __syncthreads();
+    if (tid < n) sx[o + tid] = a + red[tid + n] + red[tid + 2 * n];
+    __syncthreads();
+  }
+  for (int l = last - 1; l >= 0; --l) {
+    if (tid < T.g[l].n) {
+      const int i = (int)((uint32_t)tid / 3u);
+      const double v = sx[T.off[l] + tid] + mg_interp(T.g[l], T.g[l + 1], mg_node(T.g[l], i), tid - 3 * i, sx + T.off[l + 1]);
+      sx[T.off[l] + tid] = T.minv[l][tid] != 0.0 ? v : 0.0;
+    }
+    __syncthreads();
+  }
+  if (tid < n0) x[tid] = sx[tid];
+}
+
+// ---------------------------------------------------------------------------------
+// Coarse operators.  P is a product of one-dimensional interpolations, so P^T A P is formed one
+// direction at a time: each pass halves the rows and reads and writes each value once (1.2 GB in
+// all at 64^3), where the direct triple product reads every fine row 27 times.  A thread
+// makes the three values of one coarse row, transverse offset pair and component from nine fine
+// values.  DIR: direction coarsened; FINE: reads the block-ELL matrix with the masks of Dirichlet
+// rows and columns; LAST: applies the coarse masks, puts 1 on masked diagonals, writes the
+// inverse diagonal and rounds to the level's value type.
+// Slot of offset (dx, dy, dz) in node p's row (existing neighbours in ascending order).
+__device__ __forceinline__ int mg_slot(const MgGrid& f, const NodeXYZ& p, int dx, int dy, int dz) {
+  const int xl = p.x > 0 ? -1 : 0, yl = p.y > 0 ? -1 : 0, zl = p.z > 0 ? -1 : 0;
+  const int cx = (p.x < f.nx - 1 ? 2 : 1) - xl, cy = (p.y < f.ny - 1 ? 2 : 1) - yl;
+  return ((dz - zl) * cy + (dy - yl)) * cx + (dx - xl);
+}
+
+template <int DIR, bool FINE, bool LAST, typename TI, typename TO>
+__global__ void __launch_bounds__(256) k_mg_coarsen(MgGrid f, MgGrid g, const TI* __restrict__ A, const uint8_t* __restrict__ fixed,
+                                                   const uint8_t* __restrict__ cfixed, TO* __restrict__ out,
+                                                   double* __restrict__ minv) {
+  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t >= g.n) return;
+  const int q = (int)blockIdx.y;  // (transverse offsets, component)
+  const int k = q % 3, t1 = q / 3 % 3 - 1, t2 = q / 9 - 1;
+  const int I = (int)((uint32_t)t / 3u), c = t - 3 * I;
+  const NodeXYZ pc = mg_node(g, I);
+  const int fn[3] = {f.nx, f.ny, f.nz};
+  const int e = fn[DIR] - 1, X = DIR == 0 ? pc.x : DIR == 1 ? pc.y : pc.z;
+  const int gX = DIR == 0 ? g.nx : DIR == 1 ? g.ny : g.nz;
+  const int fX = mg_fine(X, e);
+  // transverse directions in ascending order carry the offsets (t1, t2)
+  NodeXYZ d{DIR == 0 ? 0 : t1, DIR == 1 ? 0 : (DIR == 0 ? t1 : t2), DIR == 2 ? 0 : t2};
+  const bool inside = (uint32_t)(pc.x + d.x) < (uint32_t)(DIR == 0 ? g.nx : f.nx) &&
+                      (uint32_t)(pc.y + d.y) < (uint32_t)(DIR == 1 ? g.ny : f.ny) &&
+                      (uint32_t)(pc.z + d.z) < (uint32_t)(DIR == 2 ? g.nz : f.nz);
+  double acc[3] = {0.0, 0.0, 0.0};
+  if (inside) {
+#pragma unroll
+    for (int a = -1; a <= 1; ++a) {
+      const int i = fX + a;
+      if (i < 0 || i > e) continue;
+      const double wi = mg_weight(i, fX, e);
+      if (wi == 0.0) continue;
+      const NodeXYZ pf{DIR == 0 ? i : pc.x, DIR == 1 ? i : pc.y, DIR == 2 ? i : pc.z};
+      const int node = pf.x + f.nx * (pf.y + f.ny * pf.z);
+      const int64_t row = 3 * (int64_t)node + c;
+      if (FINE && fixed[row]) continue;
+#pragma unroll
+      for (int m = -1; m <= 1; ++m) {
+        const int j = i + m;
+        if (j < 0 || j > e) continue;
+        const int dx = DIR == 0 ? m : d.x, dy = DIR == 1 ? m : d.y, dz = DIR == 2 ? m : d.z;
+        int64_t s;
+        if (FINE) {
+          const int col = node + dx + f.nx * (dy + f.ny * dz);
+          if (fixed[3 * (int64_t)col + k]) continue;
+          s = mg_slot(f, pf, dx, dy, dz);
+        } else {
+          s = (dz + 1) * 9 + (dy + 1) * 3 + dx + 1;
+        }
+        const double v = wi * (double)A[(3 * s + k) * (int64_t)f.n + row];
+#pragma unroll
+        for (int o = -1; o <= 1; ++o) {
+          const int Xo = X + o;
+          if (Xo < 0 || Xo >= gX) continue;
+          acc[o + 1] += mg_weight(j, mg_fine(Xo, e), e) * v;
+        }
+      }
+    }
+  }
+  const int64_t gn = g.n;
+#pragma unroll
+  for (int o = -1; o <= 1; ++o) {
+    const int dx = DIR == 0 ? o : d.x, dy = DIR == 1 ? o : d.y, dz = DIR == 2 ? o : d.z;
+    const int64_t s = (dz + 1) * 9 + (dy + 1) * 3 + dx + 1;
+    double v = acc[o + 1];
+    if (LAST) {
+      const bool in = inside && (uint32_t)(X + o) < (uint32_t)gX;
+      const bool diag = dx == 0 && dy == 0 && dz == 0 && k == c;
+      const bool fr = cfixed[t] != 0;
+      const bool fc = in && cfixed[3 * (int64_t)(I + dx + g.nx * (dy + g.ny * dz)) + k] != 0;
+      if (fr || fc) v = diag ? 1.0 : 0.0;
+      if (diag) minv[t] = fr ? 0.0 : 1.0 / v;
+    }
+    out[(3 * s + k) * gn + t] = (TO)v;
+  }
+}
+
+// Inverse of the last level's operator (column-major), by Gauss-Jordan elimination in LDS.  Smoothing
+// that level instead costs odd-sized boxes, whose half-width last elements pile up there, up
+// to five iterations.  The diagonal is raised by 1e-6, so that a floating box (a singular
+// operator, as where only corners are held) keeps a bounded inverse.
+// A thread keeps one row's columns q, q + 8, ... in registers; the pivot row and column pass
+// through LDS, two buffers in turn, so that a step needs one barrier.
+constexpr int INV_Q = 8, INV_C = (TAIL_LAST + INV_Q - 1) / INV_Q, INV_BS = 704;  // 8 x 81 threads in whole waves
+template <typename TM>
+__global__ void __launch_bounds__(INV_BS) k_mg_inverse(MgGrid g, const TM* __restrict__ A, double* __restrict__ inv) {
+  __shared__ double m[TAIL_LAST * TAIL_LAST], row[2][INV_Q * INV_C], col[2][TAIL_LAST];
+  const int n = g.n, tid = threadIdx.x;
+  for (int k = tid; k < n * n; k += INV_BS) m[k] = 0.0;
+  __syncthreads();
+  for (int k = tid; k < 81 * n; k += INV_BS) {
+    const int q = k / n, r = k - q * n, s = q / 3, i = r / 3;
+    const NodeXYZ p = mg_node(g, i);
+    const int x = p.x + s % 3 - 1, y = p.y + s / 3 % 3 - 1, z = p.z + s / 9 - 1;
+    if ((uint32_t)x >= (uint32_t)g.nx || (uint32_t)y >= (uint32_t)g.ny || (uint32_t)z >= (uint32_t)g.nz) continue;
+    const int c = 3 * (x + g.nx * (y + g.ny * z)) + q % 3;
+    m[c * n + r] = (double)A[k] * (c == r ? 1.0 + 1e-6 : 1.0);
+  }
+  __syncthreads();
+  const int q = tid / TAIL_LAST, r = tid - q * TAIL_LAST;
+  const bool own = q < INV_Q && r < n;
+  double v[INV_C];
+#pragma unroll
+  for (int j = 0; j < INV_C; ++j) v[j] = own && q + INV_Q * j < n ? m[(q + INV_Q * j) * n + r] : 0.0;
+#pragma unroll
+  for (int jp = 0; jp < INV_C; ++jp) {
+#pragma unroll 1
+    for (int qp = 0; qp < INV_Q; ++qp) {
+      const int p = INV_Q * jp + qp, buf = p & 1;
+      if (p >= n) break;  // uniform
+      if (own && q == qp) col[buf][r] = v[jp];
+      if (own && r == p) {
+#pragma unroll
+        for (int j = 0; j < INV_C; ++j) row[buf][q + INV_Q * j] = v[j];
+      }
+      __syncthreads();
+      if (own) {
+        const double piv = 1.0 / col[buf][p], f = r == p ? piv : -col[buf][r] * piv;
+#pragma unroll
+        for (int j = 0; j < INV_C; ++j) {
+          const double x = row[buf][q + INV_Q * j], base = r == p ? 0.0 : v[j];
+          v[j] = q + INV_Q * j == p ? f : base + f * x;
+        }
+      }
+    }
+  }
+  if (own) {
+#pragma unroll
+    for (int j = 0; j < INV_C; ++j)
+      if (q + INV_Q * j < n) inv[(q + INV_Q * j) * n + r] = v[j];
+  }
+}
+
+// Inverse diagonal of the finest level with Dirichlet dofs masked, and the Dirichlet flags of the
+// next level (those of the fine node it stands on).
+__global__ void __launch_bounds__(256) k_mg_mask(int n, const double* __restrict__ invd, const uint8_t* __restrict__ fixed,
+                                                double* __restrict__ minv) {
+  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t < n) minv[t] = fixed[t] ? 0.0 : invd[t];
+}
+__global__ void __launch_bounds__(256) k_mg_inject(MgGrid f, MgGrid g, const uint8_t* __restrict__ fixed, uint8_t* __restrict__ out) {
+  const int t = (int)(blockIdx.x * 256 + threadIdx.x);
+  if (t >= g.n) return;
+  const int I = (int)((uint32_t)t / 3u), c = t - 3 * I;
+  const NodeXYZ p = mg_node(g, I);
+  const int node = mg_fine(p.x, f.nx - 1) + f.nx * (mg_fine(p.y, f.ny - 1) + f.ny * mg_fine(p.z, f.nz - 1));
+  out[t] = fixed[3 * (int64_t)node + c];
+}
+
+static inline unsigned blocks256(int64_t n) { return (unsigned)((n + 255) / 256); }
+static inline int level_parts(int64_t n) { return n >= FLAT_ROWS ? 1 : 3; }
+static inline unsigned level_blocks(int64_t n) { return (unsigned)(level_parts(n) == 1 ? (n + 255) / 256 : (n + 63) / 64); }
+static inline int level_order(int64_t n, int rev) { return (rev & 1) | (n < PLAIN_ROWS ? 2 : 0); }
+int mg_spmv_blocks(int64_t n) { return (int)level_blocks(n); }
+
+template <typename TM>
+void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const uint8_t* is_bc,
+              double* partial, hipStream_t st) {
+  hipLaunchKernelGGL(k_mg_mask, dim3(blocks256(mg.lv[0].g.n)), dim3(256), 0, st, mg.lv[0].g.n, invd, is_bc, mg.lv[0].minv);
+  double *w1 = static_cast<double*>(mg.rap1), *w2 = static_cast<double*>(mg.rap2);
+  const uint8_t* fixed = is_bc;
+  for (int l = 0; l + 1 < mg.nl; ++l) {
+    const MgGrid f = mg.lv[l].g, g = mg.lv[l + 1].g;
+    const MgGrid gx = make_grid(g.nx, f.ny, f.nz), gy = make_grid(g.nx, g.ny, f.nz);
+    uint8_t* cfixed = reinterpret_cast<uint8_t*>(mg.lv[l + 1].r);  // flags live there until the first cycle
+    hipLaunchKernelGGL(k_mg_inject, dim3(blocks256(g.n)), dim3(256), 0, st, f, g, fixed, cfixed);
+    if (l == 0)
+      hipLaunchKernelGGL((k_mg_coarsen<0, true, false, double, double>), dim3(blocks256(gx.n), 27), dim3(256), 0, st, f, gx, vals,
+                         fixed, cfixed, w1, (double*)nullptr);
+    else
+      hipLaunchKernelGGL((k_mg_coarsen<0, false, false, TM, double>), dim3(blocks256(gx.n), 27), dim3(256), 0, st, f, gx,
+                         static_cast<const TM*>(mg.lv[l].A), fixed, cfixed, w1, (double*)nullptr);
+    hipLaunchKernelGGL((k_mg_coarsen<1, false, false, double, double>), dim3(blocks256(gy.n), 27), dim3(256), 0, st, gx, gy, w1,
+                       fixed, cfixed, w2, (double*)nullptr);
+    hipLaunchKernelGGL((k_mg_coarsen<2, false, true, double, TM>), dim3(blocks256(g.n), 27), dim3(256), 0, st, gy, g, w2, fixed,
+                       cfixed, static_cast<TM*>(mg.lv[l + 1].A), mg.lv[l + 1].minv);
+    fixed = cfixed;
+  }
+  const MgLevel& E = mg.lv[mg.nl - 1];
+  hipLaunchKernelGGL(k_mg_inverse<TM>, dim3(1), dim3(INV_BS), 0, st, E.g, static_cast<const TM*>(E.A), mg.inv);
+  // lambda_max on the second level
+  const MgLevel& L = mg.lv[1];
+  const unsigned nb = level_blocks(L.g.n);
+  double *a = L.x0, *b = L.x1;
+  hipLaunchKernelGGL(k_mg_power_start, dim3(blocks256(L.g.n)), dim3(256), 0, st, L.g, L.minv, a);
+  for (int k = 0; k < POWER_STEPS; ++k) {
+    if (level_parts(L.g.n) == 1)
+      hipLaunchKernelGGL((k_mg_power<TM, 1>), dim3(nb), dim3(MgShape<1>::BS), 0, st, BellView{}, static_cast<const TM*>(L.A), L.g,
+                         L.minv, a, b, partial, (int)nb);
+    else
+      hipLaunchKernelGGL((k_mg_power<TM, 3>), dim3(nb), dim3(MgShape<3>::BS), 0, st, BellView{}, static_cast<const TM*>(L.A), L.g,
+                         L.minv, a, b, partial, (int)nb);
+    std::swap(a, b);
+  }
+  hipLaunchKernelGGL(k_mg_power_finish, dim3(1), dim3(256), 0, st, partial, (int)nb, (int)nb, mg.lam);
+}
+
+template <typename F, typename... Args>
+static inline void timed(Prof* prof, int cls, F kernel, dim3 grid, dim3 block, hipStream_t st, Args... args) {
+  hipEvent_t a, b;
+  if (prof_sample(prof, cls, &a, &b))
+    hipExtLaunchKernelGGL(kernel, grid, block, 0, st, a, b, 0, args...);
+  else
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, args...);
+}
+
+// Smoothing of level l from its first iterate (in x0) and the residual in r; returns the buffer of
+// the last iterate.  pass: counts the passes over the finest matrix, for their direction.
+template <typename TM, bool FINE, int P>
+static double* smooth_level(const Multigrid& mg, int l, const BellView& M, const TM* A, const double* b, const Cheb& c, int deg,
+                            const int32_t* done, int* pass, hipStream_t st, Prof* prof) {
+  const MgLevel& L = mg.lv[l];
+  const dim3 grid(level_blocks(L.g.n)), block(MgShape<P>::BS);
+  const int cls = FINE ? PC_MG_FINE : PC_MG_COARSE;
+  double *cur = L.x0, *oth = L.x1;
+  for (int k = 0; k + 1 < deg; ++k) {
+    timed(prof, cls, k_mg_smooth<TM, FINE, P>, grid, block, st, M, A, L.g, (const double*)L.minv, b, (const double*)cur, oth,
+          k == 0 ? 1 : 0, c.c1[k], c.c2[k], (const double*)mg.lam, done, level_order(L.g.n, (*pass)++));
+    std::swap(cur, oth);
+  }
+  timed(prof, cls, k_mg_resid<TM, FINE, P>, grid, block, st, M, A, L.g, (const double*)L.minv, b, (const double*)cur, L.r, done,
+        level_order(L.g.n, (*pass)++));
+  return cur;
+}
+
+// One V-cycle: out = M b; level 0's first iterate is already in x0.
+template <typename TM>
+static void vcycle(const Multigrid& mg, const BellView& M, const TM* vals, const double* invd, const double* b, double* out,
+                   const int32_t* done, int* pass, hipStream_t st, Prof* prof) {
+  static const Cheb cf = cheb(DEG_FINE, 0.1), cc = cheb(DEG_COARSE, 0.1);
+  double* cur[MG_MAXL];
+  for (int l = 0; l < mg.tail; ++l) {
+    const MgLevel& L = mg.lv[l];
+    int p = 0;
+    if (l == 0) {
+      cur[0] = level_parts(L.g.n) == 1 ? smooth_level<TM, true, 1>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof)
+                                       : smooth_level<TM, true, 3>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof);
+    } else {
+      const TM* A = static_cast<const TM*>(L.A);
+      cur[l] = level_parts(L.g.n) == 1 ? smooth_level<TM, false, 1>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof)
+                                       : smooth_level<TM, false, 3>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof);
+    }
+    if (l + 1 == mg.tail) break;  // the one-block kernel restricts for itself
+    const MgLevel& C = mg.lv[l + 1];
+    timed(prof, PC_MG_COARSE, k_mg_restrict, dim3(blocks256(C.g.n)), dim3(256), st, L.g, C.g, (const double*)L.r,
+          (const double*)C.minv, C.b, C.x0, cc.ith, (const double*)mg.lam, done);
+  }
+  MgTail T{};
+  T.nl = mg.nl - mg.tail;
+  T.f = mg.lv[mg.tail - 1].g;
+  T.rf = mg.lv[mg.tail - 1].r;
+  int off = 0;
+  for (int l = 0; l < T.nl; ++l) {
+    const MgLevel& L = mg.lv[mg.tail + l];
+    T.g[l] = L.g;
+    T.A[l] = L.A;
+    T.minv[l] = L.minv;
+    T.off[l] = off;
+    off += L.g.n;
+  }
+  const MgLevel& H = mg.lv[mg.tail];
+  timed(prof, PC_MG_COARSE, k_mg_tail<TM>, dim3(1), dim3(TAIL_BS), st, T, H.x0, cc, (const double*)mg.inv, (const double*)mg.lam,
+        done);
+  const double* e = H.x0;
+  for (int l = mg.tail - 1; l >= 0; --l) {
+    const MgLevel& L = mg.lv[l];
+    double* o = l == 0 ? out : cur[l];
+    timed(prof, PC_MG_COARSE, k_mg_prolong, dim3(blocks256(L.g.n)), dim3(256), st, L.g, mg.lv[l + 1].g, e, (const double*)cur[l],
+          (const double*)L.minv, b, l == 0 ? invd : (const double*)nullptr, o, done);
+    e = o;
+  }
+}
+
+// ---------------------------------------------------------------------------------
+// BiCGSTAB with the V-cycle in the place of the diagonal scaling (recurrence and stopping rule of
+// cp_krylov.hip's header).  Three vector kernels and two products per iteration beside the two
+// cycles; sums as there: one partial per block, added by every block of the consuming kernel in
+// index order.
+
+// Sums of NSL slots over `count` partials with stride ps, returned in every thread (256 threads).
+template <int NSL>
+__device__ __forceinline__ void mg_sums(const double* __restrict__ partial, const int (&slot)[NSL], int count, int ps, double* sh,
+                                        double (&out)[NSL]) {
+  double s[NSL];
+#pragma unroll
+  for (int j = 0; j < NSL; ++j) s[j] = 0.0;
+#pragma unroll 4
+  for (int i = threadIdx.x; i < count; i += KBS) {
+#pragma unroll
+    for (int j = 0; j < NSL; ++j) s[j] += partial[slot[j] * ps + i];
+  }
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+  for (int j = 0; j < NSL; ++j) {
+    const double t = wave_sum(s[j]);
+    if (lane == 0) sh[j * (KBS / 64) + wid] = t;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < NSL; ++j) {
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < KBS / 64; ++i) t += sh[j * (KBS / 64) + i];
+    out[j] = t;
+  }
+  __syncthreads();
+}
+
+// r0 = b - A x0 = rhat = p = q, and the partials of <r,r> (= <rhat,r>) and <b,b>.
+template <int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_init(BellView M, MgGrid g, const double* __restrict__ A,
+                                                            const double* __restrict__ b, MgVec v, KrylovWork w, int order) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  __shared__ double sh[3 * (MgShape<P>::BS / 64)];
+  int r;
+  double acc, d[3] = {0.0, 0.0, 0.0};
+  if (mg_row<double, true, P>(M, g, A, v.x, order, r, acc, red)) {
+    const double bv = b[r], rv = bv - acc;
+    v.r[r] = rv;
+    v.rhat[r] = rv;
+    v.p[r] = rv;
+    v.q[r] = rv;
+    d[0] = d[1] = rv * rv;
+    d[2] = bv * bv;
+  }
+  put_partials<MgShape<P>::BS, 3>(d, {PS_RR, PS_RHR, PS_BB}, w.partial, w.ps, sh);
+}
+__global__ void __launch_bounds__(KBS) k_mgb_init2(KrylovWork w, double tol, double atol, int maxiter) {
+  __shared__ double sh[KBS / 64];
+  double s[1];
+  mg_sums<1>(w.partial, {PS_BB}, w.ps, w.ps, sh, s);
+  if (threadIdx.x == 0) {
+    KrylovScalars* sc = w.sc;
+    sc->bs = s[0];
+    sc->atol2 = fmax(tol * tol * s[0], atol * atol);
+    sc->maxiter = maxiter;
+    sc->rho2[1] = sc->alpha2[1] = sc->omega2[1] = 1.0;
+    sc->k2[1] = -1;
+    sc->done = 0;
+    sc->k = 0;
+  }
+}
+
+// Convergence test of the last iteration, beta, p and the cycle's first iterate for M p.
+__global__ void __launch_bounds__(KBS) k_mgb_p(MgVec v, KrylovWork w, int par, int iter, const double* __restrict__ minv,
+                                              double* __restrict__ y, double ith, const double* __restrict__ lam,
+                                              uint64_t* __restrict__ flag) {
+  __shared__ double sh[2 * (KBS / 64)];
+  KrylovScalars* sc = w.sc;
+  if (sc->done) return;
+  const int pv = par ^ 1;
+  const double rho = sc->rho2[pv], alpha = sc->alpha2[pv], omega = sc->omega2[pv], atol2 = sc->atol2;
+  const int kprev = sc->k2[pv], maxiter = sc->maxiter;
+  const int64_t i0 = (int64_t)blockIdx.x * KBS + threadIdx.x;
+  double sums[2];
+  mg_sums<2>(w.partial, {PS_RR, PS_RHR}, iter == 0 ? w.ps : w.nb, w.ps, sh, sums);
+  const double rs = sums[0], rho_ = sums[1];
+  int k = (omega == 0.0 || alpha == 0.0) ? -11 : kprev + 1;
+  if (rho == 0.0) k = -10;
+  const bool go = (rs > atol2) && (k < maxiter) && (k >= 0);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    sc->k2[par] = k;
+    sc->rho2[par] = rho_;
+    sc->rs = rs;
+    sc->k = k;
+    if (!go) sc->done = 1;
+    __hip_atomic_store(flag, ((uint64_t)(iter + 1) << 33) | ((uint64_t)(go ? 0 : 1) << 32) | (uint32_t)k, __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+  }
+  if (!go) return;
+  const double beta = rho_ / rho * alpha / omega, il = ith * lam[0];
+  for (int64_t i = i0; i < w.n; i += (int64_t)w.nb * KBS) {
+    const double p = __fma_rn(beta, __fma_rn(-omega, v.q[i], v.p[i]), v.r[i]);
+    v.p[i] = p;
+    y[i] = il * minv[i] * p;
+  }
+}
+
+// q = A phat and the partials of <rhat,q>.
+template <int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_q(BellView M, MgGrid g, const double* __restrict__ A, MgVec v, KrylovWork w,
+                                                         int order) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  __shared__ double sh[MgShape<P>::BS / 64];
+  const int dn = w.sc->done;
+  int r;
+  double acc, d[1] = {0.0};
+  if (mg_row<double, true, P>(M, g, A, v.phat, order, r, acc, red)) {
+    v.q[r] = acc;
+    d[0] = v.rhat[r] * acc;
+  }
+  if (dn) return;  // uniform over the grid; q is not read any more
+  put_partials<MgShape<P>::BS, 1>(d, {PS_RQ}, w.partial, w.ps, sh);
+}
+
+// alpha, s = r - alpha q and the cycle's first iterate for M s.
+__global__ void __launch_bounds__(KBS) k_mgb_s(MgVec v, KrylovWork w, int par, int nbs, const double* __restrict__ minv,
+                                              double* __restrict__ y, double ith, const double* __restrict__ lam) {
+  __shared__ double sh[KBS / 64];
+  KrylovScalars* sc = w.sc;
+  if (sc->done) return;
+  double sums[1];
+  mg_sums<1>(w.partial, {PS_RQ}, nbs, w.ps, sh, sums);
+  const double alpha = sc->rho2[par] / sums[0], il = ith * lam[0];
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->alpha2[par] = alpha;
+  for (int64_t i = (int64_t)blockIdx.x * KBS + threadIdx.x; i < w.n; i += (int64_t)w.nb * KBS) {
+    const double s = __fma_rn(-alpha, v.q[i], v.r[i]);
+    v.s[i] = s;
+    y[i] = il * minv[i] * s;
+  }
+}
+
+// t = A shat and the partials of <s,s>, <t,s>, <t,t>.
+template <int P>
+__global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_t(BellView M, MgGrid g, const double* __restrict__ A, MgVec v, KrylovWork w,
+                                                         int order) {
+  __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
+  __shared__ double sh[3 * (MgShape<P>::BS / 64)];
+  const int dn = w.sc->done;
+  int r;
+  double acc, d[3] = {0.0, 0.0, 0.0};
+  if (mg_row<double, true, P>(M, g, A, v.shat, order, r, acc, red)) {
+    const double s = v.s[r];
+    v.t[r] = acc;
+    d[0] = s * s;
+    d[1] = acc * s;
+    d[2] = acc * acc;
+  }
+  if (dn) return;  // uniform over the grid; t is not read any more
+  put_partials<MgShape<P>::BS, 3>(d, {PS_SS, PS_TS, PS_TT}, w.partial, w.ps, sh);
+}
+
+// omega, x and r, and the partials of <r,r> and <rhat,r>.
+__global__ void __launch_bounds__(KBS) k_mgb_xr(MgVec v, KrylovWork w, int par, int nbs) {
+  __shared__ double sh[3 * (KBS / 64)];
+  KrylovScalars* sc = w.sc;
+  if (sc->done) return;
+  const double alpha = sc->alpha2[par], atol2 = sc->atol2;
+  double sums[3];
+  mg_sums<3>(w.partial, {PS_SS, PS_TS, PS_TT}, nbs, w.ps, sh, sums);
+  const double omega = sums[1] / sums[2];
+  const bool early = sums[0] < atol2;
+  if (blockIdx.x == 0 && threadIdx.x == 0) sc->omega2[par] = omega;
+  double rr = 0.0, rhr = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * KBS + threadIdx.x; i < w.n; i += (int64_t)w.nb * KBS) {
+    const double s = v.s[i];
+    double r;
+    if (early) {
+      v.x[i] += alpha * v.phat[i];
+      r = s;
+    } else {
+      v.x[i] += alpha * v.phat[i] + omega * v.shat[i];
+      r = s - omega * v.t[i];
+    }
+    v.r[i] = r;
+    rr += r * r;
+    rhr += v.rhat[i] * r;
+  }
+  // (k_mgb_p adds the first w.nb partials only: nothing to clear)
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const double t0 = wave_sum(rr), t1 = wave_sum(rhr);
+  if (lane == 0) {
+    sh[wid] = t0;
+    sh[KBS / 64 + wid] = t1;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+#pragma unroll
+    for (int i = 0; i < KBS / 64; ++i) t += sh[threadIdx.x * (KBS / 64) + i];
+    w.partial[(threadIdx.x ? PS_RHR : PS_RR) * w.ps + blockIdx.x] = t;
+  }
+}
+
+void mg_krylov_init(const Multigrid& mg, const BellView& M, const double* vals, const double* b, MgVec v, KrylovWork w,
+                    double tol, double atol, int maxiter, hipStream_t st) {
+  const MgGrid g = mg.lv[0].g;
+  if (level_parts(g.n) == 1)
+    hipLaunchKernelGGL(k_mgb_init<1>, dim3((unsigned)w.nbs), dim3(MgShape<1>::BS), 0, st, M, g, vals, b, v, w, level_order(g.n, 0));
+  else
+    hipLaunchKernelGGL(k_mgb_init<3>, dim3((unsigned)w.nbs), dim3(MgShape<3>::BS), 0, st, M, g, vals, b, v, w, level_order(g.n, 0));
+  hipLaunchKernelGGL(k_mgb_init2, dim3(1), dim3(KBS), 0, st, w, tol, atol, maxiter);
+}
+
+template <typename TM>
+void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w,
+                         int iter, uint64_t* flag, hipStream_t st, Prof* prof) {
+  const MgLevel& L = mg.lv[0];
+  const MgGrid g = L.g;
+  const double ith = cheb(DEG_FINE, 0.1).ith;
+  const bool one = level_parts(g.n) == 1;
+  const dim3 vb((unsigned)w.nb), vt(KBS), sb((unsigned)w.nbs), s1(MgShape<1>::BS), s3(MgShape<3>::BS);
+  const int32_t* done = &w.sc->done;
+  const int par = iter & 1;
+  int pass = 1;  // the product that comes before walked forwards
+  timed(prof, PC_KVEC, k_mgb_p, vb, vt, st, v, w, par, iter, (const double*)L.minv, L.x0, ith, (const double*)mg.lam, flag);
+  vcycle<TM>(mg, M, valsp, v.invd, v.p, v.phat, done, &pass, st, prof);
+  if (one)
+    timed(prof, PC_SPMV, k_mgb_q<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
+  else
+    timed(prof, PC_SPMV, k_mgb_q<3>, sb, s3, st, M, g, vals, v, w, level_order(g.n, pass++));
+  timed(prof, PC_KVEC, k_mgb_s, vb, vt, st, v, w, par, w.nbs, (const double*)L.minv, L.x0, ith, (const double*)mg.lam);
+  vcycle<TM>(mg, M, valsp, v.invd, v.s, v.shat, done, &pass, st, prof);
+  if (one)
+    timed(prof, PC_SPMV, k_mgb_t<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
+  else
+    timed(prof, PC_SPMV, k_mgb_t<3>, sb, s3, st, M, g, vals, v, w, level_order(g.n, pass++));
+  timed(prof, PC_KVEC, k_mgb_xr, vb, vt, st, v, w, par, w.nbs);
+}
+
+#define CPFEM_MG_INST(TM)                                                                                                   \
+  template void mg_setup<TM>(const Multigrid&, const double*, const double*, const uint8_t*, double*, hipStream_t);         \
+  template void mg_krylov_iteration<TM>(const Multigrid&, const BellView&, const double*, const TM*, MgVec, KrylovWork, int, \
+                                        uint64_t*, hipStream_t, Prof*);
+CPFEM_MG_INST(double)
+CPFEM_MG_INST(float)
+
+}  // namespace cpfem
