@@ -111,6 +111,9 @@ struct cpfem_ctx {
   int n_slip = 0, n_slots = 0, uniform = 0;
   SlipTable<12> tab12{};
   SlipTable<24> tab24{};
+  PointTables<12> pt12{};
+  PointTables<24> pt24{};
+  void* d_tab = nullptr;  // the general form's slip table
   std::vector<int32_t> h_nslot, h_col, h_dslot;
   std::vector<double> h_sg, h_jxw;  // full per-cell geometry (host copy)
   // device: mesh and maps
@@ -125,7 +128,8 @@ struct cpfem_ctx {
   double* d_ubar = nullptr;
   // device: element work buffers
   double *d_wP = nullptr, *d_wA = nullptr, *d_KE = nullptr, *d_RE = nullptr, *d_sig = nullptr;
-  double* d_gi = nullptr;     // 1/g_old table of the Newton point kernel (allocated on first use)
+  double* d_gi = nullptr;     // scratch of the point kernels' general form (allocated on first use)
+  int64_t gi_points = 0;      // points it holds
   double* d_sconv = nullptr;  // converged stresses [6][n_qp] for the tangent kernel (Jacobian assemblies)
   int32_t* d_status = nullptr;
   unsigned long long* d_counts = nullptr;  // [0] local Newton iterations, [1] residual evaluations, [2] parked points
@@ -468,10 +472,18 @@ static int ensure_matrix_buffers(cpfem_ctx* c) {
   return CPFEM_OK;
 }
 
-// 1/g_old table of the Newton point kernel ([n_slip][n_qp]), allocated on first use
-static int ensure_point_scratch(cpfem_ctx* c) {
+// Scratch of the point kernels' general form for n points: 1/g_old ([n_slip][n]) and, where lanes
+// share a point, d dgamma / d tau as well.  Grows to the largest batch (hipFree waits for the
+// kernels that use the old one).
+static int ensure_point_scratch(cpfem_ctx* c, int64_t n) {
+  if (c->d_gi && c->gi_points >= n) return CPFEM_OK;
+  dfree(c->d_gi);
+  c->gi_points = 0;
+  // lanes share a point below a fixed count only: beyond it one table is enough
+  const int64_t doubles = std::max<int64_t>(c->n_slip * n, 2 * c->n_slip * std::min<int64_t>(n, SHARED_POINTS));
   int rc;
-  if (!c->d_gi && (rc = dalloc(&c->d_gi, (size_t)c->n_slip * c->n_qp))) return rc;
+  if ((rc = dalloc(&c->d_gi, (size_t)doubles))) return rc;
+  c->gi_points = n;
   return CPFEM_OK;
 }
 
@@ -829,8 +841,21 @@ int cpfem_create(const CpfemMesh* mesh, const CpfemSlip* slip, cpfem_ctx** out) 
         c->tab24.n[a][d] = slip->normals[3 * a + d];
       }
     }
+  c->pt12.crystal = make_slip_sys(c->tab12, &c->pt12.sys) ? 1 : 0;
+  c->pt24.crystal = make_slip_sys(c->tab24, &c->pt24.sys) ? 1 : 0;
+  const size_t tab_bytes = slip->n_slip == 12 ? sizeof(c->tab12) : sizeof(c->tab24);
   int rc;
-  if ((rc = dalloc(&c->d_cells, (size_t)8 * c->n_cells))) { cpfem_destroy(c); return rc; }
+  if ((rc = dalloc(&c->d_cells, (size_t)8 * c->n_cells)) || (rc = dalloc((uint8_t**)&c->d_tab, tab_bytes))) {
+    cpfem_destroy(c);
+    return rc;
+  }
+  if (hipMemcpy(c->d_tab, slip->n_slip == 12 ? (const void*)&c->tab12 : (const void*)&c->tab24, tab_bytes, hipMemcpyHostToDevice) !=
+      hipSuccess) {
+    cpfem_destroy(c);
+    return fail(CPFEM_EHIP, "hipMemcpy slip table");
+  }
+  c->pt12.gen = static_cast<const SlipTable<12>*>(c->d_tab);
+  c->pt24.gen = static_cast<const SlipTable<24>*>(c->d_tab);
   if (hipMemcpy(c->d_cells, mesh->cells, (size_t)32 * c->n_cells, hipMemcpyHostToDevice) != hipSuccess) {
     cpfem_destroy(c);
     return fail(CPFEM_EHIP, "hipMemcpy cells");
@@ -879,6 +904,7 @@ void cpfem_destroy(cpfem_ctx* c) {
   if (!c) return;
   (void)hipDeviceSynchronize();
   dfree(c->band.band); dfree(c->band.y); dfree(c->d_ip); dfree(c->d_bflag);
+  dfree(c->d_tab);
   dfree(c->d_cells); dfree(c->d_sg); dfree(c->d_jxw);
   dfree(c->d_col); dfree(c->d_nslot); dfree(c->d_dslot); dfree(c->d_tslot);
   dfree(c->d_cptr); dfree(c->d_clist); dfree(c->d_nptr); dfree(c->d_nlist);
@@ -957,6 +983,7 @@ int cpfem_local(cpfem_ctx* c, void* stream, int64_t n_qp, const double* u_grad, 
     if (n_qp != c->n_qp) return fail(CPFEM_EBADARG, "n_qp must equal 8 * n_cells when u_grad comes from dofs");
   }
   if (n_qp <= 0) return CPFEM_OK;
+  if ((rc = ensure_point_scratch(c, n_qp))) return rc;
   StateOut so{nullptr, nullptr, nullptr};
   if (out) {
     if (!out->Fp_inv || !out->g || !out->slip) return fail(CPFEM_EBADARG, "state_out pointers must all be set");
@@ -971,9 +998,11 @@ int cpfem_local(cpfem_ctx* c, void* stream, int64_t n_qp, const double* u_grad, 
   const SolveCfg cfg = solve_cfg(params);
   const int sl = prof_begin(&c->prof, PC_LOCAL, st);
   if (c->n_slip == 12)
-    launch_local<12>(n_qp, u_grad, G, dofs, sv, mv, c->tab12, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, st);
+    launch_local<12>(n_qp, u_grad, G, dofs, sv, mv, c->pt12, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, c->d_gi,
+                     st);
   else
-    launch_local<24>(n_qp, u_grad, G, dofs, sv, mv, c->tab24, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, st);
+    launch_local<24>(n_qp, u_grad, G, dofs, sv, mv, c->pt24, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, c->d_gi,
+                     st);
   prof_end(&c->prof, sl, st);
   HIPCHK(hipGetLastError());
   return CPFEM_OK;
@@ -985,7 +1014,7 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   int rc;
   if ((rc = check_state(c, state, params))) return rc;
   if (mat && (rc = ensure_matrix_buffers(c))) return rc;
-  if ((rc = ensure_point_scratch(c))) return rc;
+  if ((rc = ensure_point_scratch(c, c->n_qp))) return rc;
   hipStream_t st = (hipStream_t)stream;
   const Geom G = c->geom();
   const StateView sv = state_view(state, c->n_qp);
@@ -1002,24 +1031,26 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   }
   int sl = prof_begin(pf, PC_ELEMENT_QP, st);
   if (c->n_slip == 12)
-    launch_element_qp<12>(G, dofs, sv, mv, c->tab12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
+    launch_element_qp<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
   else
-    launch_element_qp<24>(G, dofs, sv, mv, c->tab24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
+    launch_element_qp<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
   prof_end(pf, sl, st);
   if (pk.lanes > 0) {
     sl = prof_begin(pf, PC_ELEMENT_PARK, st);
     if (c->n_slip == 12)
-      launch_element_qp_park<12>(G, dofs, sv, mv, c->tab12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
+      launch_element_qp_park<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi,
+                               st);
     else
-      launch_element_qp_park<24>(G, dofs, sv, mv, c->tab24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
+      launch_element_qp_park<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi,
+                               st);
     prof_end(pf, sl, st);
   }
   if (mat) {
     sl = prof_begin(pf, PC_TANGENT, st);
     if (c->n_slip == 12)
-      launch_point_tangent<12>(G, dofs, sv, mv, c->tab12, sout, wA, st);
+      launch_point_tangent<12>(G, dofs, sv, mv, c->pt12, sout, wA, c->d_gi, st);
     else
-      launch_point_tangent<24>(G, dofs, sv, mv, c->tab24, sout, wA, st);
+      launch_point_tangent<24>(G, dofs, sv, mv, c->pt24, sout, wA, c->d_gi, st);
     prof_end(pf, sl, st);
   }
   sl = prof_begin(pf, PC_ELEMENT_K, st);

@@ -5,7 +5,7 @@
 
 #include <vector>
 
-#include "cp_point.hpp"
+#include "cp_crystal.hpp"
 
 namespace cpfem {
 
@@ -70,33 +70,47 @@ struct BellView {
 // lanes = 0: no parking.
 struct PointPark {
   int32_t* idx;   // [cap] parked point index
-  double* s;      // [6][cap] its stress iterate (Voigt)
+  double* s;      // [6][cap] its iterate S' (Voigt)
   int32_t* it;    // [cap] iterations done
   uint32_t* ctr;  // [0] parked points, [1] unused
   int64_t cap;
   int lanes;
 };
 
+// Slip-system constants of the point kernels: those of the crystal-frame form by value, the general
+// form's table in device memory; crystal: the former apply (all dyads traceless).
+template <int N>
+struct PointTables {
+  SlipSys<N> sys;
+  const SlipTable<N>* gen;
+  int crystal;
+};
+
+// Lanes that share a point in the point kernels, by slip-system count and number of points: one
+// above SHARED_POINTS points.
+constexpr int64_t SHARED_POINTS = 85000;
+int point_lanes(int n_slip, int64_t n_qp);
+
 // The assembly's point kernels: launch_element_qp runs the local Newton and writes JxW P and,
-// if sout ([6][n_qp]) is set, the converged stress, keeping the 1/g_old table in gi
-// ([N][n_qp] device scratch); launch_point_tangent forms the JxW-weighted consistent tangent
-// wA ([81][n_qp]) from that stress.
+// if sout ([6][n_qp]) is set, the converged S' (points of the general form: the stress);
+// launch_point_tangent forms the JxW-weighted consistent tangent wA ([81][n_qp]) from it.
+// gs: scratch ([n_slip][n_qp], twice that where lanes share a point).
 template <int N>
-void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
+void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                        const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                       unsigned long long* counts, const PointPark& park, double* gi, hipStream_t st);
-// The second kernel over the parked points (grid sized to the device, chunks taken atomically).
+                       unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st);
+// The second kernel over the parked points (the grid covers the longest queue).
 template <int N>
-void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
+void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                             const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                            unsigned long long* counts, const PointPark& park, hipStream_t st);
+                            unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st);
 template <int N>
-void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
-                          const double* sin, double* wA, hipStream_t st);
+void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
+                          const double* sin, double* wA, double* gs, hipStream_t st);
 template <int N>
 void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u, const StateView& sv, const MatView& mv,
-                  const SlipTable<N>& tab, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
-                  const StateOut& so, int32_t* iters, int32_t* status, hipStream_t st);
+                  const PointTables<N>& tb, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
+                  const StateOut& so, int32_t* iters, int32_t* status, double* gs, hipStream_t st);
 void launch_element_K(const Geom& G, const double* wP, const double* wA, double* KE, double* RE, hipStream_t st);
 void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* cptr, const int32_t* clist, const uint8_t* is_bc,
                           double* vals, hipStream_t st);

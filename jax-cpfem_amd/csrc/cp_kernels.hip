@@ -6,6 +6,7 @@
 // models_copper.py:277-278,315): u_grad_q = sum_a u_a (x) dN_a(q);
 // r_e[a,i] = sum_q P_q,ij dN_a,j JxW_q; K_e[a i, b k] = sum_q dN_a,j A_q[ij,kl] dN_b,l JxW_q.
 #include <algorithm>
+#include <type_traits>
 
 #include "cp_internal.hpp"
 
@@ -57,7 +58,7 @@ __device__ __forceinline__ void load_point(const StateView& sv, int64_t q, doubl
   }
 }
 
-constexpr int QBS = 128;  // threads per block of the point kernels (LDS: 2 * N * QBS doubles)
+constexpr int QBS = 128;  // threads per block of the point kernels
 
 // Sum of a 32-bit count over the 64 lanes of a wave (every lane takes part).
 __device__ __forceinline__ uint32_t wave_count(uint32_t v) {
@@ -66,51 +67,72 @@ __device__ __forceinline__ uint32_t wave_count(uint32_t v) {
   return v;
 }
 
-// Point q's inputs: F = I + u_grad from the dofs, Fp_inv_old and R, and the solver set-up
-// (rotated stiffness, 1/g_old in LDS).
-// With gi (a [N][n_qp] device array) the 1/g_old table lives there instead of in LDS, and
-// sh holds only the d dgamma / d tau table.
-template <int N>
-__device__ __forceinline__ void start_point(const Geom& G, const double* __restrict__ u, const StateView& sv,
-                                            const MatView& mv, int64_t q, double* sh, Point<N>& pt, double* F,
-                                            double* Fpi, double* gi = nullptr) {
-  double H[9], R[9];
-  ugrad_from_dofs(G, u, q, H);
+// Point q's inputs: F = I + u_grad, Fp_inv_old, R and the constants.
+struct PointIn {
+  double F[9], Fpi[9], R[9];
+  PointMat m;
+  __device__ __forceinline__ void load(const double* H, const StateView& sv, const MatView& mv, int64_t q) {
 #pragma unroll
-  for (int i = 0; i < 9; ++i) F[i] = H[i] + ((i % 4) == 0 ? 1.0 : 0.0);
-  load_point(sv, q, Fpi, R);
-  const PointMat m = load_mat(mv, q);
-  if (gi)
-    pt.setup(F, Fpi, R, sv.g + q, sv.ld, m, sh + threadIdx.x, gi + q, QBS, G.n_qp);
-  else
-    pt.setup(F, Fpi, R, sv.g + q, sv.ld, m, sh + threadIdx.x, sh + N * QBS + threadIdx.x, QBS);
+    for (int i = 0; i < 9; ++i) F[i] = H[i] + ((i % 4) == 0 ? 1.0 : 0.0);
+    load_point(sv, q, Fpi, R);
+    m = load_mat(mv, q);
+  }
+  __device__ __forceinline__ void load(const Geom& G, const double* __restrict__ u, const StateView& sv, const MatView& mv,
+                                       int64_t q) {
+    double H[9];
+    ugrad_from_dofs(G, u, q, H);
+    load(H, sv, mv, q);
+  }
+};
+
+// The same index, opaque to the compiler: inputs read again behind it are not kept in registers
+// across the Newton iterations.
+__device__ __forceinline__ int64_t reread(int64_t q) {
+  int lo = (int)q, hi = (int)(q >> 32);
+  asm volatile("" : "+v"(lo), "+v"(hi));
+  return ((int64_t)hi << 32) | (uint32_t)lo;
 }
 
-// Outputs of a converged point: JxW P, JxW dP/du_grad (wA), the converged stress (sout,
-// [6][Q]), iterations, status bits.
-template <int N>
-__device__ __forceinline__ void finish_point(const Geom& G, const SlipTable<N>& tab, int64_t q, Point<N>& pt,
-                                             const double* F, const double* Fpi, const double* s, int it, int32_t st,
-                                             double* __restrict__ wP, double* __restrict__ wA,
-                                             int32_t* __restrict__ iters, int32_t* __restrict__ status,
-                                             double* __restrict__ sout = nullptr) {
-  const double w = jxw_at(G, q);
-  double P[9];
-  pk1<N>(pt, F, Fpi, s, P);
-#pragma unroll
-  for (int i = 0; i < 9; ++i) wP[i * G.n_qp + q] = w * P[i];
-  if (sout) {
-#pragma unroll
-    for (int j = 0; j < 6; ++j) sout[j * G.n_qp + q] = s[j];
+// The slip-system constants of a point kernel: its argument where a lane does a whole point (the
+// same system in every lane: scalar loads), a copy in LDS where the lanes of a point take
+// different systems.
+template <int N, int L>
+__device__ __forceinline__ const SlipSys<N>& slip_constants(const SlipSys<N>& arg, SlipSys<N>* lds) {
+  if constexpr (L == 1) {
+    return arg;
+  } else {
+    const double* src = reinterpret_cast<const double*>(&arg);
+    double* dst = reinterpret_cast<double*>(lds);
+    for (int i = threadIdx.x; i < (int)(sizeof(SlipSys<N>) / sizeof(double)); i += QBS) dst[i] = src[i];
+    __syncthreads();
+    return *lds;
   }
-  if (wA) {
-    tangent<N>(pt, tab, F, Fpi, s, [&](int m9, const double* dP) {
-#pragma unroll
-      for (int i = 0; i < 9; ++i) wA[(int64_t)(9 * i + m9) * G.n_qp + q] = w * dP[i];
-    });
-  }
-  if (iters) iters[q] = it;
-  if (st) atomicOr(status, st);
+}
+
+// LDS doubles of a point kernel's block, and the set-up of point q's crystal-frame form: d dgamma /
+// d tau in the lane's LDS column; |1/g_old| behind it where both fit two waves per SIMD, else in
+// the device array gs ([n_slip][n]).
+template <int N, int L>
+constexpr int lds_columns = N / L > 12 ? N / L : 2 * (N / L);
+template <int N, int L>
+__device__ __forceinline__ void setup_crystal(Crystal<N, L>& pt, const PointIn& in, const StateView& sv, int64_t q, int64_t n, int sub,
+                                              double* sh, double* __restrict__ gs) {
+  if (N / L > 12)
+    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, gs + q, QBS, n, sub);
+  else
+    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, sh + (N / L) * QBS + threadIdx.x, QBS, QBS, sub);
+}
+
+// Set-up of the general form (cp_point.hpp) of point q, run by the first of its lanes.  1/g_old in
+// gs ([n_slip][n]), d dgamma / d tau in the lane's LDS column, or behind 1/g_old where the
+// lanes of a point share that.
+template <int N, int L>
+__device__ __forceinline__ void setup_general(Point<N>& pt, const PointIn& in, const StateView& sv, int64_t q, int64_t n,
+                                              double* sh, double* __restrict__ gs) {
+  if (L == 1)
+    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, gs + q, QBS, n);
+  else
+    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, gs + (int64_t)N * n + q, gs + q, (int)n, n);
 }
 
 __device__ __forceinline__ void add_counts(unsigned long long* counts, uint32_t n_it, uint32_t n_ev) {
@@ -123,150 +145,234 @@ __device__ __forceinline__ void add_counts(unsigned long long* counts, uint32_t 
   }
 }
 
-constexpr double DBL_MAXV = 1.7976931348623157e308;
-
 // ---------------------------------------------------------------------------------
 // Quadrature-point kernels of the assembly.  k_element_res: H from dofs, local Newton,
-// JxW-weighted P (SoA [9][Q]) and, for Jacobian assemblies, the converged stress (sout,
-// [6][Q]); k_point_tangent then forms the JxW-weighted consistent tangent ([81][Q]: each of
-// the 81 stores of a wave writes 512 contiguous bytes) from the stored stress.  Without the
-// tangent the Newton kernel fits 256 VGPRs (a few spilled) and keeps the 1/g_old table in a
-// device array instead of LDS, so two waves share a SIMD; the tangent kernel needs ~440 VGPRs
-// (one wave per SIMD) but runs one residual evaluation and the tangent per point, no Newton
-// loop whose lanes wait on each other.  The tangent kernel re-evaluates the residual at the
-// stored stress, which gives bitwise the state the Newton kernel ended with (same inline
-// code, multiply-adds fused per source expression).
+// JxW-weighted P (SoA [9][Q]) and, for Jacobian assemblies, the converged stress (sout, [6][Q]);
+// k_point_tangent then forms the JxW-weighted consistent tangent ([81][Q]: each of the 81
+// stores of a wave writes 512 contiguous bytes) from it, re-evaluating the residual there.  Bound by FP64 VALU issue where the points fill the
+// device, by the serial chain of one point's iterations where they do not: then L lanes share a
+// point (point_lanes).
 // The lanes of a wave run their Newton iterations in lockstep; a wave whose points need very
 // different iteration counts would otherwise run until its slowest lane converges.  With
 // parking (pk.lanes > 0), once at most pk.lanes lanes of the wave are still iterating, those
-// lanes store their point's iterate in the park queue and the wave finishes the others;
+// store their point's iterate in the park queue and the wave finishes the others;
 // k_element_qp_park completes the parked points.  The iterates, and so every output, are the
-// same either way: a parked point resumes from its stored stress with the residual
-// re-evaluated there.  counts (optional): [0] += local Newton iterations, [1] += residual
-// evaluations (one atomic per wave), the measured inputs of the algorithmic flop count.
-template <int N>
-__device__ __forceinline__ void element_qp_body(const Geom& G, const double* __restrict__ u, const StateView& sv,
-                                                const MatView& mv, const SlipTable<N>& tab, const SolveCfg& cfg,
-                                                double* __restrict__ wP, double* __restrict__ sout,
-                                                int32_t* __restrict__ iters, int32_t* __restrict__ status,
-                                                unsigned long long* __restrict__ counts, const PointPark& pk, double* sh,
-                                                double* gi) {
-  const int64_t q = (int64_t)blockIdx.x * QBS + threadIdx.x;
-  const bool valid = q < G.n_qp;
+// same either way: a parked point resumes from its stored S' with the residual re-evaluated
+// there.  counts (optional): [0] += local Newton iterations, [1] += residual evaluations (one
+// atomic per wave), the measured inputs of the algorithmic flop count.
+//
+// Points that the crystal-frame form does not cover (Crystal::applies) take the general one, in a
+// function of its own, so that its registers do not weigh on the others.
+template <int N, int L>
+__device__ __attribute__((noinline)) void general_res(const Geom& G, const double* __restrict__ u, const StateView& sv,
+                                                      const MatView& mv, const SlipTable<N>& tab, const SolveCfg& cfg, int64_t q,
+                                                      double* sh, double* __restrict__ gs, double* __restrict__ wP,
+                                                      double* __restrict__ sout, int32_t* __restrict__ iters,
+                                                      int32_t* __restrict__ status, uint32_t* n_it, uint32_t* n_ev) {
+  PointIn in;
+  in.load(G, u, sv, mv, q);
   Point<N> pt;
-  double F[9], Fpi[9], s[6];
-  int it = 0;
+  double s[6], P[9];
   int32_t st = 0;
+  setup_general<N, L>(pt, in, sv, q, G.n_qp, sh, gs);
+  const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
+  pk1<N>(pt, in.F, in.Fpi, s, P);
+  const double w = jxw_at(G, q);
 #pragma unroll
-  for (int k = 0; k < 6; ++k) s[k] = 0.0;
+  for (int i = 0; i < 9; ++i) wP[i * G.n_qp + q] = w * P[i];
+  if (sout) {
+#pragma unroll
+    for (int j = 0; j < 6; ++j) sout[j * G.n_qp + q] = s[j];
+  }
+  if (iters) iters[q] = it;
+  if (st) atomicOr(status, st);
+  *n_it = (uint32_t)it;
+  *n_ev = (uint32_t)pt.nev;
+}
+
+// Outputs of a converged point: JxW P, the stress, iterations, status bits; each lane writes its
+// share.
+template <int N, int L>
+__device__ __forceinline__ void finish_point(const Geom& G, int64_t q, int sub, const Crystal<N, L>& pt, const PointIn& in,
+                                             const CrystalNewton<N, L>& nw, int32_t st, double* __restrict__ wP,
+                                             double* __restrict__ sout, int32_t* __restrict__ iters,
+                                             int32_t* __restrict__ status) {
+  const double w = jxw_at(G, q);
+  double P[9];
+  crystal_pk1(pt, in.F, in.Fpi, in.R, nw.s, P);
+#pragma unroll
+  for (int i = 0; i < 9; ++i)
+    if (L == 1 || i % L == sub) wP[i * G.n_qp + q] = w * P[i];
+  if (sout) {
+    double s[6];
+    pt.stress(nw.s, in.R, s);
+#pragma unroll
+    for (int j = 0; j < 6; ++j)
+      if (L == 1 || j % L == sub) sout[j * G.n_qp + q] = s[j];
+  }
+  if (sub == 0) {
+    if (iters) iters[q] = nw.it;
+    if (st) atomicOr(status, st);
+  }
+}
+
+template <int N, int L>
+__global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg, const SlipTable<N>* __restrict__ gen,
+              int crystal, SolveCfg cfg, double* __restrict__ wP, double* __restrict__ sout, int32_t* __restrict__ iters,
+              int32_t* __restrict__ status, unsigned long long* __restrict__ counts, PointPark pk, double* __restrict__ gs) {
+  __shared__ double sh[lds_columns<N, L> * QBS];
+  __shared__ SlipSys<L == 1 ? 3 : N> tabs;
+  const SlipSys<N>& tab = slip_constants<N, L>(arg, reinterpret_cast<SlipSys<N>*>(&tabs));
+  const int sub = L == 1 ? 0 : (int)(threadIdx.x % L);
+  const int64_t q = (int64_t)blockIdx.x * (QBS / L) + threadIdx.x / L;
+  const bool valid = q < G.n_qp;
+  Crystal<N, L> pt;
+  CrystalNewton<N, L> nw;
+  int32_t st = 0;
+  bool fits = false, act = false;
   pt.nev = 0;
   pt.nr = 0.0;
+  nw.it = 0;
+  nw.k = 0;
+  nw.lost = false;
   if (valid) {
-    start_point<N>(G, u, sv, mv, q, sh, pt, F, Fpi, gi);
-    pt.eval(tab, s);
+    PointIn in;
+    in.load(G, u, sv, mv, q);
+    fits = crystal && Crystal<N, L>::applies(in.R, in.m);
+    if (fits) {
+      setup_crystal<N, L>(pt, in, sv, q, G.n_qp, sub, sh, gs);
+      act = nw.start(pt, cfg.tol);
+    }
   }
-  bool act = valid && pt.nr > cfg.tol;
   for (;;) {  // wave-uniform exits: every lane sees the same ballot
     const int nact = __popcll(__ballot(act));
     if (nact == 0 || nact <= pk.lanes) break;
-    if (act) {
-      if (it >= cfg.max_iter) {
-        st |= PT_CAPPED;
-        act = false;
-      } else {
-        pt.newton_step(tab, cfg.max_sub_step, s);
-        ++it;
-        act = pt.nr > cfg.tol;
-      }
-    }
+    if (act) act = nw.advance(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
   }
-  const unsigned long long park = __ballot(act);
-  if (park) {  // park the lanes still iterating (one queue reservation per wave)
+  const unsigned long long park = __ballot(act && sub == 0);
+  if (park) {  // park the points still iterating (one queue reservation per wave)
     const int lane = threadIdx.x & 63;
     const int leader = __ffsll(park) - 1;
     uint32_t base = 0;
     if (lane == leader) base = atomicAdd(&pk.ctr[0], (uint32_t)__popcll(park));
     base = __shfl(base, leader, 64);
-    if (act) {
+    if (act && sub == 0) {
       const int64_t k = (int64_t)base + __popcll(park & ((1ull << lane) - 1ull));
       pk.idx[k] = (int32_t)q;
-      pk.it[k] = it;
+      pk.it[k] = nw.k ? nw.it - 1 : nw.it;  // a step whose length is still searched is formed again
 #pragma unroll
-      for (int j = 0; j < 6; ++j) pk.s[j * pk.cap + k] = s[j];
+      for (int j = 0; j < 6; ++j) pk.s[j * pk.cap + k] = nw.s[j];
     }
   }
-  uint32_t n_it = 0;
-  if (valid && !act) {
-    if (!(fabs(pt.nr) <= DBL_MAXV)) st |= PT_NONFINITE;
-    finish_point<N>(G, tab, q, pt, F, Fpi, s, it, st, wP, nullptr, iters, status, sout);
-    n_it = (uint32_t)it;
+  uint32_t n_it = 0, n_ev = fits && sub == 0 ? (uint32_t)pt.nev : 0u;
+  if (fits) fits = !nw.lost;
+  if (fits && !act) {
+    PointIn in;
+    in.load(G, u, sv, mv, reread(q));
+    CrystalNewton<N, L>::finite(pt, &st);
+    finish_point<N, L>(G, q, sub, pt, in, nw, st, wP, sout, iters, status);
+    n_it = sub == 0 ? (uint32_t)nw.it : 0u;
+  } else if (valid && !fits && sub == 0) {
+    // (its residuals here are not counted twice)
+    general_res<N, L>(G, u, sv, mv, *gen, cfg, q, sh, gs, wP, sout, iters, status, &n_it, &n_ev);
   }
-  add_counts(counts, n_it, valid ? (uint32_t)pt.nev : 0u);
+  add_counts(counts, n_it, n_ev);
 }
 
 template <int N>
-__global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipTable<N> tab, SolveCfg cfg,
-              double* __restrict__ wP, double* __restrict__ sout, int32_t* __restrict__ iters,
-              int32_t* __restrict__ status, unsigned long long* __restrict__ counts, PointPark pk,
-              double* __restrict__ gi) {
-  __shared__ double sh[N * QBS];
-  element_qp_body<N>(G, u, sv, mv, tab, cfg, wP, sout, iters, status, counts, pk, sh, gi);
-}
-
-// Consistent tangent of every point from its converged stress sin ([6][Q]).
-template <int N>
-__global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __restrict__ u, StateView sv, MatView mv,
-                                                      SlipTable<N> tab, const double* __restrict__ sin,
-                                                      double* __restrict__ wA) {
-  __shared__ double sh[2 * N * QBS];
-  const int64_t q = (int64_t)blockIdx.x * QBS + threadIdx.x;
-  if (q >= G.n_qp) return;
+__device__ __attribute__((noinline)) void general_tangent(const Geom& G, const double* __restrict__ u, const StateView& sv,
+                                                          const MatView& mv, const SlipTable<N>& tab, int64_t q,
+                                                          const double* __restrict__ sin, double* sh, double* __restrict__ gs,
+                                                          double* __restrict__ wA) {
+  PointIn in;
+  in.load(G, u, sv, mv, q);
   Point<N> pt;
-  double F[9], Fpi[9], s[6];
-  start_point<N>(G, u, sv, mv, q, sh, pt, F, Fpi);
+  double s[6];
 #pragma unroll
   for (int j = 0; j < 6; ++j) s[j] = sin[j * G.n_qp + q];
+  setup_general<N, 1>(pt, in, sv, q, G.n_qp, sh, gs);
   pt.eval(tab, s);
   const double w = jxw_at(G, q);
-  tangent<N>(pt, tab, F, Fpi, s, [&](int m9, const double* dP) {
+  tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
 #pragma unroll
     for (int i = 0; i < 9; ++i) wA[(int64_t)(9 * i + m9) * G.n_qp + q] = w * dP[i];
   });
 }
 
-// The parked points of k_element_res, one queue entry per lane: each point's stress iterate is
+// Consistent tangent of every point from its converged stress (sin, [6][Q]).
+template <int N>
+__global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __restrict__ u, StateView sv, MatView mv,
+                                                      SlipSys<N> tab, const SlipTable<N>* __restrict__ gen, int crystal,
+                                                      const double* __restrict__ sin, double* __restrict__ wA,
+                                                      double* __restrict__ gs) {
+  __shared__ double sh[lds_columns<N, 1> * QBS];
+  const int64_t q = (int64_t)blockIdx.x * QBS + threadIdx.x;
+  if (q >= G.n_qp) return;
+  PointIn in;
+  in.load(G, u, sv, mv, q);
+  bool done = false;
+  if (crystal && Crystal<N>::applies(in.R, in.m)) {
+    double s[6], x[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) s[j] = sin[j * G.n_qp + q];
+    Crystal<N>::pull_back(s, in.R, x);
+    Crystal<N> pt;
+    setup_crystal<N, 1>(pt, in, sv, q, G.n_qp, 0, sh, gs);
+    pt.eval(tab, x);
+    const double w = jxw_at(G, q);
+    done = crystal_tangent(pt, tab, in.F, in.Fpi, in.R, x, [&](int m9, const double* dP) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) wA[(int64_t)(9 * i + m9) * G.n_qp + q] = w * dP[i];
+    });
+  }
+  if (!done) general_tangent<N>(G, u, sv, mv, *gen, q, sin, sh, gs, wA);
+}
+
+// The parked points of k_element_res, one queue entry per point: each point's iterate is
 // restored, its residual re-evaluated there and its Newton iterations continued to
 // convergence.  The grid covers the longest possible queue; blocks past the queue's length
 // (final when this kernel starts: k_element_res ran before it on the same stream) exit at once,
-// so only as many blocks as parked points run, dispatched as earlier blocks retire.  (Looping
-// each wave over the queue instead costs this kernel 64 spilled registers per lane.)
-template <int N>
-__global__ void __launch_bounds__(QBS) k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv,
-                                                        SlipTable<N> tab, SolveCfg cfg, double* __restrict__ wP,
-                                                        double* __restrict__ sout, int32_t* __restrict__ iters,
-                                                        int32_t* __restrict__ status,
-                                                        unsigned long long* __restrict__ counts, PointPark pk) {
-  __shared__ double sh[2 * N * QBS];
+// so only as many blocks as parked points run, dispatched as earlier blocks retire.
+template <int N, int L>
+__global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(2, 2)))
+k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg,
+                  const SlipTable<N>* __restrict__ gen, SolveCfg cfg,
+                  double* __restrict__ wP, double* __restrict__ sout, int32_t* __restrict__ iters, int32_t* __restrict__ status,
+                  unsigned long long* __restrict__ counts, PointPark pk, double* __restrict__ gs) {
+  __shared__ double sh[lds_columns<N, L> * QBS];
+  __shared__ SlipSys<L == 1 ? 3 : N> tabs;
   const uint32_t total = __hip_atomic_load(&pk.ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  if ((int64_t)blockIdx.x * QBS >= (int64_t)total) return;  // uniform over the block
+  if ((int64_t)blockIdx.x * (QBS / L) >= (int64_t)total) return;  // uniform over the block
+  const SlipSys<N>& tab = slip_constants<N, L>(arg, reinterpret_cast<SlipSys<N>*>(&tabs));
   if (counts && blockIdx.x == 0 && threadIdx.x == 0) atomicAdd(&counts[2], (unsigned long long)total);
-  const int64_t k = (int64_t)blockIdx.x * QBS + threadIdx.x;
+  const int sub = L == 1 ? 0 : (int)(threadIdx.x % L);
+  const int64_t k = (int64_t)blockIdx.x * (QBS / L) + threadIdx.x / L;
   uint32_t n_it = 0, n_ev = 0;
   if (k < (int64_t)total) {
     const int64_t q = pk.idx[k];
-    Point<N> pt;
-    double F[9], Fpi[9], s[6];
-    start_point<N>(G, u, sv, mv, q, sh, pt, F, Fpi);
-#pragma unroll
-    for (int j = 0; j < 6; ++j) s[j] = pk.s[j * pk.cap + k];
-    pt.eval(tab, s);
-    int it = pk.it[k];
+    PointIn in;
+    Crystal<N, L> pt;
+    CrystalNewton<N, L> nw;
     int32_t st = 0;
-    pt.iterate(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &it, &st);
-    finish_point<N>(G, tab, q, pt, F, Fpi, s, it, st, wP, nullptr, iters, status, sout);
-    n_it = (uint32_t)it;
-    n_ev = (uint32_t)pt.nev;
+    in.load(G, u, sv, mv, q);
+    setup_crystal<N, L>(pt, in, sv, q, G.n_qp, sub, sh, gs);
+#pragma unroll
+    for (int j = 0; j < 6; ++j) nw.s[j] = pk.s[j * pk.cap + k];
+    nw.it = pk.it[k];
+    bool act = nw.resume(pt, tab, cfg.tol);
+    while (act) act = nw.advance(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
+    if (nw.lost) {
+      if (sub == 0) general_res<N, L>(G, u, sv, mv, *gen, cfg, q, sh, gs, wP, sout, iters, status, &n_it, &n_ev);
+    } else {
+      CrystalNewton<N, L>::finite(pt, &st);
+      in.load(G, u, sv, mv, reread(q));
+      finish_point<N, L>(G, q, sub, pt, in, nw, st, wP, sout, iters, status);
+      if (sub == 0) {
+        n_it = (uint32_t)nw.it;
+        n_ev = (uint32_t)pt.nev;
+      }
+    }
   }
   add_counts(counts, n_it, n_ev);
 }
@@ -427,68 +533,133 @@ __global__ void __launch_bounds__(256) k_element_R(Geom G, const double* __restr
 // ---------------------------------------------------------------------------------
 // Point-level update (tensor_map / update_int_vars_map, models_copper.py:263-269) on explicit
 // u_grad arrays [9][Q] (or from dofs when Hd == nullptr).  Any output pointer may be null.
-template <int N, bool TANGENT>
-__global__ void __launch_bounds__(QBS) k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G,
-                                              const double* __restrict__ u, StateView sv, MatView mv, SlipTable<N> tab,
-                                              SolveCfg cfg, int self_block, double* __restrict__ P_out,
-                                              double* __restrict__ A_out, double* __restrict__ sig_out,
-                                              StateOut so, int32_t* __restrict__ iters, int32_t* __restrict__ status) {
-  __shared__ double sh[2 * N * QBS];
-  const int64_t q = (int64_t)blockIdx.x * QBS + threadIdx.x;
-  if (q >= n_qp) return;
-  double H[9], F[9], Fpi[9], R[9];
+struct LocalOut {
+  double *P, *A, *sig;
+  StateOut so;
+  int32_t *iters, *status;
+};
+
+__device__ __forceinline__ void load_local(PointIn& in, const double* __restrict__ Hd, int64_t n_qp, const Geom& G,
+                                           const double* __restrict__ u, const StateView& sv, const MatView& mv, int64_t q) {
   if (Hd) {
+    double H[9];
 #pragma unroll
     for (int i = 0; i < 9; ++i) H[i] = Hd[i * n_qp + q];
+    in.load(H, sv, mv, q);
   } else {
-    ugrad_from_dofs(G, u, q, H);
+    in.load(G, u, sv, mv, q);
   }
-#pragma unroll
-  for (int i = 0; i < 9; ++i) F[i] = H[i] + ((i % 4) == 0 ? 1.0 : 0.0);
-  load_point(sv, q, Fpi, R);
-  const PointMat m = load_mat(mv, q);
-  double* gps = sh + threadIdx.x;
+}
+
+template <int N, bool TANGENT, int L>
+__device__ __attribute__((noinline)) void general_local(int64_t n_qp, const double* __restrict__ Hd, const Geom& G,
+                                                        const double* __restrict__ u, const StateView& sv, const MatView& mv,
+                                                        const SlipTable<N>& tab, const SolveCfg& cfg, int self_block, int64_t q,
+                                                        const LocalOut& o, double* sh, double* __restrict__ gs) {
+  PointIn in;
+  load_local(in, Hd, n_qp, G, u, sv, mv, q);
   Point<N> pt;
-  pt.setup(F, Fpi, R, sv.g + q, sv.ld, m, gps, sh + N * QBS + threadIdx.x, QBS);
-  double s[6];
+  double s[6], P[9];
   int32_t st = 0;
+  setup_general<N, L>(pt, in, sv, q, n_qp, sh, gs);
   const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
-  double P[9];
-  pk1<N>(pt, F, Fpi, s, P);
-  if (TANGENT && A_out) {  // a separate instantiation: the tangent's registers cost the others occupancy
-    tangent<N>(pt, tab, F, Fpi, s, [&](int m9, const double* dP) {
+  pk1<N>(pt, in.F, in.Fpi, s, P);
+  if (TANGENT && o.A) {
+    tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
 #pragma unroll
-      for (int i = 0; i < 9; ++i) A_out[(9 * i + m9) * n_qp + q] = dP[i];
+      for (int i = 0; i < 9; ++i) o.A[(9 * i + m9) * n_qp + q] = dP[i];
     });
   }
-  if (P_out) {
+  if (o.P) {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) P_out[i * n_qp + q] = P[i];
+    for (int i = 0; i < 9; ++i) o.P[i * n_qp + q] = P[i];
   }
-  if (sig_out) {  // sigma = P F^T / det F (compute_avg_stress, models_copper.py:308-313)
+  if (o.sig) {
     double sg[9];
-    mm3t(P, F, sg);
-    const double idF = 1.0 / det3(F);
+    mm3t(P, in.F, sg);
+    const double idF = 1.0 / det3(in.F);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) sig_out[i * n_qp + q] = sg[i] * idF;
+    for (int i = 0; i < 9; ++i) o.sig[i * n_qp + q] = sg[i] * idF;
   }
-  if (so.Fpi) {  // update_int_vars (models_copper.py:164-169,186-187)
-    double Fn[9];
-    fp_inv_new(Fpi, R, pt.Lpc, Fn);
+  if (o.so.Fpi) {
+    double Fn[9], Sc[9];
+    fp_inv_new(in.Fpi, in.R, pt.Lpc, Fn);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) so.Fpi[i * sv.ld + q] = Fn[i];
-    double Sc[9];
+    for (int i = 0; i < 9; ++i) o.so.Fpi[i * sv.ld + q] = Fn[i];
     pt.crystal_stress(s, Sc);
     for (int a = 0; a < N; ++a) {
       double dg;
       pt.slip_increment(tab, Sc, a, &dg);
-      gps[a * QBS] = dg;
-      so.slip[a * sv.ld + q] = sv.slip[a * sv.ld + q] + dg;
+      pt.gp(a) = dg;
+      o.so.slip[a * sv.ld + q] = sv.slip[a * sv.ld + q] + dg;
     }
-    hardening<N>(sv.g + q, sv.ld, gps, QBS, m, self_block, so.g + q, sv.ld);
+    hardening<N>(sv.g + q, sv.ld, pt.gpv, pt.st, in.m, self_block, o.so.g + q, sv.ld);
   }
-  if (iters) iters[q] = it;
-  if (st) atomicOr(status, st);
+  if (o.iters) o.iters[q] = it;
+  if (st) atomicOr(o.status, st);
+}
+
+template <int N, bool TANGENT, int L>
+__global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(TANGENT ? 1 : 2, TANGENT ? 1 : 2)))
+k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg,
+        const SlipTable<N>* __restrict__ gen, int crystal, SolveCfg cfg, int self_block, LocalOut o, double* __restrict__ gs) {
+  __shared__ double sh[lds_columns<N, L> * QBS];
+  __shared__ SlipSys<L == 1 ? 3 : N> tabs;
+  const SlipSys<N>& tab = slip_constants<N, L>(arg, reinterpret_cast<SlipSys<N>*>(&tabs));
+  const int sub = L == 1 ? 0 : (int)(threadIdx.x % L);
+  const int64_t q = (int64_t)blockIdx.x * (QBS / L) + threadIdx.x / L;
+  if (q >= n_qp) return;
+  PointIn in;
+  load_local(in, Hd, n_qp, G, u, sv, mv, q);
+  Crystal<N, L> pt;
+  CrystalNewton<N, L> nw;
+  int32_t st = 0;
+  bool fits = crystal && Crystal<N, L>::applies(in.R, in.m);
+  if (fits) {
+    setup_crystal<N, L>(pt, in, sv, q, n_qp, sub, sh, gs);
+    fits = nw.solve(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
+  }
+  if (fits) load_local(in, Hd, n_qp, G, u, sv, mv, reread(q));
+  if (TANGENT && fits && o.A) {  // a separate instantiation: the tangent's registers cost the others occupancy
+    fits = crystal_tangent(pt, tab, in.F, in.Fpi, in.R, nw.s, [&](int m9, const double* dP) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) o.A[(9 * i + m9) * n_qp + q] = dP[i];
+    });
+  }
+  if (!fits) {
+    if (sub == 0) general_local<N, TANGENT, L>(n_qp, Hd, G, u, sv, mv, *gen, cfg, self_block, q, o, sh, gs);
+    return;
+  }
+  // every lane of a point writes its share of the components
+  if (o.P || o.sig) {
+    double P[9];
+    crystal_pk1(pt, in.F, in.Fpi, in.R, nw.s, P);
+    if (o.P) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+        if (L == 1 || i % L == sub) o.P[i * n_qp + q] = P[i];
+    }
+    if (o.sig) {  // sigma = P F^T / det F (compute_avg_stress, models_copper.py:308-313)
+      double sg[9];
+      mm3t(P, in.F, sg);
+      const double idF = 1.0 / det3(in.F);
+#pragma unroll
+      for (int i = 0; i < 9; ++i)
+        if (L == 1 || i % L == sub) o.sig[i * n_qp + q] = sg[i] * idF;
+    }
+  }
+  if (o.so.Fpi) {  // update_int_vars (models_copper.py:164-169,186-187)
+    double Fn[9];
+    fp_inv_new(in.Fpi, in.R, pt.Lpc, Fn);
+#pragma unroll
+    for (int i = 0; i < 9; ++i)
+      if (L == 1 || i % L == sub) o.so.Fpi[i * sv.ld + q] = Fn[i];
+    crystal_history(pt, tab, nw.s, in.m, self_block, sv.g + q, sv.slip + q, sv.ld, o.so.g + q, o.so.slip + q);
+  }
+  if (sub == 0) {
+    if (o.iters) o.iters[q] = nw.it;
+    if (st) atomicOr(o.status, st);
+  }
 }
 
 // Cell average of sigma with JxW weights (models_copper.py:315)
@@ -516,42 +687,82 @@ __global__ void k_bc_x0(int64_t n, const uint8_t* __restrict__ is_bc, const doub
 
 // ---------------------------------------------------------------------------------
 // Launch helpers (host)
+
+// Lanes per point: one where the points fill the device (two waves per SIMD hold 131,072 lanes),
+// more where a launch would otherwise be one point's serial chain of iterations in a few waves.
+// Residual calls, us (FCC / BCC24), with 1, 2, 4 and 8 lanes: 4,096 points 119, 95, 67, - / 200, 150,
+// 108, 81; 13,824 points 109, 95, 92, - / 186, 157, 143, 123; 32,768 points 112, 119, 102, - / 190,
+// 201, 158, 180; 64,000 points 153, 133, 174, - / 260, 214, 249, 280; 110,592 points 161, 208, 241, -
+// / 270, 340, 374, 451.
+int point_lanes(int n_slip, int64_t n_qp) {
+  if (n_qp > SHARED_POINTS) return 1;
+  if (n_qp > 48000) return 2;
+  return n_slip == 24 && n_qp <= 20000 ? 8 : 4;
+}
+
 template <int N>
-void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
+void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                        const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                       unsigned long long* counts, const PointPark& park, double* gi, hipStream_t st) {
-  const int64_t nb = (G.n_qp + QBS - 1) / QBS;
-  hipLaunchKernelGGL(k_element_res<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tab, cfg, wP, sout, iters, status,
-                     counts, park, gi);
+                       unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st) {
+  const int L = point_lanes(N, G.n_qp);
+  const dim3 grid((unsigned)((G.n_qp * L + QBS - 1) / QBS)), block(QBS);
+  const auto go = [&](auto lanes) {
+    hipLaunchKernelGGL((k_element_res<N, decltype(lanes)::value>), grid, block, 0, st, G, u, sv, mv, tb.sys, tb.gen, tb.crystal, cfg,
+                       wP, sout, iters, status, counts, park, gs);
+  };
+  if (L == 1) go(std::integral_constant<int, 1>{});
+  if (L == 2) go(std::integral_constant<int, 2>{});
+  if (L == 4) go(std::integral_constant<int, 4>{});
+  if constexpr (N == 24) {
+    if (L == 8) go(std::integral_constant<int, 8>{});
+  }
 }
 
 template <int N>
-void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
+void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                             const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                            unsigned long long* counts, const PointPark& park, hipStream_t st) {
-  const int64_t nb = (park.cap + QBS - 1) / QBS;
-  hipLaunchKernelGGL(k_element_qp_park<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tab, cfg, wP, sout, iters,
-                     status, counts, park);
+                            unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st) {
+  const int L = point_lanes(N, G.n_qp);
+  const dim3 grid((unsigned)((park.cap * L + QBS - 1) / QBS)), block(QBS);
+  const auto go = [&](auto lanes) {
+    hipLaunchKernelGGL((k_element_qp_park<N, decltype(lanes)::value>), grid, block, 0, st, G, u, sv, mv, tb.sys, tb.gen, cfg, wP, sout,
+                       iters, status, counts, park, gs);
+  };
+  if (L == 1) go(std::integral_constant<int, 1>{});
+  if (L == 2) go(std::integral_constant<int, 2>{});
+  if (L == 4) go(std::integral_constant<int, 4>{});
+  if constexpr (N == 24) {
+    if (L == 8) go(std::integral_constant<int, 8>{});
+  }
 }
 
 template <int N>
-void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
-                          const double* sin, double* wA, hipStream_t st) {
+void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
+                          const double* sin, double* wA, double* gs, hipStream_t st) {
   const int64_t nb = (G.n_qp + QBS - 1) / QBS;
-  hipLaunchKernelGGL(k_point_tangent<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tab, sin, wA);
+  hipLaunchKernelGGL(k_point_tangent<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tb.sys, tb.gen, tb.crystal, sin, wA, gs);
 }
 
 template <int N>
 void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u, const StateView& sv, const MatView& mv,
-                  const SlipTable<N>& tab, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
-                  const StateOut& so, int32_t* iters, int32_t* status, hipStream_t st) {
-  const int64_t nb = (n_qp + QBS - 1) / QBS;
-  if (A)
-    hipLaunchKernelGGL((k_local<N, true>), dim3((unsigned)nb), dim3(QBS), 0, st, n_qp, Hd, G, u, sv, mv, tab, cfg, self_block,
-                       P, A, sig, so, iters, status);
-  else
-    hipLaunchKernelGGL((k_local<N, false>), dim3((unsigned)nb), dim3(QBS), 0, st, n_qp, Hd, G, u, sv, mv, tab, cfg,
-                       self_block, P, A, sig, so, iters, status);
+                  const PointTables<N>& tb, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
+                  const StateOut& so, int32_t* iters, int32_t* status, double* gs, hipStream_t st) {
+  const int L = A ? 1 : point_lanes(N, n_qp);
+  const dim3 grid((unsigned)((n_qp * L + QBS - 1) / QBS)), block(QBS);
+  const auto go = [&](auto tangent, auto lanes) {
+    hipLaunchKernelGGL((k_local<N, decltype(tangent)::value, decltype(lanes)::value>), grid, block, 0, st, n_qp, Hd, G, u, sv, mv,
+                       tb.sys, tb.gen, tb.crystal, cfg, self_block, LocalOut{P, A, sig, so, iters, status}, gs);
+  };
+  if (A) {
+    go(std::true_type{}, std::integral_constant<int, 1>{});
+    return;
+  }
+  if (L == 1) go(std::false_type{}, std::integral_constant<int, 1>{});
+  if (L == 2) go(std::false_type{}, std::integral_constant<int, 2>{});
+  if (L == 4) go(std::false_type{}, std::integral_constant<int, 4>{});
+  if constexpr (N == 24) {
+    if (L == 8) go(std::false_type{}, std::integral_constant<int, 8>{});
+  }
 }
 
 void launch_element_K(const Geom& G, const double* wP, const double* wA, double* KE, double* RE, hipStream_t st) {
@@ -598,17 +809,17 @@ void launch_cell_average(const Geom& G, const double* sig, double* out, hipStrea
 }
 
 #define CPFEM_INST(N)                                                                                                      \
-  template void launch_element_qp<N>(const Geom&, const double*, const StateView&, const MatView&, const SlipTable<N>&,    \
+  template void launch_element_qp<N>(const Geom&, const double*, const StateView&, const MatView&, const PointTables<N>&,  \
                                      const SolveCfg&, double*, double*, int32_t*, int32_t*, unsigned long long*,           \
                                      const PointPark&, double*, hipStream_t);                                              \
   template void launch_element_qp_park<N>(const Geom&, const double*, const StateView&, const MatView&,                    \
-                                          const SlipTable<N>&, const SolveCfg&, double*, double*, int32_t*, int32_t*,      \
-                                          unsigned long long*, const PointPark&, hipStream_t);                             \
-  template void launch_point_tangent<N>(const Geom&, const double*, const StateView&, const MatView&, const SlipTable<N>&, \
-                                        const double*, double*, hipStream_t);                                              \
+                                          const PointTables<N>&, const SolveCfg&, double*, double*, int32_t*, int32_t*,    \
+                                          unsigned long long*, const PointPark&, double*, hipStream_t);                    \
+  template void launch_point_tangent<N>(const Geom&, const double*, const StateView&, const MatView&,                      \
+                                        const PointTables<N>&, const double*, double*, double*, hipStream_t);              \
   template void launch_local<N>(int64_t, const double*, const Geom&, const double*, const StateView&, const MatView&,      \
-                                const SlipTable<N>&, const SolveCfg&, int, double*, double*, double*, const StateOut&,     \
-                                int32_t*, int32_t*, hipStream_t);
+                                const PointTables<N>&, const SolveCfg&, int, double*, double*, double*, const StateOut&,   \
+                                int32_t*, int32_t*, double*, hipStream_t);
 CPFEM_INST(12)
 CPFEM_INST(24)
 
