@@ -1111,16 +1111,14 @@ static int ensure_band(cpfem_ctx* c) {
   int32_t bw = 0;
   band_ordering(c->n_nodes, c->h_col.data(), c->h_nslot.data(), ip.data(), &bw);
   BandLU B;
-  B.n = c->n_dofs;
-  B.kl = B.ku = 3 * bw + 2;
-  B.W = B.kl + B.ku + 1;
-  const double bytes = (double)B.n * B.W * sizeof(double);
+  const double bytes = (double)c->n_dofs * (6 * bw + 5) * sizeof(double);  // of the band's entries
   if (bytes > BAND_MAX_BYTES)
     return fail(CPFEM_EBADARG, "direct solve: band storage of " + std::to_string((long long)(bytes / (1 << 20))) +
                                    " MiB exceeds the limit; use the Krylov solver ('jax_solver')");
+  band_shape(B, c->n_dofs, bw, BAND_MAX_BYTES);
   int rc;
-  if ((rc = dalloc(&c->d_ip, (size_t)c->n_nodes)) || (rc = dalloc(&c->d_bflag, 1)) || (rc = dalloc(&B.y, (size_t)B.n)) ||
-      (rc = dalloc(&B.band, (size_t)B.n * B.W)))
+  if ((rc = dalloc(&c->d_ip, (size_t)c->n_nodes)) || (rc = dalloc(&c->d_bflag, 1)) ||
+      (rc = dalloc(&B.y, (size_t)BAND_NB * B.nbk)) || (rc = dalloc(&B.band, (size_t)B.room)))
     return rc;
   HIPCHK(hipMemcpy(c->d_ip, ip.data(), ip.size() * 4, hipMemcpyHostToDevice));
   B.ip = c->d_ip;
@@ -1136,16 +1134,19 @@ int cpfem_solve_direct(cpfem_ctx* c, void* stream, const double* mat, const doub
   int rc;
   if ((rc = ensure_krylov(c, false)) || (rc = ensure_band(c))) return rc;
   hipStream_t st = (hipStream_t)stream;
-  const BandLU& B = c->band;
+  BandLU B = c->band;
   CpfemSolveInfo inf{};
   double bb;
   if ((rc = dot_host(c, st, b, b, &bb))) return rc;
   inf.b_norm = std::sqrt(bb);
-  band_assemble(B, c->bell(), mat, st);
-  band_factor(B, st);
-  HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(c->h_int, c->d_bflag, sizeof(int32_t), hipMemcpyDeviceToHost, st));
-  HIPCHK(hipStreamSynchronize(st));
+  for (;; B.nt = 0) {  // a pivot may vanish from one end of the band and not from the other
+    band_assemble(B, c->bell(), mat, st);
+    band_factor(B, st);
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipMemcpyAsync(c->h_int, c->d_bflag, sizeof(int32_t), hipMemcpyDeviceToHost, st));
+    HIPCHK(hipStreamSynchronize(st));
+    if (c->h_int[0] == 0 || B.nt == 0) break;
+  }
   if (c->h_int[0] != 0) return fail(CPFEM_EDIRECT, "direct solve: zero or non-finite pivot in the unpivoted band LU");
   band_solve(B, b, x, st);
   // x += A^-1 (b - A x), with the residual in FP64 on the block-ELL matrix

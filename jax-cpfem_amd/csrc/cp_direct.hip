@@ -2,17 +2,30 @@
 // ('umfpack_solver' in crystal_plasticity_OR_design/solver.py:100-101, used by
 // calibration_case4_UQ_polyCrystalSteel_1D_GB.py:77,90 on a 20^3 mesh).
 //
-// The block-ELL matrix (Dirichlet rows already replaced by unit rows) is copied into LAPACK-
-// style band storage under a node ordering that keeps the bandwidth small (the mesh's own
-// order or reverse Cuthill-McKee, whichever is narrower), factored in place as A = L U
-// without pivoting (right-looking, panels of BAND_NB columns: the diagonal block in one
-// wave's registers, then L21 = A21 U11^-1 and U12 = L11^-1 A12 one row / column per thread in
-// LDS, then an LDS-tiled trailing update A22 -= L21 U12), and solved with two triangular
-// sweeps of two launches per panel.  FP64 iterative refinement against the block-ELL matrix follows in the
-// caller.  Without pivoting the factorisation exists when every leading principal minor is
-// non-zero, which holds for these stiffness matrices (elastic-plastic tangents close to
-// SPD, unit Dirichlet rows); a zero or non-finite pivot is reported instead of being worked
-// round, and the caller turns it into an error.
+// The block-ELL matrix (Dirichlet rows already replaced by unit rows) is copied, under a node
+// ordering that keeps the bandwidth small (the mesh's own order or reverse Cuthill-McKee,
+// whichever is narrower), into a band of dense NB x NB tiles, factored without pivoting, and
+// solved with matrix-vector sweeps.  FP64 iterative refinement against the block-ELL matrix
+// follows in the caller.  Without pivoting the factorisation exists when the leading principal
+// minors (in the order of elimination) are non-zero, which holds for these stiffness matrices
+// (elastic-plastic tangents close to SPD, unit Dirichlet rows); a zero or non-finite pivot is
+// reported instead of being worked round, and the caller turns it into an error.
+//
+// A band of 1400 half bandwidth gives each pivot block only about a thousand tiles of work, so
+// the solve is bound by the length of the chain of dependent launches, not by operations
+// (20^3: 27783 rows, 107 GFLOP, 1.5 ms at the FP64 rate).  The chain is kept short by
+//  - elimination from both ends of the band at once (two independent fronts, which meet in a
+//    middle part of at least two half bandwidths that the first front then finishes): 239
+//    steps at 20^3 where one front has 435;
+//  - one launch per pivot block: tiles keep A_IK and A_KJ as they are and the inverse of the
+//    pivot block, A_IJ -= (A_IK A_KK^-1) A_KJ, so no launch has to solve the panel first, and
+//    the workgroup that finishes the next diagonal tile inverts it in the same launch;
+//  - sweeps over superblocks of SUP tiles: V_I = A_IS L_S^-1 and Q_J = U_S^-1 A_SJ are formed
+//    once in the factor's place (k_band_super), after which a forward sweep is
+//    y_I -= V_I y_S, one product with each superblock's own inverse, and y_S -= Q_SJ y_J, one
+//    matrix-vector launch per superblock.
+// 20^3 on an MI355X, factor and three solves: 128.6 ms with 32-wide panels from one end (four
+// launches a panel, two per panel in each sweep), 8.2 ms like this (steps 5.7, sweeps 1.8, superblocks 0.55).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -25,249 +38,509 @@
 
 namespace cpfem {
 
-constexpr int BAND_NB = 32;     // panel width
-constexpr int BAND_TILE = 64;   // trailing-update tile (rows x columns)
+constexpr int NB = BAND_NB;
+constexpr int TILE = NB * NB;
+constexpr int SUP = BAND_SUP;
+typedef double v2d __attribute__((ext_vector_type(2)));
+typedef double v4d __attribute__((ext_vector_type(4)));
 
-// Element (i, j) of the band (valid when -kl <= j - i <= ku).
-__device__ __forceinline__ int64_t bidx(int64_t i, int64_t j, int kl, int W) { return i * W + (j - i + kl); }
+// Tile (I, J), row-major, |J - I| <= hw.
+__device__ __forceinline__ double* band_tile(const BandLU& B, int I, int J) {
+  return B.band + ((int64_t)I * (2 * B.hw + 1) + (J - I + B.hw)) * TILE;
+}
 
-// Copy of the block-ELL matrix into the band under the node map ip (old -> new).
-__global__ void k_band_scatter(BellView M, const double* __restrict__ vals, const int32_t* __restrict__ ip,
-                               double* __restrict__ band, int kl, int W) {
+// Copy of the block-ELL matrix into the tiles under the node map ip (old -> new); unit rows
+// fill the last tile.
+__global__ void k_band_scatter(BellView M, const double* __restrict__ vals, BandLU B) {
   const int64_t n = 3 * M.n_nodes;
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
+  if (r >= (int64_t)NB * B.nbk) return;
+  if (r >= n) {
+    band_tile(B, B.nbk - 1, B.nbk - 1)[(r % NB) * (NB + 1)] = 1.0;
+    return;
+  }
   const int64_t i = r / 3;
   const int c = (int)(r - 3 * i);
-  const int64_t R = 3 * (int64_t)ip[i] + c;
+  const int64_t R = 3 * (int64_t)B.ip[i] + c;
+  const int I = (int)(R / NB);
   const int ns = M.nslot[i];
   for (int s = 0; s < ns; ++s) {
     const int64_t j = M.col[(int64_t)s * M.n_nodes + i];
-    const int64_t C0 = 3 * (int64_t)ip[j];
+    const int64_t C0 = 3 * (int64_t)B.ip[j];
 #pragma unroll
-    for (int k = 0; k < 3; ++k) band[bidx(R, C0 + k, kl, W)] = vals[(3 * (int64_t)s + k) * n + r];
+    for (int k = 0; k < 3; ++k)
+      band_tile(B, I, (int)((C0 + k) / NB))[(R % NB) * NB + (C0 + k) % NB] = vals[(3 * (int64_t)s + k) * n + r];
   }
 }
 
-// Diagonal block of panel k0 (nb <= BAND_NB rows and columns): A11 = L11 U11 in registers
-// of one wave, lane p holding row k0+p; the pivot row is broadcast with shuffles.  Entries
-// outside the band are zero and stay zero.
-__global__ void __launch_bounds__(64) k_band_diag(double* __restrict__ band, int kl, int ku, int W, int64_t k0, int nb,
-                                                 int32_t* __restrict__ flag) {
-  const int p = threadIdx.x;
-  double a[BAND_NB];
+// Products of 64 x 64 tiles on the matrix cores (v_mfma_f64_16x16x4: a lane holds A[l % 16][l / 16],
+// B[l / 16][l % 16] and D[4 v + l / 16][l % 16]).  A wave owns 16 rows of the left operand, kept
+// in "operand layout": x[t] = X[l % 16][4 t + l / 16].  That is both the A operand of X M and the
+// B operand of (X M)^T = M^T X^T, and the D of the latter comes out in operand layout again
+// (t = 4 c + v), so chains of right multiplications need no exchange between lanes.  M is read
+// from LDS, where a row-major tile (P = NB) has its columns exchanged in groups of 16 by row, so
+// that the four rows that one read takes lie in different banks.
+__device__ __forceinline__ int lds_swizzle(int r, int c) { return r * NB + (c ^ ((r & 3) << 4)); }
+template <int P, bool CHAIN>
+__device__ __forceinline__ void mul_tile(v4d (&acc)[4], const double (&x)[16], const double* S, int l) {
+  const double* m[4];
 #pragma unroll
-  for (int q = 0; q < BAND_NB; ++q)
-    a[q] = (p < nb && q < nb && q - p <= ku && p - q <= kl) ? band[bidx(k0 + p, k0 + q, kl, W)] : 0.0;
-  bool bad = false;
+  for (int c = 0; c < 4; ++c) m[c] = S + (P == NB ? lds_swizzle(l / 16, 16 * c + l % 16) : (l / 16) * P + 16 * c + l % 16);
+  double e[2][4];
 #pragma unroll
-  for (int c = 0; c < BAND_NB; ++c) {
-    const bool act = c < nb;  // uniform; no early exit, so a[] stays in registers
-    const double piv = __shfl(a[c], c);
-    bad |= act && !(piv != 0.0 && std::isfinite(piv));
-    const double l = act ? a[c] / piv : 0.0;
-    if (act && p > c) a[c] = l;
+  for (int c = 0; c < 4; ++c) e[0][c] = m[c][0];
 #pragma unroll
-    for (int q = c + 1; q < BAND_NB; ++q) {
-      const double u = __shfl(a[q], c);
-      if (act && p > c) a[q] -= l * u;
+  for (int t = 0; t < 16; ++t) {
+    if (t < 15) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) e[(t + 1) & 1][c] = m[c][4 * (t + 1) * P];
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      acc[c] = CHAIN ? __builtin_amdgcn_mfma_f64_16x16x4f64(e[t & 1][c], x[t], acc[c], 0, 0, 0)
+                     : __builtin_amdgcn_mfma_f64_16x16x4f64(x[t], e[t & 1][c], acc[c], 0, 0, 0);
+    // one step of LDS reads ahead is enough; the scheduler would hoist them all, and spill
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+template <int P>
+__device__ __forceinline__ void mul_chain(v4d (&acc)[4], const double (&x)[16], const double* S, int l) {
+  mul_tile<P, true>(acc, x, S, l);
+}
+template <int P>
+__device__ __forceinline__ void mul_last(v4d (&acc)[4], const double (&x)[16], const double* S, int l) {
+  mul_tile<P, false>(acc, x, S, l);
+}
+
+// A tile on its way to LDS: 256 threads, 8 x 16 bytes each.
+struct Stage {
+  v2d v[8];
+  __device__ __forceinline__ void load(const double* g) {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) v[k] = reinterpret_cast<const v2d*>(g)[threadIdx.x + 256 * k];
+  }
+  __device__ __forceinline__ void store(double* S) const {
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int e = 2 * (threadIdx.x + 256 * k);
+      *reinterpret_cast<v2d*>(S + lds_swizzle(e / NB, e % NB)) = v[k];
     }
   }
-  if (p == 0 && bad) flag[0] = 1;
+  template <int P>
+  __device__ __forceinline__ void store_transposed(double* S) const {
 #pragma unroll
-  for (int q = 0; q < BAND_NB; ++q)
-    if (p < nb && q < nb && q - p <= ku && p - q <= kl) band[bidx(k0 + p, k0 + q, kl, W)] = a[q];
-}
-
-// Rows (columns) per block of the L21 (U12) kernels: small blocks spread a panel's ~kl rows
-// over many CUs.
-constexpr int LR_BS = 64;
-
-// L21 = A21 U11^-1: one thread per row below the full panel k0..k0+BAND_NB-1, U11 and each
-// thread's row of panel entries in LDS (register arrays of this size spill).
-__global__ void __launch_bounds__(LR_BS) k_band_lrow(double* __restrict__ band, int64_t n, int kl, int ku, int W, int64_t k0) {
-  __shared__ double U[BAND_NB][BAND_NB + 1];
-  __shared__ double A[BAND_NB][LR_BS + 1];  // A[q][thread]
-  for (int e = threadIdx.x; e < BAND_NB * BAND_NB; e += LR_BS) {
-    const int p = e / BAND_NB, q = e % BAND_NB;
-    U[p][q] = (q >= p && q - p <= ku) ? band[bidx(k0 + p, k0 + q, kl, W)] : 0.0;
-  }
-  const int64_t i0 = k0 + BAND_NB + (int64_t)blockIdx.x * LR_BS, ilast = std::min<int64_t>(n - 1, k0 + BAND_NB - 1 + kl);
-  // rows read and written as contiguous lines: consecutive threads take consecutive columns
-  for (int e = threadIdx.x; e < LR_BS * BAND_NB; e += LR_BS) {
-    const int r = e / BAND_NB, q = e % BAND_NB;
-    const int64_t i = i0 + r;
-    A[q][r] = (i <= ilast && i - (k0 + q) <= kl) ? band[bidx(i, k0 + q, kl, W)] : 0.0;
-  }
-  __syncthreads();
-  const int t = threadIdx.x;
-  if (i0 + t <= ilast) {
-    for (int p = 0; p < BAND_NB; ++p) {
-      double v = A[p][t];
-      for (int q = 0; q < p; ++q) v -= A[q][t] * U[q][p];
-      A[p][t] = v / U[p][p];
+    for (int k = 0; k < 8; ++k) {
+      const int e = 2 * (threadIdx.x + 256 * k), r = e / NB, c = e % NB;
+      S[c * P + r] = v[k].x;
+      S[(c + 1) * P + r] = v[k].y;
     }
   }
-  __syncthreads();
-  for (int e = threadIdx.x; e < LR_BS * BAND_NB; e += LR_BS) {
-    const int r = e / BAND_NB, q = e % BAND_NB;
-    const int64_t i = i0 + r;
-    if (i <= ilast && i - (k0 + q) <= kl) band[bidx(i, k0 + q, kl, W)] = A[q][r];
+};
+
+// Inverse of a tile held by 256 threads in D layout (wave w: a[c][v] is row 16 w + 4 v + l / 16,
+// column 16 c + l % 16), in place, by Gauss-Jordan steps of four pivots: the four pivot rows and
+// columns go through LDS, every lane forms its column of the 4 x 4 pivot block's inverse, and the
+// rank-4 update is one matrix instruction per 16 columns, the tile column of the next pivots
+// first, the others under the next pivot block's elimination.  What bounds it is the chain LDS -
+// four reciprocals - two matrix instructions, 16 times.  Returns whether an entry that the lane
+// holds is not finite, as after a zero or non-finite pivot.
+struct InvLds {
+  double row[2][4][NB];
+  double col[2][NB][4];
+};
+__device__ __forceinline__ bool tile_inverse(v4d (&a)[4], InvLds& s) {
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63, lr = l & 15, lk = l >> 4;
+  const auto put_col = [&](int q) {
+    if (lr / 4 == q % 4) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) s.col[q & 1][16 * w + 4 * v + lk][lr % 4] = a[q / 4][v];
+    }
+  };
+  double nw = 0.0, rk[4] = {};
+  put_col(0);
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    const int pc = q / 4, pv = q % 4, buf = q & 1;  // rows 4q.. are a[.][pv] of wave pc
+    __syncthreads();
+    double p[4][4], u[4], x[4], inv[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) p[i][j] = s.col[buf][4 * q + i][j];
+    const double ci = s.col[buf][16 * w + lr][lk];
+    // x = P^-1 e_{lr % 4} by elimination without exchanges
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = lr % 4 == i ? 1.0 : 0.0;
+    const auto pivot = [&](int k) {
+      inv[k] = fast_rcp(p[k][k]);
+#pragma unroll
+      for (int i = k + 1; i < 4; ++i) {
+        const double f = p[i][k] * inv[k];
+#pragma unroll
+        for (int j = k + 1; j < 4; ++j) p[i][j] -= f * p[k][j];
+        u[i] -= f * u[k];
+      }
+    };
+    // the previous step's update of the tile columns that its successor's pivots did not need
+    if (q > 0) {
+#pragma unroll
+      for (int k = 1; k < 4; ++k) {
+        const int c = (pc + k) % 4;
+        a[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(nw, rk[c], a[c], 0, 0, 0);
+      }
+    }
+    pivot(0);
+    pivot(1);
+    if (w == pc) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) s.row[buf][lk][16 * c + lr] = a[c][pv];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < 4; ++c) rk[c] = s.row[buf][lk][16 * c + lr];
+    pivot(2);
+    pivot(3);
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+      double v = u[i];
+#pragma unroll
+      for (int j = i + 1; j < 4; ++j) v -= p[i][j] * x[j];
+      x[i] = v * inv[i];
+    }
+    // -W^T = P^-T (-A_iP)^T, with rows of the unit matrix in place of -A_iP for the pivot rows
+    // (whose old values go), as a product whose D is in operand layout
+    const bool prow = w == pc && lr / 4 == pv;
+    const double pt = lr >= 4 ? 0.0 : lk == 0 ? x[0] : lk == 1 ? x[1] : lk == 2 ? x[2] : x[3];
+    const v4d zero = {};
+    const v4d wt = __builtin_amdgcn_mfma_f64_16x16x4f64(pt, prow ? (lr % 4 == lk ? 1.0 : 0.0) : -ci, zero, 0, 0, 0);
+    nw = wt[0];
+    if (w == pc) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) a[c][pv] = 0.0;
+    }
+    if (lr / 4 == pv) {
+#pragma unroll
+      for (int v = 0; v < 4; ++v) a[pc][v] = 0.0;
+      rk[pc] = lr % 4 == lk ? 1.0 : 0.0;
+    }
+    const int pn = (q + 1) / 4 % 4;
+    a[pn] = __builtin_amdgcn_mfma_f64_16x16x4f64(nw, rk[pn], a[pn], 0, 0, 0);
+    if (q < 15) {
+      put_col(q + 1);
+    } else {
+#pragma unroll
+      for (int c = 1; c < 4; ++c) a[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(nw, rk[c], a[c], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
+  // a zero or non-finite pivot has a NaN reciprocal (fast_rcp), which reaches every entry
+  double sum = 0.0;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) sum += 0.0 * a[c][v];
+  return sum != 0.0;
 }
 
-// U12 = L11^-1 A12: one thread per column right of the full panel, L11 (unit lower) and each
-// thread's column of panel entries in LDS.
-__global__ void __launch_bounds__(LR_BS) k_band_urow(double* __restrict__ band, int64_t n, int kl, int ku, int W, int64_t k0) {
-  __shared__ double L[BAND_NB][BAND_NB + 1];
-  __shared__ double U[BAND_NB][LR_BS + 1];  // U[p][thread]
-  for (int e = threadIdx.x; e < BAND_NB * BAND_NB; e += LR_BS) {
-    const int p = e / BAND_NB, q = e % BAND_NB;
-    L[p][q] = (q < p && p - q <= kl) ? band[bidx(k0 + p, k0 + q, kl, W)] : 0.0;
-  }
-  const int t = threadIdx.x;
-  const int64_t j = k0 + BAND_NB + (int64_t)blockIdx.x * LR_BS + t;
-  const bool on = j < n && j <= k0 + BAND_NB - 1 + ku;
-  for (int p = 0; p < BAND_NB; ++p) U[p][t] = (on && j - (k0 + p) <= ku) ? band[bidx(k0 + p, j, kl, W)] : 0.0;
-  __syncthreads();
-  if (!on) return;
-  for (int p = 1; p < BAND_NB; ++p) {
-    double v = U[p][t];
-    for (int q = 0; q < p; ++q) v -= L[p][q] * U[q][t];
-    U[p][t] = v;
-  }
-  for (int p = 0; p < BAND_NB; ++p)
-    if (j - (k0 + p) <= ku) band[bidx(k0 + p, j, kl, W)] = U[p][t];
+__device__ __forceinline__ void load_d(v4d (&a)[4], const double* g, int w, int l) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) a[c][v] = g[(16 * w + 4 * v + l / 16) * NB + 16 * c + l % 16];
+}
+__device__ __forceinline__ void store_d(const v4d (&a)[4], double* g, int w, int l) {
+#pragma unroll
+  for (int v = 0; v < 4; ++v)
+#pragma unroll
+    for (int c = 0; c < 4; ++c) g[(16 * w + 4 * v + l / 16) * NB + 16 * c + l % 16] = a[c][v];
 }
 
-// Trailing update A22 -= L21 U12 over BAND_TILE x BAND_TILE tiles (256 threads, 4 x 4 each).
-__global__ void __launch_bounds__(256) k_band_trail(double* __restrict__ band, int64_t n, int kl, int ku, int W, int64_t k0,
-                                                   int nb) {
-  __shared__ double Ls[BAND_TILE][BAND_NB + 1];
-  __shared__ double Us[BAND_NB][BAND_TILE + 1];
-  const int64_t base = k0 + nb;
-  const int64_t i0 = base + (int64_t)blockIdx.y * BAND_TILE, j0 = base + (int64_t)blockIdx.x * BAND_TILE;
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  for (int e = threadIdx.x; e < BAND_TILE * BAND_NB; e += 256) {
-    const int a = e / BAND_NB, p = e % BAND_NB;  // L: row a of the tile, panel column p
-    const int64_t i = i0 + a, c = k0 + p;
-    Ls[a][p] = (p < nb && i < n && i - c <= kl) ? band[bidx(i, c, kl, W)] : 0.0;
-    const int pu = e / BAND_TILE, b = e % BAND_TILE;  // U: panel row pu, column b of the tile
-    const int64_t rr = k0 + pu, j = j0 + b;
-    Us[pu][b] = (pu < nb && j < n && j - rr <= ku) ? band[bidx(rr, j, kl, W)] : 0.0;
+// The first pivot block of each front.
+__global__ void __launch_bounds__(256) k_band_first(BandLU B) {
+  __shared__ InvLds s;
+  const int K = blockIdx.x ? B.nbk - 1 : 0, w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  double* g = band_tile(B, K, K);
+  v4d a[4];
+  load_d(a, g, w, l);
+  if (tile_inverse(a, s)) B.flag[0] = 1;
+  store_d(a, g, w, l);
+}
+
+// Elimination step t of both fronts (blockIdx.y; front 1 runs from the last tile upwards): for
+// the pivot block K, whose tile (K, K) already holds its inverse, A_IJ -= (A_IK A_KK^-1) A_KJ over
+// the cnt x cnt tiles ahead.  Workgroup 0 takes the tile of the next pivot and inverts it; the
+// others take `group` tiles of one row I, so that A_IK A_KK^-1 is formed once for them.
+// The tiles after the current one are loaded under its product.  At cnt = 22 a step of one front
+// takes 19 us, of which the chain through workgroup 0 is 17 (launch 2, loads 1.4, two products 4,
+// inverse 9); two fronts take 25 us, bound by the tiles' traffic (62 MB read and written once).
+__global__ void __launch_bounds__(256, 2) k_band_step(BandLU B, int t, int cnt, int group) {
+  __shared__ double S[2][TILE];
+  const int f = blockIdx.y, dir = f ? -1 : 1, K = f ? B.nbk - 1 - t : t;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  int i = 0, j0 = 0, j1 = 1;
+  if (blockIdx.x > 0) {
+    const int ng = (cnt + group - 1) / group, b = blockIdx.x - 1;
+    i = b / ng;
+    j0 = (b - i * ng) * group;
+    j1 = min(j0 + group, cnt);
+    if (i == 0 && j0 == 0) j0 = 1;
+    if (j0 >= j1) return;
   }
+  const int I = K + dir * (1 + i);
+  Stage st;
+  st.load(band_tile(B, K, K));
+  double x[16];
+  {
+    const double* g = band_tile(B, I, K) + (16 * w + l % 16) * NB + l / 16;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) x[k] = g[4 * k];
+  }
+  st.store(S[0]);
+  st.load(band_tile(B, K, K + dir * (1 + j0)));
+  v4d c[4];
+  load_d(c, band_tile(B, I, K + dir * (1 + j0)), w, l);
   __syncthreads();
-  double acc[4][4] = {};
-#pragma unroll 8
-  for (int p = 0; p < BAND_NB; ++p) {
-    double lv[4], uv[4];
+  {
+    v4d acc[4] = {};
+    mul_chain<NB>(acc, x, S[0], l);
 #pragma unroll
-    for (int a = 0; a < 4; ++a) lv[a] = Ls[ty + 16 * a][p];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) uv[b] = Us[p][tx + 16 * b];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] += lv[a] * uv[b];
+    for (int k = 0; k < 16; ++k) x[k] = -acc[k / 4][k % 4];
   }
-  const int64_t iend = std::min<int64_t>(k0 + nb - 1 + kl, n - 1), jend = std::min<int64_t>(k0 + nb - 1 + ku, n - 1);
+  st.store(S[1]);
+  __syncthreads();
+  if (blockIdx.x > 0) {
+    for (int j = j0, b = 1; j < j1; ++j, b ^= 1) {
+      const int J = K + dir * (1 + j);
+      const bool more = j + 1 < j1;
+      v4d next[4];
+      if (more) {
+        st.load(band_tile(B, K, J + dir));
+        load_d(next, band_tile(B, I, J + dir), w, l);
+      }
+      mul_last<NB>(c, x, S[b], l);
+      store_d(c, band_tile(B, I, J), w, l);
+      if (more) {
+        st.store(S[b ^ 1]);  // last read before the previous barrier
+        __syncthreads();
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int64_t i = i0 + ty + 16 * a;
-    if (i > iend) continue;
+        for (int k = 0; k < 4; ++k) c[k] = next[k];
+      }
+    }
+    return;
+  }
+  mul_last<NB>(c, x, S[1], l);
+  // the second front's last tile belongs to the middle part, which is eliminated later
+  if (!(f == 1 && t == B.nt - 1)) {
+    static_assert(sizeof(InvLds) <= sizeof(S[0]), "");  // S[0] is free since the second barrier
+    if (tile_inverse(c, *reinterpret_cast<InvLds*>(S[0]))) B.flag[0] = 1;
+  }
+  store_d(c, band_tile(B, I, I), w, l);
+}
+
+// Superblock u: its pivot blocks p0 + dir a, a < s, and the number of later blocks it reaches.
+// The first front's come first, then the middle part's, then the second front's.
+struct Super {
+  int p0, dir, s, cnt;
+  __device__ __forceinline__ int block(int a) const { return p0 + dir * a; }
+};
+__device__ __forceinline__ Super band_super(const BandLU& B, int u) {
+  const int na = (B.nt + B.sup - 1) / B.sup, mid = B.nbk - 2 * B.nt, nm = (mid + B.sup - 1) / B.sup;
+  Super S;
+  int off, len;
+  if (u < na || u >= na + nm) {
+    off = (u < na ? u : u - na - nm) * B.sup;
+    len = B.nt;
+    S.p0 = u < na ? off : B.nbk - 1 - off;
+    S.dir = u < na ? 1 : -1;
+  } else {
+    off = (u - na) * B.sup;
+    len = mid;
+    S.p0 = B.nt + off;
+    S.dir = 1;
+  }
+  S.s = min(B.sup, len - off);
+  const int last = S.block(S.s - 1);
+  S.cnt = min(B.wb, S.dir > 0 ? B.nbk - B.nt - 1 - last : last - B.nt);
+  return S;
+}
+
+// V_I = A_IS L_S^-1 (blockIdx.z = 0) and Q_J = U_S^-1 A_SJ (1) for one tile row or column beyond
+// superblock blockIdx.y, in place of A_IS and A_SJ, where L_S has the pivot blocks on its diagonal
+// and U_S units: block back substitution, last pivot first,
+//   V_a = (A_Ia - sum_{m > a} V_m A_ma) D_a^-1,   Q_a = D_a^-1 (A_aJ - sum_{m > a} A_am Q_m).
+// Q is formed transposed, with the tiles of S transposed on their way to LDS.  Bound by the matrix
+// cores: 0.55 ms at 20^3, ten products for each of 4800 strips, 0.32 ms at their FP64 rate.
+template <bool Q>
+__device__ __forceinline__ void super_strip(const BandLU& B, const Super& S, int I, double* sh) {
+  constexpr int P = Q ? NB + 1 : NB;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const auto tile = [&](int r, int c) { return Q ? band_tile(B, c, r) : band_tile(B, r, c); };
+  // operand layout: element (16 w + l % 16, 4 k + l / 16) of the (transposed) strip tile
+  const int o = Q ? (l / 16) * NB + 16 * w + l % 16 : (16 * w + l % 16) * NB + l / 16, os = Q ? 4 * NB : 4;
+  const auto stage = [&](const double* g) {
+    Stage st;
+    st.load(g);
+    __syncthreads();  // the tile before has been read
+    if (Q)
+      st.store_transposed<P>(sh);
+    else
+      st.store(sh);
+    __syncthreads();
+  };
+  double x[SUP][16];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int64_t j = j0 + tx + 16 * b;
-      if (j > jend || j - i > ku || i - j > kl) continue;
-      band[bidx(i, j, kl, W)] -= acc[a][b];
+  for (int a = SUP - 1; a >= 0; --a) {
+    if (a >= S.s) continue;
+    double* g = tile(I, S.block(a));
+    v4d acc[4];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) acc[k / 4][k % 4] = g[o + os * k];
+#pragma unroll
+    for (int m = SUP - 1; m > a; --m) {
+      if (m >= S.s) continue;
+      stage(tile(S.block(m), S.block(a)));
+      mul_chain<P>(acc, x[m], sh, l);
+    }
+    double y[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) y[k] = acc[k / 4][k % 4];
+    stage(band_tile(B, S.block(a), S.block(a)));
+    v4d v[4] = {};
+    mul_chain<P>(v, y, sh, l);
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+      g[o + os * k] = v[k / 4][k % 4];
+      x[a][k] = -v[k / 4][k % 4];
     }
   }
 }
 
-// Triangular sweeps, two launches per panel: one wave solves the panel rows (lane p holds
-// row k0+p with its panel row of L or U preloaded; rows are finalised in order and broadcast
-// by shuffles), then a grid over the rows the panel reaches subtracts the panel's
-// contribution.
-__global__ void __launch_bounds__(64) k_band_fwd_diag(const double* __restrict__ band, double* __restrict__ y, int kl, int W,
-                                                     int64_t k0, int nb) {
-  const int p = threadIdx.x;
-  double lr[BAND_NB];
-#pragma unroll
-  for (int q = 0; q < BAND_NB; ++q) lr[q] = (q < p && p < nb && p - q <= kl) ? band[bidx(k0 + p, k0 + q, kl, W)] : 0.0;
-  double v = p < nb ? y[k0 + p] : 0.0;
-#pragma unroll
-  for (int q = 0; q < BAND_NB; ++q) {
-    const double vq = __shfl(v, q);  // row k0+q is final here
-    v -= lr[q] * vq;
-  }
-  if (p < nb) y[k0 + p] = v;
-}
-
-// 8 lanes per row, 4 consecutive panel columns each (a row's 32 entries are one contiguous
-// 256-byte run), reduced with shuffles; 32 rows per 256-thread block, so a panel's rows spread
-// over many CUs.
-constexpr int UPD_LANES = 8;
-__global__ void __launch_bounds__(256) k_band_fwd_upd(const double* __restrict__ band, double* __restrict__ y, int64_t n, int kl,
-                                                     int W, int64_t k0, int nb) {
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t i = k0 + nb + g / UPD_LANES;
-  const int sub = (int)(g % UPD_LANES);
-  const bool on = i < n && i <= k0 + nb - 1 + kl;
-  double acc = 0.0;
-#pragma unroll
-  for (int c = 0; c < BAND_NB / UPD_LANES; ++c) {
-    const int p = sub * (BAND_NB / UPD_LANES) + c;
-    if (on && p < nb && i - (k0 + p) <= kl) acc += band[bidx(i, k0 + p, kl, W)] * y[k0 + p];
-  }
-#pragma unroll
-  for (int off = UPD_LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, UPD_LANES);
-  if (on && sub == 0) y[i] -= acc;
-}
-
-__global__ void __launch_bounds__(64) k_band_bwd_diag(const double* __restrict__ band, double* __restrict__ y, int kl, int ku,
-                                                     int W, int64_t k0, int nb) {
-  const int p = threadIdx.x;
-  double ur[BAND_NB];
-#pragma unroll
-  for (int q = 0; q < BAND_NB; ++q) ur[q] = (q >= p && q < nb && q - p <= ku) ? band[bidx(k0 + p, k0 + q, kl, W)] : 0.0;
-  double v = p < nb ? y[k0 + p] : 0.0;
-#pragma unroll
-  for (int q = BAND_NB - 1; q >= 0; --q) {
-    if (p == q && p < nb) v /= ur[q];
-    const double vq = __shfl(v, q);  // row k0+q is final here
-    if (p < q) v -= ur[q] * vq;
-  }
-  if (p < nb) y[k0 + p] = v;
-}
-
-__global__ void __launch_bounds__(256) k_band_bwd_upd(const double* __restrict__ band, double* __restrict__ y, int kl, int ku,
-                                                     int W, int64_t k0, int nb) {
-  const int64_t g = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  const int64_t i = std::max<int64_t>(0, k0 - ku) + g / UPD_LANES;
-  const int sub = (int)(g % UPD_LANES);
-  const bool on = i < k0;
-  double acc = 0.0;
-#pragma unroll
-  for (int c = 0; c < BAND_NB / UPD_LANES; ++c) {
-    const int p = sub * (BAND_NB / UPD_LANES) + c;
-    if (on && p < nb && (k0 + p) - i <= ku) acc += band[bidx(i, k0 + p, kl, W)] * y[k0 + p];
-  }
-#pragma unroll
-  for (int off = UPD_LANES / 2; off > 0; off >>= 1) acc += __shfl_xor(acc, off, UPD_LANES);
-  if (on && sub == 0) y[i] -= acc;
-}
-
-// out[new order] = in[old order] (dir = 0) or out[old] = in[new] (dir = 1), dof-wise.
-__global__ void k_band_perm(int64_t nn, const int32_t* __restrict__ ip, const double* __restrict__ in,
-                            double* __restrict__ out, int dir) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= 3 * nn) return;
-  const int64_t i = r / 3;
-  const int64_t R = 3 * (int64_t)ip[i] + (r - 3 * i);
-  if (dir == 0)
-    out[R] = in[r];
+__global__ void __launch_bounds__(256, 2) k_band_super(BandLU B) {
+  __shared__ double sh[NB * (NB + 1)];
+  const Super S = band_super(B, blockIdx.y);
+  if ((int)blockIdx.x >= S.cnt) return;
+  const int I = S.block(S.s + blockIdx.x);
+  if (blockIdx.z)
+    super_strip<true>(B, S, I, sh);
   else
-    out[r] = in[R];
+    super_strip<false>(B, S, I, sh);
+}
+
+// ---- sweeps: one launch per superblock, 4.9 us each, nearly all of it the launch and one trip to
+// memory (2.9 MB of tiles a front); tile by tile they were four times as many.  16 threads a row, 16 rows a workgroup (4 workgroups a tile row); a thread reads
+// two 16-byte pieces of each tile's row, and all of a launch's reads are in flight together.
+__device__ __forceinline__ double row_dot(const double* row, const double* y, int sub) {
+  double acc = 0.0;
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    const v2d a = reinterpret_cast<const v2d*>(row)[sub + 16 * m];
+    const v2d b = reinterpret_cast<const v2d*>(y)[sub + 16 * m];
+    acc = fma(a.x, b.x, fma(a.y, b.y, acc));
+  }
+  return acc;
+}
+__device__ __forceinline__ double sum16(double v) {
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) v += __shfl_xor(v, off, 16);
+  return v;
+}
+
+// y_I -= V_I y_S for the tile rows that superblock u0 (and, blockIdx.y = 1, u1) reaches.
+__global__ void __launch_bounds__(256) k_band_fwd(BandLU B, int u0, int u1) {
+  const Super S = band_super(B, blockIdx.y ? u1 : u0);
+  const int x = blockIdx.x / 4;
+  if (x >= S.cnt) return;
+  const int I = S.block(S.s + x), r = (blockIdx.x % 4) * 16 + threadIdx.x / 16, sub = threadIdx.x % 16;
+  double acc = 0.0;
+#pragma unroll
+  for (int a = 0; a < SUP; ++a)
+    if (a < S.s) acc += row_dot(band_tile(B, I, S.block(a)) + r * NB, B.y + (int64_t)NB * S.block(a), sub);
+  acc = sum16(acc);
+  if (sub == 0) B.y[(int64_t)NB * I + r] -= acc;
+}
+
+// y_S = A_SS^-1 y_S (of the partly eliminated matrix) for every superblock: forward and backward
+// substitution over its tiles.
+__global__ void __launch_bounds__(256) k_band_mid(BandLU B) {
+  __shared__ double y[SUP][NB];
+  __shared__ double z[NB];
+  const Super S = band_super(B, blockIdx.x);
+  const int tid = threadIdx.x, sub = tid % 16;
+  for (int e = tid; e < NB * S.s; e += 256) y[e / NB][e % NB] = B.y[(int64_t)NB * S.block(e / NB) + e % NB];
+  __syncthreads();
+  // z = (accumulated rows of tile row a), then y_a from D_a^-1 z
+  const auto times = [&](const double* g, const double* v, int k) { return row_dot(g + (16 * k + tid / 16) * NB, v, sub); };
+  for (int a = 0; a < S.s; ++a) {
+    for (int k = 0; k < 4; ++k) {
+      double acc = 0.0;
+      for (int j = 0; j < a; ++j) acc += times(band_tile(B, S.block(a), S.block(j)), y[j], k);
+      acc = sum16(acc);
+      if (sub == 0) z[16 * k + tid / 16] = y[a][16 * k + tid / 16] - acc;
+    }
+    __syncthreads();
+    for (int k = 0; k < 4; ++k) {
+      const double v = sum16(times(band_tile(B, S.block(a), S.block(a)), z, k));
+      if (sub == 0) y[a][16 * k + tid / 16] = v;
+    }
+    __syncthreads();
+  }
+  for (int a = S.s - 2; a >= 0; --a) {
+    for (int k = 0; k < 4; ++k) {
+      double acc = 0.0;
+      for (int j = a + 1; j < S.s; ++j) acc += times(band_tile(B, S.block(a), S.block(j)), y[j], k);
+      acc = sum16(acc);
+      if (sub == 0) z[16 * k + tid / 16] = acc;
+    }
+    __syncthreads();
+    for (int k = 0; k < 4; ++k) {
+      const double v = sum16(times(band_tile(B, S.block(a), S.block(a)), z, k));
+      if (sub == 0) y[a][16 * k + tid / 16] -= v;
+    }
+    __syncthreads();
+  }
+  for (int e = tid; e < NB * S.s; e += 256) B.y[(int64_t)NB * S.block(e / NB) + e % NB] = y[e / NB][e % NB];
+}
+
+// y_K -= Q_KJ y_J for the tile rows K that reach superblock u0 (blockIdx.y = 1: u1) and were
+// eliminated before it: those behind it within hw, and, for a superblock of the middle part, those
+// of the second front too.  Tiles between a superblock's reach and hw are zero.
+__global__ void __launch_bounds__(256) k_band_bwd(BandLU B, int u0, int u1) {
+  const Super S = band_super(B, blockIdx.y ? u1 : u0);
+  const int x = blockIdx.x / 4;
+  const bool mid = S.p0 >= B.nt && S.p0 < B.nbk - B.nt;
+  int K;
+  if (x < B.hw)
+    K = S.p0 - S.dir * (1 + x);
+  else {
+    K = B.nbk - B.nt + x - B.hw;
+    if (!mid || K - S.block(S.s - 1) > B.hw) return;
+  }
+  if (K < 0 || K >= B.nbk) return;
+  const int r = (blockIdx.x % 4) * 16 + threadIdx.x / 16, sub = threadIdx.x % 16;
+  double acc = 0.0;
+#pragma unroll
+  for (int a = 0; a < SUP; ++a) {
+    const int J = S.block(a);
+    if (a < S.s && abs(K - J) <= B.hw) acc += row_dot(band_tile(B, K, J) + r * NB, B.y + (int64_t)NB * J, sub);
+  }
+  acc = sum16(acc);
+  if (sub == 0) B.y[(int64_t)NB * K + r] -= acc;
+}
+
+// y[new order] = in[old order], zeros beyond the matrix (dir = 0) or out[old] = y[new] (dir = 1),
+// dof-wise.
+__global__ void k_band_perm(BandLU B, const double* __restrict__ in, double* __restrict__ out, int dir) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= B.n) {
+    if (dir == 0 && r < (int64_t)NB * B.nbk) B.y[r] = 0.0;
+    return;
+  }
+  const int64_t i = r / 3;
+  const int64_t R = 3 * (int64_t)B.ip[i] + (r - 3 * i);
+  if (dir == 0)
+    B.y[R] = in[r];
+  else
+    out[r] = B.y[R];
 }
 
 // ---------------------------------------------------------------------------------- host
@@ -360,50 +633,54 @@ int band_ordering(int64_t nn, const int32_t* col, const int32_t* nslot, int32_t*
   return 0;
 }
 
+void band_shape(BandLU& B, int64_t n, int bw, double cap) {
+  B.n = n;
+  const int kl = 3 * bw + 2;
+  B.nbk = (int)((n + NB - 1) / NB);
+  B.wb = std::min((kl + NB - 1) / NB, B.nbk - 1);
+  // a superblock's last tile reaches wb tiles on, and its first tile's row and column then store
+  // that far too; where that room is above the cap, sweeps go tile by tile
+  for (int sup : {SUP, 1}) {
+    B.sup = sup;
+    B.hw = B.wb + sup - 1;
+    B.room = (int64_t)B.nbk * (2 * B.hw + 1) * TILE;
+    if ((double)B.room * sizeof(double) <= cap) break;
+  }
+  B.nt = std::max(0, (B.nbk - 2 * B.wb) / 2);
+}
+
 void band_assemble(const BandLU& B, const BellView& M, const double* vals, hipStream_t st) {
-  (void)hipMemsetAsync(B.band, 0, (size_t)B.n * B.W * sizeof(double), st);
-  hipLaunchKernelGGL(k_band_scatter, dim3((unsigned)((B.n + 255) / 256)), dim3(256), 0, st, M, vals, B.ip, B.band, B.kl, B.W);
+  (void)hipMemsetAsync(B.band, 0, (size_t)B.room * sizeof(double), st);
+  hipLaunchKernelGGL(k_band_scatter, dim3((unsigned)((NB * (int64_t)B.nbk + 255) / 256)), dim3(256), 0, st, M, vals, B);
 }
 
 void band_factor(const BandLU& B, hipStream_t st) {
   (void)hipMemsetAsync(B.flag, 0, sizeof(int32_t), st);
-  for (int64_t k0 = 0; k0 < B.n; k0 += BAND_NB) {
-    const int nb = (int)std::min<int64_t>(BAND_NB, B.n - k0);
-    hipLaunchKernelGGL(k_band_diag, dim3(1), dim3(64), 0, st, B.band, B.kl, B.ku, B.W, k0, nb, B.flag);
-    const int64_t rest = B.n - (k0 + nb);
-    if (rest <= 0) break;  // only the last panel is narrower than BAND_NB
-    // rows k0+nb .. k0+nb-1+kl and columns k0+nb .. k0+nb-1+ku reach the panel
-    const int64_t ncol = std::min<int64_t>(rest, B.ku), nrow = std::min<int64_t>(rest, B.kl);
-    hipLaunchKernelGGL(k_band_lrow, dim3((unsigned)((nrow + LR_BS - 1) / LR_BS)), dim3(LR_BS), 0, st, B.band, B.n, B.kl, B.ku,
-                       B.W, k0);
-    hipLaunchKernelGGL(k_band_urow, dim3((unsigned)((ncol + LR_BS - 1) / LR_BS)), dim3(LR_BS), 0, st, B.band, B.n, B.kl, B.ku,
-                       B.W, k0);
-    const dim3 grid((unsigned)((ncol + BAND_TILE - 1) / BAND_TILE), (unsigned)((nrow + BAND_TILE - 1) / BAND_TILE));
-    hipLaunchKernelGGL(k_band_trail, grid, dim3(256), 0, st, B.band, B.n, B.kl, B.ku, B.W, k0, nb);
+  hipLaunchKernelGGL(k_band_first, dim3(B.nt > 0 ? 2 : 1), dim3(256), 0, st, B);
+  for (int t = 0; t + 1 < B.nbk - B.nt; ++t) {
+    const int fronts = t < B.nt ? 2 : 1, cnt = std::min(B.wb, B.nbk - B.nt - 1 - t);
+    // tiles of a row per workgroup: the fewest that leave each CU one workgroup, at most 8 (cnt =
+    // 22, two fronts: 5; with 4, 266 workgroups share CUs and a step takes 35 us instead of 29)
+    int group = 1;
+    while (group < 8 && fronts * (1 + cnt * ((cnt + group - 1) / group)) > 256) ++group;
+    hipLaunchKernelGGL(k_band_step, dim3(1 + cnt * ((cnt + group - 1) / group), fronts), dim3(256), 0, st, B, t, cnt, group);
   }
+  const int na = (B.nt + B.sup - 1) / B.sup, nm = (B.nbk - 2 * B.nt + B.sup - 1) / B.sup;
+  if (B.wb > 0) hipLaunchKernelGGL(k_band_super, dim3(B.wb, 2 * na + nm, 2), dim3(256), 0, st, B);
 }
 
 void band_solve(const BandLU& B, const double* b, double* x, hipStream_t st) {
-  const int64_t nn = B.n / 3;
-  const unsigned g = (unsigned)((B.n + 255) / 256);
-  hipLaunchKernelGGL(k_band_perm, dim3(g), dim3(256), 0, st, nn, B.ip, b, B.y, 0);
-  for (int64_t k0 = 0; k0 < B.n; k0 += BAND_NB) {
-    const int nb = (int)std::min<int64_t>(BAND_NB, B.n - k0);
-    hipLaunchKernelGGL(k_band_fwd_diag, dim3(1), dim3(64), 0, st, B.band, B.y, B.kl, B.W, k0, nb);
-    const int64_t rows = std::min<int64_t>(B.kl, B.n - (k0 + nb));
-    if (rows > 0)
-      hipLaunchKernelGGL(k_band_fwd_upd, dim3((unsigned)((rows * UPD_LANES + 255) / 256)), dim3(256), 0, st, B.band, B.y, B.n,
-                         B.kl, B.W, k0, nb);
-  }
-  for (int64_t k0 = ((B.n - 1) / BAND_NB) * BAND_NB; k0 >= 0; k0 -= BAND_NB) {
-    const int nb = (int)std::min<int64_t>(BAND_NB, B.n - k0);
-    hipLaunchKernelGGL(k_band_bwd_diag, dim3(1), dim3(64), 0, st, B.band, B.y, B.kl, B.ku, B.W, k0, nb);
-    const int64_t rows = std::min<int64_t>(B.ku, k0);
-    if (rows > 0)
-      hipLaunchKernelGGL(k_band_bwd_upd, dim3((unsigned)((rows * UPD_LANES + 255) / 256)), dim3(256), 0, st, B.band, B.y, B.kl,
-                         B.ku, B.W, k0, nb);
-  }
-  hipLaunchKernelGGL(k_band_perm, dim3(g), dim3(256), 0, st, nn, B.ip, B.y, x, 1);
+  const unsigned g = (unsigned)((NB * (int64_t)B.nbk + 255) / 256);
+  const int na = (B.nt + B.sup - 1) / B.sup, nm = (B.nbk - 2 * B.nt + B.sup - 1) / B.sup;
+  hipLaunchKernelGGL(k_band_perm, dim3(g), dim3(256), 0, st, B, b, x, 0);
+  // superblocks na + nm + u of the second front go with u of the first
+  for (int u = 0; u + 1 < na + nm; ++u)
+    hipLaunchKernelGGL(k_band_fwd, dim3(4 * B.wb, u < na ? 2 : 1), dim3(256), 0, st, B, u, na + nm + u);
+  hipLaunchKernelGGL(k_band_mid, dim3(2 * na + nm), dim3(256), 0, st, B);
+  for (int u = na + nm - 1; u > 0; --u)
+    hipLaunchKernelGGL(k_band_bwd, dim3(4 * (u < na ? B.hw : B.hw + std::min(B.hw, B.nt)), u < na ? 2 : 1), dim3(256), 0, st, B,
+                       u, na + nm + u);
+  hipLaunchKernelGGL(k_band_perm, dim3(g), dim3(256), 0, st, B, b, x, 1);
 }
 
 }  // namespace cpfem

@@ -275,17 +275,21 @@ void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* v
                          int iter, uint64_t* flag, hipStream_t st, Prof* prof);
 int mg_spmv_blocks(int64_t n);
 
-// Banded LU of the Newton matrix (direct-solve option): n dofs, half bandwidths kl = ku,
-// row-major band of width W = kl + ku + 1 under the node map ip (old -> new), work vector y,
-// pivot flag.
+// Banded LU of the Newton matrix (direct-solve option): n dofs in nbk tiles of BAND_NB, tile
+// half bandwidth wb, stored half bandwidth hw, nt pivot tiles taken from each end (0: one front),
+// sup tiles per superblock of the sweeps, room doubles of tiles at band; node map ip (old ->
+// new), work vector y of nbk tiles, pivot flag.
+constexpr int BAND_NB = 64;
+constexpr int BAND_SUP = 4;
 struct BandLU {
-  int64_t n = 0;
-  int kl = 0, ku = 0, W = 0;
+  int64_t n = 0, room = 0;
+  int nbk = 0, wb = 0, hw = 0, nt = 0, sup = 0;
   double* band = nullptr;
   const int32_t* ip = nullptr;
   double* y = nullptr;
   int32_t* flag = nullptr;
 };
+void band_shape(BandLU& B, int64_t n, int node_bandwidth, double cap);
 int band_ordering(int64_t n_nodes, const int32_t* col, const int32_t* nslot, int32_t* ip, int32_t* bandwidth);
 void band_assemble(const BandLU& B, const BellView& M, const double* vals, hipStream_t st);
 void band_factor(const BandLU& B, hipStream_t st);
