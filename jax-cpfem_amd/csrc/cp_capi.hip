@@ -128,8 +128,6 @@ struct cpfem_ctx {
   double* d_ubar = nullptr;
   // device: element work buffers
   double *d_wP = nullptr, *d_wA = nullptr, *d_KE = nullptr, *d_RE = nullptr, *d_sig = nullptr;
-  double* d_gi = nullptr;     // scratch of the point kernels' general form (allocated on first use)
-  int64_t gi_points = 0;      // points it holds
   double* d_sconv = nullptr;  // converged stresses [6][n_qp] for the tangent kernel (Jacobian assemblies)
   int32_t* d_status = nullptr;
   unsigned long long* d_counts = nullptr;  // [0] local Newton iterations, [1] residual evaluations, [2] parked points
@@ -469,21 +467,6 @@ static int ensure_matrix_buffers(cpfem_ctx* c) {
   if (!c->d_wA && (rc = dalloc(&c->d_wA, (size_t)81 * c->n_qp))) return rc;
   if (!c->d_sconv && (rc = dalloc(&c->d_sconv, (size_t)6 * c->n_qp))) return rc;
   if (!c->d_KE && (rc = dalloc(&c->d_KE, (size_t)576 * c->n_cells))) return rc;
-  return CPFEM_OK;
-}
-
-// Scratch of the point kernels' general form for n points: 1/g_old ([n_slip][n]) and, where lanes
-// share a point, d dgamma / d tau as well.  Grows to the largest batch (hipFree waits for the
-// kernels that use the old one).
-static int ensure_point_scratch(cpfem_ctx* c, int64_t n) {
-  if (c->d_gi && c->gi_points >= n) return CPFEM_OK;
-  dfree(c->d_gi);
-  c->gi_points = 0;
-  // lanes share a point below a fixed count only: beyond it one table is enough
-  const int64_t doubles = std::max<int64_t>(c->n_slip * n, 2 * c->n_slip * std::min<int64_t>(n, SHARED_POINTS));
-  int rc;
-  if ((rc = dalloc(&c->d_gi, (size_t)doubles))) return rc;
-  c->gi_points = n;
   return CPFEM_OK;
 }
 
@@ -909,7 +892,7 @@ void cpfem_destroy(cpfem_ctx* c) {
   dfree(c->d_col); dfree(c->d_nslot); dfree(c->d_dslot); dfree(c->d_tslot);
   dfree(c->d_cptr); dfree(c->d_clist); dfree(c->d_nptr); dfree(c->d_nlist);
   dfree(c->d_isbc); dfree(c->d_nobc); dfree(c->d_ubar);
-  dfree(c->d_gi); dfree(c->d_sconv);
+  dfree(c->d_sconv);
   dfree(c->d_wP); dfree(c->d_wA); dfree(c->d_KE); dfree(c->d_RE); dfree(c->d_sig); dfree(c->d_status); dfree(c->d_counts);
   dfree(c->d_park_idx); dfree(c->d_park_it); dfree(c->d_park_s); dfree(c->d_park_ctr);
   dfree(c->d_partial); dfree(c->d_scalar);
@@ -983,7 +966,6 @@ int cpfem_local(cpfem_ctx* c, void* stream, int64_t n_qp, const double* u_grad, 
     if (n_qp != c->n_qp) return fail(CPFEM_EBADARG, "n_qp must equal 8 * n_cells when u_grad comes from dofs");
   }
   if (n_qp <= 0) return CPFEM_OK;
-  if ((rc = ensure_point_scratch(c, n_qp))) return rc;
   StateOut so{nullptr, nullptr, nullptr};
   if (out) {
     if (!out->Fp_inv || !out->g || !out->slip) return fail(CPFEM_EBADARG, "state_out pointers must all be set");
@@ -998,11 +980,9 @@ int cpfem_local(cpfem_ctx* c, void* stream, int64_t n_qp, const double* u_grad, 
   const SolveCfg cfg = solve_cfg(params);
   const int sl = prof_begin(&c->prof, PC_LOCAL, st);
   if (c->n_slip == 12)
-    launch_local<12>(n_qp, u_grad, G, dofs, sv, mv, c->pt12, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, c->d_gi,
-                     st);
+    launch_local<12>(n_qp, u_grad, G, dofs, sv, mv, c->pt12, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, st);
   else
-    launch_local<24>(n_qp, u_grad, G, dofs, sv, mv, c->pt24, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, c->d_gi,
-                     st);
+    launch_local<24>(n_qp, u_grad, G, dofs, sv, mv, c->pt24, cfg, params->self_block, P, A, sigma, so, iters, c->d_status, st);
   prof_end(&c->prof, sl, st);
   HIPCHK(hipGetLastError());
   return CPFEM_OK;
@@ -1014,7 +994,6 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   int rc;
   if ((rc = check_state(c, state, params))) return rc;
   if (mat && (rc = ensure_matrix_buffers(c))) return rc;
-  if ((rc = ensure_point_scratch(c, c->n_qp))) return rc;
   hipStream_t st = (hipStream_t)stream;
   const Geom G = c->geom();
   const StateView sv = state_view(state, c->n_qp);
@@ -1031,26 +1010,24 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   }
   int sl = prof_begin(pf, PC_ELEMENT_QP, st);
   if (c->n_slip == 12)
-    launch_element_qp<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
+    launch_element_qp<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
   else
-    launch_element_qp<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi, st);
+    launch_element_qp<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
   prof_end(pf, sl, st);
   if (pk.lanes > 0) {
     sl = prof_begin(pf, PC_ELEMENT_PARK, st);
     if (c->n_slip == 12)
-      launch_element_qp_park<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi,
-                               st);
+      launch_element_qp_park<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
     else
-      launch_element_qp_park<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, c->d_gi,
-                               st);
+      launch_element_qp_park<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
     prof_end(pf, sl, st);
   }
   if (mat) {
     sl = prof_begin(pf, PC_TANGENT, st);
     if (c->n_slip == 12)
-      launch_point_tangent<12>(G, dofs, sv, mv, c->pt12, sout, wA, c->d_gi, st);
+      launch_point_tangent<12>(G, dofs, sv, mv, c->pt12, sout, wA, st);
     else
-      launch_point_tangent<24>(G, dofs, sv, mv, c->pt24, sout, wA, c->d_gi, st);
+      launch_point_tangent<24>(G, dofs, sv, mv, c->pt24, sout, wA, st);
     prof_end(pf, sl, st);
   }
   sl = prof_begin(pf, PC_ELEMENT_K, st);

@@ -18,7 +18,9 @@
 //  * dgamma and its derivative come from one power |tau/g|^(1/m - 1), without branches.
 //  * The tangent reuses G's sums sum_a g'_a z_a b_a^T as the derivative of the plastic velocity
 //    gradient, instead of six more loops over the slip systems.
-// dgamma/dtau and 1/g_old live outside the register file, as in Point, and the slip loops are rolled:
+// dgamma/dtau and 1/g_old live outside the register file, in LDS (whose 20 KB a wave at two waves
+// per SIMD hold 1/g_old of 14 of 24 systems) and, for the others, in the lane's private memory, and
+// the slip loops are rolled:
 // unrolled, with dgamma/dtau in registers, the kernels spilled 160 to 240 registers and took
 // twice the time.
 //
@@ -157,10 +159,11 @@ CPFEM_HD double rate_power(double x, double p) {
   return x > 0.0 ? w : x;
 }
 
-template <int N, int L = 1>
+template <int N, int L = 1, int KS = (N / L > 12 ? 14 : N / L)>
 struct Crystal {
   static constexpr int M = N / L;  // slip systems of this lane
   static_assert(N % L == 0 && M % 3 == 0, "a lane takes whole blocks of three slip systems");
+  static constexpr int K = KS;  // how many of them have |1/g_old| in the gi store, the others in gr
   double Ah[9];          // A R
   double B[6];           // R^T R (Voigt)
   double bb, ibb;        // its mean diagonal, and the reciprocal
@@ -168,7 +171,8 @@ struct Crystal {
   double i1, i2, i3;     // inverse: (C^-1 t)_ii = i1 t_ii - i2 tr t, shear i3 t
   double p, p1, c;       // 1/m, 1/m - 1, gamma0 dt
   double* gpv;           // d dgamma / d tau of this lane's systems, stride st
-  const double* gi;      // their |1 / g_old|, stride sti
+  const double* gi;      // |1 / g_old| of the first K, stride sti
+  const double* gr;      // of the others
   int st;
   int64_t sti;
   int a0;                // first slip system of this lane
@@ -194,7 +198,8 @@ struct Crystal {
 
   // Set-up from F, Fp_inv_old, R and the constants; stores |1/g_old| of the lane's systems at gi_store.
   CPFEM_HD void setup(const double* F, const double* Fpi_old, const double* R, const double* g_old, int64_t gstride,
-                      const PointMat& m, double* gp_store, double* gi_store, int stride, int64_t stride_gi, int sub = 0) {
+                      const PointMat& m, double* gp_store, double* gi_store, int stride, int64_t stride_gi, int sub = 0,
+                      double* gr_store = nullptr) {
     {
       double A[9];
       mm3(F, Fpi_old, A);
@@ -223,12 +228,16 @@ struct Crystal {
     st = stride;
     sti = stride_gi;
     a0 = sub * M;
+    gr = gr_store;
     nev = 0;
     double z = 0.0;
 #pragma unroll 3
     for (int j = 0; j < M; ++j) {
       const double v = fabs(1.0 / g_old[(a0 + j) * gstride]);
-      gi_store[j * stride_gi] = v;
+      if (j < K)
+        gi_store[j * stride_gi] = v;
+      else
+        gr_store[j - K] = v;
       z += 0.0 * v;
     }
     zero = lane_sum<L>(z);
@@ -297,17 +306,27 @@ struct Crystal {
 #pragma unroll
     for (int i = 0; i < 8; ++i) l[i] = 0.0;
     const double u0 = x[0] - x[2], u1 = x[1] - x[2];
-    double next = gi[0];
-#pragma unroll 2
-    for (int j = 0; j < M; ++j) {
+    const auto system = [&](int j, double gia) {
       const int a = L == 1 ? j : a0 + j;
       const double t = tab.b[a][0] * u0 + tab.b[a][1] * u1 + tab.b[a][2] * x[3] + tab.b[a][3] * x[4] + tab.b[a][4] * x[5];
-      const double gia = next;
-      next = gi[(j + 1 < M ? j + 1 : j) * sti];  // in flight during this system
       const double y = rate(fabs(t) * gia, gia), dg = y * t;
       gp(j) = p * y;
 #pragma unroll
       for (int i = 0; i < 8; ++i) l[i] += dg * tab.z[a][i];
+    };
+    double rest = K < M ? gr[0] : 0.0;
+    double next = gi[0];
+#pragma unroll 2
+    for (int j = 0; j < K; ++j) {
+      const double gia = next;
+      next = gi[(j + 1 < K ? j + 1 : j) * sti];  // in flight during this system
+      system(j, gia);
+    }
+#pragma unroll 2
+    for (int j = K; j < M; ++j) {
+      const double gia = rest;
+      rest = gr[(j + 1 < M ? j + 1 : j) - K];
+      system(j, gia);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) Lpc[i] = lane_sum<L>(l[i]);
@@ -537,8 +556,8 @@ struct CrystalNewton {
 
 // Kalidindi hardening after convergence (cp_point.hpp's hardening) and the new slips of this lane's
 // systems; x: the converged S'.
-template <int N, int L, class Tab>
-CPFEM_HD void crystal_history(const Crystal<N, L>& pt, const Tab& tab, const double* x, const PointMat& m, int self_block,
+template <int N, int L, int KS, class Tab>
+CPFEM_HD void crystal_history(const Crystal<N, L, KS>& pt, const Tab& tab, const double* x, const PointMat& m, int self_block,
                               const double* g_old, const double* slip_old, int64_t ld, double* g_new, double* slip_new) {
   constexpr int M = N / L;
   double tot = 0.0;
@@ -568,8 +587,8 @@ CPFEM_HD void crystal_history(const Crystal<N, L>& pt, const Tab& tab, const dou
 // First Piola-Kirchhoff stress P = F Y, Y = Ph S' Ph^T / (bb^2 det Fp_inv_new), Ph = Fp_inv_new R, and
 // the consistent tangent's ingredients.  Q = Fp_inv_old R, W = I - bb Lpc: Ph = Q W and
 // det Fp_inv_new = det Fp_inv_old det W.
-template <int N, int L>
-CPFEM_HD void crystal_pk1(const Crystal<N, L>& pt, const double* F, const double* Fpi_old, const double* R, const double* x,
+template <int N, int L, int KS>
+CPFEM_HD void crystal_pk1(const Crystal<N, L, KS>& pt, const double* F, const double* Fpi_old, const double* R, const double* x,
                           double* P) {
   double W[9], Q[9], Ph[9], S[9], U[9], Y[9];
 #pragma unroll
@@ -590,8 +609,8 @@ CPFEM_HD void crystal_pk1(const Crystal<N, L>& pt, const double* F, const double
 //   dP = dH Y + F dY,  dY = Ycal ds'.
 // Column m = 3 k + l (dH = e_k e_l^T) goes to sink(m, dP[9]).  False, and nothing to the sink, if the
 // factorisation needs row exchanges.
-template <int N, int L, class Tab, class Sink>
-CPFEM_HD bool crystal_tangent(const Crystal<N, L>& pt, const Tab& tab, const double* F, const double* Fpi_old, const double* R,
+template <int N, int L, int KS, class Tab, class Sink>
+CPFEM_HD bool crystal_tangent(const Crystal<N, L, KS>& pt, const Tab& tab, const double* F, const double* Fpi_old, const double* R,
                               const double* x, Sink sink) {
   double Ph[9], Yv[9], Yc[36], J[36];
   double f;  // 1 / (bb^2 det Fp_inv_new)

@@ -98,19 +98,19 @@ int point_lanes(int n_slip, int64_t n_qp);
 template <int N>
 void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                        const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                       unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st);
+                       unsigned long long* counts, const PointPark& park, hipStream_t st);
 // The second kernel over the parked points (the grid covers the longest queue).
 template <int N>
 void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                             const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                            unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st);
+                            unsigned long long* counts, const PointPark& park, hipStream_t st);
 template <int N>
 void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
-                          const double* sin, double* wA, double* gs, hipStream_t st);
+                          const double* sin, double* wA, hipStream_t st);
 template <int N>
 void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u, const StateView& sv, const MatView& mv,
                   const PointTables<N>& tb, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
-                  const StateOut& so, int32_t* iters, int32_t* status, double* gs, hipStream_t st);
+                  const StateOut& so, int32_t* iters, int32_t* status, hipStream_t st);
 void launch_element_K(const Geom& G, const double* wP, const double* wA, double* KE, double* RE, hipStream_t st);
 void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* cptr, const int32_t* clist, const uint8_t* is_bc,
                           double* vals, hipStream_t st);

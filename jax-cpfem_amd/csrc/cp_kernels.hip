@@ -109,31 +109,33 @@ __device__ __forceinline__ const SlipSys<N>& slip_constants(const SlipSys<N>& ar
   }
 }
 
-// LDS doubles of a point kernel's block, and the set-up of point q's crystal-frame form: d dgamma /
-// d tau in the lane's LDS column; |1/g_old| behind it where both fit two waves per SIMD, else in
-// the device array gs ([n_slip][n]).
+// LDS doubles per lane of a point kernel, and the set-up of point q's crystal-frame form in the
+// lane's column: d dgamma / d tau and |1/g_old| behind it, what LDS does not hold in private memory
+// (whose address escapes, or the compiler would index it in registers).
 template <int N, int L>
-constexpr int lds_columns = N / L > 12 ? N / L : 2 * (N / L);
-template <int N, int L>
-__device__ __forceinline__ void setup_crystal(Crystal<N, L>& pt, const PointIn& in, const StateView& sv, int64_t q, int64_t n, int sub,
-                                              double* sh, double* __restrict__ gs) {
-  if (N / L > 12)
-    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, gs + q, QBS, n, sub);
-  else
-    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, sh + (N / L) * QBS + threadIdx.x, QBS, QBS, sub);
+constexpr int lds_columns = Crystal<N, L>::M + Crystal<N, L>::K;
+template <int N, int L, int KS = Crystal<N, L>::K>
+struct CrystalRest {
+  static constexpr int n = N / L - KS;
+  double gi[n > 0 ? n : 1];
+};
+template <int N, int L, int KS>
+__device__ __forceinline__ void setup_crystal(Crystal<N, L, KS>& pt, const PointIn& in, const StateView& sv, int64_t q, int sub,
+                                              double* sh, CrystalRest<N, L, KS>& rest) {
+  if (rest.n > 0) asm volatile("" ::"v"(rest.gi) : "memory");
+  pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, sh + Crystal<N, L>::M * QBS + threadIdx.x, QBS, QBS, sub,
+           rest.gi);
 }
 
-// Set-up of the general form (cp_point.hpp) of point q, run by the first of its lanes.  1/g_old in
-// gs ([n_slip][n]), d dgamma / d tau in the lane's LDS column, or behind 1/g_old where the
-// lanes of a point share that.
-template <int N, int L>
-__device__ __forceinline__ void setup_general(Point<N>& pt, const PointIn& in, const StateView& sv, int64_t q, int64_t n,
-                                              double* sh, double* __restrict__ gs) {
-  if (L == 1)
-    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, sh + threadIdx.x, gs + q, QBS, n);
-  else
-    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, gs + (int64_t)N * n + q, gs + q, (int)n, n);
-}
+// d dgamma / d tau and 1/g_old of the general form (cp_point.hpp), in the lane's private memory:
+// the functions that use them are called for the points that nothing else covers.
+template <int N>
+struct GeneralStore {
+  double gp[N], gi[N];
+  __device__ __forceinline__ void setup(Point<N>& pt, const PointIn& in, const StateView& sv, int64_t q) {
+    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, gp, gi, 1, 1);
+  }
+};
 
 __device__ __forceinline__ void add_counts(unsigned long long* counts, uint32_t n_it, uint32_t n_ev) {
   if (!counts) return;
@@ -166,7 +168,7 @@ __device__ __forceinline__ void add_counts(unsigned long long* counts, uint32_t 
 template <int N, int L>
 __device__ __attribute__((noinline)) void general_res(const Geom& G, const double* __restrict__ u, const StateView& sv,
                                                       const MatView& mv, const SlipTable<N>& tab, const SolveCfg& cfg, int64_t q,
-                                                      double* sh, double* __restrict__ gs, double* __restrict__ wP,
+                                                      double* __restrict__ wP,
                                                       double* __restrict__ sout, int32_t* __restrict__ iters,
                                                       int32_t* __restrict__ status, uint32_t* n_it, uint32_t* n_ev) {
   PointIn in;
@@ -174,7 +176,8 @@ __device__ __attribute__((noinline)) void general_res(const Geom& G, const doubl
   Point<N> pt;
   double s[6], P[9];
   int32_t st = 0;
-  setup_general<N, L>(pt, in, sv, q, G.n_qp, sh, gs);
+  GeneralStore<N> store;
+  store.setup(pt, in, sv, q);
   const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
   pk1<N>(pt, in.F, in.Fpi, s, P);
   const double w = jxw_at(G, q);
@@ -220,7 +223,7 @@ template <int N, int L>
 __global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg, const SlipTable<N>* __restrict__ gen,
               int crystal, SolveCfg cfg, double* __restrict__ wP, double* __restrict__ sout, int32_t* __restrict__ iters,
-              int32_t* __restrict__ status, unsigned long long* __restrict__ counts, PointPark pk, double* __restrict__ gs) {
+              int32_t* __restrict__ status, unsigned long long* __restrict__ counts, PointPark pk) {
   __shared__ double sh[lds_columns<N, L> * QBS];
   __shared__ SlipSys<L == 1 ? 3 : N> tabs;
   const SlipSys<N>& tab = slip_constants<N, L>(arg, reinterpret_cast<SlipSys<N>*>(&tabs));
@@ -228,6 +231,7 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
   const int64_t q = (int64_t)blockIdx.x * (QBS / L) + threadIdx.x / L;
   const bool valid = q < G.n_qp;
   Crystal<N, L> pt;
+  CrystalRest<N, L> rest;
   CrystalNewton<N, L> nw;
   int32_t st = 0;
   bool fits = false, act = false;
@@ -241,7 +245,7 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
     in.load(G, u, sv, mv, q);
     fits = crystal && Crystal<N, L>::applies(in.R, in.m);
     if (fits) {
-      setup_crystal<N, L>(pt, in, sv, q, G.n_qp, sub, sh, gs);
+      setup_crystal(pt, in, sv, q, sub, sh, rest);
       act = nw.start(pt, cfg.tol);
     }
   }
@@ -275,7 +279,7 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
     n_it = sub == 0 ? (uint32_t)nw.it : 0u;
   } else if (valid && !fits && sub == 0) {
     // (its residuals here are not counted twice)
-    general_res<N, L>(G, u, sv, mv, *gen, cfg, q, sh, gs, wP, sout, iters, status, &n_it, &n_ev);
+    general_res<N, L>(G, u, sv, mv, *gen, cfg, q, wP, sout, iters, status, &n_it, &n_ev);
   }
   add_counts(counts, n_it, n_ev);
 }
@@ -283,15 +287,15 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
 template <int N>
 __device__ __attribute__((noinline)) void general_tangent(const Geom& G, const double* __restrict__ u, const StateView& sv,
                                                           const MatView& mv, const SlipTable<N>& tab, int64_t q,
-                                                          const double* __restrict__ sin, double* sh, double* __restrict__ gs,
-                                                          double* __restrict__ wA) {
+                                                          const double* __restrict__ sin, double* __restrict__ wA) {
   PointIn in;
   in.load(G, u, sv, mv, q);
   Point<N> pt;
   double s[6];
 #pragma unroll
   for (int j = 0; j < 6; ++j) s[j] = sin[j * G.n_qp + q];
-  setup_general<N, 1>(pt, in, sv, q, G.n_qp, sh, gs);
+  GeneralStore<N> store;
+  store.setup(pt, in, sv, q);
   pt.eval(tab, s);
   const double w = jxw_at(G, q);
   tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
@@ -304,9 +308,8 @@ __device__ __attribute__((noinline)) void general_tangent(const Geom& G, const d
 template <int N>
 __global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __restrict__ u, StateView sv, MatView mv,
                                                       SlipSys<N> tab, const SlipTable<N>* __restrict__ gen, int crystal,
-                                                      const double* __restrict__ sin, double* __restrict__ wA,
-                                                      double* __restrict__ gs) {
-  __shared__ double sh[lds_columns<N, 1> * QBS];
+                                                      const double* __restrict__ sin, double* __restrict__ wA) {
+  __shared__ double sh[2 * N * QBS];  // one wave per SIMD anyway
   const int64_t q = (int64_t)blockIdx.x * QBS + threadIdx.x;
   if (q >= G.n_qp) return;
   PointIn in;
@@ -317,8 +320,9 @@ __global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __r
 #pragma unroll
     for (int j = 0; j < 6; ++j) s[j] = sin[j * G.n_qp + q];
     Crystal<N>::pull_back(s, in.R, x);
-    Crystal<N> pt;
-    setup_crystal<N, 1>(pt, in, sv, q, G.n_qp, 0, sh, gs);
+    Crystal<N, 1, N> pt;
+    CrystalRest<N, 1, N> rest;
+    setup_crystal(pt, in, sv, q, 0, sh, rest);
     pt.eval(tab, x);
     const double w = jxw_at(G, q);
     done = crystal_tangent(pt, tab, in.F, in.Fpi, in.R, x, [&](int m9, const double* dP) {
@@ -326,7 +330,7 @@ __global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __r
       for (int i = 0; i < 9; ++i) wA[(int64_t)(9 * i + m9) * G.n_qp + q] = w * dP[i];
     });
   }
-  if (!done) general_tangent<N>(G, u, sv, mv, *gen, q, sin, sh, gs, wA);
+  if (!done) general_tangent<N>(G, u, sv, mv, *gen, q, sin, wA);
 }
 
 // The parked points of k_element_res, one queue entry per point: each point's iterate is
@@ -339,7 +343,7 @@ __global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(2, 2))
 k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg,
                   const SlipTable<N>* __restrict__ gen, SolveCfg cfg,
                   double* __restrict__ wP, double* __restrict__ sout, int32_t* __restrict__ iters, int32_t* __restrict__ status,
-                  unsigned long long* __restrict__ counts, PointPark pk, double* __restrict__ gs) {
+                  unsigned long long* __restrict__ counts, PointPark pk) {
   __shared__ double sh[lds_columns<N, L> * QBS];
   __shared__ SlipSys<L == 1 ? 3 : N> tabs;
   const uint32_t total = __hip_atomic_load(&pk.ctr[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -353,17 +357,18 @@ k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv
     const int64_t q = pk.idx[k];
     PointIn in;
     Crystal<N, L> pt;
+    CrystalRest<N, L> rest;
     CrystalNewton<N, L> nw;
     int32_t st = 0;
     in.load(G, u, sv, mv, q);
-    setup_crystal<N, L>(pt, in, sv, q, G.n_qp, sub, sh, gs);
+    setup_crystal(pt, in, sv, q, sub, sh, rest);
 #pragma unroll
     for (int j = 0; j < 6; ++j) nw.s[j] = pk.s[j * pk.cap + k];
     nw.it = pk.it[k];
     bool act = nw.resume(pt, tab, cfg.tol);
     while (act) act = nw.advance(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
     if (nw.lost) {
-      if (sub == 0) general_res<N, L>(G, u, sv, mv, *gen, cfg, q, sh, gs, wP, sout, iters, status, &n_it, &n_ev);
+      if (sub == 0) general_res<N, L>(G, u, sv, mv, *gen, cfg, q, wP, sout, iters, status, &n_it, &n_ev);
     } else {
       CrystalNewton<N, L>::finite(pt, &st);
       in.load(G, u, sv, mv, reread(q));
@@ -555,13 +560,14 @@ template <int N, bool TANGENT, int L>
 __device__ __attribute__((noinline)) void general_local(int64_t n_qp, const double* __restrict__ Hd, const Geom& G,
                                                         const double* __restrict__ u, const StateView& sv, const MatView& mv,
                                                         const SlipTable<N>& tab, const SolveCfg& cfg, int self_block, int64_t q,
-                                                        const LocalOut& o, double* sh, double* __restrict__ gs) {
+                                                        const LocalOut& o) {
   PointIn in;
   load_local(in, Hd, n_qp, G, u, sv, mv, q);
   Point<N> pt;
   double s[6], P[9];
   int32_t st = 0;
-  setup_general<N, L>(pt, in, sv, q, n_qp, sh, gs);
+  GeneralStore<N> store;
+  store.setup(pt, in, sv, q);
   const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
   pk1<N>(pt, in.F, in.Fpi, s, P);
   if (TANGENT && o.A) {
@@ -602,7 +608,7 @@ __device__ __attribute__((noinline)) void general_local(int64_t n_qp, const doub
 template <int N, bool TANGENT, int L>
 __global__ void __launch_bounds__(QBS) __attribute__((amdgpu_waves_per_eu(TANGENT ? 1 : 2, TANGENT ? 1 : 2)))
 k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __restrict__ u, StateView sv, MatView mv, SlipSys<N> arg,
-        const SlipTable<N>* __restrict__ gen, int crystal, SolveCfg cfg, int self_block, LocalOut o, double* __restrict__ gs) {
+        const SlipTable<N>* __restrict__ gen, int crystal, SolveCfg cfg, int self_block, LocalOut o) {
   __shared__ double sh[lds_columns<N, L> * QBS];
   __shared__ SlipSys<L == 1 ? 3 : N> tabs;
   const SlipSys<N>& tab = slip_constants<N, L>(arg, reinterpret_cast<SlipSys<N>*>(&tabs));
@@ -612,11 +618,12 @@ k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __res
   PointIn in;
   load_local(in, Hd, n_qp, G, u, sv, mv, q);
   Crystal<N, L> pt;
+  CrystalRest<N, L> rest;
   CrystalNewton<N, L> nw;
   int32_t st = 0;
   bool fits = crystal && Crystal<N, L>::applies(in.R, in.m);
   if (fits) {
-    setup_crystal<N, L>(pt, in, sv, q, n_qp, sub, sh, gs);
+    setup_crystal(pt, in, sv, q, sub, sh, rest);
     fits = nw.solve(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
   }
   if (fits) load_local(in, Hd, n_qp, G, u, sv, mv, reread(q));
@@ -627,7 +634,7 @@ k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __res
     });
   }
   if (!fits) {
-    if (sub == 0) general_local<N, TANGENT, L>(n_qp, Hd, G, u, sv, mv, *gen, cfg, self_block, q, o, sh, gs);
+    if (sub == 0) general_local<N, TANGENT, L>(n_qp, Hd, G, u, sv, mv, *gen, cfg, self_block, q, o);
     return;
   }
   // every lane of a point writes its share of the components
@@ -703,12 +710,12 @@ int point_lanes(int n_slip, int64_t n_qp) {
 template <int N>
 void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                        const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                       unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st) {
+                       unsigned long long* counts, const PointPark& park, hipStream_t st) {
   const int L = point_lanes(N, G.n_qp);
   const dim3 grid((unsigned)((G.n_qp * L + QBS - 1) / QBS)), block(QBS);
   const auto go = [&](auto lanes) {
     hipLaunchKernelGGL((k_element_res<N, decltype(lanes)::value>), grid, block, 0, st, G, u, sv, mv, tb.sys, tb.gen, tb.crystal, cfg,
-                       wP, sout, iters, status, counts, park, gs);
+                       wP, sout, iters, status, counts, park);
   };
   if (L == 1) go(std::integral_constant<int, 1>{});
   if (L == 2) go(std::integral_constant<int, 2>{});
@@ -721,12 +728,12 @@ void launch_element_qp(const Geom& G, const double* u, const StateView& sv, cons
 template <int N>
 void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                             const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
-                            unsigned long long* counts, const PointPark& park, double* gs, hipStream_t st) {
+                            unsigned long long* counts, const PointPark& park, hipStream_t st) {
   const int L = point_lanes(N, G.n_qp);
   const dim3 grid((unsigned)((park.cap * L + QBS - 1) / QBS)), block(QBS);
   const auto go = [&](auto lanes) {
     hipLaunchKernelGGL((k_element_qp_park<N, decltype(lanes)::value>), grid, block, 0, st, G, u, sv, mv, tb.sys, tb.gen, cfg, wP, sout,
-                       iters, status, counts, park, gs);
+                       iters, status, counts, park);
   };
   if (L == 1) go(std::integral_constant<int, 1>{});
   if (L == 2) go(std::integral_constant<int, 2>{});
@@ -738,20 +745,20 @@ void launch_element_qp_park(const Geom& G, const double* u, const StateView& sv,
 
 template <int N>
 void launch_point_tangent(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
-                          const double* sin, double* wA, double* gs, hipStream_t st) {
+                          const double* sin, double* wA, hipStream_t st) {
   const int64_t nb = (G.n_qp + QBS - 1) / QBS;
-  hipLaunchKernelGGL(k_point_tangent<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tb.sys, tb.gen, tb.crystal, sin, wA, gs);
+  hipLaunchKernelGGL(k_point_tangent<N>, dim3((unsigned)nb), dim3(QBS), 0, st, G, u, sv, mv, tb.sys, tb.gen, tb.crystal, sin, wA);
 }
 
 template <int N>
 void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u, const StateView& sv, const MatView& mv,
                   const PointTables<N>& tb, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
-                  const StateOut& so, int32_t* iters, int32_t* status, double* gs, hipStream_t st) {
+                  const StateOut& so, int32_t* iters, int32_t* status, hipStream_t st) {
   const int L = A ? 1 : point_lanes(N, n_qp);
   const dim3 grid((unsigned)((n_qp * L + QBS - 1) / QBS)), block(QBS);
   const auto go = [&](auto tangent, auto lanes) {
     hipLaunchKernelGGL((k_local<N, decltype(tangent)::value, decltype(lanes)::value>), grid, block, 0, st, n_qp, Hd, G, u, sv, mv,
-                       tb.sys, tb.gen, tb.crystal, cfg, self_block, LocalOut{P, A, sig, so, iters, status}, gs);
+                       tb.sys, tb.gen, tb.crystal, cfg, self_block, LocalOut{P, A, sig, so, iters, status});
   };
   if (A) {
     go(std::true_type{}, std::integral_constant<int, 1>{});
@@ -811,15 +818,15 @@ void launch_cell_average(const Geom& G, const double* sig, double* out, hipStrea
 #define CPFEM_INST(N)                                                                                                      \
   template void launch_element_qp<N>(const Geom&, const double*, const StateView&, const MatView&, const PointTables<N>&,  \
                                      const SolveCfg&, double*, double*, int32_t*, int32_t*, unsigned long long*,           \
-                                     const PointPark&, double*, hipStream_t);                                              \
+                                     const PointPark&, hipStream_t);                                              \
   template void launch_element_qp_park<N>(const Geom&, const double*, const StateView&, const MatView&,                    \
                                           const PointTables<N>&, const SolveCfg&, double*, double*, int32_t*, int32_t*,    \
-                                          unsigned long long*, const PointPark&, double*, hipStream_t);                    \
+                                          unsigned long long*, const PointPark&, hipStream_t);                    \
   template void launch_point_tangent<N>(const Geom&, const double*, const StateView&, const MatView&,                      \
-                                        const PointTables<N>&, const double*, double*, double*, hipStream_t);              \
+                                        const PointTables<N>&, const double*, double*, hipStream_t);              \
   template void launch_local<N>(int64_t, const double*, const Geom&, const double*, const StateView&, const MatView&,      \
                                 const PointTables<N>&, const SolveCfg&, int, double*, double*, double*, const StateOut&,   \
-                                int32_t*, int32_t*, double*, hipStream_t);
+                                int32_t*, int32_t*, hipStream_t);
 CPFEM_INST(12)
 CPFEM_INST(24)
 

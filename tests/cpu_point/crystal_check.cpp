@@ -39,7 +39,7 @@ static int64_t run(int crystal, int64_t Q, const double* H, const double* Fpi, c
     if (crystal && fits) {
       Crystal<N> pt;
       CrystalNewton<N, 1> nw;
-      pt.setup(F, Fo, Rq, go, 1, m, gp.data(), gi.data(), 1, 1);
+      pt.setup(F, Fo, Rq, go, 1, m, gp.data(), gi.data(), 1, 1, 0, gi.data() + Crystal<N>::K);
       done = nw.solve(pt, sys, tol, max_sub, max_iter, &status[q]) && crystal_tangent(pt, sys, F, Fo, Rq, nw.s, sink);
       if (done) {
         iters[q] = nw.it;
