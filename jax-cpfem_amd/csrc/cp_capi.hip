@@ -1340,9 +1340,9 @@ int cpfem_local_vjp(cpfem_ctx* c, void* stream, const double* dofs, const CpfemS
   const MatView mv = mat_view(params);
   const SolveCfg cfg = solve_cfg(params);
   if (c->n_slip == 12)
-    launch_local_vjp<12>(G, dofs, sv, mv, c->tab12, cfg, params->self_block, va, st);
+    launch_local_vjp<12>(G, dofs, sv, mv, c->pt12, cfg, params->self_block, va, st);
   else
-    launch_local_vjp<24>(G, dofs, sv, mv, c->tab24, cfg, params->self_block, va, st);
+    launch_local_vjp<24>(G, dofs, sv, mv, c->pt24, cfg, params->self_block, va, st);
   HIPCHK(hipGetLastError());
   return CPFEM_OK;
 }

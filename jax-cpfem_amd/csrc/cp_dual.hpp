@@ -1,6 +1,7 @@
-// Forward-mode dual numbers and the per-point map written once for any scalar type, used by
-// the reverse-mode (adjoint) kernel: with T = Dual, one evaluation gives the derivative of the
-// residual and of every output in one seeded input direction.
+// Forward-mode dual numbers and the per-point map written once for any scalar type: with T = Dual,
+// one evaluation gives the derivative of the residual and of every output in one seeded input
+// direction.  The CPU oracle's adjoint and the checks of the kernels' reverse sweep
+// (cp_reverse.hpp) use it.
 //
 // local_fn follows singlecrystal_copper/models_copper.py:155-200 (and the per-point-parameter
 // variants calibration/case1.py:152-200, models_DPsteel_inhomo.py:240-294):

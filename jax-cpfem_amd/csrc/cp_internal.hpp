@@ -92,9 +92,8 @@ constexpr int64_t SHARED_POINTS = 85000;
 int point_lanes(int n_slip, int64_t n_qp);
 
 // The assembly's point kernels: launch_element_qp runs the local Newton and writes JxW P and,
-// if sout ([6][n_qp]) is set, the converged S' (points of the general form: the stress);
-// launch_point_tangent forms the JxW-weighted consistent tangent wA ([81][n_qp]) from it.
-// gs: scratch ([n_slip][n_qp], twice that where lanes share a point).
+// if sout ([6][n_qp]) is set, the converged stress; launch_point_tangent forms the JxW-weighted
+// consistent tangent wA ([81][n_qp]) from it.
 template <int N>
 void launch_element_qp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                        const SolveCfg& cfg, double* wP, double* sout, int32_t* iters, int32_t* status,
@@ -138,7 +137,7 @@ struct VjpArgs {
 };
 
 template <int N>
-void launch_local_vjp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const SlipTable<N>& tab,
+void launch_local_vjp(const Geom& G, const double* u, const StateView& sv, const MatView& mv, const PointTables<N>& tb,
                       const SolveCfg& cfg, int self_block, const VjpArgs& va, hipStream_t st);
 void launch_grad_field(const Geom& G, const double* lam, const uint8_t* is_bc, double scale_by_w, double* out, hipStream_t st);
 void launch_transpose(const BellView& M, const int32_t* tslot, const double* A, double* At, hipStream_t st);
