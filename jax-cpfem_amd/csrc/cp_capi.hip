@@ -725,8 +725,9 @@ static bool ensure_mg(cpfem_ctx* c) {
   }
   int64_t n1 = 0, n2 = 0;
   mg_scratch(mg, &n1, &n2);
-  ok = ok && (mg.rap1 = get((size_t)n1)) && (mg.rap2 = get((size_t)n2)) && (mg.lam = get(8)) &&
-       (mg.inv = get((size_t)mg.lv[mg.nl - 1].g.n * mg.lv[mg.nl - 1].g.n));
+  ok = ok && (mg.rap1 = get((size_t)n1)) && (mg.rap2 = get((size_t)n2)) && (mg.lam = get(8));
+  const size_t nt = (size_t)mg_dense_tiles(mg.lv[mg.nl - 1].g.n), tile = (size_t)BAND_NB * BAND_NB;
+  ok = ok && (mg.dense[0] = get(nt * nt * tile)) && (mg.dense[1] = get(nt * nt * tile)) && (mg.dpiv = get(2 * tile));
   if (ok && !c->h_flag && hipHostMalloc((void**)&c->h_flag, sizeof(uint64_t)) != hipSuccess) {
     (void)hipGetLastError();
     ok = false;

@@ -245,10 +245,10 @@ struct MgLevel {
 };
 struct Multigrid {
   int nl = 0;    // levels
-  int tail = 0;  // first level of the one-block kernel
   MgLevel lv[MG_MAXL];
   void *rap1 = nullptr, *rap2 = nullptr;  // triple-product intermediates
-  double* inv = nullptr;                  // inverse of the last level's operator
+  double* dense[2] = {};                  // last level's operator in dense tiles, and its inverse
+  double* dpiv = nullptr;                 // two pivot tiles' inverses
   double* lam = nullptr;                  // [0] = 1 / lambda_max of the scaled operator
   int state = 0;                          // 0: no buffers yet, 1: allocated, -1: does not apply
 };
@@ -273,6 +273,7 @@ template <typename TM>
 void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w,
                          int iter, uint64_t* flag, hipStream_t st, Prof* prof);
 int mg_spmv_blocks(int64_t n);
+int mg_dense_tiles(int64_t n);  // tiles per side of the last level's n rows
 
 // Banded LU of the Newton matrix (direct-solve option): n dofs in nbk tiles of BAND_NB, tile
 // half bandwidth wb, stored half bandwidth hw, nt pivot tiles taken from each end (0: one front),

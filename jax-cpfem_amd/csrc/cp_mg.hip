@@ -11,14 +11,16 @@
 // Cycle: levels coarsen every direction by two (node 2I; an odd last element stays as one),
 // trilinear interpolation P, coarse operators P^T A P, Dirichlet dofs masked out on every level
 // (they are scaled by the diagonal alone); before the coarse correction a Chebyshev polynomial
-// of the diagonally scaled operator over [0.1, 1.1] lambda_max, none after it.  With
-// scalar-diagonal smoothing before the correction only, degree 4 on the finest and 3 on the
-// coarser levels needs the fewest matrix passes (per iteration 2 + 2 x 4 on the finest level;
-// degree 2 takes 16 iterations, 3 takes 12, 4 takes 10; smoothing after the correction as well,
-// 3x3 block diagonals and W-cycles gain nothing).  The last level (at most 81 rows) is inverted.
+// of the diagonally scaled operator over [0.1, 1.1] lambda_max (coarser levels: [0.07, 1.1]), none
+// after it.  With scalar-diagonal smoothing before the correction only, degree 4 needs the fewest
+// matrix passes (per iteration 2 + 2 x 4 on the finest level; degree 2 takes 16 iterations, 3 takes
+// 12, 4 takes 10; smoothing after the correction as well, 3x3 block diagonals and W-cycles gain
+// nothing).  Degree 4 over the wider range on the coarser levels takes 664 iterations for 72
+// systems of 24 shapes, where degree 3 over [0.1, 1.1] takes 731, and 16.3 ms at 64^3 (17.5), 3.0 at
+// 40^3 (3.2).  The last level is the first of at most DENSE_ROWS rows; its inverse is formed by
+// tiles (k_dense_step) and applied as one dense product.
 // lambda_max comes from a power iteration on the second level (the levels' values differ by a
-// few percent, the polynomial's range by ten).  Levels of at most TAIL_ROWS rows run in one
-// block, whose barriers are cheaper than launches.
+// few percent, the polynomial's range by ten).
 //
 // The polynomial is run as the three-term recurrence on the iterate,
 //   x' = x + c1 (x - x_prev) + c2 D^-1 (b - A x),
@@ -29,11 +31,13 @@
 #include <type_traits>
 
 #include "cp_krylov.hpp"
+#include "cp_tiles.hpp"
 
 namespace cpfem {
 
-constexpr int DEG_FINE = 4, DEG_COARSE = 3;
-constexpr int TAIL_ROWS = 384, TAIL_LAST = 81, TAIL_SUM = 768, TAIL_BS = 2 * TAIL_ROWS;
+constexpr int DEG_FINE = 4, DEG_COARSE = 4;
+constexpr double LOW_FINE = 0.1, LOW_COARSE = 0.07;  // the polynomials' ranges start at this times lambda_max
+constexpr int DENSE_ROWS = 768;    // the first level of at most this many rows is the last, and is inverted
 constexpr int POWER_STEPS = 12;
 constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
 constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
@@ -82,19 +86,11 @@ bool mg_plan(const int64_t box[3], Multigrid* mg) {
     mg->lv[mg->nl].g = make_grid(m[0], m[1], m[2]);
     ++mg->nl;
     const int64_t c[3] = {coarse_nodes(m[0]), coarse_nodes(m[1]), coarse_nodes(m[2])};
-    if (3 * m[0] * m[1] * m[2] <= 81 || (c[0] == m[0] && c[1] == m[1] && c[2] == m[2])) break;
+    if (3 * m[0] * m[1] * m[2] <= DENSE_ROWS || (c[0] == m[0] && c[1] == m[1] && c[2] == m[2])) break;
     if (mg->nl == MG_MAXL) break;
     for (int d = 0; d < 3; ++d) m[d] = c[d];
   }
-  mg->tail = mg->nl - 1;
-  int64_t sum = mg->lv[mg->tail].g.n;
-  if (sum > TAIL_LAST) return false;
-  // the first level of the block holds its matrix in registers (two threads per row), the others
-  // take three threads per row
-  while (mg->tail > 1 && mg->lv[mg->tail].g.n * 3 <= TAIL_BS && mg->lv[mg->tail - 1].g.n <= TAIL_ROWS &&
-         sum + mg->lv[mg->tail - 1].g.n <= TAIL_SUM)
-    sum += mg->lv[--mg->tail].g.n;
-  return mg->nl >= 2;
+  return mg->nl >= 2 && mg->lv[mg->nl - 1].g.n <= DENSE_ROWS;
 }
 
 void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2) {
@@ -375,166 +371,6 @@ __global__ void __launch_bounds__(256) k_mg_prolong(MgGrid f, MgGrid g, const do
   out[t] = minv[t] != 0.0 ? v : (invd ? b[t] * invd[t] : 0.0);
 }
 
-// The levels of at most TAIL_ROWS rows in one block, their vectors in LDS.  Bound by latency: one
-// CU reads 64 B per clock from the L2, so the first of these levels (375 rows, 243 KB at 64^3)
-// keeps its matrix in registers, half a row per thread, and reads it once per cycle instead
-// of once per product; the last level (at most 81 rows) is solved with its inverse, staged in LDS.
-// (Reading it for each product, one thread per row: 56 us per cycle.)
-struct MgTail {
-  int nl;
-  MgGrid f;  // the level above, whose residual is restricted first
-  const double* rf;
-  MgGrid g[MG_MAXL];
-  const void* A[MG_MAXL];
-  const double* minv[MG_MAXL];
-  int off[MG_MAXL];
-};
-
-// One thread's share of a row of the block's first level: slots [S0, S0 + 14) (13 in the second
-// half).  Rows off the box read a node of the box against a zero.
-constexpr int TAIL_SLOTS = 14;
-struct TailRow {
-  int i3, xm, xp, ym, yp, zm, zp;  // three times the node, and the steps to its neighbours (0: none)
-  __device__ TailRow(const MgGrid& g, int r) {
-    const int i = (int)((uint32_t)r / 3u);
-    const NodeXYZ p = mg_node(g, i);
-    i3 = 3 * i;
-    xm = p.x > 0 ? 3 : 0;
-    xp = p.x < g.nx - 1 ? 3 : 0;
-    ym = p.y > 0 ? 3 * g.nx : 0;
-    yp = p.y < g.ny - 1 ? 3 * g.nx : 0;
-    zm = p.z > 0 ? 3 * g.nx * g.ny : 0;
-    zp = p.z < g.nz - 1 ? 3 * g.nx * g.ny : 0;
-  }
-};
-template <typename TM, int S0>
-__device__ __forceinline__ void tail_load(const TM* __restrict__ A, int n, int r, TM (&a)[3 * TAIL_SLOTS]) {
-#pragma unroll
-  for (int k = 0; k < 3 * TAIL_SLOTS; ++k) a[k] = 3 * S0 + k < 81 ? A[(3 * S0 + k) * (int64_t)n + r] : (TM)0;
-}
-template <typename TM, int S0>
-__device__ __forceinline__ double tail_dot(const TailRow& t, const TM (&a)[3 * TAIL_SLOTS], const double* __restrict__ v) {
-  double acc = 0.0;
-#pragma unroll
-  for (int k = 0; k < TAIL_SLOTS; ++k) {
-    constexpr int last = 26;
-    const int s = S0 + k < last ? S0 + k : last;
-    const int dz = s / 9 - 1, dy = s / 3 % 3 - 1, dx = s % 3 - 1;
-    const double* w = v + t.i3 + (dz < 0 ? -t.zm : dz > 0 ? t.zp : 0) + (dy < 0 ? -t.ym : dy > 0 ? t.yp : 0) +
-                      (dx < 0 ? -t.xm : dx > 0 ? t.xp : 0);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) acc += (double)a[3 * k + c] * w[c];
-  }
-  return acc;
-}
-
-template <typename TM>
-__global__ void __launch_bounds__(TAIL_BS) k_mg_tail(MgTail T, double* __restrict__ x, Cheb cc, const double* __restrict__ inv,
-                                                     const double* __restrict__ lam, const int32_t* __restrict__ done) {
-  __shared__ double sb[TAIL_SUM], sx[TAIL_SUM], so[TAIL_SUM], red[TAIL_BS];
-  __shared__ double sI[TAIL_LAST * TAIL_LAST];
-  const int tid = threadIdx.x;
-  const int dn = *done;
-  const double il = lam[0];
-  const BellView none{};
-  const int last = T.nl - 1;
-  // the first level's matrix (threads below TAIL_ROWS: first half of the row's slots), the last
-  // level's inverse into LDS
-  const int n0 = T.g[0].n, half = __builtin_amdgcn_readfirstlane(tid >= TAIL_ROWS ? 1 : 0), r0 = tid - half * TAIL_ROWS;
-  const bool own0 = r0 < n0 && last > 0;
-  const TailRow row0(T.g[0], own0 ? r0 : 0);
-  TM a0[3 * TAIL_SLOTS];
-  if (own0) {
-    if (half)
-      tail_load<TM, TAIL_SLOTS>(static_cast<const TM*>(T.A[0]), n0, r0, a0);
-    else
-      tail_load<TM, 0>(static_cast<const TM*>(T.A[0]), n0, r0, a0);
-  }
-  for (int k = tid; k < T.g[last].n * T.g[last].n; k += TAIL_BS) sI[k] = inv[k];
-  if (tid < n0) {
-    const double v = mg_restrict_row(T.f, T.g[0], tid, T.rf);
-    sb[tid] = T.minv[0][tid] != 0.0 ? v : 0.0;
-  }
-  if (dn) return;  // uniform
-  // A v of the level's rows in the threads tid < n
-  const auto product = [&](int l, const double* v) -> double {
-    const int n = T.g[l].n;
-    double a = 0.0, y = 0.0;
-    if (l == 0 && last > 0) {
-      if (own0) a = half ? tail_dot<TM, TAIL_SLOTS>(row0, a0, v) : tail_dot<TM, 0>(row0, a0, v);
-      red[tid] = a;
-      __syncthreads();
-      if (tid < n) y = a + red[tid + TAIL_ROWS];
-    } else {
-      const TM* A = static_cast<const TM*>(T.A[l]);
-      const int part = tid / n, r = tid - part * n;  // 3 n <= TAIL_BS below the first level
-      if (part < 3) a = mg_dot<TM, false, 3>(none, T.g[l], A, v, r, part);
-      red[tid] = a;
-      __syncthreads();
-      if (tid < n) y = a + red[tid + n] + red[tid + 2 * n];
-    }
-    __syncthreads();
-    return y;
-  };
-  // Chebyshev polynomial of degree deg from zero; the result's buffer alternates between sx and so
-  const auto smooth = [&](int l, int deg, const Cheb& c) -> double* {
-    const int n = T.g[l].n, o = T.off[l];
-    double *cur = sx + o, *oth = so + o;
-    const double mi = tid < n ? T.minv[l][tid] : 0.0;
-    if (tid < n) {
-      cur[tid] = c.ith * il * mi * sb[o + tid];
-      oth[tid] = 0.0;
-    }
-    __syncthreads();
-    for (int k = 0; k + 1 < deg; ++k) {
-      const double y = product(l, cur);
-      if (tid < n) oth[tid] = cur[tid] + (c.c1[k] * (cur[tid] - oth[tid]) + c.c2[k] * il * mi * (sb[o + tid] - y));
-      __syncthreads();
-      double* s = cur;
-      cur = oth;
-      oth = s;
-    }
-    return cur;
-  };
-  __syncthreads();
-  for (int l = 0; l < last; ++l) {
-    const double* cur = smooth(l, DEG_COARSE, cc);
-    const int n = T.g[l].n, o = T.off[l];
-    const double y = product(l, cur);
-    double v = 0.0;
-    if (tid < n) {
-      v = cur[tid];
-      so[o + tid] = T.minv[l][tid] != 0.0 ? sb[o + tid] - y : 0.0;  // residual
-      sx[o + tid] = v;                                               // iterate
-    }
-    __syncthreads();
-    const int nc = T.g[l + 1].n;
-    if (tid < nc) sb[T.off[l + 1] + tid] = T.minv[l + 1][tid] != 0.0 ? mg_restrict_row(T.g[l], T.g[l + 1], tid, so + o) : 0.0;
-    __syncthreads();
-  }
-  {  // the last level exactly, a row's columns over three threads
-    const int n = T.g[last].n, o = T.off[last], w = (n + 2) / 3;
-    const int part = tid / n, r = tid - part * n;
-    double a = 0.0;
-    if (part < 3) {
-      for (int c = part * w; c < min(n, (part + 1) * w); ++c) a += sI[c * n + r] * sb[o + c];
-    }
-    red[tid] = a;
-    __syncthreads();
-    if (tid < n) sx[o + tid] = a + red[tid + n] + red[tid + 2 * n];
-    __syncthreads();
-  }
-  for (int l = last - 1; l >= 0; --l) {
-    if (tid < T.g[l].n) {
-      const int i = (int)((uint32_t)tid / 3u);
-      const double v = sx[T.off[l] + tid] + mg_interp(T.g[l], T.g[l + 1], mg_node(T.g[l], i), tid - 3 * i, sx + T.off[l + 1]);
-      sx[T.off[l] + tid] = T.minv[l][tid] != 0.0 ? v : 0.0;
-    }
-    __syncthreads();
-  }
-  if (tid < n0) x[tid] = sx[tid];
-}
-
 // ---------------------------------------------------------------------------------
 // Coarse operators.  P is a product of one-dimensional interpolations, so P^T A P is formed one
 // direction at a time: each pass halves the rows and reads and writes each value once (1.2 GB in
@@ -622,60 +458,108 @@ __global__ void __launch_bounds__(256) k_mg_coarsen(MgGrid f, MgGrid g, const TI
   }
 }
 
-// Inverse of the last level's operator (column-major), by Gauss-Jordan elimination in LDS.  Smoothing
-// that level instead costs odd-sized boxes, whose half-width last elements pile up there, up
-// to five iterations.  The diagonal is raised by 1e-6, so that a floating box (a singular
-// operator, as where only corners are held) keeps a bounded inverse.
-// A thread keeps one row's columns q, q + 8, ... in registers; the pivot row and column pass
-// through LDS, two buffers in turn, so that a step needs one barrier.
-constexpr int INV_Q = 8, INV_C = (TAIL_LAST + INV_Q - 1) / INV_Q, INV_BS = 704;  // 8 x 81 threads in whole waves
+// ---------------------------------------------------------------------------------
+// The last level: n rows in nt x nt dense tiles (unit rows beyond n), inverted by Gauss-Jordan
+// steps over the tiles, one launch each, between two buffers:
+//   A_kk' = D, A_kj' = D A_kj, A_ik' = -A_ik D, A_ij' = A_ij - (A_ik D) A_kj,  D = A_kk^-1,
+// where the workgroup that finishes the next diagonal tile inverts it too.  The diagonal is raised
+// by 1e-6, so that a floating box (a singular operator, as where only corners are held) keeps a
+// bounded inverse.  Bound by the chain through the diagonal tiles, 17 us a step.
+// Applying the inverse is one launch (375 rows 7 us, 648 rows 10), and takes the place of smoothing
+// this level and the ones below it, 375 rows in one block of one CU 21 us, 648 rows in launches 45;
+// forming it takes 6 x 17 or 11 x 18 us, where the inverse of 81 rows took 67.
 template <typename TM>
-__global__ void __launch_bounds__(INV_BS) k_mg_inverse(MgGrid g, const TM* __restrict__ A, double* __restrict__ inv) {
-  __shared__ double m[TAIL_LAST * TAIL_LAST], row[2][INV_Q * INV_C], col[2][TAIL_LAST];
-  const int n = g.n, tid = threadIdx.x;
-  for (int k = tid; k < n * n; k += INV_BS) m[k] = 0.0;
-  __syncthreads();
-  for (int k = tid; k < 81 * n; k += INV_BS) {
-    const int q = k / n, r = k - q * n, s = q / 3, i = r / 3;
-    const NodeXYZ p = mg_node(g, i);
-    const int x = p.x + s % 3 - 1, y = p.y + s / 3 % 3 - 1, z = p.z + s / 9 - 1;
-    if ((uint32_t)x >= (uint32_t)g.nx || (uint32_t)y >= (uint32_t)g.ny || (uint32_t)z >= (uint32_t)g.nz) continue;
-    const int c = 3 * (x + g.nx * (y + g.ny * z)) + q % 3;
-    m[c * n + r] = (double)A[k] * (c == r ? 1.0 + 1e-6 : 1.0);
+__global__ void __launch_bounds__(256) k_dense_fill(MgGrid g, int nt, const TM* __restrict__ A, double* __restrict__ out) {
+  const int c = (int)(blockIdx.x * 256 + threadIdx.x), r = (int)blockIdx.y, ld = nt * NB;
+  if (c >= ld) return;
+  double v = r == c ? 1.0 : 0.0;
+  if (r < g.n && c < g.n) {
+    const NodeXYZ p = mg_node(g, (int)((uint32_t)r / 3u)), q = mg_node(g, (int)((uint32_t)c / 3u));
+    const int dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
+    v = 0.0;
+    if (abs(dx) <= 1 && abs(dy) <= 1 && abs(dz) <= 1)
+      v = (double)A[(3 * ((dz + 1) * 9 + (dy + 1) * 3 + dx + 1) + c % 3) * (int64_t)g.n + r] * (r == c ? 1.0 + 1e-6 : 1.0);
   }
-  __syncthreads();
-  const int q = tid / TAIL_LAST, r = tid - q * TAIL_LAST;
-  const bool own = q < INV_Q && r < n;
-  double v[INV_C];
+  out[((int64_t)(r / NB) * nt + c / NB) * TILE + (r % NB) * NB + c % NB] = v;
+}
+
+__global__ void __launch_bounds__(256) k_dense_first(const double* __restrict__ A, double* __restrict__ D) {
+  __shared__ InvLds s;
+  const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  v4d a[4];
+  load_d(a, A, w, l);
+  (void)tile_inverse(a, s);
+  store_d(a, D, w, l);
+}
+
+// Step k: `in` to `out`; D holds the inverse of tile (k, k), the next one goes to Dn.
+__global__ void __launch_bounds__(256, 2) k_dense_step(int nt, int k, const double* __restrict__ in, double* __restrict__ out,
+                                                       const double* __restrict__ D, double* __restrict__ Dn) {
+  __shared__ double S[2][TILE];
+  const int i = (int)blockIdx.y, j = (int)blockIdx.x, w = threadIdx.x >> 6, l = threadIdx.x & 63;
+  const auto tile = [&](const double* m, int r, int c) { return m + ((int64_t)r * nt + c) * TILE; };
+  double* o = out + ((int64_t)i * nt + j) * TILE;
+  v4d c[4] = {};
+  if (i == k && j == k) {  // uniform over the block, as the other cases
+    load_d(c, D, w, l);
+    store_d(c, o, w, l);
+    return;
+  }
+  Stage st;
+  double x[16];
+  // left operand: rows of D (row k), else of A_ik
+  const double* g = (i == k ? D : tile(in, i, k)) + (16 * w + l % 16) * NB + l / 16;
 #pragma unroll
-  for (int j = 0; j < INV_C; ++j) v[j] = own && q + INV_Q * j < n ? m[(q + INV_Q * j) * n + r] : 0.0;
+  for (int t = 0; t < 16; ++t) x[t] = g[4 * t];
+  if (i == k || j == k) {
+    st.load(i == k ? tile(in, k, j) : D);
+    st.store(S[0]);
+    __syncthreads();
+    mul_last<NB>(c, x, S[0], l);
+    if (j == k) {
 #pragma unroll
-  for (int jp = 0; jp < INV_C; ++jp) {
-#pragma unroll 1
-    for (int qp = 0; qp < INV_Q; ++qp) {
-      const int p = INV_Q * jp + qp, buf = p & 1;
-      if (p >= n) break;  // uniform
-      if (own && q == qp) col[buf][r] = v[jp];
-      if (own && r == p) {
-#pragma unroll
-        for (int j = 0; j < INV_C; ++j) row[buf][q + INV_Q * j] = v[j];
-      }
-      __syncthreads();
-      if (own) {
-        const double piv = 1.0 / col[buf][p], f = r == p ? piv : -col[buf][r] * piv;
-#pragma unroll
-        for (int j = 0; j < INV_C; ++j) {
-          const double x = row[buf][q + INV_Q * j], base = r == p ? 0.0 : v[j];
-          v[j] = q + INV_Q * j == p ? f : base + f * x;
-        }
-      }
+      for (int q = 0; q < 4; ++q) c[q] = -c[q];
     }
-  }
-  if (own) {
+  } else {
+    st.load(D);
+    st.store(S[0]);
+    st.load(tile(in, k, j));
+    load_d(c, tile(in, i, j), w, l);
+    __syncthreads();
+    {
+      v4d acc[4] = {};
+      mul_chain<NB>(acc, x, S[0], l);
 #pragma unroll
-    for (int j = 0; j < INV_C; ++j)
-      if (q + INV_Q * j < n) inv[(q + INV_Q * j) * n + r] = v[j];
+      for (int t = 0; t < 16; ++t) x[t] = -acc[t / 4][t % 4];
+    }
+    st.store(S[1]);
+    __syncthreads();
+    mul_last<NB>(c, x, S[1], l);
   }
+  store_d(c, o, w, l);
+  if (i == k + 1 && j == k + 1) {
+    static_assert(sizeof(InvLds) <= sizeof(S[0]), "");  // S[0] is free since the second barrier
+    (void)tile_inverse(c, *reinterpret_cast<InvLds*>(S[0]));
+    store_d(c, Dn, w, l);
+  }
+}
+
+// x = inverse (P^T rf) of the last level, P^T rf formed by every workgroup for itself (its right-hand
+// side in LDS), 16 rows a workgroup, 16 threads a row.
+__global__ void __launch_bounds__(256) k_mg_dense(MgGrid f, MgGrid g, int nt, const double* __restrict__ rf,
+                                                  const double* __restrict__ minv, const double* __restrict__ inv,
+                                                  double* __restrict__ x, const int32_t* __restrict__ done) {
+  __shared__ __align__(16) double b[DENSE_ROWS];
+  const int dn = *done;
+  for (int t = threadIdx.x; t < nt * NB; t += 256) b[t] = t < g.n && minv[t] != 0.0 ? mg_restrict_row(f, g, t, rf) : 0.0;
+  __syncthreads();
+  const int r = (int)blockIdx.x * 16 + threadIdx.x / 16, sub = threadIdx.x % 16;
+  const double* row = inv + (int64_t)(r / NB) * nt * TILE + (r % NB) * NB;
+  double acc = 0.0;
+  for (int j = 0; j < nt; ++j) acc += row_dot(row + (int64_t)j * TILE, b + j * NB, sub);
+  acc = sum16(acc);
+  if (dn) return;
+  if (sub == 0 && r < g.n) x[r] = acc;
 }
 
 // Inverse diagonal of the finest level with Dirichlet dofs masked, and the Dirichlet flags of the
@@ -699,6 +583,7 @@ static inline int level_parts(int64_t n) { return n >= FLAT_ROWS ? 1 : 3; }
 static inline unsigned level_blocks(int64_t n) { return (unsigned)(level_parts(n) == 1 ? (n + 255) / 256 : (n + 63) / 64); }
 static inline int level_order(int64_t n, int rev) { return (rev & 1) | (n < PLAIN_ROWS ? 2 : 0); }
 int mg_spmv_blocks(int64_t n) { return (int)level_blocks(n); }
+int mg_dense_tiles(int64_t n) { return (int)((n + NB - 1) / NB); }
 
 template <typename TM>
 void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const uint8_t* is_bc,
@@ -724,7 +609,13 @@ void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const
     fixed = cfixed;
   }
   const MgLevel& E = mg.lv[mg.nl - 1];
-  hipLaunchKernelGGL(k_mg_inverse<TM>, dim3(1), dim3(INV_BS), 0, st, E.g, static_cast<const TM*>(E.A), mg.inv);
+  const int nt = mg_dense_tiles(E.g.n);
+  hipLaunchKernelGGL(k_dense_fill<TM>, dim3((unsigned)((nt * NB + 255) / 256), (unsigned)(nt * NB)), dim3(256), 0, st, E.g, nt,
+                     static_cast<const TM*>(E.A), mg.dense[0]);
+  hipLaunchKernelGGL(k_dense_first, dim3(1), dim3(256), 0, st, mg.dense[0], mg.dpiv);
+  for (int k = 0; k < nt; ++k)
+    hipLaunchKernelGGL(k_dense_step, dim3((unsigned)nt, (unsigned)nt), dim3(256), 0, st, nt, k, mg.dense[k & 1],
+                       mg.dense[(k & 1) ^ 1], mg.dpiv + (k & 1) * TILE, mg.dpiv + ((k & 1) ^ 1) * TILE);
   // lambda_max on the second level
   const MgLevel& L = mg.lv[1];
   const unsigned nb = level_blocks(L.g.n);
@@ -774,9 +665,10 @@ static double* smooth_level(const Multigrid& mg, int l, const BellView& M, const
 template <typename TM>
 static void vcycle(const Multigrid& mg, const BellView& M, const TM* vals, const double* invd, const double* b, double* out,
                    const int32_t* done, int* pass, hipStream_t st, Prof* prof) {
-  static const Cheb cf = cheb(DEG_FINE, 0.1), cc = cheb(DEG_COARSE, 0.1);
+  static const Cheb cf = cheb(DEG_FINE, LOW_FINE), cc = cheb(DEG_COARSE, LOW_COARSE);
   double* cur[MG_MAXL];
-  for (int l = 0; l < mg.tail; ++l) {
+  const int last = mg.nl - 1;
+  for (int l = 0; l < last; ++l) {
     const MgLevel& L = mg.lv[l];
     int p = 0;
     if (l == 0) {
@@ -787,29 +679,17 @@ static void vcycle(const Multigrid& mg, const BellView& M, const TM* vals, const
       cur[l] = level_parts(L.g.n) == 1 ? smooth_level<TM, false, 1>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof)
                                        : smooth_level<TM, false, 3>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof);
     }
-    if (l + 1 == mg.tail) break;  // the one-block kernel restricts for itself
+    if (l + 1 == last) break;  // the last level's kernel restricts for itself
     const MgLevel& C = mg.lv[l + 1];
     timed(prof, PC_MG_COARSE, k_mg_restrict, dim3(blocks256(C.g.n)), dim3(256), st, L.g, C.g, (const double*)L.r,
           (const double*)C.minv, C.b, C.x0, cc.ith, (const double*)mg.lam, done);
   }
-  MgTail T{};
-  T.nl = mg.nl - mg.tail;
-  T.f = mg.lv[mg.tail - 1].g;
-  T.rf = mg.lv[mg.tail - 1].r;
-  int off = 0;
-  for (int l = 0; l < T.nl; ++l) {
-    const MgLevel& L = mg.lv[mg.tail + l];
-    T.g[l] = L.g;
-    T.A[l] = L.A;
-    T.minv[l] = L.minv;
-    T.off[l] = off;
-    off += L.g.n;
-  }
-  const MgLevel& H = mg.lv[mg.tail];
-  timed(prof, PC_MG_COARSE, k_mg_tail<TM>, dim3(1), dim3(TAIL_BS), st, T, H.x0, cc, (const double*)mg.inv, (const double*)mg.lam,
-        done);
-  const double* e = H.x0;
-  for (int l = mg.tail - 1; l >= 0; --l) {
+  const MgLevel &A = mg.lv[last - 1], &E = mg.lv[last];
+  const int nt = mg_dense_tiles(E.g.n);
+  timed(prof, PC_MG_COARSE, k_mg_dense, dim3((unsigned)((E.g.n + 15) / 16)), dim3(256), st, A.g, E.g, nt, (const double*)A.r,
+        (const double*)E.minv, (const double*)mg.dense[nt & 1], E.x0, done);
+  const double* e = E.x0;
+  for (int l = last - 1; l >= 0; --l) {
     const MgLevel& L = mg.lv[l];
     double* o = l == 0 ? out : cur[l];
     timed(prof, PC_MG_COARSE, k_mg_prolong, dim3(blocks256(L.g.n)), dim3(256), st, L.g, mg.lv[l + 1].g, e, (const double*)cur[l],
@@ -1034,7 +914,7 @@ void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* v
                          int iter, uint64_t* flag, hipStream_t st, Prof* prof) {
   const MgLevel& L = mg.lv[0];
   const MgGrid g = L.g;
-  const double ith = cheb(DEG_FINE, 0.1).ith;
+  const double ith = cheb(DEG_FINE, LOW_FINE).ith;
   const bool one = level_parts(g.n) == 1;
   const dim3 vb((unsigned)w.nb), vt(KBS), sb((unsigned)w.nbs), s1(MgShape<1>::BS), s3(MgShape<3>::BS);
   const int32_t* done = &w.sc->done;
