@@ -88,7 +88,11 @@ k_local_vjp(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Slip
       load_point(sv, reread(q), Fpi, R);
       pt.stress(nw.s, R, s);
     } else if (sub == 0) {
-      general_stress<N>(G, u, sv, mv, *gen, cfg, q, s);
+      const OutOfLine f{G, sv, mv, cfg};
+      double sg[6];
+      general_stress<N>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, sg);
+#pragma unroll
+      for (int i = 0; i < 6; ++i) s[i] = sg[i];
     }
   }
   __syncthreads();  // the sweep's columns are shared out by point, not by lane

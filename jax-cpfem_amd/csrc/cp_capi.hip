@@ -121,7 +121,8 @@ struct cpfem_ctx {
   double* d_sg = nullptr;
   double* d_jxw = nullptr;
   int32_t *d_col = nullptr, *d_nslot = nullptr, *d_dslot = nullptr, *d_tslot = nullptr;
-  int32_t *d_cptr = nullptr, *d_clist = nullptr;
+  uint16_t* d_slots = nullptr;  // (cell, a, b) -> slot, rank
+  int slot_ranks = 1;
   int32_t *d_nptr = nullptr, *d_nlist = nullptr;
   uint8_t* d_isbc = nullptr;
   uint8_t* d_nobc = nullptr;  // all-zero flags (raw residual / matrix)
@@ -381,39 +382,35 @@ static int build_maps(cpfem_ctx* c, const int32_t* cells) {
       const auto& v = nb[i];
       tslot[(size_t)s * nn + j] = (int32_t)(std::lower_bound(v.begin(), v.end(), (int32_t)j) - v.begin());
     }
-  // (node i, slot s) -> element blocks (cell*64 + a*8 + b), ascending cell
-  const int64_t nkey = (int64_t)maxs * nn;
-  std::vector<int32_t> cptr(nkey + 1, 0), clist((size_t)nc * 64);
-  auto slot_of = [&](int64_t i, int32_t j) {
-    const auto& v = nb[i];
-    return (int)(std::lower_bound(v.begin(), v.end(), j) - v.begin());
-  };
-  std::vector<int32_t> keys((size_t)nc * 64);
-  for (int64_t e = 0; e < nc; ++e)
-    for (int a = 0; a < 8; ++a)
-      for (int b = 0; b < 8; ++b) {
-        const int64_t i = cells[e * 8 + a];
-        const int s = slot_of(i, cells[e * 8 + b]);
-        const int64_t key = (int64_t)s * nn + i;
-        keys[e * 64 + a * 8 + b] = (int32_t)key;
-        cptr[key + 1]++;
-      }
-  for (int64_t k = 0; k < nkey; ++k) cptr[k + 1] += cptr[k];
-  {
-    std::vector<int32_t> fill(cptr.begin(), cptr.end() - 1);
-    for (int64_t t = 0; t < nc * 64; ++t) clist[fill[keys[t]]++] = (int32_t)t;
+  // (cell, a, b) -> slot of node b in node a's row, and its rank among the cell's earlier equal nodes
+  if (maxs >= GATHER_RANK) return fail(CPFEM_EBADARG, "a node has " + std::to_string(maxs) + " neighbours");
+  std::vector<uint16_t> slots((size_t)nc * 64);
+  int ranks = 1;
+  for (int64_t e = 0; e < nc; ++e) {
+    int rank[8];
+    for (int b = 0; b < 8; ++b) {
+      rank[b] = 0;
+      for (int d = 0; d < b; ++d) rank[b] += cells[e * 8 + d] == cells[e * 8 + b];
+      ranks = std::max(ranks, rank[b] + 1);
+    }
+    for (int a = 0; a < 8; ++a) {
+      const auto& v = nb[cells[e * 8 + a]];
+      for (int b = 0; b < 8; ++b)
+        slots[e * 64 + a * 8 + b] =
+            (uint16_t)((std::lower_bound(v.begin(), v.end(), cells[e * 8 + b]) - v.begin()) + GATHER_RANK * rank[b]);
+    }
   }
+  c->slot_ranks = ranks;
   int rc;
   if ((rc = dalloc(&c->d_nptr, nptr.size())) || (rc = dalloc(&c->d_nlist, nlist.size())) ||
-      (rc = dalloc(&c->d_cptr, cptr.size())) || (rc = dalloc(&c->d_clist, clist.size())) ||
+      (rc = dalloc(&c->d_slots, slots.size())) ||
       (rc = dalloc(&c->d_col, c->h_col.size())) || (rc = dalloc(&c->d_nslot, c->h_nslot.size())) ||
       (rc = dalloc(&c->d_dslot, c->h_dslot.size())) || (rc = dalloc(&c->d_tslot, tslot.size())))
     return rc;
   HIPCHK(hipMemcpy(c->d_tslot, tslot.data(), tslot.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nptr, nptr.data(), nptr.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nlist, nlist.data(), nlist.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->d_cptr, cptr.data(), cptr.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->d_clist, clist.data(), clist.size() * 4, hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(c->d_slots, slots.data(), slots.size() * 2, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_col, c->h_col.data(), c->h_col.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nslot, c->h_nslot.data(), c->h_nslot.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_dslot, c->h_dslot.data(), c->h_dslot.size() * 4, hipMemcpyHostToDevice));
@@ -891,7 +888,7 @@ void cpfem_destroy(cpfem_ctx* c) {
   dfree(c->d_tab);
   dfree(c->d_cells); dfree(c->d_sg); dfree(c->d_jxw);
   dfree(c->d_col); dfree(c->d_nslot); dfree(c->d_dslot); dfree(c->d_tslot);
-  dfree(c->d_cptr); dfree(c->d_clist); dfree(c->d_nptr); dfree(c->d_nlist);
+  dfree(c->d_slots); dfree(c->d_nptr); dfree(c->d_nlist);
   dfree(c->d_isbc); dfree(c->d_nobc); dfree(c->d_ubar);
   dfree(c->d_sconv);
   dfree(c->d_wP); dfree(c->d_wA); dfree(c->d_KE); dfree(c->d_RE); dfree(c->d_sig); dfree(c->d_status); dfree(c->d_counts);
@@ -1040,7 +1037,7 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   prof_end(pf, sl, st);
   if (mat) {
     sl = prof_begin(pf, PC_GATHER_MAT, st);
-    launch_gather_matrix(c->bell(), c->d_KE, c->d_cptr, c->d_clist, isbc, mat, st);
+    launch_gather_matrix(c->bell(), c->d_KE, c->d_nptr, c->d_nlist, c->d_slots, c->slot_ranks, c->d_dslot, isbc, mat, st);
     prof_end(pf, sl, st);
   }
   HIPCHK(hipGetLastError());

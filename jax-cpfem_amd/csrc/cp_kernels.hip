@@ -162,7 +162,10 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
     n_it = sub == 0 ? (uint32_t)nw.it : 0u;
   } else if (valid && !fits && sub == 0) {
     // (its residuals here are not counted twice)
-    general_res<N, L>(G, u, sv, mv, *gen, cfg, q, wP, sout, iters, status, &n_it, &n_ev);
+    OutOfLine f{G, sv, mv, cfg};
+    general_res<N, L>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, wP, sout, iters, status, &f.n_it, &f.n_ev);
+    n_it = f.n_it;
+    n_ev = f.n_ev;
   }
   add_counts(counts, n_it, n_ev);
 }
@@ -213,7 +216,10 @@ __global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __r
       for (int i = 0; i < 9; ++i) wA[(int64_t)(9 * i + m9) * G.n_qp + q] = w * dP[i];
     });
   }
-  if (!done) general_tangent<N>(G, u, sv, mv, *gen, q, sin, wA);
+  if (!done) {
+    const OutOfLine f{G, sv, mv, {}};
+    general_tangent<N>(f.G, u, f.sv, f.mv, *gen, q, sin, wA);
+  }
 }
 
 // The parked points of k_element_res, one queue entry per point: each point's iterate is
@@ -251,7 +257,12 @@ k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv
     bool act = nw.resume(pt, tab, cfg.tol);
     while (act) act = nw.advance(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
     if (nw.lost) {
-      if (sub == 0) general_res<N, L>(G, u, sv, mv, *gen, cfg, q, wP, sout, iters, status, &n_it, &n_ev);
+      if (sub == 0) {
+        OutOfLine f{G, sv, mv, cfg};
+        general_res<N, L>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, wP, sout, iters, status, &f.n_it, &f.n_ev);
+        n_it = f.n_it;
+        n_ev = f.n_ev;
+      }
     } else {
       CrystalNewton<N, L>::finite(pt, &st);
       in.load(G, u, sv, mv, reread(q));
@@ -266,118 +277,155 @@ k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv
 }
 
 // ---------------------------------------------------------------------------------
-// Element stiffness / residual: one thread per (cell, local node a); writes the 8 node-pair
-// blocks of row-block a (KE[cell][a][b][i][k]) and r_e[cell][a][i].  A block takes 16 cells
-// (128 points, contiguous in the [component][Q] layouts) and stages their JxW P and, one
-// row index i at a time, the 27 tangent components dP_(ij)/dH_(kl) of all 128 points in LDS
-// with coalesced loads: each value is read from HBM once, where eight threads of a cell
-// reading it from global memory re-fetched the tangent ~7 times (L2 misses) per launch.
+// Element stiffness / residual: one thread per (cell, local node a) and row index i; writes the 24
+// values (b, k) of its row (KE[cell][a][i][b][k]) and r_e[cell][a][i].  A block takes 16 cells (128
+// points, contiguous in the [component][Q] layouts) and one i, and stages their JxW P_ij and
+// the 27 tangent components dP_(ij)/dH_(kl) in LDS with coalesced loads: each value is read
+// once.  The rows leave through the same LDS, 192 contiguous bytes each.  The three i of a cell are
+// blocks of the same XCD, which then finds the cells' gradients in its L2.
+// Bound by memory (2.6 GB at 64^3).  64^3: 950 us; with the three i in one thread's 72 accumulators
+// and 16-byte stores 576 bytes apart, 1550.  19x14x11 (183 blocks of that kind): 24 us, 52.
 constexpr int EK_CELLS = 16;
 constexpr int EK_BS = 8 * EK_CELLS;  // threads = points per block
+constexpr int EK_PITCH = 25;         // doubles between the rows in LDS
+constexpr int XCDS = 8;
 
-// Two waves per SIMD: 256 VGPRs with 12 B of spills (one wave per SIMD at 258 registers
-// without the bound).
-__global__ void __launch_bounds__(EK_BS) __attribute__((amdgpu_waves_per_eu(2, 2)))
-k_element_K(Geom G, const double* __restrict__ wP, const double* __restrict__ wA, double* __restrict__ KE,
-            double* __restrict__ RE) {
-  __shared__ double sP[9][EK_BS];
-  __shared__ double sA[27][EK_BS];
-  const int64_t q0 = (int64_t)blockIdx.x * EK_BS;  // first point of the block
+template <bool UNIFORM>
+__global__ void __launch_bounds__(EK_BS) k_element_K(Geom G, const double* __restrict__ wP, const double* __restrict__ wA,
+                                                    double* __restrict__ KE, double* __restrict__ RE) {
+  static_assert(EK_PITCH * EK_BS <= 27 * EK_BS, "the rows use the tangents' LDS");
+  __shared__ double sP[3][EK_BS];
+  __shared__ double sA[27 * EK_BS];
+  __shared__ double sG[UNIFORM ? 192 : 1];
+  const int i = (int)(blockIdx.x / XCDS) % 3;
+  const int64_t q0 = ((int64_t)(blockIdx.x / (3 * XCDS)) * XCDS + blockIdx.x % XCDS) * EK_BS;  // first point of the block
   const int tid = threadIdx.x;
-  const int64_t t = q0 + tid;                      // (cell, a) of this thread
+  const int64_t t = q0 + tid;  // (cell, a) of this thread
   const bool valid = t < G.n_qp;
   const int64_t cell = t >> 3;
   const int a = tid & 7;
   const int cl = tid >> 3;  // cell within the block
 #pragma unroll
-  for (int c = 0; c < 9; ++c) sP[c][tid] = valid ? wP[c * G.n_qp + t] : 0.0;
-  double K[72];
+  for (int j = 0; j < 3; ++j) sP[j][tid] = valid ? wP[(3 * i + j) * G.n_qp + t] : 0.0;
 #pragma unroll
-  for (int k = 0; k < 72; ++k) K[k] = 0.0;
-  double re[3] = {0.0, 0.0, 0.0};
-#pragma unroll  // i indexes the register arrays K and re: unrolled, no scratch
-  for (int i = 0; i < 3; ++i) {
-    __syncthreads();  // sA free (previous i), sP written
+  for (int c = 0; c < 27; ++c) sA[c * EK_BS + tid] = valid ? wA[(int64_t)(27 * i + c) * G.n_qp + t] : 0.0;
+  if (UNIFORM)
+    for (int e = tid; e < 192; e += EK_BS) sG[e] = G.sg[e];
+  __syncthreads();
+  double K[24], re = 0.0;
 #pragma unroll
-    for (int c = 0; c < 27; ++c) sA[c][tid] = valid ? wA[(int64_t)(27 * i + c) * G.n_qp + t] : 0.0;
-    __syncthreads();
-    if (valid) {
+  for (int k = 0; k < 24; ++k) K[k] = 0.0;
+  if (valid) {
 #pragma unroll 1
-      for (int q = 0; q < 8; ++q) {
-        const int p = 8 * cl + q;
-        const int64_t qp = cell * 8 + q;
-        double ga[3], gb[24];
+    for (int q = 0; q < 8; ++q) {
+      const int p = 8 * cl + q;
+      const int64_t qp = cell * 8 + q;
+      double ga[3], gb[24];
 #pragma unroll
-        for (int c = 0; c < 24; ++c) gb[c] = sg_at(G, c, qp);
-        ga[0] = sg_at(G, 3 * a, qp);
-        ga[1] = sg_at(G, 3 * a + 1, qp);
-        ga[2] = sg_at(G, 3 * a + 2, qp);
-        double sr = 0.0;
+      for (int c = 0; c < 24; ++c) gb[c] = UNIFORM ? G.sg[c * 8 + q] : G.sg[c * G.n_qp + qp];
 #pragma unroll
-        for (int j = 0; j < 3; ++j) sr += sP[3 * i + j][p] * ga[j];
-        re[i] += sr;
-        double Z[9];  // Z[k][l] = sum_j ga_j A[(i j),(k l)]
+      for (int j = 0; j < 3; ++j) ga[j] = UNIFORM ? sG[(3 * a + j) * 8 + q] : G.sg[(3 * a + j) * G.n_qp + qp];
+      double sr = 0.0;
 #pragma unroll
-        for (int kl = 0; kl < 9; ++kl) {
-          double z = 0.0;
+      for (int j = 0; j < 3; ++j) sr += sP[j][p] * ga[j];
+      re += sr;
+      double Z[9];  // Z[k][l] = sum_j ga_j A[(i j),(k l)]
 #pragma unroll
-          for (int j = 0; j < 3; ++j) z += ga[j] * sA[9 * j + kl][p];
-          Z[kl] = z;
-        }
+      for (int kl = 0; kl < 9; ++kl) {
+        double z = 0.0;
 #pragma unroll
-        for (int b = 0; b < 8; ++b)
-#pragma unroll
-          for (int k = 0; k < 3; ++k)
-            K[b * 9 + i * 3 + k] += Z[3 * k] * gb[3 * b] + Z[3 * k + 1] * gb[3 * b + 1] + Z[3 * k + 2] * gb[3 * b + 2];
+        for (int j = 0; j < 3; ++j) z += ga[j] * sA[(9 * j + kl) * EK_BS + p];
+        Z[kl] = z;
       }
+#pragma unroll
+      for (int b = 0; b < 8; ++b)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) K[b * 3 + k] += Z[3 * k] * gb[3 * b] + Z[3 * k + 1] * gb[3 * b + 1] + Z[3 * k + 2] * gb[3 * b + 2];
     }
+    RE[t * 3 + i] = re;
   }
-  if (!valid) return;
-  double2* out = reinterpret_cast<double2*>(KE + t * 72);
+  __syncthreads();  // the tangents have been read
 #pragma unroll
-  for (int k = 0; k < 36; ++k) out[k] = make_double2(K[2 * k], K[2 * k + 1]);
+  for (int k = 0; k < 24; ++k) sA[tid * EK_PITCH + k] = K[k];
+  __syncthreads();
+  const int n = (int)std::max<int64_t>(0, std::min<int64_t>(EK_BS, G.n_qp - q0)) * 12;
 #pragma unroll
-  for (int k = 0; k < 3; ++k) RE[t * 3 + k] = re[k];
+  for (int m = 0; m < 12; ++m) {
+    const int e = tid + m * EK_BS, r = e / 12, c = 2 * (e % 12);
+    if (e < n)
+      *reinterpret_cast<double2*>(KE + ((q0 + r) * 3 + i) * 24 + c) = make_double2(sA[r * EK_PITCH + c], sA[r * EK_PITCH + c + 1]);
+  }
 }
 
 // ---------------------------------------------------------------------------------
-// Block-ELL gather: thread per (slot s, scalar row r = 3 i + c), padding slots included.
-// Sums the element blocks
-// that touch (node i, node col[s][i]) in ascending cell order (the order in which scipy's
-// COO->CSR sum_duplicates adds them, solver.py:281-282), then applies the row elimination
-// of get_A (solver.py:290-293): a Dirichlet row becomes zero with a unit diagonal.
-__global__ void __launch_bounds__(256) k_gather_matrix(BellView M, const double* __restrict__ KE,
-                                                      const int32_t* __restrict__ cptr, const int32_t* __restrict__ clist,
-                                                      const uint8_t* __restrict__ is_bc, double* __restrict__ vals) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t nrow = 3 * M.n_nodes;
-  if (t >= nrow * M.n_slots) return;
-  const int s = (int)(t / nrow);
-  const int64_t r = t - (int64_t)s * nrow;
-  const int64_t i = r / 3;
-  const int c = (int)(r - 3 * i);
-  double v0 = 0.0, v1 = 0.0, v2 = 0.0;
-  if (s >= M.nslot[i]) {
-    // padding slot (column = own node): explicit zeros so the SpMV can run a fixed slot count
-  } else if (is_bc[r]) {
-    const int64_t j = M.col[(int64_t)s * M.n_nodes + i];
-    if (j == i) {
-      v0 = (c == 0) ? 1.0 : 0.0;
-      v1 = (c == 1) ? 1.0 : 0.0;
-      v2 = (c == 2) ? 1.0 : 0.0;
+// Block-ELL gather.  A block takes 16 nodes and sums, in ascending cell order (the order in which
+// scipy's COO->CSR sum_duplicates adds them, solver.py:281-282), the rows of the element matrices
+// at each node into an LDS tile of 27 slots (in turns where a pattern has more); a node's rows in one
+// cell are 576 contiguous bytes.  24 lanes (b, c) take a node, two nodes a wave; slots: the slot of
+// node b in the row of node a, per (cell, a, b), and above it (GATHER_RANK) the number of earlier b
+// of the same cell with the same node (degenerate cells only, ranks > 1), which take turns.
+// The tile leaves with the row elimination of get_A (solver.py:290-293): a Dirichlet row becomes zero
+// with a unit diagonal.
+// Bound by memory (1.2 GB of element matrices read, 0.53 GB written at 64^3): 565 us; with a thread per
+// (slot, row), whose reads of 72 bytes use their lines about half, 620.
+constexpr int GN = 16, GBS = 32 * GN, GPITCH = 3 * GN + 1;
+__global__ void __launch_bounds__(GBS) k_gather_matrix(BellView M, const double* __restrict__ KE, const int32_t* __restrict__ nptr,
+                                                      const int32_t* __restrict__ nlist, const uint16_t* __restrict__ slots, int ranks,
+                                                      const int32_t* __restrict__ dslot, const uint8_t* __restrict__ is_bc,
+                                                      double* __restrict__ vals) {
+  __shared__ double T[81 * GPITCH];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int64_t node0 = (int64_t)blockIdx.x * GN, nrow = 3 * M.n_nodes;
+  const int half = lane / 24, j = lane - 24 * half, b = j / 3, c = j - 3 * b;
+  for (int s0 = 0; s0 < M.n_slots; s0 += 27) {
+    for (int e = tid; e < 81 * GPITCH; e += GBS) T[e] = 0.0;
+    __syncthreads();
+    const int nl = 2 * wave + half;
+    const int64_t i = node0 + nl;
+    if (half < 2 && i < M.n_nodes) {
+      const int e1 = nptr[i + 1];
+      for (int e0 = nptr[i]; e0 < e1; e0 += 8) {
+        double v[8][3];
+        int sl[8];
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          sl[m] = -1;
+          if (e0 + m < e1) {
+            const int64_t ca = nlist[e0 + m];
+            const double* src = KE + (ca * 3 + c) * 24 + 3 * b;
+            sl[m] = slots[ca * 8 + b];
+            v[m][0] = src[0];
+            v[m][1] = src[1];
+            v[m][2] = src[2];
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < 8; ++m) {
+          const int s = (sl[m] & (GATHER_RANK - 1)) - s0;
+          for (int r = 0; r < ranks; ++r) {
+            if (sl[m] >= 0 && sl[m] / GATHER_RANK == r && s >= 0 && s < 27) {
+              double* d = T + 3 * s * GPITCH + 3 * nl + c;
+              d[0] += v[m][0];
+              d[GPITCH] += v[m][1];
+              d[2 * GPITCH] += v[m][2];
+            }
+            asm volatile("" ::: "memory");  // another lane may add to the same entry next: LDS keeps a wave's order
+          }
+        }
+      }
     }
-  } else {
-    const int64_t e0 = cptr[(int64_t)s * M.n_nodes + i], e1 = cptr[(int64_t)s * M.n_nodes + i + 1];
-    for (int64_t e = e0; e < e1; ++e) {
-      const double* blk = KE + (int64_t)clist[e] * 9 + 3 * c;
-      v0 += blk[0];
-      v1 += blk[1];
-      v2 += blk[2];
+    __syncthreads();
+    const int rows = 3 * min(27, M.n_slots - s0);
+    for (int e = tid; e < rows * 3 * GN; e += GBS) {
+      const int row = e / (3 * GN), col = e - row * (3 * GN);
+      const int64_t r = 3 * node0 + col;
+      if (r >= nrow) continue;
+      double v = T[row * GPITCH + col];
+      if (is_bc[r]) v = s0 + row / 3 == dslot[node0 + col / 3] && row % 3 == col % 3 ? 1.0 : 0.0;
+      vals[(3 * (int64_t)s0 + row) * nrow + r] = v;
     }
+    __syncthreads();  // before the tile is cleared for the next slots
   }
-  vals[(3 * (int64_t)s + 0) * nrow + r] = v0;
-  vals[(3 * (int64_t)s + 1) * nrow + r] = v1;
-  vals[(3 * (int64_t)s + 2) * nrow + r] = v2;
 }
 
 // Residual gather + apply_bc_vec (solver.py:119-133): res[bc] = u[bc] - ubar.
@@ -517,7 +565,11 @@ k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __res
     });
   }
   if (!fits) {
-    if (sub == 0) general_local<N, TANGENT, L>(n_qp, Hd, G, u, sv, mv, *gen, cfg, self_block, q, o);
+    if (sub == 0) {
+      const OutOfLine f{G, sv, mv, cfg};
+      const LocalOut out = o;
+      general_local<N, TANGENT, L>(n_qp, Hd, f.G, u, f.sv, f.mv, *gen, f.cfg, self_block, q, out);
+    }
     return;
   }
   // every lane of a point writes its share of the components
@@ -659,16 +711,16 @@ void launch_element_K(const Geom& G, const double* wP, const double* wA, double*
   const int bs = 256;
   const int64_t nb = (G.n_qp + bs - 1) / bs;
   if (wA)
-    hipLaunchKernelGGL(k_element_K, dim3((unsigned)((G.n_qp + EK_BS - 1) / EK_BS)), dim3(EK_BS), 0, st, G, wP, wA, KE, RE);
+    hipLaunchKernelGGL(G.uniform ? k_element_K<true> : k_element_K<false>,
+                       dim3((unsigned)((G.n_qp + XCDS * EK_BS - 1) / (XCDS * EK_BS) * 3 * XCDS)), dim3(EK_BS), 0, st, G, wP, wA, KE, RE);
   else
     hipLaunchKernelGGL(k_element_R, dim3((unsigned)nb), dim3(bs), 0, st, G, wP, RE);
 }
 
-void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* cptr, const int32_t* clist, const uint8_t* is_bc,
-                          double* vals, hipStream_t st) {
-  const int bs = 256;
-  const int64_t n = 3 * M.n_nodes * M.n_slots;
-  hipLaunchKernelGGL(k_gather_matrix, dim3((unsigned)((n + bs - 1) / bs)), dim3(bs), 0, st, M, KE, cptr, clist, is_bc, vals);
+void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint16_t* slots,
+                          int ranks, const int32_t* dslot, const uint8_t* is_bc, double* vals, hipStream_t st) {
+  hipLaunchKernelGGL(k_gather_matrix, dim3((unsigned)((M.n_nodes + GN - 1) / GN)), dim3(GBS), 0, st, M, KE, nptr, nlist, slots, ranks,
+                     dslot, is_bc, vals);
 }
 
 void launch_gather_residual(int64_t n_nodes, const double* RE, const int32_t* nptr, const int32_t* nlist, const uint8_t* is_bc,

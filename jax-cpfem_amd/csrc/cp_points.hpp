@@ -113,6 +113,17 @@ __device__ __forceinline__ void setup_crystal(Crystal<N, L, KS>& pt, const Point
            rest.gi);
 }
 
+// Kernel arguments that go to a function out of line by reference, copied in the branch that calls it:
+// the arguments themselves would be stored to every lane's private memory at the kernel's start
+// (0.5 GB a launch at 64^3).
+struct OutOfLine {
+  Geom G;
+  StateView sv;
+  MatView mv;
+  SolveCfg cfg;
+  uint32_t n_it = 0, n_ev = 0;
+};
+
 // d dgamma / d tau and 1/g_old of the general form (cp_point.hpp), in the lane's private memory:
 // the functions that use them are called for the points that nothing else covers.
 template <int N>
