@@ -133,6 +133,12 @@ enum { CPFEM_APPLY_BC = 1 };
 int cpfem_assemble(cpfem_ctx* ctx, void* stream, const double* dofs, const CpfemState* state,
                    const CpfemParams* params, double* res, double* mat, int32_t* iters, int32_t flags);
 
+/* cpfem_assemble in two parts, for a caller that evaluates residuals at several dofs and wants the
+   matrix at one of them (a line search): with res, the residual, and the points' converged stresses
+   in stress ([6][n_qp], device); with mat, the matrix at the dofs whose stresses stress holds. */
+int cpfem_assemble_state(cpfem_ctx* ctx, void* stream, const double* dofs, const CpfemState* state,
+                         const CpfemParams* params, double* stress, double* res, double* mat, int32_t flags);
+
 /* Cell-averaged Cauchy stress (n_cells, 3, 3), device. */
 int cpfem_cell_stress(cpfem_ctx* ctx, void* stream, const double* dofs, const CpfemState* state,
                       const CpfemParams* params, double* sigma_cells);

@@ -72,6 +72,8 @@ _SIGS = {
                                    ctypes.POINTER(CpfemParams), vp, vp, vp, ctypes.POINTER(CpfemStateOut), vp]),
     "cpfem_assemble": (ctypes.c_int, [vp, vp, vp, ctypes.POINTER(CpfemState), ctypes.POINTER(CpfemParams),
                                       vp, vp, vp, ctypes.c_int32]),
+    "cpfem_assemble_state": (ctypes.c_int, [vp, vp, vp, ctypes.POINTER(CpfemState), ctypes.POINTER(CpfemParams),
+                                            vp, vp, vp, ctypes.c_int32]),
     "cpfem_cell_stress": (ctypes.c_int, [vp, vp, vp, ctypes.POINTER(CpfemState), ctypes.POINTER(CpfemParams), vp]),
     "cpfem_update_state": (ctypes.c_int, [vp, vp, vp, ctypes.POINTER(CpfemState), ctypes.POINTER(CpfemParams),
                                           ctypes.POINTER(CpfemStateOut)]),

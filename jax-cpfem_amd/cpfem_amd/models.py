@@ -259,15 +259,33 @@ class CrystalPlasticity(Problem):
         st, pr, keep = self._marshal(params)
         dofs = dofs.detach()
         res = torch.empty(self.ctx.n_dofs, dtype=torch.float64, device=device())
-        mat = None
-        if want_matrix:
-            if getattr(self, "_mat_buf", None) is None:
-                self._mat_buf = torch.empty(self.ctx.mat_len, dtype=torch.float64, device=device())
-            mat = self._mat_buf
+        mat = self._matrix_buffer() if want_matrix else None
         N.check(self.ctx._lib.cpfem_assemble(self.ctx.h, stream_handle(), ptr(dofs), ctypes.byref(st),
                                              ctypes.byref(pr), ptr(res), ptr(mat), ptr(iters),
                                              N.APPLY_BC if apply_bc else 0))
         return res, mat
+
+    def _matrix_buffer(self):
+        if getattr(self, "_mat_buf", None) is None:
+            self._mat_buf = torch.empty(self.ctx.mat_len, dtype=torch.float64, device=device())
+        return self._mat_buf
+
+    def residual_state(self, dofs, stress):
+        """Residual at dofs with the Dirichlet rows applied; the points' converged stresses go to
+        stress (6, n_qp)."""
+        st, pr, keep = self._marshal(self.internal_vars)
+        res = torch.empty(self.ctx.n_dofs, dtype=torch.float64, device=device())
+        N.check(self.ctx._lib.cpfem_assemble_state(self.ctx.h, stream_handle(), ptr(dofs.detach()), ctypes.byref(st),
+                                                   ctypes.byref(pr), ptr(stress), ptr(res), ptr(None), N.APPLY_BC))
+        return res
+
+    def matrix_at(self, dofs, stress):
+        """Jacobian values at dofs, from the stresses that residual_state stored there."""
+        st, pr, keep = self._marshal(self.internal_vars)
+        mat = self._matrix_buffer()
+        N.check(self.ctx._lib.cpfem_assemble_state(self.ctx.h, stream_handle(), ptr(dofs.detach()), ctypes.byref(st),
+                                                   ctypes.byref(pr), ptr(stress), ptr(None), ptr(mat), N.APPLY_BC))
+        return mat
 
     def newton_update(self, sol_list):
         """Raw residual list; the Jacobian is kept as ``self.A`` (jax-fem newton_update)."""

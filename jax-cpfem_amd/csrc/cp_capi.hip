@@ -986,55 +986,57 @@ int cpfem_local(cpfem_ctx* c, void* stream, int64_t n_qp, const double* u_grad, 
   return CPFEM_OK;
 }
 
-int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemState* state, const CpfemParams* params,
-                   double* res, double* mat, int32_t* iters, int32_t flags) {
-  if (!c || !dofs || !res) return fail(CPFEM_EBADARG, "null argument");
+// The assembly's passes.  res: local Newton, whose converged stresses go to `stress` if that is set, and
+// the residual; mat: the matrix from the stresses of an earlier or the same call.
+static int assemble_passes(cpfem_ctx* c, hipStream_t st, const double* dofs, const CpfemState* state, const CpfemParams* params,
+                           double* stress, double* res, double* mat, int32_t* iters, int32_t flags) {
   int rc;
-  if ((rc = check_state(c, state, params))) return rc;
-  if (mat && (rc = ensure_matrix_buffers(c))) return rc;
-  hipStream_t st = (hipStream_t)stream;
   const Geom G = c->geom();
   const StateView sv = state_view(state, c->n_qp);
   const MatView mv = mat_view(params);
   const SolveCfg cfg = solve_cfg(params);
   double* wA = mat ? c->d_wA : nullptr;
-  double* sout = mat ? c->d_sconv : nullptr;  // converged stresses for the tangent kernel
   Prof* pf = &c->prof;
-  PointPark pk{c->d_park_idx, c->d_park_s, c->d_park_it, c->d_park_ctr, c->n_qp, c->park_lanes};
-  if (pk.lanes > 0) {
-    if ((rc = ensure_park(c))) return rc;
-    pk = PointPark{c->d_park_idx, c->d_park_s, c->d_park_it, c->d_park_ctr, c->n_qp, c->park_lanes};
-    launch_zero_words(pk.ctr, 2, st);
-  }
-  int sl = prof_begin(pf, PC_ELEMENT_QP, st);
-  if (c->n_slip == 12)
-    launch_element_qp<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
-  else
-    launch_element_qp<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
-  prof_end(pf, sl, st);
-  if (pk.lanes > 0) {
-    sl = prof_begin(pf, PC_ELEMENT_PARK, st);
+  int sl;
+  if (res) {
+    PointPark pk{c->d_park_idx, c->d_park_s, c->d_park_it, c->d_park_ctr, c->n_qp, c->park_lanes};
+    if (pk.lanes > 0) {
+      if ((rc = ensure_park(c))) return rc;
+      pk = PointPark{c->d_park_idx, c->d_park_s, c->d_park_it, c->d_park_ctr, c->n_qp, c->park_lanes};
+      launch_zero_words(pk.ctr, 2, st);
+    }
+    sl = prof_begin(pf, PC_ELEMENT_QP, st);
     if (c->n_slip == 12)
-      launch_element_qp_park<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
+      launch_element_qp<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, stress, iters, c->d_status, c->d_counts, pk, st);
     else
-      launch_element_qp_park<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, sout, iters, c->d_status, c->d_counts, pk, st);
+      launch_element_qp<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, stress, iters, c->d_status, c->d_counts, pk, st);
     prof_end(pf, sl, st);
+    if (pk.lanes > 0) {
+      sl = prof_begin(pf, PC_ELEMENT_PARK, st);
+      if (c->n_slip == 12)
+        launch_element_qp_park<12>(G, dofs, sv, mv, c->pt12, cfg, c->d_wP, stress, iters, c->d_status, c->d_counts, pk, st);
+      else
+        launch_element_qp_park<24>(G, dofs, sv, mv, c->pt24, cfg, c->d_wP, stress, iters, c->d_status, c->d_counts, pk, st);
+      prof_end(pf, sl, st);
+    }
   }
   if (mat) {
     sl = prof_begin(pf, PC_TANGENT, st);
     if (c->n_slip == 12)
-      launch_point_tangent<12>(G, dofs, sv, mv, c->pt12, sout, wA, st);
+      launch_point_tangent<12>(G, dofs, sv, mv, c->pt12, stress, wA, st);
     else
-      launch_point_tangent<24>(G, dofs, sv, mv, c->pt24, sout, wA, st);
+      launch_point_tangent<24>(G, dofs, sv, mv, c->pt24, stress, wA, st);
     prof_end(pf, sl, st);
   }
   sl = prof_begin(pf, PC_ELEMENT_K, st);
-  launch_element_K(G, c->d_wP, wA, c->d_KE, c->d_RE, st);
+  launch_element_K(G, c->d_wP, wA, c->d_KE, c->d_RE, st);  // (without res, the residual's part is not used)
   prof_end(pf, sl, st);
   const uint8_t* isbc = (flags & CPFEM_APPLY_BC) ? c->d_isbc : c->d_nobc;
-  sl = prof_begin(pf, PC_GATHER_RES, st);
-  launch_gather_residual(c->n_nodes, c->d_RE, c->d_nptr, c->d_nlist, isbc, c->d_ubar, dofs, res, st);
-  prof_end(pf, sl, st);
+  if (res) {
+    sl = prof_begin(pf, PC_GATHER_RES, st);
+    launch_gather_residual(c->n_nodes, c->d_RE, c->d_nptr, c->d_nlist, isbc, c->d_ubar, dofs, res, st);
+    prof_end(pf, sl, st);
+  }
   if (mat) {
     sl = prof_begin(pf, PC_GATHER_MAT, st);
     launch_gather_matrix(c->bell(), c->d_KE, c->d_nptr, c->d_nlist, c->d_slots, c->slot_ranks, c->d_dslot, isbc, mat, st);
@@ -1042,6 +1044,24 @@ int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemSt
   }
   HIPCHK(hipGetLastError());
   return CPFEM_OK;
+}
+
+int cpfem_assemble(cpfem_ctx* c, void* stream, const double* dofs, const CpfemState* state, const CpfemParams* params,
+                   double* res, double* mat, int32_t* iters, int32_t flags) {
+  if (!c || !dofs || !res) return fail(CPFEM_EBADARG, "null argument");
+  int rc;
+  if ((rc = check_state(c, state, params))) return rc;
+  if (mat && (rc = ensure_matrix_buffers(c))) return rc;
+  return assemble_passes(c, (hipStream_t)stream, dofs, state, params, mat ? c->d_sconv : nullptr, res, mat, iters, flags);
+}
+
+int cpfem_assemble_state(cpfem_ctx* c, void* stream, const double* dofs, const CpfemState* state, const CpfemParams* params,
+                         double* stress, double* res, double* mat, int32_t flags) {
+  if (!c || !dofs || !stress || (!res && !mat)) return fail(CPFEM_EBADARG, "null argument");
+  int rc;
+  if ((rc = check_state(c, state, params))) return rc;
+  if (mat && (rc = ensure_matrix_buffers(c))) return rc;
+  return assemble_passes(c, (hipStream_t)stream, dofs, state, params, stress, res, mat, nullptr, flags);
 }
 
 int cpfem_cell_stress(cpfem_ctx* c, void* stream, const double* dofs, const CpfemState* state, const CpfemParams* params,

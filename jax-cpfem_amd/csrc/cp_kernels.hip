@@ -457,10 +457,16 @@ __global__ void __launch_bounds__(256) k_element_R(Geom G, const double* __restr
 #pragma unroll 1
   for (int q = 0; q < 8; ++q) {
     const int64_t qp = cell * 8 + q;
-    const double g0 = sg_at(G, 3 * a, qp), g1 = sg_at(G, 3 * a + 1, qp), g2 = sg_at(G, 3 * a + 2, qp);
+    double ga[3];
 #pragma unroll
-    for (int i = 0; i < 3; ++i)
-      re[i] += wP[(3 * i) * G.n_qp + qp] * g0 + wP[(3 * i + 1) * G.n_qp + qp] * g1 + wP[(3 * i + 2) * G.n_qp + qp] * g2;
+    for (int j = 0; j < 3; ++j) ga[j] = sg_at(G, 3 * a + j, qp);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      double sr = 0.0;  // the sum of k_element_K, to the bit
+#pragma unroll
+      for (int j = 0; j < 3; ++j) sr += wP[(3 * i + j) * G.n_qp + qp] * ga[j];
+      re[i] += sr;
+    }
   }
 #pragma unroll
   for (int i = 0; i < 3; ++i) RE[t * 3 + i] = re[i];
