@@ -316,7 +316,8 @@ struct Crystal {
     };
     double rest = K < M ? gr[0] : 0.0;
     double next = gi[0];
-#pragma unroll 2
+    // (a lane of three systems evaluates them together: their chains fill each other's latency)
+#pragma unroll(M == 3 ? 3 : 2)
     for (int j = 0; j < K; ++j) {
       const double gia = next;
       next = gi[(j + 1 < K ? j + 1 : j) * sti];  // in flight during this system
@@ -344,7 +345,7 @@ struct Crystal {
   CPFEM_HD void dyads(const Tab& tab, double* Z) const {
 #pragma unroll
     for (int i = 0; i < 40; ++i) Z[i] = 0.0;
-#pragma unroll 1
+#pragma unroll(M == 3 ? 3 : 1)
     for (int m = 0; m < M; ++m) {
       const int a = L == 1 ? m : a0 + m;
       const double g = gp(m);
