@@ -760,11 +760,11 @@ static int run_mg(cpfem_ctx* c, hipStream_t st, const double* mat, const TM* mat
   __atomic_store_n(c->h_flag, (uint64_t)0, __ATOMIC_RELEASE);
   mg_krylov_init(mg, M, mat, b, v, w, tol, atol, std::min(maxiter, MG_MAXITER), st);
   HIPCHK(hipGetLastError());
-  // An iteration's first kernel reports the convergence test in the pinned word; the next
-  // iteration is queued once it has, while the rest of this one runs.
+  // An iteration's first kernel reports the convergence test in the pinned word; the rest of the
+  // iteration is queued once it has, while the finest level is smoothed.
   uint64_t f = 0;
   for (int it = 0; it <= MG_MAXITER + 1; ++it) {
-    mg_krylov_iteration<TM>(mg, M, mat, matp, v, w, it, c->h_flag, st, &c->prof);
+    mg_krylov_begin<TM>(mg, M, matp, v, w, it, c->h_flag, st, &c->prof);
     HIPCHK(hipGetLastError());
     for (unsigned spin = 0;; ++spin) {
       f = __atomic_load_n(c->h_flag, __ATOMIC_ACQUIRE);
@@ -779,6 +779,7 @@ static int run_mg(cpfem_ctx* c, hipStream_t st, const double* mat, const TM* mat
       }
     }
     if (f >> 32 & 1) break;
+    mg_krylov_finish<TM>(mg, M, mat, matp, v, w, it, st, &c->prof);
   }
   launch_residual64(M, mat, x, b, c->d_tmp64, st);
   launch_residual_norm(c->n_dofs, c->d_tmp64, c->d_tmp64, c->d_partial, c->nb, c->d_scalar, st);

@@ -268,11 +268,15 @@ struct MgVec {
 };
 void mg_krylov_init(const Multigrid& mg, const BellView& M, const double* vals, const double* b, MgVec v, KrylovWork w,
                     double tol, double atol, int maxiter, hipStream_t st);
-// One iteration; vals: FP64 operator, valsp: the preconditioner's values of the same matrix.
-// flag: host word that the first kernel sets to (iteration + 1) << 33 | done << 32 | k.
+// One iteration, in two parts; vals: FP64 operator, valsp: the preconditioner's values of the same
+// matrix.  flag: host word that the first kernel of mg_krylov_begin sets to
+// (iteration + 1) << 33 | done << 32 | k.
 template <typename TM>
-void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w,
-                         int iter, uint64_t* flag, hipStream_t st, Prof* prof);
+void mg_krylov_begin(const Multigrid& mg, const BellView& M, const TM* valsp, MgVec v, KrylovWork w, int iter, uint64_t* flag,
+                     hipStream_t st, Prof* prof);
+template <typename TM>
+void mg_krylov_finish(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w, int iter,
+                      hipStream_t st, Prof* prof);
 int mg_spmv_blocks(int64_t n);
 int mg_dense_tiles(int64_t n);  // tiles per side of the last level's n rows
 

@@ -211,7 +211,10 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_smooth(BellView M, const 
                                                              double c1, double c2, const double* __restrict__ lam,
                                                              const int32_t* __restrict__ done, int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
-  const int dn = *done;  // tested when the product is there: one round trip less per pass
+  // tested when the product is there, one round trip less per pass; but a pass over the finest matrix
+  // (14 us at 32^3, 108 at 64^3) is not made for nothing
+  const int dn = *done;
+  if (FINE && P == 1 && dn) return;
   const double c2l = c2 * lam[0];
   int r;
   double acc;
@@ -228,6 +231,7 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_resid(BellView M, const T
                                                             const int32_t* __restrict__ done, int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
   const int dn = *done;
+  if (FINE && P == 1 && dn) return;
   int r;
   double acc;
   if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red) || dn) return;
@@ -661,20 +665,27 @@ static double* smooth_level(const Multigrid& mg, int l, const BellView& M, const
   return cur;
 }
 
-// One V-cycle: out = M b; level 0's first iterate is already in x0.
+// Smoothing of the finest level from its first iterate in x0, the first part of a V-cycle.
 template <typename TM>
-static void vcycle(const Multigrid& mg, const BellView& M, const TM* vals, const double* invd, const double* b, double* out,
-                   const int32_t* done, int* pass, hipStream_t st, Prof* prof) {
-  static const Cheb cf = cheb(DEG_FINE, LOW_FINE), cc = cheb(DEG_COARSE, LOW_COARSE);
+static double* smooth_fine(const Multigrid& mg, const BellView& M, const TM* vals, const double* b, const int32_t* done, int* pass,
+                           hipStream_t st, Prof* prof) {
+  static const Cheb cf = cheb(DEG_FINE, LOW_FINE);
+  return level_parts(mg.lv[0].g.n) == 1 ? smooth_level<TM, true, 1>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof)
+                                        : smooth_level<TM, true, 3>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof);
+}
+
+// The rest of the V-cycle: out = M b, from the finest level's iterate and its residual.
+template <typename TM>
+static void vcycle(const Multigrid& mg, const BellView& M, double* iterate, const double* invd, const double* b, double* out,
+                   const int32_t* done, hipStream_t st, Prof* prof) {
+  static const Cheb cc = cheb(DEG_COARSE, LOW_COARSE);
   double* cur[MG_MAXL];
   const int last = mg.nl - 1;
+  cur[0] = iterate;
   for (int l = 0; l < last; ++l) {
     const MgLevel& L = mg.lv[l];
     int p = 0;
-    if (l == 0) {
-      cur[0] = level_parts(L.g.n) == 1 ? smooth_level<TM, true, 1>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof)
-                                       : smooth_level<TM, true, 3>(mg, 0, M, vals, b, cf, DEG_FINE, done, pass, st, prof);
-    } else {
+    if (l > 0) {
       const TM* A = static_cast<const TM*>(L.A);
       cur[l] = level_parts(L.g.n) == 1 ? smooth_level<TM, false, 1>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof)
                                        : smooth_level<TM, false, 3>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof);
@@ -909,9 +920,22 @@ void mg_krylov_init(const Multigrid& mg, const BellView& M, const double* vals, 
   hipLaunchKernelGGL(k_mgb_init2, dim3(1), dim3(KBS), 0, st, w, tol, atol, maxiter);
 }
 
+// An iteration in two parts, so that the host can read the first one's convergence test before it
+// queues the second: what a converged solve has queued in vain is then the smoothing of one level
+// and not an iteration (16^3: 18 of 115 us).
 template <typename TM>
-void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w,
-                         int iter, uint64_t* flag, hipStream_t st, Prof* prof) {
+void mg_krylov_begin(const Multigrid& mg, const BellView& M, const TM* valsp, MgVec v, KrylovWork w, int iter, uint64_t* flag,
+                     hipStream_t st, Prof* prof) {
+  const MgLevel& L = mg.lv[0];
+  const double ith = cheb(DEG_FINE, LOW_FINE).ith;
+  int pass = 1;  // the product that comes before walked forwards
+  timed(prof, PC_KVEC, k_mgb_p, dim3((unsigned)w.nb), dim3(KBS), st, v, w, iter & 1, iter, (const double*)L.minv, L.x0, ith,
+        (const double*)mg.lam, flag);
+  smooth_fine<TM>(mg, M, valsp, v.p, &w.sc->done, &pass, st, prof);
+}
+template <typename TM>
+void mg_krylov_finish(const Multigrid& mg, const BellView& M, const double* vals, const TM* valsp, MgVec v, KrylovWork w, int iter,
+                      hipStream_t st, Prof* prof) {
   const MgLevel& L = mg.lv[0];
   const MgGrid g = L.g;
   const double ith = cheb(DEG_FINE, LOW_FINE).ith;
@@ -919,15 +943,15 @@ void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* v
   const dim3 vb((unsigned)w.nb), vt(KBS), sb((unsigned)w.nbs), s1(MgShape<1>::BS), s3(MgShape<3>::BS);
   const int32_t* done = &w.sc->done;
   const int par = iter & 1;
-  int pass = 1;  // the product that comes before walked forwards
-  timed(prof, PC_KVEC, k_mgb_p, vb, vt, st, v, w, par, iter, (const double*)L.minv, L.x0, ith, (const double*)mg.lam, flag);
-  vcycle<TM>(mg, M, valsp, v.invd, v.p, v.phat, done, &pass, st, prof);
+  int pass = 1 + DEG_FINE;  // those of mg_krylov_begin
+  vcycle<TM>(mg, M, (DEG_FINE - 1) & 1 ? L.x1 : L.x0, v.invd, v.p, v.phat, done, st, prof);
   if (one)
     timed(prof, PC_SPMV, k_mgb_q<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
   else
     timed(prof, PC_SPMV, k_mgb_q<3>, sb, s3, st, M, g, vals, v, w, level_order(g.n, pass++));
   timed(prof, PC_KVEC, k_mgb_s, vb, vt, st, v, w, par, w.nbs, (const double*)L.minv, L.x0, ith, (const double*)mg.lam);
-  vcycle<TM>(mg, M, valsp, v.invd, v.s, v.shat, done, &pass, st, prof);
+  double* it = smooth_fine<TM>(mg, M, valsp, v.s, done, &pass, st, prof);
+  vcycle<TM>(mg, M, it, v.invd, v.s, v.shat, done, st, prof);
   if (one)
     timed(prof, PC_SPMV, k_mgb_t<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
   else
@@ -937,8 +961,10 @@ void mg_krylov_iteration(const Multigrid& mg, const BellView& M, const double* v
 
 #define CPFEM_MG_INST(TM)                                                                                                   \
   template void mg_setup<TM>(const Multigrid&, const double*, const double*, const uint8_t*, double*, hipStream_t);         \
-  template void mg_krylov_iteration<TM>(const Multigrid&, const BellView&, const double*, const TM*, MgVec, KrylovWork, int, \
-                                        uint64_t*, hipStream_t, Prof*);
+  template void mg_krylov_begin<TM>(const Multigrid&, const BellView&, const TM*, MgVec, KrylovWork, int, uint64_t*,          \
+                                    hipStream_t, Prof*);                                                                    \
+  template void mg_krylov_finish<TM>(const Multigrid&, const BellView&, const double*, const TM*, MgVec, KrylovWork, int,   \
+                                     hipStream_t, Prof*);
 CPFEM_MG_INST(double)
 CPFEM_MG_INST(float)
 
