@@ -8,7 +8,7 @@ seeded uniform-SO(3) orientations, 20% of the grains hard (g0 x4, h0 x2), FP64.
 A step is one load step (load step 1: 1e-3 strain, dt = 1 s) re-run from its snapshot (the
 state before it), with all of its work: the global Newton to the reference tolerances with
 the dual-phase driver's line search (per-point Kalidindi update + consistent tangent, hex8
-assembly into the block-ELL Jacobian, Jacobi-BiCGSTAB solves, line-search residuals), then
+assembly into the block-ELL Jacobian, multigrid-preconditioned BiCGSTAB solves, line-search residuals), then
 the cell-averaged Cauchy stress and the history update, through the drop-in
 ``solver(problem, solver_options)`` loop.  (The reference algorithm, local Newton from S = 0
 with cut-half backtracking, does not get through load step 2 of this workload from 24^3 up:
@@ -21,7 +21,8 @@ timed with HIP events on its launch stream; ``detail`` carries the mixed-precisi
 the adjoint gradients (this workload's load step w.r.t. its 900 Euler angles, and the
 calibration workload's 50-step history w.r.t. five hardening parameters), and the point
 kernel's FP64 roofline.  ``cpu_baseline`` times the C++/OpenMP restatement of the same
-algorithm on the host's cores on a bounded sample of the same state.
+algorithm on the host's cores on a bounded sample of the same state; its Krylov iterations are
+those of the reference's Jacobi-BiCGSTAB, counted in an untimed load step with that solver.
 """
 import argparse
 import ctypes
@@ -68,6 +69,18 @@ def spmv_bytes(prob, value_bytes=8, computed_columns=False, one_operand=False):
             idx -= 4 * 27 * (nx - 2) * (ny - 2) * (nz - 2)
     vec = (7 + 6) / 2 if one_operand else (7 + 5) / 2
     return round(9 * value_bytes * nnzb + idx + vec * 8 * n), nnzb
+
+
+def mg_bytes(prob, value_bytes=8, vectors=3.0):
+    """Algorithmic HBM bytes of one product with the finest matrix in the multigrid solve: as
+    spmv_bytes, with the columns of the nodes off the box's faces computed, and `vectors` FP64 row
+    vectors: 3 in the Krylov products (k_mgb_q: phat, rhat, q; k_mgb_t: shat, s, t), and in the
+    smoother 19/4, the mean of three k_mg_smooth (iterate, previous iterate, right-hand side, inverse
+    diagonal, result) and one k_mg_resid (iterate, right-hand side, mask, residual)."""
+    nslot, _ = prob.ctx.pattern()
+    nnzb = int(nslot.sum())
+    nx, ny, nz = prob.ctx.box_numbering()
+    return round(9 * value_bytes * nnzb + 4 * (nnzb - 27 * (nx - 2) * (ny - 2) * (nz - 2)) + vectors * 8 * prob.ctx.n_dofs)
 
 
 def point_flops(n_slip, tangent_points, newton_iters, residual_evals):
@@ -149,14 +162,17 @@ class StepRunner:
         self.prob, self.w, self.index = prob, w, index
         self.params, self.sol = params, sol
 
-    def run(self, precision, on_step=None):
+    def run(self, precision, on_step=None, jacobi=False):
         from cpfem_amd import configs
-        return configs.run_steps(self.prob, self.w, self.params, [self.sol[0]], self.index, self.index + 1,
-                                 {"precision": precision}, on_step=on_step)
+        opts = {"precision": precision}
+        if jacobi:  # the reference's preconditioner
+            opts["jax_solver"] = {"precond": "jacobi"}
+        return configs.run_steps(self.prob, self.w, self.params, [self.sol[0]], self.index, self.index + 1, opts,
+                                 on_step=on_step)
 
 
 # ------------------------------------------------------------------------------ adjoints
-def step_adjoint(prob, w, index, szz_ref, precision):
+def step_adjoint(prob, w, index, szz_ref, precision, jacobi=False):
     """Gradient of (mean szz after load step `index` - target)^2 w.r.t. the per-grain z-y-x
     Euler angles (the orientation-design loss of poly_sensitivity_rot_mesh2.py:179-239, with
     R = R_euler(theta) R_quat per grain as at :203), through the forward load step and its
@@ -177,11 +193,14 @@ def step_adjoint(prob, w, index, szz_ref, precision):
     theta = torch.zeros(len(w.quat), 3, dtype=torch.float64, device="cuda", requires_grad=True)
     target = 1.05 * szz_ref
     opts = dict(w.solver_options, precision=precision)
+    adjoint_opts = {"precision": precision}
+    if jacobi:
+        opts["jax_solver"] = adjoint_opts["jax_solver"] = {"precond": "jacobi"}
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     R = alpha_rotate_tensor_rank_2(rotate_theta_transfer(theta), Rq)[gid].unsqueeze(1).expand(nc, 8, 3, 3)
     szz = C.simulate(prob, load, g0, mat8, R, checkpoint_every=5, solver_options=opts,
-                     adjoint_solver_options={"precision": precision})[-1, 2, 2]
+                     adjoint_solver_options=adjoint_opts)[-1, 2, 2]
     loss = (szz - target) ** 2
     torch.cuda.synchronize()
     t1 = time.perf_counter()
@@ -268,10 +287,10 @@ def cpu_baseline(prob, w, params, sol, index, per_step, krylov_iters=40, adjoint
     on a bounded sample of the timed load step: one full assembly (every point's local Newton
     and tangent, element stiffness, CSR gather), one residual-only assembly (the line search's),
     one point pass without tangent and `krylov_iters` Jacobi-BiCGSTAB iterations on the
-    assembled CSR matrix at the converged state, scaled by the GPU run's per-step counts of
+    assembled CSR matrix at the converged state, scaled by the reference algorithm's per-step counts of
     Jacobian assemblies, residual-only assemblies, point passes (cell stress, history update)
-    and Krylov iterations.  With adjoint_krylov_iters (the GPU backward's transposed-solve
-    iterations of the load-step adjoint) also one per-point VJP pass, and the adjoint gradient
+    and Krylov iterations (per_step).  With adjoint_krylov_iters (its transposed-solve
+    iterations in the backward of the load-step adjoint) also one per-point VJP pass, and the adjoint gradient
     is estimated as the load step plus its backward: two VJP passes, one Jacobian assembly at
     the converged state and the transposed solve."""
     from oracle.cpu import cpu_ref
@@ -300,7 +319,7 @@ def cpu_baseline(prob, w, params, sol, index, per_step, krylov_iters=40, adjoint
                        f"gather; {info['newton_iters'] / Q:.2f} local iterations per point), one residual-only "
                        f"assembly ({t_res:.2f} s), one point pass without tangent ({t_post:.2f} s) and {krylov_iters} "
                        f"Jacobi-BiCGSTAB iterations on the {info['n_dofs']}-dof CSR matrix ({t_it * 1e3:.1f} "
-                       f"ms/iteration), scaled by the GPU run's per-step counts ({per_step['assemblies']:.1f} Jacobian "
+                       f"ms/iteration), scaled by the reference algorithm's per-step counts ({per_step['assemblies']:.1f} Jacobian "
                        f"assemblies, {per_step['residual_assemblies']:.1f} residual-only assemblies, 2 point passes, "
                        f"{per_step['krylov_iters']:.0f} Krylov iterations): est. {step_s:.1f} s per load step"),
                load_step_s=step_s)
@@ -442,8 +461,10 @@ def main():
     log(f"[bench] timed {K} steps in {T:.3f}s ({T / K:.3f} s/step); newton {counts['newton'] / K:.1f}/step; "
         "profile: " + ", ".join(f"{c}={kp[c]['est_total_ms']:.1f}ms/{kp[c]['launches']}" for c in kp))
     assemblies = counts["newton"] + K  # one Jacobian assembly per Newton iteration plus the initial one
-    # every assembly launches the point kernel once; the others are the line search's residuals
-    res_assemblies = max(kp["element_qp"]["launches"] - assemblies, 0)
+    # the point kernel runs once per residual: in each assembly and each trial of the line search, where
+    # the accepted trial is the next iteration's assembly too (the reference solves its points again)
+    line_search = bool(w.solver_options.get("line_search_flag", False))
+    res_assemblies = max(kp["element_qp"]["launches"] - (K if line_search else assemblies), 0)
     per_step = dict(assemblies=assemblies / K, residual_assemblies=res_assemblies / K,
                     krylov_iters=sum(max(k, 0) for k in kry) / K)
 
@@ -456,10 +477,13 @@ def main():
     cus = torch.cuda.get_device_properties(0).multi_processor_count
     tm = "float" if vb == 4 else "double"
     names = spmv_kernel_names(form, tm)
+    multigrid = kp["mg_fine"]["launches"] > 0
+    if multigrid:
+        sb, names = mg_bytes(prob), ["cpfem::k_mgb_q", "cpfem::k_mgb_t"]
     tkey = f"c{args.config}_{n_mesh}"
     point_ms = lambda: (kp["element_qp"]["est_total_ms"] + kp["element_qp_park"]["est_total_ms"]
                         + kp["point_tangent"]["est_total_ms"])
-    dom = max(("krylov_spmv", "element_qp", "element_K", "gather_matrix", "krylov_vector", "point_local"),
+    dom = max(("krylov_spmv", "element_qp", "element_K", "gather_matrix", "krylov_vector", "point_local", "mg_fine", "mg_coarse"),
               key=lambda c: point_ms() if c == "element_qp" else kp[c]["est_total_ms"])
     # Launches that move the matrix: two per BiCGSTAB iteration plus the initial residual of each
     # solve (the launches queued past convergence return at once and move nothing, so the class
@@ -474,14 +498,29 @@ def main():
                          frac=round(ach / HBM_PEAK_GBS, 4), traffic=(round(traffic) if traffic else None),
                          traffic_source=(f"rocprofv3 FETCH_SIZE+WRITE_SIZE per dispatch, copy-kernel scaled "
                                          f"(profiles/traffic_{tkey}.txt)" if traffic else None),
-                         kernel=f"{names[0]} / {names[1]} (BiCGSTAB SpMV with fused p/s updates and dots)",
+                         kernel=f"{names[0]} / {names[1]} (BiCGSTAB SpMV with fused "
+                                f"{'dots' if multigrid else 'p/s updates and dots'})",
                          bytes_per_launch=sb, avg_launch_us=round(t_launch * 1e3, 2), working_launches=working,
                          timing="hipExtLaunchKernelGGL start/stop events (kernel-bound) on every "
                                 f"{args.profile_sample}th launch of the class, on its launch stream")
+    mg_roof = None
+    if multigrid and kp["mg_fine"]["avg_ms"] and kry:
+        # four products per V-cycle, two cycles per iteration; the smoothing queued with a solve's last
+        # test returns at once, or counts as time of the working ones
+        mg_working = 8 * sum(max(k, 0) for k in kry)
+        mb = mg_bytes(prob, vb, 19 / 4)
+        t_launch = kp["mg_fine"]["est_total_ms"] / mg_working
+        ach = mb / (t_launch * 1e-3) / 1e9
+        mg_roof = dict(bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS, unit="GB/s", frac=round(ach / HBM_PEAK_GBS, 4),
+                       traffic=None, kernel=f"cpfem::k_mg_smooth<{tm}> / cpfem::k_mg_resid<{tm}> (Chebyshev smoothing of the "
+                                            "finest level)",
+                       bytes_per_launch=mb, avg_launch_us=round(t_launch * 1e3, 2), working_launches=mg_working,
+                       timing="hipExtLaunchKernelGGL start/stop events (kernel-bound) on every "
+                              f"{args.profile_sample}th launch of the class, on its launch stream")
     point_roof = None
     qp = kp["element_qp"]
     if qp["avg_ms"] and qp["launches"]:
-        tangent_launches = assemblies  # one Jacobian assembly per Newton iteration plus the initial one
+        tangent_launches = kp["point_tangent"]["launches"]
         flops = point_flops(prob.num_slip_sys, Q * tangent_launches, work["newton_iters"], work["residual_evals"])
         t_ms = point_ms()
         ach_tf = flops / (t_ms * 1e-3) / 1e12
@@ -497,7 +536,7 @@ def main():
                           residual_evals_per_point_launch=round(work["residual_evals"] / (Q * qp["launches"]), 3),
                           flop_model="F_res(N)=41N+350 per residual evaluation, F_jac(N)=165N+2574 + F_LU=648 per "
                                      "iteration, F_tan=9300 per tangent (reference algorithm counts)")
-    roof = spmv_roof if dom == "krylov_spmv" else (point_roof if dom == "element_qp" else
+    roof = spmv_roof if dom == "krylov_spmv" else mg_roof if dom == "mg_fine" else (point_roof if dom == "element_qp" else
                                                     dict(bound=None, achieved=None, peak=None, unit=None, frac=None,
                                                          traffic=None, kernel=dom))
     szz = [float(s[2, 2]) for s in sigs]
@@ -505,7 +544,7 @@ def main():
         kernel_profile=kp, dominant=dom, newton_per_step=counts["newton"] / K, krylov_per_solve=kry[: 40],
         per_step=per_step, point_work=work, sigma_bar_zz=szz[0], sigma_bar_zz_spread=max(szz) - min(szz),
         nnz_blocks=nnzb, n_dofs=prob.ctx.n_dofs, krylov_form=form, spmv_bytes_per_launch=sb, load_step_s=T / K,
-        spmv_roofline=spmv_roof, point_roofline=point_roof)
+        spmv_roofline=spmv_roof, mg_roofline=mg_roof, point_roofline=point_roof)
 
     if args.mixed_steps > 0:
         other = "mixed" if args.precision == "fp64" else "fp64"
@@ -567,8 +606,12 @@ def main():
     if not args.no_cpu:
         log("[bench] CPU baseline (C++/OpenMP restatement) ...")
         adj = detail.get("adjoint_load_step")
-        cpu = cpu_baseline(prob, w, runner.params, [final_sol[0]], S, per_step,
-                           adjoint_krylov_iters=adj["backward_krylov_iters"] if adj else None)
+        # the reference's iteration counts: one untimed load step (and gradient) with its preconditioner
+        prob.solver_info.clear()
+        runner.run(args.precision, jacobi=True)
+        reference = dict(per_step, krylov_iters=sum(max(d["iterations"], 0) for d in prob.solver_info))
+        back = step_adjoint(prob, w, S, szz[0], args.precision, jacobi=True)["backward_krylov_iters"] if adj else None
+        cpu = cpu_baseline(prob, w, runner.params, [final_sol[0]], S, reference, adjoint_krylov_iters=back)
         detail["speedup_vs_cpu_load_step"] = cpu["load_step_s"] / (T / K)
         if adj:
             detail["speedup_vs_cpu_adjoint_grad"] = dict(fp64=cpu["adjoint_grad_s"] / adj["grad_s"],
@@ -586,7 +629,8 @@ def main():
         "dtype": "f64" if args.precision == "fp64" else "f64+f32-krylov",
         "data": "synthetic (seeded Voronoi polycrystal, uniform SO(3) orientations)",
         "config": {"workload": w.name, "n_qp": Q, "load_step": f"{S + 1} of {len(w.ts) - 1}, re-run from its snapshot",
-                   "precision": args.precision, "solver": "row-elimination Newton, Jacobi-BiCGSTAB tol=atol=1e-10",
+                   "precision": args.precision, "solver": f"row-elimination Newton, {'multigrid' if multigrid else 'Jacobi'}-preconditioned BiCGSTAB "
+                             "tol=atol=1e-10",
                    "solver_options": w.solver_options},
         "roofline": roof,
         "cpu_baseline": cpu,
