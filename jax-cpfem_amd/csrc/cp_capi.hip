@@ -121,7 +121,7 @@ struct cpfem_ctx {
   double* d_sg = nullptr;
   double* d_jxw = nullptr;
   int32_t *d_col = nullptr, *d_nslot = nullptr, *d_dslot = nullptr, *d_tslot = nullptr;
-  uint16_t* d_slots = nullptr;  // (cell, a, b) -> slot, rank
+  uint32_t* d_slots = nullptr;  // (cell, a, b) -> slot, rank
   int slot_ranks = 1;
   int32_t *d_nptr = nullptr, *d_nlist = nullptr;
   uint8_t* d_isbc = nullptr;
@@ -383,8 +383,7 @@ static int build_maps(cpfem_ctx* c, const int32_t* cells) {
       tslot[(size_t)s * nn + j] = (int32_t)(std::lower_bound(v.begin(), v.end(), (int32_t)j) - v.begin());
     }
   // (cell, a, b) -> slot of node b in node a's row, and its rank among the cell's earlier equal nodes
-  if (maxs >= GATHER_RANK) return fail(CPFEM_EBADARG, "a node has " + std::to_string(maxs) + " neighbours");
-  std::vector<uint16_t> slots((size_t)nc * 64);
+  std::vector<uint32_t> slots((size_t)nc * 64);
   int ranks = 1;
   for (int64_t e = 0; e < nc; ++e) {
     int rank[8];
@@ -397,7 +396,7 @@ static int build_maps(cpfem_ctx* c, const int32_t* cells) {
       const auto& v = nb[cells[e * 8 + a]];
       for (int b = 0; b < 8; ++b)
         slots[e * 64 + a * 8 + b] =
-            (uint16_t)((std::lower_bound(v.begin(), v.end(), cells[e * 8 + b]) - v.begin()) + GATHER_RANK * rank[b]);
+            (uint32_t)((std::lower_bound(v.begin(), v.end(), cells[e * 8 + b]) - v.begin()) + GATHER_RANK * rank[b]);
     }
   }
   c->slot_ranks = ranks;
@@ -410,7 +409,7 @@ static int build_maps(cpfem_ctx* c, const int32_t* cells) {
   HIPCHK(hipMemcpy(c->d_tslot, tslot.data(), tslot.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nptr, nptr.data(), nptr.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nlist, nlist.data(), nlist.size() * 4, hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->d_slots, slots.data(), slots.size() * 2, hipMemcpyHostToDevice));
+  HIPCHK(hipMemcpy(c->d_slots, slots.data(), slots.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_col, c->h_col.data(), c->h_col.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_nslot, c->h_nslot.data(), c->h_nslot.size() * 4, hipMemcpyHostToDevice));
   HIPCHK(hipMemcpy(c->d_dslot, c->h_dslot.data(), c->h_dslot.size() * 4, hipMemcpyHostToDevice));

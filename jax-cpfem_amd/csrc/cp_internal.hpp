@@ -111,8 +111,8 @@ void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u
                   const PointTables<N>& tb, const SolveCfg& cfg, int self_block, double* P, double* A, double* sig,
                   const StateOut& so, int32_t* iters, int32_t* status, hipStream_t st);
 void launch_element_K(const Geom& G, const double* wP, const double* wA, double* KE, double* RE, hipStream_t st);
-constexpr int GATHER_RANK = 1 << 13;  // slots entries: slot + GATHER_RANK x rank among equal nodes of the cell
-void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint16_t* slots,
+constexpr int GATHER_RANK = 1 << 28;  // slots entries: slot + GATHER_RANK x rank among equal nodes of the cell
+void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint32_t* slots,
                           int ranks, const int32_t* dslot, const uint8_t* is_bc, double* vals, hipStream_t st);
 void launch_gather_residual(int64_t n_nodes, const double* RE, const int32_t* nptr, const int32_t* nlist, const uint8_t* is_bc,
                             const double* ubar, const double* u, double* res, hipStream_t st);

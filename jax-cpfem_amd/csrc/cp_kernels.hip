@@ -370,7 +370,7 @@ __global__ void __launch_bounds__(EK_BS) k_element_K(Geom G, const double* __res
 // (slot, row), whose reads of 72 bytes use their lines about half, 620.
 constexpr int GN = 16, GBS = 32 * GN, GPITCH = 3 * GN + 1;
 __global__ void __launch_bounds__(GBS) k_gather_matrix(BellView M, const double* __restrict__ KE, const int32_t* __restrict__ nptr,
-                                                      const int32_t* __restrict__ nlist, const uint16_t* __restrict__ slots, int ranks,
+                                                      const int32_t* __restrict__ nlist, const uint32_t* __restrict__ slots, int ranks,
                                                       const int32_t* __restrict__ dslot, const uint8_t* __restrict__ is_bc,
                                                       double* __restrict__ vals) {
   __shared__ double T[81 * GPITCH];
@@ -393,7 +393,7 @@ __global__ void __launch_bounds__(GBS) k_gather_matrix(BellView M, const double*
           if (e0 + m < e1) {
             const int64_t ca = nlist[e0 + m];
             const double* src = KE + (ca * 3 + c) * 24 + 3 * b;
-            sl[m] = slots[ca * 8 + b];
+            sl[m] = (int)slots[ca * 8 + b];
             v[m][0] = src[0];
             v[m][1] = src[1];
             v[m][2] = src[2];
@@ -723,7 +723,7 @@ void launch_element_K(const Geom& G, const double* wP, const double* wA, double*
     hipLaunchKernelGGL(k_element_R, dim3((unsigned)nb), dim3(bs), 0, st, G, wP, RE);
 }
 
-void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint16_t* slots,
+void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint32_t* slots,
                           int ranks, const int32_t* dslot, const uint8_t* is_bc, double* vals, hipStream_t st) {
   hipLaunchKernelGGL(k_gather_matrix, dim3((unsigned)((M.n_nodes + GN - 1) / GN)), dim3(GBS), 0, st, M, KE, nptr, nlist, slots, ranks,
                      dslot, is_bc, vals);
