@@ -448,23 +448,33 @@ __global__ void __launch_bounds__(256) k_gather_residual(int64_t n_nodes, const 
 }
 
 // Element residual only: thread per (cell, a)
-__global__ void __launch_bounds__(256) k_element_R(Geom G, const double* __restrict__ wP, double* __restrict__ RE) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= G.n_qp) return;
-  const int64_t cell = t >> 3;
-  const int a = (int)(t & 7);
+// A block stages the JxW P of its 128 points in LDS with coalesced loads (read from memory by each
+// of a cell's eight threads, eight lines per load: 33 us at 40^3, now 14).
+template <bool UNIFORM>
+__global__ void __launch_bounds__(EK_BS) k_element_R(Geom G, const double* __restrict__ wP, double* __restrict__ RE) {
+  __shared__ double sP[9][EK_BS];
+  __shared__ double sG[UNIFORM ? 192 : 1];
+  const int tid = threadIdx.x, a = tid & 7, cl = tid >> 3;
+  const int64_t t = (int64_t)blockIdx.x * EK_BS + tid, cell = t >> 3;
+  const bool valid = t < G.n_qp;
+#pragma unroll
+  for (int c = 0; c < 9; ++c) sP[c][tid] = valid ? wP[c * G.n_qp + t] : 0.0;
+  if (UNIFORM)
+    for (int e = tid; e < 192; e += EK_BS) sG[e] = G.sg[e];
+  __syncthreads();
+  if (!valid) return;
   double re[3] = {0.0, 0.0, 0.0};
-#pragma unroll 1
+#pragma unroll 4
   for (int q = 0; q < 8; ++q) {
-    const int64_t qp = cell * 8 + q;
+    const int p = 8 * cl + q;
     double ga[3];
 #pragma unroll
-    for (int j = 0; j < 3; ++j) ga[j] = sg_at(G, 3 * a + j, qp);
+    for (int j = 0; j < 3; ++j) ga[j] = UNIFORM ? sG[(3 * a + j) * 8 + q] : G.sg[(3 * a + j) * G.n_qp + cell * 8 + q];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       double sr = 0.0;  // the sum of k_element_K, to the bit
 #pragma unroll
-      for (int j = 0; j < 3; ++j) sr += wP[(3 * i + j) * G.n_qp + qp] * ga[j];
+      for (int j = 0; j < 3; ++j) sr += sP[3 * i + j][p] * ga[j];
       re[i] += sr;
     }
   }
@@ -714,13 +724,12 @@ void launch_local(int64_t n_qp, const double* Hd, const Geom& G, const double* u
 }
 
 void launch_element_K(const Geom& G, const double* wP, const double* wA, double* KE, double* RE, hipStream_t st) {
-  const int bs = 256;
-  const int64_t nb = (G.n_qp + bs - 1) / bs;
   if (wA)
     hipLaunchKernelGGL(G.uniform ? k_element_K<true> : k_element_K<false>,
                        dim3((unsigned)((G.n_qp + XCDS * EK_BS - 1) / (XCDS * EK_BS) * 3 * XCDS)), dim3(EK_BS), 0, st, G, wP, wA, KE, RE);
   else
-    hipLaunchKernelGGL(k_element_R, dim3((unsigned)nb), dim3(bs), 0, st, G, wP, RE);
+    hipLaunchKernelGGL(G.uniform ? k_element_R<true> : k_element_R<false>, dim3((unsigned)((G.n_qp + EK_BS - 1) / EK_BS)), dim3(EK_BS),
+                       0, st, G, wP, RE);
 }
 
 void launch_gather_matrix(const BellView& M, const double* KE, const int32_t* nptr, const int32_t* nlist, const uint32_t* slots,
