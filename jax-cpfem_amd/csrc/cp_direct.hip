@@ -86,7 +86,9 @@ __global__ void __launch_bounds__(256) k_band_first(BandLU B) {
 // others take `group` tiles of one row I, so that A_IK A_KK^-1 is formed once for them.
 // The tiles after the current one are loaded under its product.  At cnt = 22 a step of one front
 // takes 19 us, of which the chain through workgroup 0 is 17 (launch 2, loads 1.4, two products 4,
-// inverse 9); two fronts take 25 us, bound by the tiles' traffic (62 MB read and written once).
+// inverse 9); two fronts take 25 us, with 62 MB of tiles read and written.  (Visiting a tile in every
+// second step only, for two pivots, halves that traffic and takes 32 us: the second inverse's
+// product comes before the first tile's.)
 __global__ void __launch_bounds__(256, 2) k_band_step(BandLU B, int t, int cnt, int group) {
   __shared__ double S[2][TILE];
   const int f = blockIdx.y, dir = f ? -1 : 1, K = f ? B.nbk - 1 - t : t;
