@@ -200,6 +200,7 @@ struct KrylovScalars {
   int32_t done;  // read by the host together with k
   int32_t maxiter;
   int32_t pad;
+  double rs0;    // <r,r> at the first test (multigrid solve)
 };
 
 struct KrylovWork {

@@ -38,7 +38,17 @@ namespace cpfem {
 constexpr int DEG_FINE = 4, DEG_COARSE = 4;
 constexpr double LOW_FINE = 0.1, LOW_COARSE = 0.07;  // the polynomials' ranges start at this times lambda_max
 constexpr int DENSE_ROWS = 768;    // the first level of at most this many rows is the last, and is inverted
+// Steps of the power iteration: BiCGSTAB iterations over 24 shapes at 6, 8, 10, 12, 14, 16, 20 steps:
+// 4991 (some solves run to the limit), 737, 670, 664, 667, 669, 669.
 constexpr int POWER_STEPS = 12;
+// When the iteration gives up. Elements ten times as long as wide and thin plates are not for this
+// preconditioner (point smoothing, coarsening in all directions), and ran through MG_MAXITER iterations
+// before the Jacobi solve began: 24^3 of 1:1:10 elements 27.0 ms, now 18.0, Jacobi alone 15.3; of 1:3:10
+// 26.8, now 20.8 (13.8); 32x32x4 of 1:1:0.4 13.6, now 8.1 (6.1). What converges is left alone: 24
+// shapes of 1:1:1 elements, and 1:1:3 (32 iterations), 1:1:0.1 (37) take the iterations they took.
+constexpr int STALL_FROM = 7;
+constexpr int STALL_LIMIT = 60;       // MG_MAXITER; not the caller's own limit, which may be lower
+constexpr float STALL_SLACK = 6.65f;  // log2(100)
 constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
 constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
 
@@ -795,11 +805,19 @@ __global__ void __launch_bounds__(KBS) k_mgb_p(MgVec v, KrylovWork w, int par, i
   const double rs = sums[0], rho_ = sums[1];
   int k = (omega == 0.0 || alpha == 0.0) ? -11 : kprev + 1;
   if (rho == 0.0) k = -10;
+  // A solve that is not on its way to the threshold within STALL_LIMIT iterations is left to the Jacobi
+  // solve: from STALL_FROM on, the squared residual has to be under a straight line (in its logarithm)
+  // from a hundredfold of the first one. See STALL_FROM for what it costs without this.
+  if (k >= STALL_FROM && rs > atol2) {
+    const float line = log2f(fmaxf((float)(atol2 / sc->rs0), 1e-30f)) * ((float)k / (float)STALL_LIMIT);
+    if (log2f((float)(rs / sc->rs0)) > STALL_SLACK + line) k = -12;
+  }
   const bool go = (rs > atol2) && (k < maxiter) && (k >= 0);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     sc->k2[par] = k;
     sc->rho2[par] = rho_;
     sc->rs = rs;
+    if (iter == 0) sc->rs0 = rs;
     sc->k = k;
     if (!go) sc->done = 1;
     __hip_atomic_store(flag, ((uint64_t)(iter + 1) << 33) | ((uint64_t)(go ? 0 : 1) << 32) | (uint32_t)k, __ATOMIC_RELAXED,

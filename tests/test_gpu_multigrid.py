@@ -124,3 +124,55 @@ def test_nan_matrix_fails_as_the_jacobi_solve_does():
         linear_solver(prob, bad, b, x0, {"jax_solver": {}})
     linear_solver(prob, mat, b, x0, {"jax_solver": {}})
     assert prob.solver_info[-1]["iterations"] <= 30
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n, size", [((24, 24, 24), (1, 1, 10)), ((32, 32, 4), (1, 1, 0.05))])
+def test_stretched_elements_are_left_to_the_jacobi_solve(n, size, precision):
+    """Where the preconditioner is no good the solve gives up early, and the Jacobi solve starts from
+    x0: nothing of the attempt is left in the result, so it and its iterations are krylov_solve's, to
+    the last bit."""
+    from cpfem_amd.solver import krylov_solve, multigrid_solve
+    prob, mat, b, x0 = _elastic(n, size)
+    opts = {"precision": precision}
+    xj = krylov_solve(prob, mat, b, x0, opts)
+    kj = prob.solver_info[-1]["iterations"]
+    assert kj > 60
+    x = multigrid_solve(prob, mat, b, x0, opts)
+    assert prob.solver_info[-1]["iterations"] == kj
+    assert torch.equal(x, xj)
+
+
+@pytest.mark.parametrize("n, size", [((16, 16, 16), (1, 1, 1)), ((24, 24, 24), (1, 1, 3)), ((24, 24, 24), (1, 1, 0.1))])
+def test_a_low_limit_does_not_make_the_multigrid_solve_give_up(n, size):
+    """Solves that need 9 to 40 iterations take the same with just these allowed: the line that a
+    solve has to stay under is not drawn from the caller's limit."""
+    from cpfem_amd.solver import multigrid_solve
+    prob, mat, b, x0 = _elastic(n, size)
+    x = multigrid_solve(prob, mat, b, x0, {})
+    k = prob.solver_info[-1]["iterations"]
+    assert 5 < k < 60
+    y = multigrid_solve(prob, mat, b, x0, {"krylov_maxiter": k})
+    assert prob.solver_info[-1]["iterations"] == k
+    assert torch.equal(x, y)
+
+
+def _elastic(n, size):
+    """The first Newton system of a copper polycrystal box (elements of any proportions)."""
+    import cpfem_amd as C
+    from cpfem_amd.solver import bc_x0
+    rng = np.random.default_rng(0)
+    m = C.box_mesh(*n, *size)
+    mesh = C.Mesh(m.points, m.cells_dict["hexahedron"])
+    at = lambda d, v: (lambda p: np.isclose(p[d], v, atol=1e-6))
+    zero, top = (lambda p: 0.0), (lambda p: 1e-3 * size[2])
+    info = [[at(0, 0), at(1, 0), at(2, 0), at(2, size[2])], [0, 1, 2, 2], [zero, zero, zero, top]]
+    quat = rng.normal(size=(40, 4))
+    quat /= np.linalg.norm(quat, axis=1, keepdims=True)
+    prob = C.CrystalPlasticity(mesh, dirichlet_bc_info=info, additional_info=(quat, rng.integers(0, 40, len(mesh.cells))),
+                               material=C.CALIB_COPPER)
+    prob.dt = 0.1
+    prob.set_params(prob.internal_vars)
+    dofs = bc_x0(prob, torch.zeros(prob.fes[0].num_total_nodes * 3, dtype=torch.float64, device="cuda"))
+    res, mat = prob.assemble(dofs)
+    return prob, mat.clone(), -res, torch.zeros_like(res)
