@@ -213,6 +213,15 @@ __device__ __forceinline__ bool mg_row(const BellView& M, const MgGrid& g, const
   }
 }
 
+// The finest level is smoothed once more while the host waits for the convergence test (see
+// mg_krylov_begin): a pass over its matrix (14 us at 32^3, 108 at 64^3) is not made when that has ended
+// the solve.  Smaller levels make theirs: it is shorter than the test's round trip to memory.  No kernel
+// in flight writes `done`, so it is the same in every wave of the grid.
+template <bool FINE, int P>
+__device__ __forceinline__ bool mg_idle(const int32_t* __restrict__ done) {
+  return FINE && P == 1 && *done;
+}
+
 // One Chebyshev step: xo <- x + c1 (x - xo) + c2 D^-1 (b - A x) (first: xo counts as zero).
 template <typename TM, bool FINE, int P>
 __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_smooth(BellView M, const TM* __restrict__ A, MgGrid g,
@@ -221,14 +230,11 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_smooth(BellView M, const 
                                                              double c1, double c2, const double* __restrict__ lam,
                                                              const int32_t* __restrict__ done, int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
-  // tested when the product is there, one round trip less per pass; but a pass over the finest matrix
-  // (14 us at 32^3, 108 at 64^3) is not made for nothing
-  const int dn = *done;
-  if (FINE && P == 1 && dn) return;
+  if (mg_idle<FINE, P>(done)) return;
   const double c2l = c2 * lam[0];
   int r;
   double acc;
-  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red) || dn) return;
+  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red)) return;
   const double xv = x[r], xp = first ? 0.0 : xo[r];
   xo[r] = xv + (c1 * (xv - xp) + c2l * minv[r] * (b[r] - acc));
 }
@@ -240,11 +246,10 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_resid(BellView M, const T
                                                             const double* __restrict__ x, double* __restrict__ out,
                                                             const int32_t* __restrict__ done, int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
-  const int dn = *done;
-  if (FINE && P == 1 && dn) return;
+  if (mg_idle<FINE, P>(done)) return;
   int r;
   double acc;
-  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red) || dn) return;
+  if (!mg_row<TM, FINE, P>(M, g, A, x, order, r, acc, red)) return;
   out[r] = minv[r] != 0.0 ? b[r] - acc : 0.0;
 }
 
@@ -329,14 +334,11 @@ __device__ __forceinline__ double mg_restrict_row(const MgGrid& f, const MgGrid&
 // Restriction b_c = P^T r and the first coarse iterate x_c = ith D^-1 b_c.
 __global__ void __launch_bounds__(256) k_mg_restrict(MgGrid f, MgGrid g, const double* __restrict__ rf,
                                                     const double* __restrict__ minv, double* __restrict__ b,
-                                                    double* __restrict__ x, double ith, const double* __restrict__ lam,
-                                                    const int32_t* __restrict__ done) {
+                                                    double* __restrict__ x, double ith, const double* __restrict__ lam) {
   const int t = (int)(blockIdx.x * 256 + threadIdx.x);
   if (t >= g.n) return;
-  const int dn = *done;
   const double il = ith * lam[0], mi = minv[t];
   double acc = mg_restrict_row(f, g, t, rf);
-  if (dn) return;
   acc = mi != 0.0 ? acc : 0.0;
   b[t] = acc;
   x[t] = il * mi * acc;
@@ -373,15 +375,12 @@ __device__ __forceinline__ double mg_interp(const MgGrid& f, const MgGrid& g, co
 // out = x + P e on the free dofs; on Dirichlet dofs b / diagonal (finest level) or 0.
 __global__ void __launch_bounds__(256) k_mg_prolong(MgGrid f, MgGrid g, const double* __restrict__ e, const double* __restrict__ x,
                                                    const double* __restrict__ minv, const double* __restrict__ b,
-                                                   const double* __restrict__ invd, double* __restrict__ out,
-                                                   const int32_t* __restrict__ done) {
+                                                   const double* __restrict__ invd, double* __restrict__ out) {
   const int t = (int)(blockIdx.x * 256 + threadIdx.x);
   if (t >= f.n) return;
-  const int dn = *done;
   const int i = (int)((uint32_t)t / 3u);
   const NodeXYZ p = mg_node(f, i);
   const double v = x[t] + mg_interp(f, g, p, t - 3 * i, e);
-  if (dn) return;
   out[t] = minv[t] != 0.0 ? v : (invd ? b[t] * invd[t] : 0.0);
 }
 
@@ -562,9 +561,8 @@ __global__ void __launch_bounds__(256, 2) k_dense_step(int nt, int k, const doub
 // side in LDS), 16 rows a workgroup, 16 threads a row.
 __global__ void __launch_bounds__(256) k_mg_dense(MgGrid f, MgGrid g, int nt, const double* __restrict__ rf,
                                                   const double* __restrict__ minv, const double* __restrict__ inv,
-                                                  double* __restrict__ x, const int32_t* __restrict__ done) {
+                                                  double* __restrict__ x) {
   __shared__ __align__(16) double b[DENSE_ROWS];
-  const int dn = *done;
   for (int t = threadIdx.x; t < nt * NB; t += 256) b[t] = t < g.n && minv[t] != 0.0 ? mg_restrict_row(f, g, t, rf) : 0.0;
   __syncthreads();
   const int r = (int)blockIdx.x * 16 + threadIdx.x / 16, sub = threadIdx.x % 16;
@@ -572,7 +570,6 @@ __global__ void __launch_bounds__(256) k_mg_dense(MgGrid f, MgGrid g, int nt, co
   double acc = 0.0;
   for (int j = 0; j < nt; ++j) acc += row_dot(row + (int64_t)j * TILE, b + j * NB, sub);
   acc = sum16(acc);
-  if (dn) return;
   if (sub == 0 && r < g.n) x[r] = acc;
 }
 
@@ -687,7 +684,7 @@ static double* smooth_fine(const Multigrid& mg, const BellView& M, const TM* val
 // The rest of the V-cycle: out = M b, from the finest level's iterate and its residual.
 template <typename TM>
 static void vcycle(const Multigrid& mg, const BellView& M, double* iterate, const double* invd, const double* b, double* out,
-                   const int32_t* done, hipStream_t st, Prof* prof) {
+                   hipStream_t st, Prof* prof) {
   static const Cheb cc = cheb(DEG_COARSE, LOW_COARSE);
   double* cur[MG_MAXL];
   const int last = mg.nl - 1;
@@ -697,24 +694,24 @@ static void vcycle(const Multigrid& mg, const BellView& M, double* iterate, cons
     int p = 0;
     if (l > 0) {
       const TM* A = static_cast<const TM*>(L.A);
-      cur[l] = level_parts(L.g.n) == 1 ? smooth_level<TM, false, 1>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof)
-                                       : smooth_level<TM, false, 3>(mg, l, M, A, L.b, cc, DEG_COARSE, done, &p, st, prof);
+      cur[l] = level_parts(L.g.n) == 1 ? smooth_level<TM, false, 1>(mg, l, M, A, L.b, cc, DEG_COARSE, nullptr, &p, st, prof)
+                                       : smooth_level<TM, false, 3>(mg, l, M, A, L.b, cc, DEG_COARSE, nullptr, &p, st, prof);
     }
     if (l + 1 == last) break;  // the last level's kernel restricts for itself
     const MgLevel& C = mg.lv[l + 1];
     timed(prof, PC_MG_COARSE, k_mg_restrict, dim3(blocks256(C.g.n)), dim3(256), st, L.g, C.g, (const double*)L.r,
-          (const double*)C.minv, C.b, C.x0, cc.ith, (const double*)mg.lam, done);
+          (const double*)C.minv, C.b, C.x0, cc.ith, (const double*)mg.lam);
   }
   const MgLevel &A = mg.lv[last - 1], &E = mg.lv[last];
   const int nt = mg_dense_tiles(E.g.n);
   timed(prof, PC_MG_COARSE, k_mg_dense, dim3((unsigned)((E.g.n + 15) / 16)), dim3(256), st, A.g, E.g, nt, (const double*)A.r,
-        (const double*)E.minv, (const double*)mg.dense[nt & 1], E.x0, done);
+        (const double*)E.minv, (const double*)mg.dense[nt & 1], E.x0);
   const double* e = E.x0;
   for (int l = last - 1; l >= 0; --l) {
     const MgLevel& L = mg.lv[l];
     double* o = l == 0 ? out : cur[l];
     timed(prof, PC_MG_COARSE, k_mg_prolong, dim3(blocks256(L.g.n)), dim3(256), st, L.g, mg.lv[l + 1].g, e, (const double*)cur[l],
-          (const double*)L.minv, b, l == 0 ? invd : (const double*)nullptr, o, done);
+          (const double*)L.minv, b, l == 0 ? invd : (const double*)nullptr, o);
     e = o;
   }
 }
@@ -794,8 +791,8 @@ __global__ void __launch_bounds__(KBS) k_mgb_p(MgVec v, KrylovWork w, int par, i
                                               double* __restrict__ y, double ith, const double* __restrict__ lam,
                                               uint64_t* __restrict__ flag) {
   __shared__ double sh[2 * (KBS / 64)];
+  // (`done` is written here and so not read: blocks of this launch would see either value)
   KrylovScalars* sc = w.sc;
-  if (sc->done) return;
   const int pv = par ^ 1;
   const double rho = sc->rho2[pv], alpha = sc->alpha2[pv], omega = sc->omega2[pv], atol2 = sc->atol2;
   const int kprev = sc->k2[pv], maxiter = sc->maxiter;
@@ -838,14 +835,12 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_q(BellView M, MgGrid g, 
                                                          int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
   __shared__ double sh[MgShape<P>::BS / 64];
-  const int dn = w.sc->done;
   int r;
   double acc, d[1] = {0.0};
   if (mg_row<double, true, P>(M, g, A, v.phat, order, r, acc, red)) {
     v.q[r] = acc;
     d[0] = v.rhat[r] * acc;
   }
-  if (dn) return;  // uniform over the grid; q is not read any more
   put_partials<MgShape<P>::BS, 1>(d, {PS_RQ}, w.partial, w.ps, sh);
 }
 
@@ -854,7 +849,6 @@ __global__ void __launch_bounds__(KBS) k_mgb_s(MgVec v, KrylovWork w, int par, i
                                               double* __restrict__ y, double ith, const double* __restrict__ lam) {
   __shared__ double sh[KBS / 64];
   KrylovScalars* sc = w.sc;
-  if (sc->done) return;
   double sums[1];
   mg_sums<1>(w.partial, {PS_RQ}, nbs, w.ps, sh, sums);
   const double alpha = sc->rho2[par] / sums[0], il = ith * lam[0];
@@ -872,7 +866,6 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_t(BellView M, MgGrid g, 
                                                          int order) {
   __shared__ double red[P > 1 ? (P - 1) * 64 : 1];
   __shared__ double sh[3 * (MgShape<P>::BS / 64)];
-  const int dn = w.sc->done;
   int r;
   double acc, d[3] = {0.0, 0.0, 0.0};
   if (mg_row<double, true, P>(M, g, A, v.shat, order, r, acc, red)) {
@@ -882,7 +875,6 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_t(BellView M, MgGrid g, 
     d[1] = acc * s;
     d[2] = acc * acc;
   }
-  if (dn) return;  // uniform over the grid; t is not read any more
   put_partials<MgShape<P>::BS, 3>(d, {PS_SS, PS_TS, PS_TT}, w.partial, w.ps, sh);
 }
 
@@ -890,7 +882,6 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_t(BellView M, MgGrid g, 
 __global__ void __launch_bounds__(KBS) k_mgb_xr(MgVec v, KrylovWork w, int par, int nbs) {
   __shared__ double sh[3 * (KBS / 64)];
   KrylovScalars* sc = w.sc;
-  if (sc->done) return;
   const double alpha = sc->alpha2[par], atol2 = sc->atol2;
   double sums[3];
   mg_sums<3>(w.partial, {PS_SS, PS_TS, PS_TT}, nbs, w.ps, sh, sums);
@@ -959,17 +950,16 @@ void mg_krylov_finish(const Multigrid& mg, const BellView& M, const double* vals
   const double ith = cheb(DEG_FINE, LOW_FINE).ith;
   const bool one = level_parts(g.n) == 1;
   const dim3 vb((unsigned)w.nb), vt(KBS), sb((unsigned)w.nbs), s1(MgShape<1>::BS), s3(MgShape<3>::BS);
-  const int32_t* done = &w.sc->done;
   const int par = iter & 1;
   int pass = 1 + DEG_FINE;  // those of mg_krylov_begin
-  vcycle<TM>(mg, M, (DEG_FINE - 1) & 1 ? L.x1 : L.x0, v.invd, v.p, v.phat, done, st, prof);
+  vcycle<TM>(mg, M, (DEG_FINE - 1) & 1 ? L.x1 : L.x0, v.invd, v.p, v.phat, st, prof);
   if (one)
     timed(prof, PC_SPMV, k_mgb_q<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
   else
     timed(prof, PC_SPMV, k_mgb_q<3>, sb, s3, st, M, g, vals, v, w, level_order(g.n, pass++));
   timed(prof, PC_KVEC, k_mgb_s, vb, vt, st, v, w, par, w.nbs, (const double*)L.minv, L.x0, ith, (const double*)mg.lam);
-  double* it = smooth_fine<TM>(mg, M, valsp, v.s, done, &pass, st, prof);
-  vcycle<TM>(mg, M, it, v.invd, v.s, v.shat, done, st, prof);
+  double* it = smooth_fine<TM>(mg, M, valsp, v.s, &w.sc->done, &pass, st, prof);
+  vcycle<TM>(mg, M, it, v.invd, v.s, v.shat, st, prof);
   if (one)
     timed(prof, PC_SPMV, k_mgb_t<1>, sb, s1, st, M, g, vals, v, w, level_order(g.n, pass++));
   else
