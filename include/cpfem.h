@@ -156,7 +156,8 @@ int cpfem_solve(cpfem_ctx* ctx, void* stream, const double* mat, const double* b
 
 /* cpfem_solve with a geometric multigrid V-cycle in the place of the Jacobi scaling, where that
    applies: systems of at least 1500 rows on meshes whose nodes are numbered as a full box (see
-   cpfem_box_numbering; every node, on the faces too, coupled to all its neighbours).  Same
+   cpfem_box_numbering; every node, on the faces too, coupled to all its neighbours) whose
+   elements and Dirichlet dofs let it be the shorter one (cpfem_multigrid_pays).  Same
    recurrence, stopping rule, arguments and errors; info->iterations counts its (far fewer)
    iterations.  precision CPFEM_MIXED: FP32 values inside the preconditioner, FP64 operator.  On
    other systems, and from x0 anew where the multigrid solve breaks down, does not meet the
@@ -203,6 +204,13 @@ int cpfem_band_order(int64_t n_nodes, const int32_t* col, const int32_t* nslot, 
    instead of loading them.  No counterpart in the reference (a property of the mesh's node
    numbering; the reference's box meshes have it). */
 int cpfem_box_numbering(int64_t n_nodes, const int32_t* col, const int32_t* nslot, int64_t* dims);
+
+/* Whether cpfem_solve_mg tries multigrid on a box mesh of dims = (nx, ny, nz) nodes at points
+   ([n_nodes][3]) with n Dirichlet dofs, all host arrays:
+   *pays = 1 where the iterations expected of it from the elements' proportions cost less than
+   those expected of the Jacobi solve from the way to the nearest held node.  No counterpart in
+   the reference. */
+int cpfem_multigrid_pays(const int64_t* dims, const double* points, int64_t n, const int64_t* dofs, int32_t* pays);
 
 /* y = A x on the block-ELL matrix (device). */
 int cpfem_spmv(cpfem_ctx* ctx, void* stream, const double* mat, const double* x, double* y);

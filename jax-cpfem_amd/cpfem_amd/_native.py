@@ -87,6 +87,7 @@ _SIGS = {
     "cpfem_solve_direct": (ctypes.c_int, [vp, vp, vp, vp, vp, ctypes.c_int32, ctypes.POINTER(CpfemSolveInfo)]),
     "cpfem_band_order": (ctypes.c_int, [ctypes.c_int64, vp, vp, vp, vp]),
     "cpfem_box_numbering": (ctypes.c_int, [ctypes.c_int64, vp, vp, vp]),
+    "cpfem_multigrid_pays": (ctypes.c_int, [vp, vp, ctypes.c_int64, vp, ctypes.POINTER(ctypes.c_int32)]),
     "cpfem_norm": (ctypes.c_int, [vp, vp, vp, ctypes.POINTER(ctypes.c_double), ctypes.POINTER(ctypes.c_int32)]),
     "cpfem_axpby": (ctypes.c_int, [vp, vp, ctypes.c_double, vp, ctypes.c_double, vp]),
     "cpfem_to_csr": (ctypes.c_int, [vp, vp, vp, vp, vp, vp]),

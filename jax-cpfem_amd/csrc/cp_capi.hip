@@ -164,6 +164,8 @@ struct cpfem_ctx {
   Multigrid mg;                // multigrid preconditioner (buffers allocated on first use)
   std::vector<void*> mg_mem;   // its device allocations
   bool box_full = false;       // every row of the pattern holds exactly the node's neighbours in the box
+  MgMesh mg_shape;             // of a full box: its elements, for the choice of the preconditioner
+  bool mg_use = false;         // that choice, for the present Dirichlet dofs
   uint64_t* h_flag = nullptr;  // progress word written by its BiCGSTAB (pinned)
   double* scratch = nullptr;  // device address of the fixed workspace array on this context's device
 
@@ -696,7 +698,7 @@ static bool ensure_mg(cpfem_ctx* c) {
   Multigrid& mg = c->mg;
   if (mg.state) return mg.state > 0;
   mg.state = -1;
-  if (!c->box_full || c->n_slots != 27 || c->n_dofs < MG_MIN_ROWS || !mg_plan(c->box, &mg)) return false;
+  if (c->n_slots != 27 || c->n_dofs < MG_MIN_ROWS || !mg_plan(c->box, &mg)) return false;
   const auto get = [&](size_t doubles) -> double* {
     void* p = nullptr;
     if (hipMalloc(&p, doubles * sizeof(double)) != hipSuccess) {
@@ -847,6 +849,10 @@ int cpfem_create(const CpfemMesh* mesh, const CpfemSlip* slip, cpfem_ctx** out) 
     g_err = e;
     return rc;
   }
+  if (c->box_full) {
+    c->mg_shape = mg_mesh(c->box, mesh->points);
+    c->mg_use = mg_pays(c->box, c->mg_shape, 0, nullptr);
+  }
   if ((rc = scratch_address(&c->scratch))) {
     const std::string e = g_err;
     cpfem_destroy(c);
@@ -947,6 +953,7 @@ int cpfem_set_dirichlet(cpfem_ctx* c, void* stream, int64_t n, const int64_t* do
     isbc[dofs[k]] = 1;
     ubar[dofs[k]] = vals[k];
   }
+  c->mg_use = c->box_full && mg_pays(c->box, c->mg_shape, n, dofs);
   hipStream_t st = (hipStream_t)stream;
   HIPCHK(hipMemcpyAsync(c->d_isbc, isbc.data(), c->n_dofs, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(c->d_ubar, ubar.data(), 8 * c->n_dofs, hipMemcpyHostToDevice, st));
@@ -1088,6 +1095,15 @@ int cpfem_update_state(cpfem_ctx* c, void* stream, const double* dofs, const Cpf
 int cpfem_band_order(int64_t n_nodes, const int32_t* col, const int32_t* nslot, int32_t* ip, int32_t* bandwidth) {
   if (n_nodes <= 0 || !col || !nslot || !ip || !bandwidth) return fail(CPFEM_EBADARG, "null argument");
   return band_ordering(n_nodes, col, nslot, ip, bandwidth);
+}
+
+int cpfem_multigrid_pays(const int64_t* dims, const double* points, int64_t n, const int64_t* dofs, int32_t* pays) {
+  if (!dims || !points || !pays || (n > 0 && !dofs)) return fail(CPFEM_EBADARG, "null argument");
+  if (dims[0] < 2 || dims[1] < 2 || dims[2] < 2) return fail(CPFEM_EBADARG, "a box has at least two nodes a side");
+  for (int64_t k = 0; k < n; ++k)
+    if (dofs[k] < 0 || dofs[k] >= 3 * dims[0] * dims[1] * dims[2]) return fail(CPFEM_EBADARG, "Dirichlet dof out of range");
+  *pays = mg_pays(dims, mg_mesh(dims, points), n, dofs) ? 1 : 0;
+  return CPFEM_OK;
 }
 
 int cpfem_box_numbering(int64_t n_nodes, const int32_t* col, const int32_t* nslot, int64_t* dims) {
@@ -1257,7 +1273,7 @@ int cpfem_solve_mg(cpfem_ctx* c, void* stream, const double* mat, const double* 
   if (!c || !mat || !b || !x) return fail(CPFEM_EBADARG, "null argument");
   if (precision != CPFEM_FP64 && precision != CPFEM_MIXED) return fail(CPFEM_EBADARG, "unknown precision");
   if (maxiter < 0) return fail(CPFEM_EBADARG, "maxiter must be >= 0");
-  if (ensure_mg(c)) {
+  if (c->mg_use && ensure_mg(c)) {
     int rc;
     hipStream_t st = (hipStream_t)stream;
     if ((rc = ensure_krylov(c, precision == CPFEM_MIXED))) return rc;

@@ -254,6 +254,17 @@ struct Multigrid {
   double* lam = nullptr;                  // [0] = 1 / lambda_max of the scaled operator
   int state = 0;                          // 0: no buffers yet, 1: allocated, -1: does not apply
 };
+// What the choice between the multigrid and the Jacobi preconditioner needs to know of a box mesh:
+// mean element length of each box direction, the coordinate that it runs along, and the iterations that
+// a multigrid solve is expected to take (the most over the elements).
+struct MgMesh {
+  double h[3] = {0.0, 0.0, 0.0};
+  int axis[3] = {0, 1, 2};
+  double its = 0.0;
+};
+MgMesh mg_mesh(const int64_t box[3], const double* points);
+// Whether the multigrid solve is expected to be the shorter one, for these n Dirichlet dofs (host).
+bool mg_pays(const int64_t box[3], const MgMesh& mesh, int64_t n, const int64_t* dofs);
 // Levels of a box of nx x ny x nz nodes (host; no buffers). False if the box is too thin.
 bool mg_plan(const int64_t box[3], Multigrid* mg);
 // Doubles of the two triple-product intermediates of the plan.

@@ -28,7 +28,9 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
+#include <vector>
 
 #include "cp_krylov.hpp"
 #include "cp_tiles.hpp"
@@ -41,11 +43,11 @@ constexpr int DENSE_ROWS = 768;    // the first level of at most this many rows 
 // Steps of the power iteration: BiCGSTAB iterations over 24 shapes at 6, 8, 10, 12, 14, 16, 20 steps:
 // 4991 (some solves run to the limit), 737, 670, 664, 667, 669, 669.
 constexpr int POWER_STEPS = 12;
-// When the iteration gives up. Elements ten times as long as wide and thin plates are not for this
-// preconditioner (point smoothing, coarsening in all directions), and ran through MG_MAXITER iterations
-// before the Jacobi solve began: 24^3 of 1:1:10 elements 27.0 ms, now 18.0, Jacobi alone 15.3; of 1:3:10
-// 26.8, now 20.8 (13.8); 32x32x4 of 1:1:0.4 13.6, now 8.1 (6.1). What converges is left alone: 24
-// shapes of 1:1:1 elements, and 1:1:3 (32 iterations), 1:1:0.1 (37) take the iterations they took.
+// When the iteration gives up.  mg_pays keeps most systems that are not for this preconditioner from it;
+// for those that it lets through (48^3 of 1:1:0.1 elements, 3x20x20 of 1:1:4 held on two faces) this bounds
+// what the attempt costs: 24^3 of 1:1:10, tried all the same, 27.0 ms with all MG_MAXITER iterations, 18.0
+// with this, Jacobi alone 15.3.  What converges is left alone: 24 shapes of 1:1:1 elements, and 1:1:3
+// (32 iterations), 1:1:0.1 (37) take the iterations they took.
 constexpr int STALL_FROM = 7;
 constexpr int STALL_LIMIT = 60;       // MG_MAXITER; not the caller's own limit, which may be lower
 constexpr float STALL_SLACK = 6.65f;  // log2(100)
@@ -107,6 +109,99 @@ void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2) {
   const MgGrid &f = mg.lv[0].g, &c = mg.lv[1].g;
   *n1 = 81LL * 3 * c.nx * f.ny * f.nz;
   *n2 = 81LL * 3 * c.nx * c.ny * f.nz;
+}
+
+// ---------------------------------------------------------------------------------
+// Which preconditioner (host).  Multigrid wants elements that are not too stretched (point smoothing,
+// coarsening in all directions), and a system that is hard for the Jacobi iteration: held on close
+// faces, that one needs a few dozen iterations, each a fraction of a multigrid one.  Both counts are
+// estimated from the mesh and its Dirichlet dofs.
+//
+// Multigrid, from elements of proportions a <= b <= c: 2.5 + 4.6 c/a + 1.2 (c/b - 1), measured 6..8 for
+// cubes, 12 for 1:1:2, 18 for 1:1:3, 25 for 1:1:4, 31 for 1:1:5, 53 for 1:1:10, 24 for 1:5:5 and 49 for
+// 1:10:10.  Above 40 some run into MG_MAXITER; they are let through to 50 only where the longest way to a
+// held node (below) runs in the direction of the displacement itself.
+//
+// Jacobi, from the longest way to a node where a displacement component is held, over components and
+// directions, in elements: 38 + 6 w along the component, w weighted by the square root of
+// the element's length over the shortest one; 35 + 9 w across it (a bar held at its ends), w weighted by
+// that length.  These are low estimates: 24^3 under symmetry planes 182 (measured 233..239), 16^3 134
+// (156..192), 24x24x6 182 (165..177), 24^3 held on two faces 143 (182..199), 24x24x6 62 (64), 32x32x4 53
+// (45), 24^3 of 1:1:10 266 (385..410), of 1:10:10 493 (815).
+//
+// A multigrid iteration takes the time of 4.5 Jacobi ones with two levels (10^3), 6.8 with three (16^3),
+// 8 with four (24^3; 5.5 to 7 where the finest level's passes outweigh the launches), its set-up that of about
+// fifteen.
+// Without this, against the Jacobi solve: 24x24x6 held on two faces 1.29 -> 2.70 ms, 16^3 so held of
+// 1:1:0.2 1.77 -> 3.10, 24^3 of 1:1:10 9.4 -> 10.3, 16^3 of it 4.5 -> 5.8, each now the Jacobi solve.  Of
+// 1:1:4 elements 24^3 would gain 1.5, and takes the Jacobi solve too.
+static double mg_iterations(double x, double y, double z) {
+  const double a = std::min({x, y, z}), c = std::max({x, y, z}), b = std::max(std::min(x, y), std::min(std::max(x, y), z));
+  return a > 0.0 ? 2.5 + 4.6 * c / a + 1.2 * (c / b - 1.0) : 1e30;
+}
+
+MgMesh mg_mesh(const int64_t box[3], const double* points) {
+  MgMesh m;
+  const int64_t step[3] = {1, box[0], box[0] * box[1]};
+  double run[3][3] = {}, count[3] = {};
+  for (int64_t z = 0, i = 0; z < box[2]; ++z)
+    for (int64_t y = 0; y < box[1]; ++y)
+      for (int64_t x = 0; x < box[0]; ++x, ++i) {
+        const bool in[3] = {x + 1 < box[0], y + 1 < box[1], z + 1 < box[2]};
+        double len[3];
+        for (int d = 0; d < 3; ++d) {
+          if (!in[d]) continue;
+          double s = 0.0;
+          for (int c = 0; c < 3; ++c) {
+            const double v = points[3 * (i + step[d]) + c] - points[3 * i + c];
+            s += v * v;
+            run[d][c] += std::fabs(v);
+          }
+          len[d] = std::sqrt(s);
+          m.h[d] += len[d];
+          count[d] += 1.0;
+        }
+        if (in[0] && in[1] && in[2]) m.its = std::max(m.its, mg_iterations(len[0], len[1], len[2]));
+      }
+  for (int d = 0; d < 3; ++d) {
+    m.h[d] /= std::max(count[d], 1.0);
+    m.axis[d] = (int)(std::max_element(run[d], run[d] + 3) - run[d]);
+  }
+  return m;
+}
+
+bool mg_pays(const int64_t box[3], const MgMesh& mesh, int64_t n, const int64_t* dofs) {
+  const double h0 = std::min({mesh.h[0], mesh.h[1], mesh.h[2]});
+  Multigrid plan;
+  if (!(h0 > 0.0) || !mg_plan(box, &plan)) return false;
+  std::vector<uint8_t> held[3][3];  // coordinates of the nodes where a component is held
+  for (int c = 0; c < 3; ++c)
+    for (int d = 0; d < 3; ++d) held[c][d].assign((size_t)box[d], 0);
+  for (int64_t k = 0; k < n; ++k) {
+    const int64_t i = dofs[k] / 3, z = i / (box[0] * box[1]), y = i / box[0] % box[1], x = i % box[0];
+    std::vector<uint8_t>* h = held[dofs[k] % 3];
+    h[0][x] = h[1][y] = h[2][z] = 1;
+  }
+  double jacobi = 0.0;
+  bool along = true;
+  for (int c = 0; c < 3; ++c) {
+    for (int d = 0; d < 3; ++d) {
+      int64_t far = 0, last = -1;  // last: the held coordinate before
+      for (int64_t k = 0; k <= box[d]; ++k) {
+        if (k < box[d] && !held[c][d][k]) continue;
+        const bool open = last < 0 || k == box[d];  // an end of the box, not held
+        far = std::max(far, last < 0 && k == box[d] ? box[d] - 1 : open ? (last < 0 ? k : k - 1 - last) : (k - last) / 2);
+        last = k;
+      }
+      const double l = mesh.h[d] / h0;
+      const double it = mesh.axis[d] == c ? 38.0 + 6.0 * (double)far * std::sqrt(l) : 35.0 + 9.0 * (double)far * l;
+      if (it > jacobi) {
+        jacobi = it;
+        along = mesh.axis[d] == c;
+      }
+    }
+  }
+  return mesh.its <= (along ? 50.0 : 40.0) && jacobi >= 15.0 + std::min(8.0, 0.4 + 2.2 * plan.nl) * mesh.its;
 }
 
 // ---------------------------------------------------------------------------------
