@@ -251,7 +251,7 @@ struct Multigrid {
   void *rap1 = nullptr, *rap2 = nullptr;  // triple-product intermediates
   double* dense[2] = {};                  // last level's operator in dense tiles, and its inverse
   double* dpiv = nullptr;                 // two pivot tiles' inverses
-  double* lam = nullptr;                  // [0] = 1 / lambda_max of the scaled operator
+  double* lam = nullptr;                  // 1 / lambda_max of the scaled operator: used, of the second level, of the finest
   int state = 0;                          // 0: no buffers yet, 1: allocated, -1: does not apply
 };
 // What the choice between the multigrid and the Jacobi preconditioner needs to know of a box mesh:
@@ -269,10 +269,14 @@ bool mg_pays(const int64_t box[3], const MgMesh& mesh, int64_t n, const int64_t*
 bool mg_plan(const int64_t box[3], Multigrid* mg);
 // Doubles of the two triple-product intermediates of the plan.
 void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2);
-// Coarse operators, diagonals and the spectral bound for the matrix vals (fine values in TM).
+// Boxes of fewer than eight elements in a direction.
+bool mg_thin(const Multigrid& mg);
+// For the matrix vals (M: its pattern): second level and spectral bound, and then the other levels.
 template <typename TM>
-void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const uint8_t* is_bc, double* partial,
-              hipStream_t st);
+void mg_setup_range(const Multigrid& mg, const BellView& M, const double* vals, const double* invd, const uint8_t* is_bc,
+                    double* partial, hipStream_t st);
+template <typename TM>
+void mg_setup_rest(const Multigrid& mg, hipStream_t st);
 // Vectors of the multigrid-preconditioned BiCGSTAB.
 struct MgVec {
   double *x, *r, *rhat, *p, *q, *phat, *s, *shat, *t;

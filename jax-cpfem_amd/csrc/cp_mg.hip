@@ -19,8 +19,11 @@
 // systems of 24 shapes, where degree 3 over [0.1, 1.1] takes 731, and 16.3 ms at 64^3 (17.5), 3.0 at
 // 40^3 (3.2).  The last level is the first of at most DENSE_ROWS rows; its inverse is formed by
 // tiles (k_dense_step) and applied as one dense product.
-// lambda_max comes from a power iteration on the second level (the levels' values differ by a
-// few percent, the polynomial's range by ten).
+// lambda_max comes from a power iteration on the second level: on boxes of eight and more elements a
+// side the levels' values differ by a few percent, the polynomial's range by ten.  On thinner ones the
+// second level has one to three elements across, between faces that may both be held, and its value
+// can lie far below the finest level's (a polynomial over too short a range amplifies instead of
+// smoothing): there the finest level's own value is found too, and the larger one taken.
 //
 // The polynomial is run as the three-term recurrence on the iterate,
 //   x' = x + c1 (x - x_prev) + c2 D^-1 (b - A x),
@@ -51,6 +54,7 @@ constexpr int POWER_STEPS = 12;
 constexpr int STALL_FROM = 7;
 constexpr int STALL_LIMIT = 60;       // MG_MAXITER; not the caller's own limit, which may be lower
 constexpr float STALL_SLACK = 6.65f;  // log2(100)
+constexpr int THIN = 8;              // nodes a side up to which the finest level's lambda_max is found too
 constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
 constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
 
@@ -349,7 +353,7 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_resid(BellView M, const T
 }
 
 // Power iteration: xo = D^-1 A x, and the partial sums of <xo, xo> and <x, x>.
-template <typename TM, int P>
+template <typename TM, bool FINE, int P>
 __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_power(BellView M, const TM* __restrict__ A, MgGrid g,
                                                             const double* __restrict__ minv, const double* __restrict__ x,
                                                             double* __restrict__ xo, double* __restrict__ partial, int ps) {
@@ -357,7 +361,7 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mg_power(BellView M, const T
   __shared__ double sh[2 * (MgShape<P>::BS / 64)];
   int r;
   double acc, v[2] = {0.0, 0.0};
-  if (mg_row<TM, false, P>(M, g, A, x, 0, r, acc, red)) {
+  if (mg_row<TM, FINE, P>(M, g, A, x, 0, r, acc, red)) {
     const double y = minv[r] * acc;
     xo[r] = y;
     v[0] = y * y;
@@ -378,7 +382,8 @@ __global__ void __launch_bounds__(256) k_mg_power_start(MgGrid g, const double* 
   const double s = ((p.x + p.y + p.z) & 1) ? -1.0 : 1.0;
   x[r] = minv[r] != 0.0 ? s * (0.5 + (double)(h >> 8) * (1.0 / 16777216.0)) : 0.0;
 }
-__global__ void __launch_bounds__(256) k_mg_power_finish(const double* __restrict__ partial, int count, int ps,
+// lam[1 + which] = 1 / lambda_max; lam[0] the least of those found.
+__global__ void __launch_bounds__(256) k_mg_power_finish(const double* __restrict__ partial, int count, int ps, int which,
                                                         double* __restrict__ lam) {
   __shared__ double sh[2 * 4];
   double v[2] = {0.0, 0.0};
@@ -393,7 +398,11 @@ __global__ void __launch_bounds__(256) k_mg_power_finish(const double* __restric
     if (lane == 0) sh[j * 4 + wid] = s;
   }
   __syncthreads();
-  if (threadIdx.x == 0) lam[0] = sqrt((sh[4] + sh[5] + sh[6] + sh[7]) / (sh[0] + sh[1] + sh[2] + sh[3]));
+  if (threadIdx.x == 0) {
+    const double il = sqrt((sh[4] + sh[5] + sh[6] + sh[7]) / (sh[0] + sh[1] + sh[2] + sh[3]));
+    lam[1 + which] = il;
+    lam[0] = which ? fmin(lam[0], il) : il;
+  }
 }
 
 // P^T r at coarse row t (res: the residual of grid f).
@@ -689,18 +698,18 @@ static inline int level_parts(int64_t n) { return n >= FLAT_ROWS ? 1 : 3; }
 static inline unsigned level_blocks(int64_t n) { return (unsigned)(level_parts(n) == 1 ? (n + 255) / 256 : (n + 63) / 64); }
 static inline int level_order(int64_t n, int rev) { return (rev & 1) | (n < PLAIN_ROWS ? 2 : 0); }
 int mg_spmv_blocks(int64_t n) { return (int)level_blocks(n); }
+// Dirichlet flags of a coarse level, in its residual until the first cycle.
+static inline uint8_t* level_flags(const Multigrid& mg, int l) { return reinterpret_cast<uint8_t*>(mg.lv[l].r); }
 int mg_dense_tiles(int64_t n) { return (int)((n + NB - 1) / NB); }
 
+// Coarse operators of levels first + 1 to last; fixed: Dirichlet flags of level `first`.
 template <typename TM>
-void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const uint8_t* is_bc,
-              double* partial, hipStream_t st) {
-  hipLaunchKernelGGL(k_mg_mask, dim3(blocks256(mg.lv[0].g.n)), dim3(256), 0, st, mg.lv[0].g.n, invd, is_bc, mg.lv[0].minv);
+static void coarsen(const Multigrid& mg, int first, int last, const double* vals, const uint8_t* fixed, hipStream_t st) {
   double *w1 = static_cast<double*>(mg.rap1), *w2 = static_cast<double*>(mg.rap2);
-  const uint8_t* fixed = is_bc;
-  for (int l = 0; l + 1 < mg.nl; ++l) {
+  for (int l = first; l < last; ++l) {
     const MgGrid f = mg.lv[l].g, g = mg.lv[l + 1].g;
     const MgGrid gx = make_grid(g.nx, f.ny, f.nz), gy = make_grid(g.nx, g.ny, f.nz);
-    uint8_t* cfixed = reinterpret_cast<uint8_t*>(mg.lv[l + 1].r);  // flags live there until the first cycle
+    uint8_t* cfixed = level_flags(mg, l + 1);
     hipLaunchKernelGGL(k_mg_inject, dim3(blocks256(g.n)), dim3(256), 0, st, f, g, fixed, cfixed);
     if (l == 0)
       hipLaunchKernelGGL((k_mg_coarsen<0, true, false, double, double>), dim3(blocks256(gx.n), 27), dim3(256), 0, st, f, gx, vals,
@@ -714,6 +723,42 @@ void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const
                        cfixed, static_cast<TM*>(mg.lv[l + 1].A), mg.lv[l + 1].minv);
     fixed = cfixed;
   }
+}
+
+// Power iteration on one level; which: 0 the second level's, 1 the finest one's, after it.
+template <typename TM, bool FINE>
+static void power(const Multigrid& mg, int l, const BellView& M, const TM* A, int which, double* partial, hipStream_t st) {
+  const MgLevel& L = mg.lv[l];
+  const unsigned nb = level_blocks(L.g.n);
+  double *a = L.x0, *b = L.x1;
+  hipLaunchKernelGGL(k_mg_power_start, dim3(blocks256(L.g.n)), dim3(256), 0, st, L.g, L.minv, a);
+  for (int k = 0; k < POWER_STEPS; ++k) {
+    if (level_parts(L.g.n) == 1)
+      hipLaunchKernelGGL((k_mg_power<TM, FINE, 1>), dim3(nb), dim3(MgShape<1>::BS), 0, st, M, A, L.g, L.minv, a, b, partial, (int)nb);
+    else
+      hipLaunchKernelGGL((k_mg_power<TM, FINE, 3>), dim3(nb), dim3(MgShape<3>::BS), 0, st, M, A, L.g, L.minv, a, b, partial, (int)nb);
+    std::swap(a, b);
+  }
+  hipLaunchKernelGGL(k_mg_power_finish, dim3(1), dim3(256), 0, st, partial, (int)nb, (int)nb, which, mg.lam);
+}
+
+bool mg_thin(const Multigrid& mg) {
+  const MgGrid& g = mg.lv[0].g;
+  return std::min({g.nx, g.ny, g.nz}) <= THIN;
+}
+
+template <typename TM>
+void mg_setup_range(const Multigrid& mg, const BellView& M, const double* vals, const double* invd, const uint8_t* is_bc,
+                    double* partial, hipStream_t st) {
+  hipLaunchKernelGGL(k_mg_mask, dim3(blocks256(mg.lv[0].g.n)), dim3(256), 0, st, mg.lv[0].g.n, invd, is_bc, mg.lv[0].minv);
+  coarsen<TM>(mg, 0, 1, vals, is_bc, st);
+  power<TM, false>(mg, 1, BellView{}, static_cast<const TM*>(mg.lv[1].A), 0, partial, st);
+  if (mg_thin(mg)) power<double, true>(mg, 0, M, vals, 1, partial, st);
+}
+
+template <typename TM>
+void mg_setup_rest(const Multigrid& mg, hipStream_t st) {
+  coarsen<TM>(mg, 1, mg.nl - 1, nullptr, level_flags(mg, 1), st);
   const MgLevel& E = mg.lv[mg.nl - 1];
   const int nt = mg_dense_tiles(E.g.n);
   hipLaunchKernelGGL(k_dense_fill<TM>, dim3((unsigned)((nt * NB + 255) / 256), (unsigned)(nt * NB)), dim3(256), 0, st, E.g, nt,
@@ -722,21 +767,6 @@ void mg_setup(const Multigrid& mg, const double* vals, const double* invd, const
   for (int k = 0; k < nt; ++k)
     hipLaunchKernelGGL(k_dense_step, dim3((unsigned)nt, (unsigned)nt), dim3(256), 0, st, nt, k, mg.dense[k & 1],
                        mg.dense[(k & 1) ^ 1], mg.dpiv + (k & 1) * TILE, mg.dpiv + ((k & 1) ^ 1) * TILE);
-  // lambda_max on the second level
-  const MgLevel& L = mg.lv[1];
-  const unsigned nb = level_blocks(L.g.n);
-  double *a = L.x0, *b = L.x1;
-  hipLaunchKernelGGL(k_mg_power_start, dim3(blocks256(L.g.n)), dim3(256), 0, st, L.g, L.minv, a);
-  for (int k = 0; k < POWER_STEPS; ++k) {
-    if (level_parts(L.g.n) == 1)
-      hipLaunchKernelGGL((k_mg_power<TM, 1>), dim3(nb), dim3(MgShape<1>::BS), 0, st, BellView{}, static_cast<const TM*>(L.A), L.g,
-                         L.minv, a, b, partial, (int)nb);
-    else
-      hipLaunchKernelGGL((k_mg_power<TM, 3>), dim3(nb), dim3(MgShape<3>::BS), 0, st, BellView{}, static_cast<const TM*>(L.A), L.g,
-                         L.minv, a, b, partial, (int)nb);
-    std::swap(a, b);
-  }
-  hipLaunchKernelGGL(k_mg_power_finish, dim3(1), dim3(256), 0, st, partial, (int)nb, (int)nb, mg.lam);
 }
 
 template <typename F, typename... Args>
@@ -1063,7 +1093,9 @@ void mg_krylov_finish(const Multigrid& mg, const BellView& M, const double* vals
 }
 
 #define CPFEM_MG_INST(TM)                                                                                                   \
-  template void mg_setup<TM>(const Multigrid&, const double*, const double*, const uint8_t*, double*, hipStream_t);         \
+  template void mg_setup_range<TM>(const Multigrid&, const BellView&, const double*, const double*, const uint8_t*,         \
+                                   double*, hipStream_t);                                                                  \
+  template void mg_setup_rest<TM>(const Multigrid&, hipStream_t);                                                          \
   template void mg_krylov_begin<TM>(const Multigrid&, const BellView&, const TM*, MgVec, KrylovWork, int, uint64_t*,          \
                                     hipStream_t, Prof*);                                                                    \
   template void mg_krylov_finish<TM>(const Multigrid&, const BellView&, const double*, const TM*, MgVec, KrylovWork, int,   \

@@ -60,6 +60,39 @@ def test_no_multigrid_work_where_the_jacobi_solve_is_faster(n, h, held):
     assert torch.equal(x, xj)
 
 
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n, h", [((24, 24, 6), (1, 1, 0.3)), ((80, 80, 3), (1, 1, 1)), ((24, 24, 7), (1, 1, 0.5))])
+def test_thin_boxes_whose_second_level_has_a_lower_spectrum(n, h, precision):
+    """The second level's lambda_max is 1.13 to 1.2 times below the finest one's, beyond what the
+    polynomial's range allows for: the range has to be the finest level's.  The bars are those of the other
+    comparisons with the Jacobi solve: |r| <= 1e-11 (|b| + |r0|) where both solves stop at 1e-12."""
+    import cpfem_amd as C
+    from cpfem_amd.solver import krylov_solve, multigrid_solve
+    prob, mat, b, x0 = _system(n, h, False)
+    opts = {"krylov_tol": 1e-12, "krylov_atol": 1e-14, "precision": precision}
+    xj = krylov_solve(prob, mat, b, x0, opts).cpu().numpy()
+    x = multigrid_solve(prob, mat, b, x0, opts).cpu().numpy()
+    k = prob.solver_info[-1]["iterations"]
+    A = C.BlockEllMatrix(prob.ctx, mat).to_scipy()
+    bh = b.cpu().numpy()
+    r, bar = np.linalg.norm(A @ x - bh), 1e-11 * (np.linalg.norm(bh) + np.linalg.norm(bh - A @ x0.cpu().numpy()))
+    print(n, h, precision, k, f"|Ax - b| {r:.2e} (bar {bar:.2e})", flush=True)
+    assert 0 < k <= 30
+    assert r <= bar
+    assert np.linalg.norm(x - xj) <= 1e-7 * np.linalg.norm(xj)
+
+
+@pytest.mark.parametrize("n, h", [((32, 32, 4), (1, 1, 0.5)), ((2, 2, 60), (1, 1, 1.4))])
+def test_thin_boxes_whose_second_level_is_no_coarse_form(n, h):
+    """Where the second level's lambda_max lies further below, no iteration is begun."""
+    from cpfem_amd.solver import krylov_solve, multigrid_solve
+    prob, mat, b, x0 = _system(n, h, False)
+    xj = krylov_solve(prob, mat, b, x0)
+    x, launches = _launches(prob, lambda: multigrid_solve(prob, mat, b, x0))
+    assert launches["mg_setup"] > 0 and launches["mg_fine"] == 0
+    assert torch.equal(x, xj)
+
+
 def test_an_attempt_in_vain_leaves_nothing_behind():
     """A system that the estimates let through and multigrid does not solve: the Jacobi solve starts from x0."""
     from cpfem_amd.solver import krylov_solve, multigrid_solve
