@@ -698,6 +698,7 @@ static bool ensure_mg(cpfem_ctx* c) {
   Multigrid& mg = c->mg;
   if (mg.state) return mg.state > 0;
   mg.state = -1;
+  mg.fine_range = mg_fine_range(c->box, c->mg_shape);
   if (c->n_slots != 27 || c->n_dofs < MG_MIN_ROWS || !mg_plan(c->box, &mg)) return false;
   const auto get = [&](size_t doubles) -> double* {
     void* p = nullptr;
@@ -748,9 +749,9 @@ static int run_mg(cpfem_ctx* c, hipStream_t st, const double* mat, const TM* mat
   launch_inv_diag(M, mat, c->d_dslot, c->kv64[8], 1, st);
   int sl = prof_begin(&c->prof, PC_MG_SETUP, st);
   mg_setup_range<TM>(mg, M, mat, c->kv64[8], c->d_isbc, c->d_kpartial, st);
-  if (mg_thin(mg)) {
+  if (mg.fine_range) {
     // A second level whose lambda_max lies a fifth below the finest one's is no coarse form of it (its few
-    // nodes across the box are held): 32x32x4 of 1:1:0.4, 1.26 times, of 1:1:0.7 1.31; 24x24x6 of cubes 1.01.
+    // nodes across the box are held): 32x32x4 of 1:1:0.4, 1.26 times, of 1:1:0.7 1.31; 24x24x6 of 1:1:2 1.01.
     HIPCHK(hipMemcpyAsync(c->h_dbl, mg.lam, 3 * sizeof(double), hipMemcpyDeviceToHost, st));
     HIPCHK(hipStreamSynchronize(st));
     if (!(c->h_dbl[1] <= 1.2 * c->h_dbl[2])) {

@@ -252,6 +252,7 @@ struct Multigrid {
   double* dense[2] = {};                  // last level's operator in dense tiles, and its inverse
   double* dpiv = nullptr;                 // two pivot tiles' inverses
   double* lam = nullptr;                  // 1 / lambda_max of the scaled operator: used, of the second level, of the finest
+  bool fine_range = false;                // the finest level's lambda_max is found too
   int state = 0;                          // 0: no buffers yet, 1: allocated, -1: does not apply
 };
 // What the choice between the multigrid and the Jacobi preconditioner needs to know of a box mesh:
@@ -261,6 +262,7 @@ struct MgMesh {
   double h[3] = {0.0, 0.0, 0.0};
   int axis[3] = {0, 1, 2};
   double its = 0.0;
+  double stretch = 1.0;  // longest over shortest edge of an element, the most over the elements
 };
 MgMesh mg_mesh(const int64_t box[3], const double* points);
 // Whether the multigrid solve is expected to be the shorter one, for these n Dirichlet dofs (host).
@@ -269,8 +271,8 @@ bool mg_pays(const int64_t box[3], const MgMesh& mesh, int64_t n, const int64_t*
 bool mg_plan(const int64_t box[3], Multigrid* mg);
 // Doubles of the two triple-product intermediates of the plan.
 void mg_scratch(const Multigrid& mg, int64_t* n1, int64_t* n2);
-// Boxes of fewer than eight elements in a direction.
-bool mg_thin(const Multigrid& mg);
+// Whether the finest level's lambda_max has to be found too.
+bool mg_fine_range(const int64_t box[3], const MgMesh& mesh);
 // For the matrix vals (M: its pattern): second level and spectral bound, and then the other levels.
 template <typename TM>
 void mg_setup_range(const Multigrid& mg, const BellView& M, const double* vals, const double* invd, const uint8_t* is_bc,

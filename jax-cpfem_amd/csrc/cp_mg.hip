@@ -23,7 +23,7 @@
 // side the levels' values differ by a few percent, the polynomial's range by ten.  On thinner ones the
 // second level has one to three elements across, between faces that may both be held, and its value
 // can lie far below the finest level's (a polynomial over too short a range amplifies instead of
-// smoothing): there the finest level's own value is found too, and the larger one taken.
+// smoothing): there (mg_fine_range) the finest level's own value is found too, and the larger one taken.
 //
 // The polynomial is run as the three-term recurrence on the iterate,
 //   x' = x + c1 (x - x_prev) + c2 D^-1 (b - A x),
@@ -54,7 +54,6 @@ constexpr int POWER_STEPS = 12;
 constexpr int STALL_FROM = 7;
 constexpr int STALL_LIMIT = 60;       // MG_MAXITER; not the caller's own limit, which may be lower
 constexpr float STALL_SLACK = 6.65f;  // log2(100)
-constexpr int THIN = 8;              // nodes a side up to which the finest level's lambda_max is found too
 constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
 constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
 
@@ -165,13 +164,24 @@ MgMesh mg_mesh(const int64_t box[3], const double* points) {
           m.h[d] += len[d];
           count[d] += 1.0;
         }
-        if (in[0] && in[1] && in[2]) m.its = std::max(m.its, mg_iterations(len[0], len[1], len[2]));
+        if (in[0] && in[1] && in[2]) {
+          m.its = std::max(m.its, mg_iterations(len[0], len[1], len[2]));
+          m.stretch = std::max(m.stretch, std::max({len[0], len[1], len[2]}) / std::min({len[0], len[1], len[2]}));
+        }
       }
   for (int d = 0; d < 3; ++d) {
     m.h[d] /= std::max(count[d], 1.0);
     m.axis[d] = (int)(std::max_element(run[d], run[d] + 3) - run[d]);
   }
   return m;
+}
+
+// Boxes of fewer than eight elements in a direction, if the elements are not nearly cubes, and of fewer than
+// four: there the second level's lambda_max was up to 1.8 times below the finest one's; cubes, four to
+// seven across between held faces, 1.01 to 1.04.
+bool mg_fine_range(const int64_t box[3], const MgMesh& mesh) {
+  const int64_t across = std::min({box[0], box[1], box[2]}) - 1;
+  return across < 4 || (across < 8 && mesh.stretch > 1.25);
 }
 
 bool mg_pays(const int64_t box[3], const MgMesh& mesh, int64_t n, const int64_t* dofs) {
@@ -742,18 +752,13 @@ static void power(const Multigrid& mg, int l, const BellView& M, const TM* A, in
   hipLaunchKernelGGL(k_mg_power_finish, dim3(1), dim3(256), 0, st, partial, (int)nb, (int)nb, which, mg.lam);
 }
 
-bool mg_thin(const Multigrid& mg) {
-  const MgGrid& g = mg.lv[0].g;
-  return std::min({g.nx, g.ny, g.nz}) <= THIN;
-}
-
 template <typename TM>
 void mg_setup_range(const Multigrid& mg, const BellView& M, const double* vals, const double* invd, const uint8_t* is_bc,
                     double* partial, hipStream_t st) {
   hipLaunchKernelGGL(k_mg_mask, dim3(blocks256(mg.lv[0].g.n)), dim3(256), 0, st, mg.lv[0].g.n, invd, is_bc, mg.lv[0].minv);
   coarsen<TM>(mg, 0, 1, vals, is_bc, st);
   power<TM, false>(mg, 1, BellView{}, static_cast<const TM*>(mg.lv[1].A), 0, partial, st);
-  if (mg_thin(mg)) power<double, true>(mg, 0, M, vals, 1, partial, st);
+  if (mg.fine_range) power<double, true>(mg, 0, M, vals, 1, partial, st);
 }
 
 template <typename TM>
