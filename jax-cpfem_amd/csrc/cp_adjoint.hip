@@ -17,17 +17,17 @@ namespace cpfem {
 constexpr int VBS = 64;  // threads per block of the point VJP kernel: one wave
 
 // Converged stress of a point that the crystal-frame form does not cover.
-template <int N>
+template <int N, int L>
 __device__ __attribute__((noinline)) void general_stress(const Geom& G, const double* __restrict__ u, const StateView& sv,
-                                                         const MatView& mv, const SlipTable<N>& tab, const SolveCfg& cfg, int64_t q,
-                                                         double* s) {
+                                                         const MatView& mv, const SlipTable<N>* table, const SolveCfg& cfg, int64_t q,
+                                                         int sub, LdsDouble* sh, double* s) {
   PointIn in;
   in.load(G, u, sv, mv, q);
-  Point<N> pt;
   int32_t st = 0;
-  GeneralStore<N> store;
-  store.setup(pt, in, sv, q);
-  pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
+  Point<N, L, Crystal<N, L>::K> pt;
+  CrystalRest<N, L> rest;
+  setup_general<VBS>(pt, in, sv, q, sub, sh, rest);
+  pt.solve(uniform_table(table), cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
 }
 
 // A point's inputs, read from memory again at each load().
@@ -56,7 +56,7 @@ struct PointRead {
 // Fpibar [9][Q], 4 g_old -> gbar_old [N][Q], 8 material -> pbar [8][Q], 16 R -> Rbar [9][Q].
 //
 // The local Newton is solved again (by L lanes a point, as in the other point kernels); the first
-// lane of a point then runs the reverse sweep, with 261 to 318 registers spilled outside its loops
+// lane of a point then runs the reverse sweep, with 269 to 318 registers spilled outside its loops
 // (two waves per SIMD are worth more to the re-solve).  16^3, FCC: 174 us, half of it the re-solve;
 // 1938 us with one forward evaluation of the map per input direction.
 template <int N, int L>
@@ -87,10 +87,10 @@ k_local_vjp(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Slip
       double R[9], Fpi[9];
       load_point(sv, reread(q), Fpi, R);
       pt.stress(nw.s, R, s);
-    } else if (sub == 0) {
+    } else {
       const OutOfLine f{G, sv, mv, cfg};
       double sg[6];
-      general_stress<N>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, sg);
+      general_stress<N, L>(f.G, u, f.sv, f.mv, gen, f.cfg, q, sub, (LdsDouble*)sh, sg);
 #pragma unroll
       for (int i = 0; i < 6; ++i) s[i] = sg[i];
     }

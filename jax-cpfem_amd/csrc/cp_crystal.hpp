@@ -28,8 +28,6 @@
 // a row, the sums are exchanged by DPP in an order that gives every lane the same bits, and
 // everything else is computed by all of them alike.
 #pragma once
-#include <type_traits>
-
 #include "cp_point.hpp"
 
 namespace cpfem {
@@ -57,24 +55,6 @@ inline bool make_slip_sys(const SlipTable<N>& t, SlipSys<N>* o) {
     ok = ok && fabs(d[0] * n[0] + d[1] * n[1] + d[2] * n[2]) <= 1e-15;
   }
   return ok;
-}
-
-// Sum over the L lanes of a point, the same bits in each.
-template <int L>
-CPFEM_HD double lane_sum(double v) {
-#if defined(__HIP_DEVICE_COMPILE__)
-  const auto from = [](double x, auto ctrl) {
-    constexpr int C = decltype(ctrl)::value;
-    const long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, C, 0xf, 0xf, true);
-    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), C, 0xf, 0xf, true);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-  };
-  if constexpr (L >= 2) v += from(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
-  if constexpr (L >= 4) v += from(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
-  if constexpr (L >= 8) v += from(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
-#endif
-  return v;
 }
 
 // a b + c for a constant c.  On the device the instruction is written out: the compiler otherwise
@@ -554,36 +534,6 @@ struct CrystalNewton {
     if (!(fabs(pt.nr) <= 1.7976931348623157e308)) *stat |= PT_NONFINITE;
   }
 };
-
-// Kalidindi hardening after convergence (cp_point.hpp's hardening) and the new slips of this lane's
-// systems; x: the converged S'.
-template <int N, int L, int KS, class Tab>
-CPFEM_HD void crystal_history(const Crystal<N, L, KS>& pt, const Tab& tab, const double* x, const PointMat& m, int self_block,
-                              const double* g_old, const double* slip_old, int64_t ld, double* g_new, double* slip_new) {
-  constexpr int M = N / L;
-  double tot = 0.0;
-#pragma unroll 2
-  for (int j = 0; j < M; ++j) {
-    const int64_t o = (pt.a0 + j) * ld;
-    const double dg = pt.increment(tab, j, x);
-    slip_new[o] = slip_old[o] + dg;
-    const double y = 1.0 - g_old[o] / m.tsat;
-    const double t = m.h * fabs(dg) * pow_pos(fabs(y), m.gss_a) * sgn(y);
-    pt.gp(j) = t;  // (used up)
-    tot += t;
-  }
-  tot = lane_sum<L>(tot);
-#pragma unroll 1
-  for (int k = 0; k < M; k += 3) {
-    double inc = m.r * tot;
-    if (self_block) inc += (1.0 - m.r) * (pt.gp(k) + pt.gp(k + 1) + pt.gp(k + 2));
-#pragma unroll
-    for (int j = k; j < k + 3; ++j) {
-      const int64_t o = (pt.a0 + j) * ld;
-      g_new[o] = g_old[o] + inc;
-    }
-  }
-}
 
 // First Piola-Kirchhoff stress P = F Y, Y = Ph S' Ph^T / (bb^2 det Fp_inv_new), Ph = Fp_inv_new R, and
 // the consistent tangent's ingredients.  Q = Fp_inv_old R, W = I - bb Lpc: Ph = Q W and

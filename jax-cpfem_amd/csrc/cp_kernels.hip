@@ -46,30 +46,35 @@ __device__ __forceinline__ void add_counts(unsigned long long* counts, uint32_t 
 // there.  counts (optional): [0] += local Newton iterations, [1] += residual evaluations (one
 // atomic per wave), the measured inputs of the algorithmic flop count.
 //
-// Points that the crystal-frame form does not cover (Crystal::applies) take the general one, in a
-// function of its own, so that its registers do not weigh on the others.
+// Points that the crystal-frame form does not cover (Crystal::applies) take the general one, by the same lanes
+// in a function of its own (cp_points.hpp).
 template <int N, int L>
 __device__ __attribute__((noinline)) void general_res(const Geom& G, const double* __restrict__ u, const StateView& sv,
-                                                      const MatView& mv, const SlipTable<N>& tab, const SolveCfg& cfg, int64_t q,
-                                                      double* __restrict__ wP,
+                                                      const MatView& mv, const SlipTable<N>* table, const SolveCfg& cfg, int64_t q,
+                                                      int sub, LdsDouble* sh, double* __restrict__ wP,
                                                       double* __restrict__ sout, int32_t* __restrict__ iters,
                                                       int32_t* __restrict__ status, uint32_t* n_it, uint32_t* n_ev) {
   PointIn in;
   in.load(G, u, sv, mv, q);
-  Point<N> pt;
   double s[6], P[9];
   int32_t st = 0;
-  GeneralStore<N> store;
-  store.setup(pt, in, sv, q);
+  ConstTable<N>& tab = uniform_table(table);
+  Point<N, L, Crystal<N, L>::K> pt;
+  CrystalRest<N, L> rest;
+  setup_general<QBS>(pt, in, sv, q, sub, sh, rest);
   const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
-  pk1<N>(pt, in.F, in.Fpi, s, P);
+  in.load(G, u, sv, mv, reread(q));
+  pk1(pt, in.F, in.Fpi, s, P);
   const double w = jxw_at(G, q);
 #pragma unroll
-  for (int i = 0; i < 9; ++i) wP[i * G.n_qp + q] = w * P[i];
+  for (int i = 0; i < 9; ++i)
+    if (L == 1 || i % L == sub) wP[i * G.n_qp + q] = w * P[i];
   if (sout) {
 #pragma unroll
-    for (int j = 0; j < 6; ++j) sout[j * G.n_qp + q] = s[j];
+    for (int j = 0; j < 6; ++j)
+      if (L == 1 || j % L == sub) sout[j * G.n_qp + q] = s[j];
   }
+  if (sub != 0) return;
   if (iters) iters[q] = it;
   if (st) atomicOr(status, st);
   *n_it = (uint32_t)it;
@@ -160,10 +165,10 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
     CrystalNewton<N, L>::finite(pt, &st);
     finish_point<N, L>(G, q, sub, pt, in, nw, st, wP, sout, iters, status);
     n_it = sub == 0 ? (uint32_t)nw.it : 0u;
-  } else if (valid && !fits && sub == 0) {
+  } else if (valid && !fits) {
     // (its residuals here are not counted twice)
     OutOfLine f{G, sv, mv, cfg};
-    general_res<N, L>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, wP, sout, iters, status, &f.n_it, &f.n_ev);
+    general_res<N, L>(f.G, u, f.sv, f.mv, gen, f.cfg, q, sub, (LdsDouble*)sh, wP, sout, iters, status, &f.n_it, &f.n_ev);
     n_it = f.n_it;
     n_ev = f.n_ev;
   }
@@ -172,16 +177,17 @@ k_element_res(Geom G, const double* __restrict__ u, StateView sv, MatView mv, Sl
 
 template <int N>
 __device__ __attribute__((noinline)) void general_tangent(const Geom& G, const double* __restrict__ u, const StateView& sv,
-                                                          const MatView& mv, const SlipTable<N>& tab, int64_t q,
+                                                          const MatView& mv, const SlipTable<N>* table, int64_t q, LdsDouble* sh,
                                                           const double* __restrict__ sin, double* __restrict__ wA) {
   PointIn in;
   in.load(G, u, sv, mv, q);
-  Point<N> pt;
   double s[6];
 #pragma unroll
   for (int j = 0; j < 6; ++j) s[j] = sin[j * G.n_qp + q];
-  GeneralStore<N> store;
-  store.setup(pt, in, sv, q);
+  ConstTable<N>& tab = uniform_table(table);
+  Point<N> pt;
+  CrystalRest<N, 1, N> rest;
+  setup_general<QBS>(pt, in, sv, q, 0, sh, rest);
   pt.eval(tab, s);
   const double w = jxw_at(G, q);
   tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
@@ -218,7 +224,7 @@ __global__ void __launch_bounds__(QBS) k_point_tangent(Geom G, const double* __r
   }
   if (!done) {
     const OutOfLine f{G, sv, mv, {}};
-    general_tangent<N>(f.G, u, f.sv, f.mv, *gen, q, sin, wA);
+    general_tangent<N>(f.G, u, f.sv, f.mv, gen, q, (LdsDouble*)sh, sin, wA);
   }
 }
 
@@ -257,12 +263,10 @@ k_element_qp_park(Geom G, const double* __restrict__ u, StateView sv, MatView mv
     bool act = nw.resume(pt, tab, cfg.tol);
     while (act) act = nw.advance(pt, tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, &st);
     if (nw.lost) {
-      if (sub == 0) {
-        OutOfLine f{G, sv, mv, cfg};
-        general_res<N, L>(f.G, u, f.sv, f.mv, *gen, f.cfg, q, wP, sout, iters, status, &f.n_it, &f.n_ev);
-        n_it = f.n_it;
-        n_ev = f.n_ev;
-      }
+      OutOfLine f{G, sv, mv, cfg};
+      general_res<N, L>(f.G, u, f.sv, f.mv, gen, f.cfg, q, sub, (LdsDouble*)sh, wP, sout, iters, status, &f.n_it, &f.n_ev);
+      n_it = f.n_it;
+      n_ev = f.n_ev;
     } else {
       CrystalNewton<N, L>::finite(pt, &st);
       in.load(G, u, sv, mv, reread(q));
@@ -506,48 +510,50 @@ __device__ __forceinline__ void load_local(PointIn& in, const double* __restrict
 template <int N, bool TANGENT, int L>
 __device__ __attribute__((noinline)) void general_local(int64_t n_qp, const double* __restrict__ Hd, const Geom& G,
                                                         const double* __restrict__ u, const StateView& sv, const MatView& mv,
-                                                        const SlipTable<N>& tab, const SolveCfg& cfg, int self_block, int64_t q,
-                                                        const LocalOut& o) {
+                                                        const SlipTable<N>* table, const SolveCfg& cfg, int self_block, int64_t q,
+                                                        int sub, LdsDouble* sh, const LocalOut& o) {
   PointIn in;
   load_local(in, Hd, n_qp, G, u, sv, mv, q);
-  Point<N> pt;
   double s[6], P[9];
   int32_t st = 0;
-  GeneralStore<N> store;
-  store.setup(pt, in, sv, q);
+  ConstTable<N>& tab = uniform_table(table);
+  Point<N, L, Crystal<N, L>::K> pt;
+  CrystalRest<N, L> rest;
+  setup_general<QBS>(pt, in, sv, q, sub, sh, rest);
   const int it = pt.solve(tab, cfg.tol, cfg.max_sub_step, cfg.max_iter, s, &st);
-  pk1<N>(pt, in.F, in.Fpi, s, P);
-  if (TANGENT && o.A) {
-    tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
+  load_local(in, Hd, n_qp, G, u, sv, mv, reread(q));
+  pk1(pt, in.F, in.Fpi, s, P);
+  if constexpr (TANGENT) {
+    if (o.A) {
+      tangent<N>(pt, tab, in.F, in.Fpi, s, [&](int m9, const double* dP) {
 #pragma unroll
-      for (int i = 0; i < 9; ++i) o.A[(9 * i + m9) * n_qp + q] = dP[i];
-    });
+        for (int i = 0; i < 9; ++i) o.A[(9 * i + m9) * n_qp + q] = dP[i];
+      });
+    }
   }
   if (o.P) {
 #pragma unroll
-    for (int i = 0; i < 9; ++i) o.P[i * n_qp + q] = P[i];
+    for (int i = 0; i < 9; ++i)
+      if (L == 1 || i % L == sub) o.P[i * n_qp + q] = P[i];
   }
   if (o.sig) {
     double sg[9];
     mm3t(P, in.F, sg);
     const double idF = 1.0 / det3(in.F);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) o.sig[i * n_qp + q] = sg[i] * idF;
+    for (int i = 0; i < 9; ++i)
+      if (L == 1 || i % L == sub) o.sig[i * n_qp + q] = sg[i] * idF;
   }
   if (o.so.Fpi) {
     double Fn[9], Sc[9];
     fp_inv_new(in.Fpi, in.R, pt.Lpc, Fn);
 #pragma unroll
-    for (int i = 0; i < 9; ++i) o.so.Fpi[i * sv.ld + q] = Fn[i];
+    for (int i = 0; i < 9; ++i)
+      if (L == 1 || i % L == sub) o.so.Fpi[i * sv.ld + q] = Fn[i];
     pt.crystal_stress(s, Sc);
-    for (int a = 0; a < N; ++a) {
-      double dg;
-      pt.slip_increment(tab, Sc, a, &dg);
-      pt.gp(a) = dg;
-      o.so.slip[a * sv.ld + q] = sv.slip[a * sv.ld + q] + dg;
-    }
-    hardening<N>(sv.g + q, sv.ld, pt.gpv, pt.st, in.m, self_block, o.so.g + q, sv.ld);
+    point_history<N, L>(pt, tab, Sc, in.m, self_block, sv.g + q, sv.slip + q, sv.ld, o.so.g + q, o.so.slip + q);
   }
+  if (sub != 0) return;
   if (o.iters) o.iters[q] = it;
   if (st) atomicOr(o.status, st);
 }
@@ -581,11 +587,9 @@ k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __res
     });
   }
   if (!fits) {
-    if (sub == 0) {
-      const OutOfLine f{G, sv, mv, cfg};
-      const LocalOut out = o;
-      general_local<N, TANGENT, L>(n_qp, Hd, f.G, u, f.sv, f.mv, *gen, f.cfg, self_block, q, out);
-    }
+    const OutOfLine f{G, sv, mv, cfg};
+    const LocalOut out = o;
+    general_local<N, TANGENT, L>(n_qp, Hd, f.G, u, f.sv, f.mv, gen, f.cfg, self_block, q, sub, (LdsDouble*)sh, out);
     return;
   }
   // every lane of a point writes its share of the components
@@ -612,7 +616,7 @@ k_local(int64_t n_qp, const double* __restrict__ Hd, Geom G, const double* __res
 #pragma unroll
     for (int i = 0; i < 9; ++i)
       if (L == 1 || i % L == sub) o.so.Fpi[i * sv.ld + q] = Fn[i];
-    crystal_history(pt, tab, nw.s, in.m, self_block, sv.g + q, sv.slip + q, sv.ld, o.so.g + q, o.so.slip + q);
+    point_history<N, L>(pt, tab, nw.s, in.m, self_block, sv.g + q, sv.slip + q, sv.ld, o.so.g + q, o.so.slip + q);
   }
   if (sub == 0) {
     if (o.iters) o.iters[q] = nw.it;

@@ -26,6 +26,8 @@
 #include <math.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
 #define CPFEM_HD __host__ __device__ __forceinline__
@@ -266,19 +268,44 @@ CPFEM_HD void lu6_solve(const double* J, const int* piv, double* b) {
   }
 }
 
+// Sum over the L lanes of a point, the same bits in each.
+template <int L>
+CPFEM_HD double lane_sum(double v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  const auto from = [](double x, auto ctrl) {
+    constexpr int C = decltype(ctrl)::value;
+    const long long b = __double_as_longlong(x);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, C, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), C, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+  };
+  if constexpr (L >= 2) v += from(v, std::integral_constant<int, 0xB1>{});   // quad_perm [1,0,3,2]
+  if constexpr (L >= 4) v += from(v, std::integral_constant<int, 0x4E>{});   // quad_perm [2,3,0,1]
+  if constexpr (L >= 8) v += from(v, std::integral_constant<int, 0x141>{});  // row_half_mirror
+#endif
+  return v;
+}
+
 // Per-point solver state.  The per-slip-system arrays (1/g_old and d dgamma/d tau) live
 // outside the register file: in LDS on the device (column [a * stride + lane]), in a plain
 // array in the host build, so the slip loops need not be unrolled.
-template <int N>
+// L lanes (adjacent, a power of two up to 8) may share one point: each takes N / L slip systems in
+// a row, lane_sum gives every lane the same sums, and everything else is computed by all of them alike.
+// K of a lane's 1/g_old are in the first store, the others in a second one.
+template <int N, int L = 1, int K = N / L>
 struct Point {
+  static constexpr int M = N / L;  // slip systems of this lane
+  static_assert(N % L == 0 && M % 3 == 0, "a lane takes whole blocks of three slip systems");
   double R[9];    // rotation (as given, not re-orthonormalised)
   double A[9];    // F Fp_inv_old
   double C6[21];  // rotated stiffness, packed symmetric Voigt
   double p, c;    // 1/m, gamma0 dt
-  double* gpv;    // d dgamma_a / d tau_a   [a * st]
-  double* giv;    // 1 / g_old_a            [a * sti]
+  double* gpv;    // d dgamma / d tau of this lane's systems   [j * st]
+  double* giv;    // 1 / g_old of the first K                  [j * sti]
+  double* grv;    // of the others
   int st;
   int64_t sti;
+  int a0;         // first slip system of this lane
   // results of the last residual evaluation
   double Lpc[9];  // sum_a dgamma_a d_a (x) n_a   (crystal frame)
   double Fe[9];
@@ -286,14 +313,22 @@ struct Point {
   double nr;
   int nev;        // residual evaluations since setup (work counter)
 
-  CPFEM_HD double& gp(int a) { return gpv[a * st]; }
-  CPFEM_HD double& gi(int a) { return giv[a * sti]; }
+  CPFEM_HD double& gp(int j) { return gpv[j * st]; }
+  CPFEM_HD double gi(int j) const {
+    if (K >= M) return giv[j * sti];
+    const double u = giv[(j < K ? j : 0) * sti], v = grv[j < K ? 0 : j - K];  // (one address for both stores is a flat one)
+    return j < K ? u : v;
+  }
 
-  // gp_store / gi_store: the per-slip arrays, at stride `stride` and `stride_gi` (-1: the same)
+  // gp_store / gi_store: the per-slip arrays, at stride `stride` and `stride_gi` (-1: the same); sub: this
+  // lane among the point's; gr_store: 1/g_old beyond the first K.
   CPFEM_HD void setup(const double* F, const double* Fpi_old, const double* Rin, const double* g_old, int64_t gstride,
-                      const PointMat& m, double* gp_store, double* gi_store, int stride, int64_t stride_gi = -1) {
+                      const PointMat& m, double* gp_store, double* gi_store, int stride, int64_t stride_gi = -1, int sub = 0,
+                      double* gr_store = nullptr) {
     gpv = gp_store;
     giv = gi_store;
+    grv = gr_store;
+    a0 = sub * M;
     st = stride;
     sti = stride_gi < 0 ? stride : stride_gi;
 #pragma unroll
@@ -301,7 +336,13 @@ struct Point {
     mm3(F, Fpi_old, A);
     rotated_stiffness(R, m.C11, m.C12, m.C44, C6);
 #pragma unroll 2
-    for (int a = 0; a < N; ++a) gi(a) = 1.0 / g_old[a * gstride];
+    for (int j = 0; j < M; ++j) {
+      const double v = 1.0 / g_old[(a0 + j) * gstride];
+      if (j < K)
+        giv[j * sti] = v;
+      else
+        grv[j - K] = v;
+    }
     p = m.p;
     c = m.c;
     nev = 0;
@@ -316,27 +357,36 @@ struct Point {
   }
 
   // Residual at symmetric S (Voigt 6); fills gp, Lpc, Fe, r, nr.
-  CPFEM_HD void eval(const SlipTable<N>& tab, const double* s) {
+  template <class Tab>
+  CPFEM_HD void eval(const Tab& tab, const double* s) {
     ++nev;
     double Sc[9];
     crystal_stress(s, Sc);
 #pragma unroll
     for (int i = 0; i < 9; ++i) Lpc[i] = 0.0;
-#pragma unroll 2
-    for (int a = 0; a < N; ++a) {
+    const auto system = [&](int j, double gia) {
+      const int a = L == 1 ? j : a0 + j;
       const double d0 = tab.d[a][0], d1 = tab.d[a][1], d2 = tab.d[a][2];
       const double n0 = tab.n[a][0], n1 = tab.n[a][1], n2 = tab.n[a][2];
       const double v0 = Sc[0] * n0 + Sc[1] * n1 + Sc[2] * n2;
       const double v1 = Sc[3] * n0 + Sc[4] * n1 + Sc[5] * n2;
       const double v2 = Sc[6] * n0 + Sc[7] * n1 + Sc[8] * n2;
       const double tau = d0 * v0 + d1 * v1 + d2 * v2;
-      const double ax = fabs(tau * gi(a));
+      const double ax = fabs(tau * gia);
       const double pw = pow_pos(ax, p);
       const double dg = c * pw * sgn(tau);
-      gp(a) = (tau != 0.0) ? c * p * pw / fabs(tau) : (p == 1.0 ? c * gi(a) : 0.0);
+      gp(j) = (tau != 0.0) ? c * p * pw / fabs(tau) : (p == 1.0 ? c * gia : 0.0);
       Lpc[0] += dg * d0 * n0; Lpc[1] += dg * d0 * n1; Lpc[2] += dg * d0 * n2;
       Lpc[3] += dg * d1 * n0; Lpc[4] += dg * d1 * n1; Lpc[5] += dg * d1 * n2;
       Lpc[6] += dg * d2 * n0; Lpc[7] += dg * d2 * n1; Lpc[8] += dg * d2 * n2;
+    };
+#pragma unroll 2
+    for (int j = 0; j < K; ++j) system(j, giv[j * sti]);
+#pragma unroll 2
+    for (int j = K; j < M; ++j) system(j, grv[j - K]);
+    if (L > 1) {
+#pragma unroll
+      for (int i = 0; i < 9; ++i) Lpc[i] = lane_sum<L>(Lpc[i]);
     }
     // Fe = A (I - R Lpc R^T)
     double X[9], Y[9], Z[9];
@@ -360,28 +410,38 @@ struct Point {
     nr = sqrt(r[0] * r[0] + r[1] * r[1] + r[2] * r[2] + 2.0 * (r[3] * r[3] + r[4] * r[4] + r[5] * r[5]));
   }
 
-  // Slip increments at symmetric S (same arithmetic as eval).
-  CPFEM_HD void slip_increment(const SlipTable<N>& tab, const double* Sc, int a, double* dg) {
+  // Slip increment of this lane's system j at the crystal-frame stress Sc (same arithmetic as eval).
+  template <class Tab>
+  CPFEM_HD double increment(const Tab& tab, int j, const double* Sc) {
+    double dg;
+    slip_increment(tab, Sc, j, &dg);
+    return dg;
+  }
+  template <class Tab>
+  CPFEM_HD void slip_increment(const Tab& tab, const double* Sc, int j, double* dg) {
+    const int a = L == 1 ? j : a0 + j;
     const double d0 = tab.d[a][0], d1 = tab.d[a][1], d2 = tab.d[a][2];
     const double n0 = tab.n[a][0], n1 = tab.n[a][1], n2 = tab.n[a][2];
     const double v0 = Sc[0] * n0 + Sc[1] * n1 + Sc[2] * n2;
     const double v1 = Sc[3] * n0 + Sc[4] * n1 + Sc[5] * n2;
     const double v2 = Sc[6] * n0 + Sc[7] * n1 + Sc[8] * n2;
     const double tau = d0 * v0 + d1 * v1 + d2 * v2;
-    *dg = c * pow_pos(fabs(tau * gi(a)), p) * sgn(tau);
+    *dg = c * pow_pos(fabs(tau * gi(j)), p) * sgn(tau);
   }
 
   // Jacobian dr/ds (6x6, row-major) at the last evaluated point:
   // J = I + C6 * sum_a g'_a W_a b_a^T with W_a = 2 sym(M R d_a (x) R n_a) (engineering form),
-  // b_a = d tau_a / d s, M = Fe^T A.
-  CPFEM_HD void jac(const SlipTable<N>& tab, double* J) {
-    double M[9], MR[9];
-    mtm3(Fe, A, M);
-    mm3(M, R, MR);
+  // b_a = d tau_a / d s, M = Fe^T A (FA).
+  template <class Tab>
+  CPFEM_HD void jac(const Tab& tab, double* J) {
+    double FA[9], MR[9];
+    mtm3(Fe, A, FA);
+    mm3(FA, R, MR);
 #pragma unroll
     for (int i = 0; i < 36; ++i) J[i] = 0.0;
 #pragma unroll 2
-    for (int a = 0; a < N; ++a) {
+    for (int k = 0; k < M; ++k) {
+      const int a = L == 1 ? k : a0 + k;
       const double d0 = tab.d[a][0], d1 = tab.d[a][1], d2 = tab.d[a][2];
       const double n0 = tab.n[a][0], n1 = tab.n[a][1], n2 = tab.n[a][2];
       const double m0 = MR[0] * d0 + MR[1] * d1 + MR[2] * d2;
@@ -393,7 +453,7 @@ struct Point {
       const double u0 = R[0] * n0 + R[1] * n1 + R[2] * n2;
       const double u1 = R[3] * n0 + R[4] * n1 + R[5] * n2;
       const double u2 = R[6] * n0 + R[7] * n1 + R[8] * n2;
-      const double g = gp(a);
+      const double g = gp(k);
       double w[6], b[6];
       w[0] = g * m0 * u0; w[1] = g * m1 * u1; w[2] = g * m2 * u2;
       w[3] = g * (m1 * u2 + m2 * u1); w[4] = g * (m0 * u2 + m2 * u0); w[5] = g * (m0 * u1 + m1 * u0);
@@ -403,6 +463,10 @@ struct Point {
       for (int i = 0; i < 6; ++i)
 #pragma unroll
         for (int j = 0; j < 6; ++j) J[6 * i + j] += w[i] * b[j];
+    }
+    if (L > 1) {
+#pragma unroll
+      for (int i = 0; i < 36; ++i) J[i] = lane_sum<L>(J[i]);
     }
     // in place, column by column: J[:, j] <- e_j + C6 * G[:, j]
 #pragma unroll
@@ -423,7 +487,8 @@ struct Point {
   // One local Newton iteration from the last evaluated point s (models_copper.py:218-247):
   // d = -J^-1 r, then trials s + lam d for lam = 1, 1/2, ... until |r_trial| < |r| or
   // max_sub_step trials; the last trial is accepted (s <- trial, r and nr are its residual).
-  CPFEM_HD void newton_step(const SlipTable<N>& tab, int max_sub_step, double* s) {
+  template <class Tab>
+  CPFEM_HD void newton_step(const Tab& tab, int max_sub_step, double* s) {
     double dlt[6];
     {
       double J[36];
@@ -451,7 +516,8 @@ struct Point {
 
   // Iterations from the current evaluated point while |r| > tol, counted in *it, up to it_end;
   // sets PT_CAPPED if it_end is reached unconverged and PT_NONFINITE on a non-finite |r|.
-  CPFEM_HD void iterate(const SlipTable<N>& tab, double tol, int max_sub_step, int it_end, double* s, int* it,
+  template <class Tab>
+  CPFEM_HD void iterate(const Tab& tab, double tol, int max_sub_step, int it_end, double* s, int* it,
                         int32_t* stat) {
     while (nr > tol) {
       if (*it >= it_end) { *stat |= PT_CAPPED; break; }
@@ -463,7 +529,8 @@ struct Point {
 
   // Local Newton from S = 0 with cut-half backtracking (models_copper.py:204-249).
   // Returns the iteration count; status bits in *stat; s holds the converged stress.
-  CPFEM_HD int solve(const SlipTable<N>& tab, double tol, int max_sub_step, int max_iter, double* s, int32_t* stat) {
+  template <class Tab>
+  CPFEM_HD int solve(const Tab& tab, double tol, int max_sub_step, int max_iter, double* s, int32_t* stat) {
 #pragma unroll
     for (int q = 0; q < 6; ++q) s[q] = 0.0;
     eval(tab, s);
@@ -485,8 +552,8 @@ CPFEM_HD void fp_inv_new(const double* Fpi_old, const double* R, const double* L
 
 // First Piola-Kirchhoff stress P = F Fp_inv S Fp_inv^T / det Fp_inv at the converged point
 // (equal to det F (Fe S Fe^T / det Fe) F^-T of models_copper.py:160-161 since Fe = F Fp_inv).
-template <int N>
-CPFEM_HD void pk1(const Point<N>& pt, const double* F, const double* Fpi_old, const double* s, double* P) {
+template <int N, int L, int K>
+CPFEM_HD void pk1(const Point<N, L, K>& pt, const double* F, const double* Fpi_old, const double* s, double* P) {
   double Fpi[9], S[9], SFt[9], Y[9];
   fp_inv_new(Fpi_old, pt.R, pt.Lpc, Fpi);
   const double idFp = 1.0 / det3(Fpi);
@@ -504,8 +571,8 @@ CPFEM_HD void pk1(const Point<N>& pt, const double* F, const double* Fpi_old, co
 // Ycal is formed once from six unit stress directions; the nine dH = e_k e_l^T columns then
 // cost one 6x6 solve each.  All loops over directions are unrolled so every array index is a
 // compile-time constant (register resident).  Column m = 3k+l goes to sink(m, dP[9]).
-template <int N, class Sink>
-CPFEM_HD void tangent(Point<N>& pt, const SlipTable<N>& tab, const double* F, const double* Fpi_old, const double* s,
+template <int N, int K, class Tab, class Sink>
+CPFEM_HD void tangent(Point<N, 1, K>& pt, const Tab& tab, const double* F, const double* Fpi_old, const double* s,
                       Sink sink) {
   double Fpi[9];
   fp_inv_new(Fpi_old, pt.R, pt.Lpc, Fpi);
@@ -624,6 +691,36 @@ CPFEM_HD void hardening(const double* g_old, int64_t gstride, double* tmp, int t
       inc += (1.0 - m.r) * blk;
     }
     g_new[a * ostride] = g_old[a * gstride] + inc;
+  }
+}
+
+// Kalidindi hardening after convergence (the sums of hardening) and the new slips of this lane's systems, for
+// either form of a point; x: the converged stress in the crystal's frame, as its increment() takes it.
+template <int N, int L, class Pt, class Tab>
+CPFEM_HD void point_history(Pt& pt, const Tab& tab, const double* x, const PointMat& m, int self_block, const double* g_old,
+                            const double* slip_old, int64_t ld, double* g_new, double* slip_new) {
+  constexpr int M = N / L;
+  double tot = 0.0;
+#pragma unroll 2
+  for (int j = 0; j < M; ++j) {
+    const int64_t o = (pt.a0 + j) * ld;
+    const double dg = pt.increment(tab, j, x);
+    slip_new[o] = slip_old[o] + dg;
+    const double y = 1.0 - g_old[o] / m.tsat;
+    const double t = m.h * fabs(dg) * pow_pos(fabs(y), m.gss_a) * sgn(y);
+    pt.gp(j) = t;  // (used up)
+    tot += t;
+  }
+  tot = lane_sum<L>(tot);
+#pragma unroll 1
+  for (int k = 0; k < M; k += 3) {
+    double inc = m.r * tot;
+    if (self_block) inc += (1.0 - m.r) * (pt.gp(k) + pt.gp(k + 1) + pt.gp(k + 2));
+#pragma unroll
+    for (int j = k; j < k + 3; ++j) {
+      const int64_t o = (pt.a0 + j) * ld;
+      g_new[o] = g_old[o] + inc;
+    }
   }
 }
 

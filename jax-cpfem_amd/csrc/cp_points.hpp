@@ -124,14 +124,31 @@ struct OutOfLine {
   uint32_t n_it = 0, n_ev = 0;
 };
 
-// d dgamma / d tau and 1/g_old of the general form (cp_point.hpp), in the lane's private memory:
-// the functions that use them are called for the points that nothing else covers.
+// The general form (cp_point.hpp) runs in functions out of line, so that its registers do not weigh on the
+// points of the crystal-frame form; the lanes of a point and their LDS columns are the same.  What crosses
+// the call keeps its address space, or every access would be a flat one: the columns are an LDS pointer, the
+// slip table one to constant memory, the same in every lane (scalar loads where a lane does a whole point).
+// Batches whose every R is a rotation to 32 bits only, and so of this form, us per call (the crystal-frame
+// form's call; one lane of each point at work, gp and 1/g_old in private memory, flat accesses): stress map of 4,096
+// FCC points 101 (82; 251), residual 8^3 98 (61; 249), 16^3 BCC24 135 (86; 292), 40^3 BCC24 748 (378; 1076),
+// assembly 64^3 BCC24 8,680 (5,510; 11,990), stress and history 32^3 842 (510; 1143).
+typedef __attribute__((address_space(3))) double LdsDouble;
 template <int N>
-struct GeneralStore {
-  double gp[N], gi[N];
-  __device__ __forceinline__ void setup(Point<N>& pt, const PointIn& in, const StateView& sv, int64_t q) {
-    pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, gp, gi, 1, 1);
-  }
-};
+using ConstTable = const __attribute__((address_space(4))) SlipTable<N>;
+
+template <int N>
+__device__ __forceinline__ ConstTable<N>& uniform_table(const SlipTable<N>* table) {
+  const uint64_t t = (uint64_t)table;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)t), hi = __builtin_amdgcn_readfirstlane((uint32_t)(t >> 32));
+  return *(ConstTable<N>*)((uint64_t)hi << 32 | lo);
+}
+// (rest: no member of the point, whose registers it would drag into memory)
+template <int BS, int N, int L, int KS>
+__device__ __forceinline__ void setup_general(Point<N, L, KS>& pt, const PointIn& in, const StateView& sv, int64_t q, int sub,
+                                              LdsDouble* sh, CrystalRest<N, L, KS>& rest) {
+  if (rest.n > 0) asm volatile("" ::"v"(rest.gi) : "memory");
+  pt.setup(in.F, in.Fpi, in.R, sv.g + q, sv.ld, in.m, (double*)sh + threadIdx.x, (double*)sh + Point<N, L, KS>::M * BS + threadIdx.x,
+           BS, BS, sub, rest.n > 0 ? rest.gi : nullptr);
+}
 
 }  // namespace cpfem

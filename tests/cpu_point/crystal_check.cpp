@@ -44,7 +44,7 @@ static int64_t run(int crystal, int64_t Q, const double* H, const double* Fpi, c
       if (done) {
         iters[q] = nw.it;
         crystal_pk1(pt, F, Fo, Rq, nw.s, P + 9 * q);
-        crystal_history(pt, sys, nw.s, m, self_block, go, slip + N * q, 1, gn + N * q, sn + N * q);
+        point_history<N, 1>(pt, sys, nw.s, m, self_block, go, slip + N * q, 1, gn + N * q, sn + N * q);
         pt.stress(nw.s, Rq, s);
       } else {
         --used;
