@@ -183,10 +183,12 @@ int cpfem_solve_noalloc(cpfem_ctx* ctx, void* stream, const double* mat, const d
 
 /* Direct solve of A x = b (replaces umfpack_solve, crystal_plasticity_OR_design/solver.py:50-60,
    selected by solver_options 'umfpack_solver' at :100-101): LU of the band form of A under a
-   bandwidth-reducing node order (unpivoted; a zero pivot returns CPFEM_EDIRECT), then `refine`
-   (0..10) steps of FP64 iterative refinement.  x need not hold a guess.  The band storage,
-   n_dofs x (4 * (3 * node bandwidth + 2) + 1) doubles under 64 GiB, is allocated on first use
-   and kept with the context.  info->residual = |A x - b|, info->iterations = refine. */
+   bandwidth-reducing node order (unpivoted, from both ends of the band, and again from its
+   beginning alone where a pivot vanishes or the solution's backward error exceeds 1e-13; a zero
+   pivot then returns CPFEM_EDIRECT), then `refine` (0..10) steps of FP64 iterative refinement.
+   x need not hold a guess.  The band's entries, n_dofs x (6 * node bandwidth + 5) doubles, have
+   to stay under 64 GiB; they are kept in 64 x 64 tiles with the context, allocated on first use.
+   info->residual = |A x - b|, info->iterations = refine. */
 int cpfem_solve_direct(cpfem_ctx* ctx, void* stream, const double* mat, const double* b, double* x, int32_t refine,
                        CpfemSolveInfo* info);
 

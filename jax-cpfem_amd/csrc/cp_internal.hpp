@@ -336,6 +336,9 @@ void launch_residual_norm(int64_t n, const double* a, const double* b, double* p
 void launch_axpby(int64_t n, double alpha, const double* x, double beta, double* y, hipStream_t st);
 void launch_cast_f32(int64_t n, const double* x, float* y, hipStream_t st);
 void launch_residual64(const BellView& M, const double* vals, const double* x, const double* b, double* r, hipStream_t st);
+// r = b - A x, and the largest |r| / (|A| |x| + |b|) over the rows (NaN if any is) to *omega (device).
+void launch_backward_error(const BellView& M, const double* vals, const double* x, const double* b, double* r, double* omega,
+                           hipStream_t st);
 void launch_copy(int64_t n, const double* x, double* y, hipStream_t st);
 // y[i] = v for i < n
 void launch_fill(int64_t n, double v, double* y, hipStream_t st);

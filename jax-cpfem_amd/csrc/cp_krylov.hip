@@ -102,6 +102,30 @@ __global__ void __launch_bounds__(KBS) k_residual64(BellView M, const double* __
   r[i] = b[i] - spmv_row<double>(M, vals, x, i);
 }
 
+// The same, and the componentwise backward error |r| / (|A| |x| + |b|) of each row; their maximum, through
+// its bits (the order of positive doubles, NaN above all), to *omega.
+__global__ void __launch_bounds__(KBS) k_backward_error(BellView M, const double* __restrict__ vals, const double* __restrict__ x,
+                                                       const double* __restrict__ b, double* __restrict__ r,
+                                                       unsigned long long* __restrict__ omega) {
+  const int64_t i = (int64_t)blockIdx.x * KBS + threadIdx.x, nrow = 3 * M.n_nodes;
+  double w = 0.0;
+  if (i < nrow) {
+    const int64_t node = i / 3;
+    const double v = b[i] - spmv_row<double>(M, vals, x, i);
+    r[i] = v;
+    double scale = fabs(b[i]);
+    for (int s = 0; s < M.nslot[node]; ++s) {
+      const int64_t j = 3 * (int64_t)M.col[(int64_t)s * M.n_nodes + node];
+      for (int c = 0; c < 3; ++c) scale += fabs(vals[(3 * (int64_t)s + c) * nrow + i] * x[j + c]);
+    }
+    w = v == 0.0 ? 0.0 : fabs(v / scale);
+  }
+  unsigned long long m = (unsigned long long)__double_as_longlong(w);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, (unsigned long long)__shfl_xor((long long)m, o, 64));
+  if ((threadIdx.x & 63) == 0 && m) atomicMax(omega, m);
+}
+
 __global__ void __launch_bounds__(KBS) k_inv_diag(BellView M, const double* __restrict__ vals, const int32_t* __restrict__ dslot,
                                                  double* __restrict__ invd, int precond) {
   const int64_t r = (int64_t)blockIdx.x * KBS + threadIdx.x;
@@ -1213,6 +1237,12 @@ void launch_cast_f32(int64_t n, const double* x, float* y, hipStream_t st) {
 }
 void launch_residual64(const BellView& M, const double* vals, const double* x, const double* b, double* r, hipStream_t st) {
   hipLaunchKernelGGL(k_residual64, dim3(nblk(3 * M.n_nodes)), dim3(KBS), 0, st, M, vals, x, b, r);
+}
+void launch_backward_error(const BellView& M, const double* vals, const double* x, const double* b, double* r, double* omega,
+                           hipStream_t st) {
+  launch_zero_words(reinterpret_cast<uint32_t*>(omega), 2, st);
+  hipLaunchKernelGGL(k_backward_error, dim3(nblk(3 * M.n_nodes)), dim3(KBS), 0, st, M, vals, x, b, r,
+                     reinterpret_cast<unsigned long long*>(omega));
 }
 
 template void krylov_init<double>(const BellView&, const double*, const double*, KVec, KrylovWork, hipStream_t);
