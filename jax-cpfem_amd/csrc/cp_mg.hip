@@ -504,8 +504,9 @@ __global__ void __launch_bounds__(256) k_mg_prolong(MgGrid f, MgGrid g, const do
 // all at 64^3), where the direct triple product reads every fine row 27 times.  A thread
 // makes the three values of one coarse row, transverse offset pair and component from nine fine
 // values.  DIR: direction coarsened; FINE: reads the block-ELL matrix with the masks of Dirichlet
-// rows and columns; LAST: applies the coarse masks, puts 1 on masked diagonals, writes the
-// inverse diagonal and rounds to the level's value type.
+// rows and columns; LAST: applies the coarse masks, writes the inverse diagonal and rounds to the level's
+// value type.  Masked rows and columns are zero, their diagonals too: a number put there would be carried into
+// the free dofs of the levels below, in units that are not the matrix's (k_dense_fill puts 1 there).
 // Slot of offset (dx, dy, dz) in node p's row (existing neighbours in ascending order).
 __device__ __forceinline__ int mg_slot(const MgGrid& f, const NodeXYZ& p, int dx, int dy, int dz) {
   const int xl = p.x > 0 ? -1 : 0, yl = p.y > 0 ? -1 : 0, zl = p.z > 0 ? -1 : 0;
@@ -578,8 +579,8 @@ __global__ void __launch_bounds__(256) k_mg_coarsen(MgGrid f, MgGrid g, const TI
       const bool diag = dx == 0 && dy == 0 && dz == 0 && k == c;
       const bool fr = cfixed[t] != 0;
       const bool fc = in && cfixed[3 * (int64_t)(I + dx + g.nx * (dy + g.ny * dz)) + k] != 0;
-      if (fr || fc) v = diag ? 1.0 : 0.0;
       if (diag) minv[t] = fr ? 0.0 : 1.0 / v;
+      if (fr || fc) v = 0.0;
     }
     out[(3 * s + k) * gn + t] = (TO)v;
   }
@@ -596,11 +597,12 @@ __global__ void __launch_bounds__(256) k_mg_coarsen(MgGrid f, MgGrid g, const TI
 // this level and the ones below it, 375 rows in one block of one CU 21 us, 648 rows in launches 45;
 // forming it takes 6 x 17 or 11 x 18 us, where the inverse of 81 rows took 67.
 template <typename TM>
-__global__ void __launch_bounds__(256) k_dense_fill(MgGrid g, int nt, const TM* __restrict__ A, double* __restrict__ out) {
+__global__ void __launch_bounds__(256) k_dense_fill(MgGrid g, int nt, const TM* __restrict__ A, const double* __restrict__ minv,
+                                                    double* __restrict__ out) {
   const int c = (int)(blockIdx.x * 256 + threadIdx.x), r = (int)blockIdx.y, ld = nt * NB;
   if (c >= ld) return;
   double v = r == c ? 1.0 : 0.0;
-  if (r < g.n && c < g.n) {
+  if (r < g.n && c < g.n && (r != c || minv[r] != 0.0)) {
     const NodeXYZ p = mg_node(g, (int)((uint32_t)r / 3u)), q = mg_node(g, (int)((uint32_t)c / 3u));
     const int dx = q.x - p.x, dy = q.y - p.y, dz = q.z - p.z;
     v = 0.0;
@@ -767,7 +769,7 @@ void mg_setup_rest(const Multigrid& mg, hipStream_t st) {
   const MgLevel& E = mg.lv[mg.nl - 1];
   const int nt = mg_dense_tiles(E.g.n);
   hipLaunchKernelGGL(k_dense_fill<TM>, dim3((unsigned)((nt * NB + 255) / 256), (unsigned)(nt * NB)), dim3(256), 0, st, E.g, nt,
-                     static_cast<const TM*>(E.A), mg.dense[0]);
+                     static_cast<const TM*>(E.A), (const double*)E.minv, mg.dense[0]);
   hipLaunchKernelGGL(k_dense_first, dim3(1), dim3(256), 0, st, mg.dense[0], mg.dpiv);
   for (int k = 0; k < nt; ++k)
     hipLaunchKernelGGL(k_dense_step, dim3((unsigned)nt, (unsigned)nt), dim3(256), 0, st, nt, k, mg.dense[k & 1],
