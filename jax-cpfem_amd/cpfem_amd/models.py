@@ -301,6 +301,9 @@ class CrystalPlasticity(Problem):
         return self.unflatten_fn_sol_list(res)
 
 
+OWN_ASSEMBLE = CrystalPlasticity.assemble  # residual_state and matrix_at are its parts
+
+
 def local_full(problem, u_grad, params):
     """Every output of the point kernel for a batch (P, dP/du_grad, new history, iterations)
     from explicit u_grad (Q, 3, 3) and per-point params (each (Q, ...)); for tests and

@@ -153,10 +153,11 @@ def line_search(problem, dofs, inc):
 
 def _splits_assembly(problem):
     """Whether problem's residual and matrix may be formed apart: it assembles as the framework's
-    own class does, by no method of a subclass or of the instance."""
-    from .models import CrystalPlasticity
+    own class does, by no method of a subclass, of the instance or put in the class's place, and
+    the Newton step and its line search are this module's own."""
+    from .models import OWN_ASSEMBLE, CrystalPlasticity
     return (isinstance(problem, CrystalPlasticity) and "assemble" not in vars(problem)
-            and type(problem).assemble is CrystalPlasticity.assemble)
+            and type(problem).assemble is OWN_ASSEMBLE and (line_search, linear_incremental_solver) == _OWN_STEP)
 
 
 def _line_search_state(problem, dofs, inc, status):
@@ -197,6 +198,9 @@ def linear_incremental_solver(problem, res, mat, dofs, solver_options):
     if solver_options.get("line_search_flag", False):
         return line_search(problem, dofs, inc)
     return dofs + inc
+
+
+_OWN_STEP = (line_search, linear_incremental_solver)  # what _line_search_state stands for
 
 
 def solver(problem, solver_options={}):
