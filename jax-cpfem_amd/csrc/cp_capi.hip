@@ -1293,10 +1293,10 @@ int cpfem_solve_mg(cpfem_ctx* c, void* stream, const double* mat, const double* 
   if (!c || !mat || !b || !x) return fail(CPFEM_EBADARG, "null argument");
   if (precision != CPFEM_FP64 && precision != CPFEM_MIXED) return fail(CPFEM_EBADARG, "unknown precision");
   if (maxiter < 0) return fail(CPFEM_EBADARG, "maxiter must be >= 0");
+  int rc;  // (what either solve needs is allocated before what one can do without)
+  if ((rc = ensure_krylov(c, precision == CPFEM_MIXED))) return rc;
   if (c->mg_use && ensure_mg(c)) {
-    int rc;
     hipStream_t st = (hipStream_t)stream;
-    if ((rc = ensure_krylov(c, precision == CPFEM_MIXED))) return rc;
     launch_copy(c->n_dofs, x, c->kv64[9], st);  // x0, for the solve that takes over
     CpfemSolveInfo inf{};
     bool converged = false;
