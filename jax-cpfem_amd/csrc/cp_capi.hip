@@ -96,8 +96,17 @@ template <typename T>
 static int dalloc(T** p, size_t n) {
   *p = nullptr;
   if (n == 0) n = 1;
-  HIPCHK(hipMalloc((void**)p, n * sizeof(T)));
-  return CPFEM_OK;
+  const hipError_t e = hipMalloc((void**)p, n * sizeof(T));
+  if (e == hipSuccess) return CPFEM_OK;
+  (void)hipGetLastError();  // reported here, not by the next call's check of its launches
+  return fail(CPFEM_EHIP, std::string("hipMalloc((void**)p, n * sizeof(T)): ") + hipGetErrorString(e));
+}
+
+// The same for a buffer of the context that is allocated on first use: one that is there stays, so that a call
+// after one that ran out of memory half way allocates the others.
+template <typename T>
+static int need(T** p, size_t n) {
+  return *p ? CPFEM_OK : dalloc(p, n);
 }
 
 template <typename T>
@@ -462,17 +471,17 @@ static SolveCfg solve_cfg(const CpfemParams* p) {
 
 static int ensure_matrix_buffers(cpfem_ctx* c) {
   int rc;
-  if (!c->d_wA && (rc = dalloc(&c->d_wA, (size_t)81 * c->n_qp))) return rc;
-  if (!c->d_sconv && (rc = dalloc(&c->d_sconv, (size_t)6 * c->n_qp))) return rc;
-  if (!c->d_KE && (rc = dalloc(&c->d_KE, (size_t)576 * c->n_cells))) return rc;
+  if ((rc = need(&c->d_wA, (size_t)81 * c->n_qp)) || (rc = need(&c->d_sconv, (size_t)6 * c->n_qp)) ||
+      (rc = need(&c->d_KE, (size_t)576 * c->n_cells)))
+    return rc;
   return CPFEM_OK;
 }
 
 static int ensure_park(cpfem_ctx* c) {
   int rc;
   if (c->d_park_ctr) return CPFEM_OK;
-  if ((rc = dalloc(&c->d_park_idx, (size_t)c->n_qp)) || (rc = dalloc(&c->d_park_it, (size_t)c->n_qp)) ||
-      (rc = dalloc(&c->d_park_s, (size_t)6 * c->n_qp)) || (rc = dalloc(&c->d_park_ctr, 2)))
+  if ((rc = need(&c->d_park_idx, (size_t)c->n_qp)) || (rc = need(&c->d_park_it, (size_t)c->n_qp)) ||
+      (rc = need(&c->d_park_s, (size_t)6 * c->n_qp)) || (rc = need(&c->d_park_ctr, 2)))
     return rc;
   return CPFEM_OK;
 }
@@ -480,14 +489,14 @@ static int ensure_park(cpfem_ctx* c) {
 static int ensure_krylov(cpfem_ctx* c, bool mixed) {
   int rc;
   const int64_t n = c->n_dofs;
-  if (!c->d_ksc) {
-    if ((rc = dalloc(&c->d_ksc, 1)) || (rc = dalloc(&c->d_kpartial, (size_t)8 * krylov_stride_max(n)))) return rc;
+  if (!c->d_ksc) {  // the last of them
+    if ((rc = need(&c->d_kpartial, (size_t)8 * krylov_stride_max(n)))) return rc;
     for (int i = 0; i < 12; ++i)
-      if ((rc = dalloc(&c->kv64[i], i >= 10 ? 2 * n : n))) return rc;
-    if ((rc = dalloc(&c->d_r64, n)) || (rc = dalloc(&c->d_tmp64, n))) return rc;
+      if ((rc = need(&c->kv64[i], i >= 10 ? 2 * n : n))) return rc;
+    if ((rc = need(&c->d_r64, n)) || (rc = need(&c->d_tmp64, n)) || (rc = need(&c->d_ksc, 1))) return rc;
     HIPCHK(hipMemset(c->d_ksc, 0, sizeof(KrylovScalars)));
   }
-  if (mixed && !c->d_mat32 && (rc = dalloc(&c->d_mat32, c->mat_len()))) return rc;
+  if (mixed && (rc = need(&c->d_mat32, c->mat_len()))) return rc;
   return CPFEM_OK;
 }
 
@@ -1141,10 +1150,12 @@ static int ensure_band(cpfem_ctx* c) {
                                    " MiB exceeds the limit; use the Krylov solver ('jax_solver')");
   band_shape(B, c->n_dofs, bw, BAND_MAX_BYTES);
   int rc;
-  if ((rc = dalloc(&c->d_ip, (size_t)c->n_nodes)) || (rc = dalloc(&c->d_bflag, 1)) ||
-      (rc = dalloc(&B.y, (size_t)BAND_NB * B.nbk)) || (rc = dalloc(&B.band, (size_t)B.room)))
+  if ((rc = need(&c->d_ip, (size_t)c->n_nodes)) || (rc = need(&c->d_bflag, 1)) ||
+      (rc = need(&c->band.y, (size_t)BAND_NB * B.nbk)))
     return rc;
   HIPCHK(hipMemcpy(c->d_ip, ip.data(), ip.size() * 4, hipMemcpyHostToDevice));
+  if ((rc = dalloc(&B.band, (size_t)B.room))) return rc;
+  B.y = c->band.y;
   B.ip = c->d_ip;
   B.flag = c->d_bflag;
   c->band = B;

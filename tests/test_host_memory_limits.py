@@ -1,6 +1,6 @@
 """What the Krylov solves allocate when device memory is short, with a HIP runtime that only keeps books
 (tests/fake_hip): buffers a solve cannot do without come before the optional ones of the multigrid
-preconditioner."""
+preconditioner, and a call that failed leaves nothing half done behind."""
 import os
 import subprocess
 import sys
@@ -79,6 +79,47 @@ for precision in (0, 1):
 print("done")
 '''
 
+RETRY = CHILD + r'''
+krylov, _ = sizes(0)
+for part in (0.02, 0.3, 0.7, 0.95):
+    ctx = create()
+    base = fake.fake_used()
+    fake.fake_limit(base + int(part * krylov))
+    assert solve(ctx, False) == N.EHIP, L.cpfem_last_error()
+    fake.fake_limit(2 ** 62)
+    assert solve(ctx, False) == 0
+    assert fake.fake_used() == base + krylov, (part, fake.fake_used() - base, krylov)
+    count = fake.fake_mallocs()
+    assert solve(ctx, False) == 0 and fake.fake_mallocs() == count
+    L.cpfem_destroy(ctx)
+    assert fake.fake_used() == 0
+print("done")
+'''
+
+
+DIRECT = CHILD + r'''
+def direct(ctx):
+    info = N.CpfemSolveInfo()
+    return L.cpfem_solve_direct(ctx, None, mat.ctypes.data, v.ctypes.data, v.ctypes.data, 0, ctypes.byref(info))
+
+ctx = create()
+base = fake.fake_used()
+assert direct(ctx) == 0, L.cpfem_last_error()
+whole = fake.fake_used() - base
+L.cpfem_destroy(ctx)
+for part in (0.01, 0.5, 0.9, 0.999):
+    ctx = create()
+    fake.fake_limit(base + int(part * whole))
+    assert direct(ctx) == N.EHIP
+    fake.fake_limit(2 ** 62)
+    assert direct(ctx) == 0, L.cpfem_last_error()
+    assert fake.fake_used() == base + whole, (part, fake.fake_used() - base, whole)
+    L.cpfem_destroy(ctx)
+    assert fake.fake_used() == 0
+print("done")
+'''
+
+
 @pytest.fixture(scope="module")
 def fake(tmp_path_factory):
     if not os.path.exists(LIB):
@@ -97,3 +138,9 @@ def _run(script, fake):
 def test_krylov_vectors_come_before_multigrid_buffers(fake):
     _run(ORDER, fake)
 
+def test_a_failed_allocation_is_made_up_for_by_the_next_call(fake):
+    _run(RETRY, fake)
+
+
+def test_a_failed_direct_solve_is_made_up_for_by_the_next_call(fake):
+    _run(DIRECT, fake)
