@@ -693,8 +693,6 @@ static int solve_impl(cpfem_ctx* c, hipStream_t st, const KBufs& kb, const doubl
 // ------------------------------------------------------------------------- multigrid solve
 // Systems of at least MG_MIN_ROWS rows on full box patterns take the multigrid preconditioner.
 constexpr int64_t MG_MIN_ROWS = 1500;
-// Iterations it gets before the Jacobi-preconditioned solve takes over (it needs about 10).
-constexpr int MG_MAXITER = 60;
 
 static void mg_free(cpfem_ctx* c) {
   for (void* p : c->mg_mem) (void)hipFree(p);

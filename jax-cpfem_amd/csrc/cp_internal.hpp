@@ -237,6 +237,8 @@ struct MgGrid {
   double inv_a, inv_b;  // 1 / (nx ny), 1 / nx
 };
 constexpr int MG_MAXL = 12;
+// Iterations a multigrid solve gets before the Jacobi-preconditioned one takes over (it needs about 10).
+constexpr int MG_MAXITER = 60;
 // One level: operator (level 0: the caller's block-ELL matrix; coarser levels: 27 offsets in
 // lexicographic order, value (o, k) of row r at (3 o + k) n + r, zero outside the box), the
 // inverse diagonal (0 on Dirichlet dofs), right-hand side, two iterates and the residual.

@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(KBS) k_kinit(BellView M, const TM* __restrict_
 __global__ void __launch_bounds__(KBS) k_kinit2(KrylovWork w) {
   __shared__ double sh[2 * (KBS / 64)];
   double sums[2];
-  get_sums<KBS, 2>(w.partial, {PS_BB, PS_RR}, w.ps, sh, sums);
+  get_sums<KBS, 2>(w.partial, {PS_BB, PS_RR}, w.ps, w.ps, sh, sums);
   const double bb = sums[0];
   if (threadIdx.x == 0) {
     KrylovScalars* sc = w.sc;
@@ -946,7 +946,7 @@ __global__ void __launch_bounds__(KBS) k_kxr1(KVec v, KrylovWork w, int par) {
   }
   if (done) return;
   double sums[5];
-  get_sums<KBS, 5>(w.partial, {PS_SS, PS_TS, PS_TT, PS_RS, PS_RT}, w.ps, sh, sums);
+  get_sums<KBS, 5>(w.partial, {PS_SS, PS_TS, PS_TT, PS_RS, PS_RT}, w.ps, w.ps, sh, sums);
   const double ss = sums[0];
   const double omega = sums[1] / sums[2];
   const double beta = (sums[3] - omega * sums[4]) / rho * alpha / omega;  // of the next iteration
@@ -997,7 +997,7 @@ __global__ void __launch_bounds__(KBS) k_kxr(KVec v, KrylovWork w, int par) {
   }
   if (done) return;
   double sums[3];
-  get_sums<KBS, 3>(w.partial, {PS_SS, PS_TS, PS_TT}, w.ps, sh, sums);
+  get_sums<KBS, 3>(w.partial, {PS_SS, PS_TS, PS_TT}, w.ps, w.ps, sh, sums);
   const double ss = sums[0];
   const double omega = sums[1] / sums[2];
   const bool early = ss < atol2;

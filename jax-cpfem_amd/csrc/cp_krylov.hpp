@@ -68,17 +68,18 @@ __device__ __forceinline__ void put_partials(const double (&v)[NSL], const int (
   }
 }
 
-// Sums of NSL partial slots, computed by the whole block (all slots' loads in one pass);
-// returned in every thread, identical in every block.
+// Sums of the first `count` entries of NSL partial slots (stride ps), computed by the whole block (all
+// slots' loads in one pass); returned in every thread, identical in every block.
 template <int BS, int NSL>
-__device__ __forceinline__ void get_sums(const double* partial, const int (&slot)[NSL], int ps, double* sh, double (&out)[NSL]) {
+__device__ __forceinline__ void get_sums(const double* __restrict__ partial, const int (&slot)[NSL], int count, int ps, double* sh,
+                                         double (&out)[NSL]) {
   double s[NSL];
 #pragma unroll
   for (int j = 0; j < NSL; ++j) s[j] = 0.0;
   // unrolled so that several iterations' loads are in flight together (the flat SpMV form
   // leaves thousands of partials per sum); the additions keep their order
 #pragma unroll 4
-  for (int i = threadIdx.x; i < ps; i += BS) {
+  for (int i = threadIdx.x; i < count; i += BS) {
 #pragma unroll
     for (int j = 0; j < NSL; ++j) s[j] += partial[slot[j] * ps + i];
   }

@@ -52,7 +52,6 @@ constexpr int POWER_STEPS = 12;
 // with this, Jacobi alone 15.3.  What converges is left alone: 24 shapes of 1:1:1 elements, and 1:1:3
 // (32 iterations), 1:1:0.1 (37) take the iterations they took.
 constexpr int STALL_FROM = 7;
-constexpr int STALL_LIMIT = 60;       // MG_MAXITER; not the caller's own limit, which may be lower
 constexpr float STALL_SLACK = 6.65f;  // log2(100)
 constexpr int FLAT_ROWS = 60000;   // one thread per row from here on; below, three waves per 64 rows
 constexpr int PLAIN_ROWS = 700000; // row blocks in launch order from here on; below, XCD-local ranges
@@ -854,35 +853,6 @@ static void vcycle(const Multigrid& mg, const BellView& M, double* iterate, cons
 // cycles; sums as there: one partial per block, added by every block of the consuming kernel in
 // index order.
 
-// Sums of NSL slots over `count` partials with stride ps, returned in every thread (256 threads).
-template <int NSL>
-__device__ __forceinline__ void mg_sums(const double* __restrict__ partial, const int (&slot)[NSL], int count, int ps, double* sh,
-                                        double (&out)[NSL]) {
-  double s[NSL];
-#pragma unroll
-  for (int j = 0; j < NSL; ++j) s[j] = 0.0;
-#pragma unroll 4
-  for (int i = threadIdx.x; i < count; i += KBS) {
-#pragma unroll
-    for (int j = 0; j < NSL; ++j) s[j] += partial[slot[j] * ps + i];
-  }
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int j = 0; j < NSL; ++j) {
-    const double t = wave_sum(s[j]);
-    if (lane == 0) sh[j * (KBS / 64) + wid] = t;
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < NSL; ++j) {
-    double t = 0.0;
-#pragma unroll
-    for (int i = 0; i < KBS / 64; ++i) t += sh[j * (KBS / 64) + i];
-    out[j] = t;
-  }
-  __syncthreads();
-}
-
 // r0 = b - A x0 = rhat = p = q, and the partials of <r,r> (= <rhat,r>) and <b,b>.
 template <int P>
 __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_init(BellView M, MgGrid g, const double* __restrict__ A,
@@ -905,7 +875,7 @@ __global__ void __launch_bounds__(MgShape<P>::BS) k_mgb_init(BellView M, MgGrid 
 __global__ void __launch_bounds__(KBS) k_mgb_init2(KrylovWork w, double tol, double atol, int maxiter) {
   __shared__ double sh[KBS / 64];
   double s[1];
-  mg_sums<1>(w.partial, {PS_BB}, w.ps, w.ps, sh, s);
+  get_sums<KBS, 1>(w.partial, {PS_BB}, w.ps, w.ps, sh, s);
   if (threadIdx.x == 0) {
     KrylovScalars* sc = w.sc;
     sc->bs = s[0];
@@ -930,15 +900,16 @@ __global__ void __launch_bounds__(KBS) k_mgb_p(MgVec v, KrylovWork w, int par, i
   const int kprev = sc->k2[pv], maxiter = sc->maxiter;
   const int64_t i0 = (int64_t)blockIdx.x * KBS + threadIdx.x;
   double sums[2];
-  mg_sums<2>(w.partial, {PS_RR, PS_RHR}, iter == 0 ? w.ps : w.nb, w.ps, sh, sums);
+  get_sums<KBS, 2>(w.partial, {PS_RR, PS_RHR}, iter == 0 ? w.ps : w.nb, w.ps, sh, sums);
   const double rs = sums[0], rho_ = sums[1];
   int k = (omega == 0.0 || alpha == 0.0) ? -11 : kprev + 1;
   if (rho == 0.0) k = -10;
-  // A solve that is not on its way to the threshold within STALL_LIMIT iterations is left to the Jacobi
-  // solve: from STALL_FROM on, the squared residual has to be under a straight line (in its logarithm)
-  // from a hundredfold of the first one. See STALL_FROM for what it costs without this.
+  // A solve that is not on its way to the threshold within MG_MAXITER iterations (not the caller's own
+  // limit, which may be lower) is left to the Jacobi solve: from STALL_FROM on, the squared residual has to
+  // be under a straight line (in its logarithm) from a hundredfold of the first one.  See STALL_FROM for
+  // what it costs without this.
   if (k >= STALL_FROM && rs > atol2) {
-    const float line = log2f(fmaxf((float)(atol2 / sc->rs0), 1e-30f)) * ((float)k / (float)STALL_LIMIT);
+    const float line = log2f(fmaxf((float)(atol2 / sc->rs0), 1e-30f)) * ((float)k / (float)MG_MAXITER);
     if (log2f((float)(rs / sc->rs0)) > STALL_SLACK + line) k = -12;
   }
   const bool go = (rs > atol2) && (k < maxiter) && (k >= 0);
@@ -982,7 +953,7 @@ __global__ void __launch_bounds__(KBS) k_mgb_s(MgVec v, KrylovWork w, int par, i
   __shared__ double sh[KBS / 64];
   KrylovScalars* sc = w.sc;
   double sums[1];
-  mg_sums<1>(w.partial, {PS_RQ}, nbs, w.ps, sh, sums);
+  get_sums<KBS, 1>(w.partial, {PS_RQ}, nbs, w.ps, sh, sums);
   const double alpha = sc->rho2[par] / sums[0], il = ith * lam[0];
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->alpha2[par] = alpha;
   for (int64_t i = (int64_t)blockIdx.x * KBS + threadIdx.x; i < w.n; i += (int64_t)w.nb * KBS) {
@@ -1016,7 +987,7 @@ __global__ void __launch_bounds__(KBS) k_mgb_xr(MgVec v, KrylovWork w, int par, 
   KrylovScalars* sc = w.sc;
   const double alpha = sc->alpha2[par], atol2 = sc->atol2;
   double sums[3];
-  mg_sums<3>(w.partial, {PS_SS, PS_TS, PS_TT}, nbs, w.ps, sh, sums);
+  get_sums<KBS, 3>(w.partial, {PS_SS, PS_TS, PS_TT}, nbs, w.ps, sh, sums);
   const double omega = sums[1] / sums[2];
   const bool early = sums[0] < atol2;
   if (blockIdx.x == 0 && threadIdx.x == 0) sc->omega2[par] = omega;
