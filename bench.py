@@ -83,9 +83,27 @@ def mg_bytes(prob, value_bytes=8, vectors=3.0):
     return round(9 * value_bytes * nnzb + 4 * (nnzb - 27 * (nx - 2) * (ny - 2) * (nz - 2)) + vectors * 8 * prob.ctx.n_dofs)
 
 
+# FP64 operations of the crystal-frame point form (cp_crystal.hpp) per unit of work, as (per slip system, fixed): FMA
+# = 2, each other + - * / sqrt = 1, a rate's power with its series; counted by tests/cpu_point/op_count.cpp.
+POINT_OPS = dict(residual=(94, 137), elastic_residual=(0, 80), jacobian=(85, 529), setup=(3, 136), outputs=(0, 381),
+                 tangent=(179, 3564))
+TRIAL_OPS, GRADIENT_OPS = 12, 144  # a trial stress; the displacement gradient of eight nodes
+
+
+def point_ops(n_slip, points, tangent_points, newton_iters, residual_evals):
+    """FP64 operations that the assembly's point kernels (k_element_res, the parked points' k_element_qp_park and
+    k_point_tangent) execute, from measured totals over `points` point updates: the first residual of each is the
+    elastic one, at S' = 0 without slip, and the first step takes no Jacobian.  (Points of the general form,
+    which the workloads here do not have, would count as points of this one.)"""
+    ops = {k: a * n_slip + b for k, (a, b) in POINT_OPS.items()}
+    return (points * (GRADIENT_OPS + ops["setup"] + ops["elastic_residual"] + ops["outputs"])
+            + max(residual_evals - points, 0) * (ops["residual"] + TRIAL_OPS) + max(newton_iters - points, 0) * ops["jacobian"]
+            + tangent_points * (GRADIENT_OPS + ops["setup"] + ops["tangent"]))
+
+
 def point_flops(n_slip, tangent_points, newton_iters, residual_evals):
-    """Algorithmic FP64 flops of the assembly's point kernels (k_element_res, the parked points'
-    k_element_qp_park and k_point_tangent) from measured totals: the reference algorithm's per-unit counts
+    """FP64 flops that the reference's algorithm would take for the work of the assembly's point kernels, from
+    measured totals (an equivalent work rate, not what the kernels execute: point_ops): its per-unit counts
     (FMA = 2 flops; div, abs, sign, pow, sqrt = 1 each), F_res(N) = 41 N + 350 per residual
     evaluation, F_jac(N) = 165 N + 2574 per local Jacobian and F_LU = 648 per 9x9 LU and solve
     (once per iteration), F_tan = 9300 per consistent tangent (assemblies with the Jacobian
@@ -521,7 +539,8 @@ def main():
     qp = kp["element_qp"]
     if qp["avg_ms"] and qp["launches"]:
         tangent_launches = kp["point_tangent"]["launches"]
-        flops = point_flops(prob.num_slip_sys, Q * tangent_launches, work["newton_iters"], work["residual_evals"])
+        flops = point_ops(prob.num_slip_sys, Q * qp["launches"], Q * tangent_launches, work["newton_iters"], work["residual_evals"])
+        ref_flops = point_flops(prob.num_slip_sys, Q * tangent_launches, work["newton_iters"], work["residual_evals"])
         t_ms = point_ms()
         ach_tf = flops / (t_ms * 1e-3) / 1e12
         point_roof = dict(bound="fp64 valu", achieved=round(ach_tf, 3), peak=FP64_PEAK_TFLOPS, unit="TFLOP/s",
@@ -534,8 +553,10 @@ def main():
                           flops_per_point_launch=round(flops / (Q * qp["launches"]), 1),
                           newton_iters_per_point_launch=round(work["newton_iters"] / (Q * qp["launches"]), 3),
                           residual_evals_per_point_launch=round(work["residual_evals"] / (Q * qp["launches"]), 3),
-                          flop_model="F_res(N)=41N+350 per residual evaluation, F_jac(N)=165N+2574 + F_LU=648 per "
-                                     "iteration, F_tan=9300 per tangent (reference algorithm counts)")
+                          flop_model="operations executed by the crystal-frame form (bench.point_ops)",
+                          reference_equivalent_tflops=round(ref_flops / (t_ms * 1e-3) / 1e12, 3),
+                          reference_flop_model="F_res(N)=41N+350 per residual evaluation, F_jac(N)=165N+2574 + F_LU=648 per "
+                                               "iteration, F_tan=9300 per tangent")
     roof = spmv_roof if dom == "krylov_spmv" else mg_roof if dom == "mg_fine" else (point_roof if dom == "element_qp" else
                                                     dict(bound=None, achieved=None, peak=None, unit=None, frac=None,
                                                          traffic=None, kernel=dom))
