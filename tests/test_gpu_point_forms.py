@@ -179,6 +179,33 @@ def test_point_vjp_at_every_lane_count(N, n):
         assert err < 5e-8
 
 
+@pytest.mark.parametrize("N", [12, 24])
+def test_tangents_of_a_batch(N):
+    """Point updates with their tangents, of either form, among them unstrained points (converged before the first
+    iteration) and one whose resistance is not a number, which does not reach its neighbours."""
+    from cpfem_amd.models import local_full
+    from oracle import cp_local
+    H, Fp, g, slip, R, xm = (a.copy() for a in _states(N, False))
+    H[64:96] = 0.0
+    Fp[64:96] = np.eye(3)
+    xm[64:96] = 0.02  # (at m = 1 the rate has a slope at zero stress; |x| is given none by the oracle)
+    ref = cp_local.local_update(H, Fp, g, slip, R, _oracle_material(N, xm), 0.5)
+    bad = 77
+    g[bad, 5] = np.nan
+    prob = _problem(N, 2)[0]
+    out = local_full(prob, H, _params((H, Fp, g, slip, R, xm), np.arange(B)))
+    rest = np.delete(np.arange(B), bad)
+    strained = np.setdiff1d(rest, np.arange(64, 96))
+    assert np.isnan(out["P"][bad]).any() and np.isfinite(out["A"][rest]).all()
+    assert np.all(out["iters"][strained] > 0) and np.all(out["iters"][np.setdiff1d(np.arange(64, 96), [bad])] == 0)
+    assert _rel(out["A"][rest], ref["A"].reshape(B, 9, 9)[rest]).max() < 1e-10
+    assert _rel(out["P"][strained], ref["P"][strained]).max() < 1e-10
+    assert np.abs(out["P"][np.setdiff1d(np.arange(64, 96), [bad])]).max() == 0.0
+    assert _rel(out["Fp_inv_new"][rest], ref["Fp_inv_new"][rest]).max() < 1e-12
+    assert _rel(out["g_new"][rest], ref["g_new"][rest]).max() < 1e-12
+    np.testing.assert_allclose(out["slip_new"][rest], ref["slip_new"][rest], rtol=1e-9, atol=1e-15)
+
+
 def test_parking_of_a_batch_with_one_lane_a_point():
     """Parking changes the time only, at the batch size it is made for (85,184 points, one lane each), with
     points of either form in every wave."""
