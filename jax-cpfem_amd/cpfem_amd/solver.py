@@ -14,7 +14,7 @@ with FP64 refinement), 'krylov_tol'/'krylov_atol' (1e-10), 'krylov_maxiter' (100
 band LU under a bandwidth-reducing node order plus FP64 iterative refinement, 'refine' steps,
 default 2); 'jax_solver' with precond True (the default) runs the reference's BiCGSTAB to its
 stopping rule with a multigrid cycle in the place of the Jacobi scaling on box-numbered meshes
-(multigrid_solve; 'jacobi', or a 'krylov_maxiter', keeps the scaling); 'petsc_solver' (an iterative Krylov solve in the reference, bcgsl + ilu by default)
+whose elements and Dirichlet dofs let that be the shorter solve (multigrid_solve; 'jacobi', or a 'krylov_maxiter', keeps the scaling); 'petsc_solver' (an iterative Krylov solve in the reference, bcgsl + ilu by default)
 by the same solve at the same 1e-10 tolerance.
 """
 import ctypes
@@ -74,8 +74,8 @@ def krylov_solve(problem, mat, b, x0, solver_options=None, precond=True):
 
 
 def multigrid_solve(problem, mat, b, x0, solver_options=None):
-    """krylov_solve with the multigrid preconditioner where the mesh allows it (cpfem_solve_mg):
-    the same system to the same stopping rule in about ten iterations; elsewhere, and where it
+    """krylov_solve with the multigrid preconditioner where mesh and Dirichlet dofs let it be the shorter
+    solve (cpfem_solve_mg): the same system to the same stopping rule in about ten iterations; elsewhere, and where it
     does not converge, the Jacobi-preconditioned solve."""
     solver_options = solver_options or {}
     x = x0.clone()

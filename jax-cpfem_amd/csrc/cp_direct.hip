@@ -8,8 +8,9 @@
 // solved with matrix-vector sweeps.  FP64 iterative refinement against the block-ELL matrix
 // follows in the caller.  Without pivoting the factorisation exists when the leading principal
 // minors (in the order of elimination) are non-zero, which holds for these stiffness matrices
-// (elastic-plastic tangents close to SPD, unit Dirichlet rows); a zero or non-finite pivot is
-// reported instead of being worked round, and the caller turns it into an error.
+// (elastic-plastic tangents close to SPD, unit Dirichlet rows).  A zero or non-finite pivot is
+// reported instead of being worked round: the caller factors once more with one front (nt = 0), as it
+// does where the solution's backward error is large, and turns a second one into an error.
 //
 // A band of 1400 half bandwidth gives each pivot block only about a thousand tiles of work, so
 // the solve is bound by the length of the chain of dependent launches, not by operations

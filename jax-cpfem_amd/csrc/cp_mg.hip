@@ -10,7 +10,7 @@
 //
 // Cycle: levels coarsen every direction by two (node 2I; an odd last element stays as one),
 // trilinear interpolation P, coarse operators P^T A P, Dirichlet dofs masked out on every level
-// (they are scaled by the diagonal alone); before the coarse correction a Chebyshev polynomial
+// (on the finest they are scaled by the diagonal alone, on the others they stay zero); before the coarse correction a Chebyshev polynomial
 // of the diagonally scaled operator over [0.1, 1.1] lambda_max (coarser levels: [0.07, 1.1]), none
 // after it.  With scalar-diagonal smoothing before the correction only, degree 4 needs the fewest
 // matrix passes (per iteration 2 + 2 x 4 on the finest level; degree 2 takes 16 iterations, 3 takes

@@ -5,7 +5,7 @@ Both stop at |r| <= 1e-12 |b| of their recurrence; the bar on the true residual,
 1e-11 |r0|, leaves a decade for the recurrence's drift (observed below 1e-12 |r0| in either
 solve).  Sizes sit at the edges of the level plan: odd and even counts, thin boxes, both sides
 of the row count from which a level runs one row per thread (60,000 rows: 26^3 and 27^3
-elements), one and several levels in the one-block kernel."""
+elements), one and several levels above the inverted one."""
 import numpy as np
 import pytest
 
